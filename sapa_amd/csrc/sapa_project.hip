@@ -37,6 +37,12 @@ typedef u32 u32x2 __attribute__((ext_vector_type(2)));
 typedef u32 u32x4 __attribute__((ext_vector_type(4)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 
+// The result stores of the buffer kernels below carry their whole offset in the vector operand:
+// with a scalar offset register the compiler leaves no wait state between a 16-byte buffer store
+// and an instruction that overwrites its data registers, and the first dword of a piece was then
+// now and then stored with the overwriting value (once a second workgroup on the CU kept the store
+// waiting: 16-bit planes, 16 images of 200 x 336 pixels, 5000 of 69 M results).
+
 template <typename T> struct Mma;
 template <> struct Mma<f16_t> {
     typedef _Float16 v4 __attribute__((ext_vector_type(4)));
@@ -319,7 +325,7 @@ project16p_kernel(const T *__restrict__ x, const T *__restrict__ w, const T *__r
                 for (int j = 0; j < (16 * O / 8 + 63) / 64; ++j) {
                     const int i = j * 64 + lane, row = i / (O / 8), col = i % (O / 8);
                     if (16 * O / 8 % 64 == 0 || i < 16 * O / 8)
-                        __builtin_amdgcn_raw_buffer_store_b128(*(const u32x4 *)(xt + row * OW + 4 * col), ro, (u32)(i * 16), obase, 2);
+                        __builtin_amdgcn_raw_buffer_store_b128(*(const u32x4 *)(xt + row * OW + 4 * col), ro, (u32)(i * 16) + obase, 0, 2);
                 }
             }
         } else {
@@ -337,7 +343,7 @@ project16p_kernel(const T *__restrict__ x, const T *__restrict__ w, const T *__r
                 for (int j = 0; j < 2; ++j) {
                     const int row = 8 * j + (lane >> 3), col = lane & 7;
                     const u32 off = t * 64 + 8 * col < HW ? (u32)(row * HW + 8 * col) * 2u : 0x80000000u;
-                    __builtin_amdgcn_raw_buffer_store_b128(*(const u32x4 *)(xt + row * PW + 4 * col), ro, off, obase, 2);
+                    __builtin_amdgcn_raw_buffer_store_b128(*(const u32x4 *)(xt + row * PW + 4 * col), ro, off + obase, 0, 2);
                 }
             }
         }
@@ -556,7 +562,7 @@ project32_kernel(const float *__restrict__ x, const float *__restrict__ w, const
                 for (int j = 0; j < 2; ++j) {
                     const int row = 8 * j + (lane >> 3), col = lane & 7;
                     const u32 off = t * 32 + 4 * col < HW ? (u32)(row * HW + 4 * col) * 4u : 0x80000000u;
-                    __builtin_amdgcn_raw_buffer_store_b128(*(const u32x4 *)(rt + row * PS + 4 * col), ro, off, obase, 2);
+                    __builtin_amdgcn_raw_buffer_store_b128(*(const u32x4 *)(rt + row * PS + 4 * col), ro, off + obase, 0, 2);
                 }
             }
             continue;
@@ -574,7 +580,7 @@ project32_kernel(const float *__restrict__ x, const float *__restrict__ w, const
             for (int j = 0; j < (16 * O / 4 + 63) / 64; ++j) {
                 const int i = j * 64 + lane, row = i / (O / 4), col = i % (O / 4);
                 if (16 * O / 4 % 64 == 0 || i < 16 * O / 4)
-                    __builtin_amdgcn_raw_buffer_store_b128(*(const u32x4 *)(rt + row * OS + 4 * col), ro, (u32)(i * 16), obase, 2);
+                    __builtin_amdgcn_raw_buffer_store_b128(*(const u32x4 *)(rt + row * OS + 4 * col), ro, (u32)(i * 16) + obase, 0, 2);
             }
         }
     }
