@@ -171,6 +171,21 @@ int sapa_fused_backward_attn(const void *grad_out, const void *query, const void
                              int d, int C, int H, int W, int K, int s, int dtype,
                              void *stream);
 
+/* The same gradients straight from the four operands in two kernels on the 16-bit
+ * matrix instructions, with no K*K tensor in memory: `stats` is scratch of
+ * 3 floats per output pixel (12*B*sH*sW bytes, 16-byte aligned).  channels_last:
+ * every tensor in [B,H,W,C] order, else contiguous.  f16 / bf16, K = 5, s = 2;
+ * SAPA_ERR_UNSUPPORTED (nothing written) for shapes that
+ * sapa_fused_backward_direct_serves does not name and for tensors not aligned to
+ * 16 bytes: sapa_fused_backward serves those. */
+int sapa_fused_backward_direct_serves(int d, int C, int H, int W, int K, int s,
+                                      int channels_last, int dtype);
+int sapa_fused_backward_direct(const void *grad_out, const void *query, const void *key,
+                               const void *value, void *stats, void *grad_query,
+                               void *grad_key, void *grad_value, int B, int d, int C,
+                               int H, int W, int K, int s, int channels_last, int dtype,
+                               void *stream);
+
 /* Softmax over the middle axis of x [N,R,M] -> y [N,R,M] (max-subtracted,
  * fp32 arithmetic for 16-bit types).  Covers the reference's
  * F.softmax(logits, dim=1) on [B,K*K,sH,sW] (sapa_base.py:39: N=B, R=K*K,

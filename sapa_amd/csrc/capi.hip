@@ -301,6 +301,13 @@ static int fused_backward_impl(const void *grad_out, const void *query, const vo
     if (B == 0) return SAPA_OK;
     if (!grad_out || !query || !key || !value || !workspace) return SAPA_ERR_INVALID_ARGUMENT;
     hipStream_t st = (hipStream_t)stream;
+    if (!attn_given) {
+        // 16-bit tensors: two kernels from the four operands, no K*K tensors (they take 3 floats per
+        // pixel of the workspace)
+        const hipError_t e = sapa_b_bwd16_launch(query, key, value, grad_out, workspace, grad_query, grad_key,
+                                                 grad_value, B, d, C, H, W, K, s, dtype, st);
+        if (e != hipErrorNotSupported) return finish(e);
+    }
     float *grad_logits = (float *)workspace + (attn_given ? 0LL : (long long)B * K * K * H * s * W * s);
     const float *attn = attn_given ? attn_given : (const float *)workspace;
     // every stage on the LDS-tiled kernels with fp32 K*K tensors; a stage they do
@@ -341,6 +348,25 @@ int sapa_fused_backward(const void *grad_out, const void *query, const void *key
                         int d, int C, int H, int W, int K, int s, int dtype, void *stream) {
     return fused_backward_impl(grad_out, query, key, value, nullptr, workspace, grad_query, grad_key,
                                grad_value, B, d, C, H, W, K, s, dtype, stream);
+}
+
+int sapa_fused_backward_direct_serves(int d, int C, int H, int W, int K, int s, int channels_last, int dtype) {
+    if (d <= 0 || C <= 0 || H <= 0 || W <= 0) return 0;
+    return !channels_last && sapa_b_bwd16_serves(d, C, H, W, K, s, dtype);
+}
+
+int sapa_fused_backward_direct(const void *grad_out, const void *query, const void *key, const void *value,
+                               void *stats, void *grad_query, void *grad_key, void *grad_value, int B, int d,
+                               int C, int H, int W, int K, int s, int channels_last, int dtype, void *stream) {
+    const int rc = check_window_args(B, d, C, H, W, K, s, dtype);
+    if (rc != SAPA_OK) return rc;
+    if (B == 0) return SAPA_OK;
+    if (!grad_out || !query || !key || !value || !stats) return SAPA_ERR_INVALID_ARGUMENT;
+    const hipError_t e = channels_last ? hipErrorNotSupported
+                                       : sapa_b_bwd16_launch(query, key, value, grad_out, stats, grad_query, grad_key,
+                                                             grad_value, B, d, C, H, W, K, s, dtype, (hipStream_t)stream);
+    if (e == hipErrorNotSupported) return SAPA_ERR_UNSUPPORTED;
+    return finish(e);
 }
 
 int sapa_fused_forward_attn(const void *query, const void *key, const void *value, void *attn,

@@ -206,11 +206,41 @@ def qk_softmax(query, key, kernel_size, scale_factor):
     return _qk_softmax_forward(query, key, kernel_size, scale_factor, nhwc)
 
 
+def _direct_serves(query, key, value, K, s, nhwc):
+    """Whether the gradients of these operands come from sapa_fused_backward_direct, which forms the
+    attention weights itself (nothing to keep from the forward pass)."""
+    return (value.dtype in (torch.float16, torch.bfloat16) and query.dtype == key.dtype == value.dtype
+            and bool(_lib.lib().sapa_fused_backward_direct_serves(key.size(1), value.size(1), key.size(2), key.size(3),
+                                                                  K, s, int(nhwc), _lib.dtype_code(value))))
+
+
+def _direct_backward(grad_output, query, key, value, K, s, needs):
+    """The gradients through sapa_fused_backward_direct (16-bit tensors in one memory order; the
+    output's gradient is brought into it); None where that entry point does not serve the call."""
+    nhwc = all(_lib.is_channels_last(t) for t in (query, key, value))
+    if not (nhwc or all(t.is_contiguous() for t in (query, key, value))):
+        return None
+    if grad_output.dtype != value.dtype or not _direct_serves(query, key, value, K, s, nhwc):
+        return None
+    grad_output = _lib.layout_copy(grad_output, nhwc)
+    n, c, h, w = value.size()
+    stats = torch.empty((3, n, h * s, w * s), dtype=torch.float32, device=value.device)
+    grads = [_lib.new_out(t, channels_last=nhwc) if need else None for t, need in zip((query, key, value), needs)]
+    status = _lib.call_status('sapa_fused_backward_direct', value.device, _lib.ptr(grad_output), _lib.ptr(query),
+                              _lib.ptr(key), _lib.ptr(value), _lib.ptr(stats), _lib.ptr(grads[0]),
+                              _lib.ptr(grads[1]), _lib.ptr(grads[2]), n, key.size(1), c, h, w, K, s, int(nhwc),
+                              _lib.dtype_code(value))
+    return None if status == _lib.UNSUPPORTED else tuple(grads)
+
+
 def _fused_backward(grad_output, query, key, value, K, s, needs=(True, True, True), attn=None):
     """Gradients of av(softmax(qk(query, key)), value): the attention weights
     are recomputed (one launch) unless the forward pass kept them (`attn`, fp32),
     then the three operators' gradients chain."""
     need_q, need_k, need_v = needs
+    grads = _direct_backward(grad_output, query, key, value, K, s, needs)
+    if grads is not None:
+        return grads
     cl = [_lib.is_channels_last(t) for t in (query, key, value)]
     if any(cl) or _lib.is_channels_last(grad_output) or _lib.is_channels_last(attn):
         # the gradient kernels take contiguous tensors: operands in channels-last order are
@@ -293,7 +323,8 @@ class SAPAFusedFunction(Function):
     """av(softmax(qk(query, key), dim=1), value) -- SAPA.attention
     (sapa_base.py:38-40) -- as one launch in the forward pass.  When a gradient
     is wanted and `save_attention` is set (the default, SAVE_ATTENTION), the
-    forward pass runs as two launches that leave the fp32 attention weights
+    forward pass of operands that sapa_fused_backward_direct does not serve (fp32)
+    runs as two launches that leave the fp32 attention weights
     [B,K*K,sH,sW] behind for the backward pass, as the reference's autograd graph
     does; otherwise the backward pass recomputes them (one launch more, nothing
     kept alive but the operands).  Then the three operators' gradients chain.
@@ -332,7 +363,11 @@ class SAPAFusedFunction(Function):
             query = query + query_bias[:, :, None, None]
             query_bias = None
         output = _lib.new_out(value, (n, c, h * scale_factor, w * scale_factor), nhwc)
-        if wants_grad and not nhwc and (SAVE_ATTENTION if save_attention is None else save_attention):
+        # (where the gradients come straight from the operands the weights are kept on request only)
+        if save_attention is None:
+            save_attention = SAVE_ATTENTION and not (
+                wants_grad and _direct_serves(query, key, value, kernel_size, scale_factor, nhwc))
+        if wants_grad and not nhwc and save_attention:
             attn = torch.empty((n, kernel_size * kernel_size, h * scale_factor, w * scale_factor),
                                dtype=torch.float32, device=value.device)
             status = _lib.call_status('sapa_fused_forward_attn', value.device, _lib.ptr(query), _lib.ptr(key),
