@@ -451,9 +451,9 @@ def main():
         import sapa_amd
         go = torch.randn(B, C, H * s, W * s, device=dev).to(dtype)
         if args.layout == 'channels_last':
-            # the forward runs on the channels-last kernels; the backward pass has no
-            # channels-last kernels: autograd copies its operands to contiguous order and
-            # the gradients come back in that order (the step below includes those copies)
+            # the forward runs on the channels-last kernels, and so does the backward pass of
+            # 16-bit tensors; for fp32 autograd copies its operands to contiguous order and the
+            # gradients come back in that order (the step below includes those copies)
             go = go.contiguous(memory_format=torch.channels_last)
         leaves = [t.requires_grad_() for t in ((q, key, v, off) if deform else (q, key, v))]
         if deform:
@@ -622,7 +622,7 @@ def main():
         what = what.replace('forward', 'forward + backward')
         kern = 'several (see profiles/)'
         if args.layout == 'channels_last':
-            kern += '; forward on the channels-last kernels, backward through contiguous copies'
+            kern += '; forward on the channels-last kernels; backward on them too for 16-bit tensors, through contiguous copies for fp32'
     traffic = traffic_source = None
     if not train:
         tlayout = 'nchw_reference_order' if deform and args.layout == 'nchw' and args.reference_order else args.layout

@@ -352,7 +352,7 @@ int sapa_fused_backward(const void *grad_out, const void *query, const void *key
 
 int sapa_fused_backward_direct_serves(int d, int C, int H, int W, int K, int s, int channels_last, int dtype) {
     if (d <= 0 || C <= 0 || H <= 0 || W <= 0) return 0;
-    return !channels_last && sapa_b_bwd16_serves(d, C, H, W, K, s, dtype);
+    return channels_last ? sapa_b_nhwc_bwd16_serves(d, C, H, W, K, s, dtype) : sapa_b_bwd16_serves(d, C, H, W, K, s, dtype);
 }
 
 int sapa_fused_backward_direct(const void *grad_out, const void *query, const void *key, const void *value,
@@ -362,9 +362,9 @@ int sapa_fused_backward_direct(const void *grad_out, const void *query, const vo
     if (rc != SAPA_OK) return rc;
     if (B == 0) return SAPA_OK;
     if (!grad_out || !query || !key || !value || !stats) return SAPA_ERR_INVALID_ARGUMENT;
-    const hipError_t e = channels_last ? hipErrorNotSupported
-                                       : sapa_b_bwd16_launch(query, key, value, grad_out, stats, grad_query, grad_key,
-                                                             grad_value, B, d, C, H, W, K, s, dtype, (hipStream_t)stream);
+    const hipError_t e = (channels_last ? sapa_b_nhwc_bwd16_launch : sapa_b_bwd16_launch)(
+        query, key, value, grad_out, stats, grad_query, grad_key, grad_value, B, d, C, H, W, K, s, dtype,
+        (hipStream_t)stream);
     if (e == hipErrorNotSupported) return SAPA_ERR_UNSUPPORTED;
     return finish(e);
 }

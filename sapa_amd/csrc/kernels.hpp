@@ -61,6 +61,12 @@ hipError_t sapa_b_bwd16_launch(const void *q, const void *key, const void *value
                                void *grad_q, void *grad_key, void *grad_value, int B, int d, int C, int H, int W,
                                int K, int s, int dtype, hipStream_t st);
 
+// sapa_b_nhwc_bwd16.hip: the same for channels-last tensors
+bool sapa_b_nhwc_bwd16_serves(int d, int C, int H, int W, int K, int s, int dtype);
+hipError_t sapa_b_nhwc_bwd16_launch(const void *q, const void *key, const void *value, const void *grad_out,
+                                    void *stats, void *grad_q, void *grad_key, void *grad_value, int B, int d,
+                                    int C, int H, int W, int K, int s, int dtype, hipStream_t st);
+
 // sapa_moments.hip: per (image, channel) mean and variance of a feature map
 long channel_moments_workspace(int B, int C, long HW, bool channels_last);
 hipError_t channel_moments_launch(const void *x, void *workspace, float *mean_var, int B, int C,

@@ -31,13 +31,16 @@ def _rel(got, want):
 
 
 @pytest.mark.parametrize('dtype', [torch.bfloat16, torch.float16])
-@pytest.mark.parametrize('B,d,C,H,W', [
-    (1, 16, 16, 4, 16),      # the smallest width served
-    (2, 24, 40, 5, 18),      # ragged channel chunks, rows of 4 k + 2 cells, a last row of blocks of one row
-    (1, 32, 64, 33, 30),     # one tile of cell blocks, its last one past the image
-    (1, 40, 24, 3, 66),      # several tiles, fewer rows than a block
+@pytest.mark.parametrize('channels_last,B,d,C,H,W', [
+    (False, 1, 16, 16, 4, 16),      # the smallest width served
+    (False, 2, 24, 40, 5, 18),      # ragged channel chunks, rows of 4 k + 2 cells, a last row of blocks of one row
+    (False, 1, 32, 64, 33, 30),     # one tile of cell blocks, its last one past the image
+    (False, 1, 40, 24, 3, 66),      # several tiles, fewer rows than a block
+    (True, 1, 8, 8, 1, 3),          # the smallest tensors served
+    (True, 2, 72, 40, 9, 17),       # ragged channel chunks, odd extents
+    (True, 1, 64, 136, 15, 62),     # whole and partial tiles in both directions
 ])
-def test_fused_backward_from_operands(dtype, B, d, C, H, W):
+def test_fused_backward_from_operands(dtype, channels_last, B, d, C, H, W):
     """The two-kernel backward of 16-bit tensors (sapa_fused_backward_direct) against the fp64
     operators, all gradients and one at a time.  Bar: one rounding of the result to its type leaves a
     relative error of eps / 2 / sqrt(3) at most; the 16-bit weight pairs and fp32 sums are far below."""
@@ -45,13 +48,14 @@ def test_fused_backward_from_operands(dtype, B, d, C, H, W):
     from sapa_amd.sapa_func import _direct_serves
     g = torch.Generator(device='cuda').manual_seed(H * W)
     shapes = ((B, d, 2 * H, 2 * W), (B, d, H, W), (B, C, H, W), (B, C, 2 * H, 2 * W))
-    *ops, go = (torch.randn(s, generator=g, device='cuda').mul(0.6).to(dtype) for s in shapes)
-    assert _direct_serves(*ops, 5, 2, False)
-    wide = [t.double().requires_grad_() for t in ops]
-    want = torch.autograd.grad(sapa_amd.sapa_fused(*wide, 5, 2), wide, go.double())
+    fmt = torch.channels_last if channels_last else torch.contiguous_format
+    *ops, go = (torch.randn(s, generator=g, device='cuda').mul(0.6).to(dtype).contiguous(memory_format=fmt) for s in shapes)
+    assert _direct_serves(*ops, 5, 2, channels_last)
+    wide = [t.double().contiguous().requires_grad_() for t in ops]
+    want = torch.autograd.grad(sapa_amd.sapa_fused(*wide, 5, 2), wide, go.double().contiguous())
     bar = torch.finfo(dtype).eps / 2 / 3 ** 0.5 * 1.2
     for needs in ((True, True, True), (True, False, False), (False, True, False), (False, False, True)):
-        leaves = [t.clone().requires_grad_(n) for t, n in zip(ops, needs)]
+        leaves = [t.clone(memory_format=torch.preserve_format).requires_grad_(n) for t, n in zip(ops, needs)]
         got = torch.autograd.grad(sapa_amd.sapa_fused(*leaves, 5, 2), [t for t in leaves if t.requires_grad], go)
         for a, b in zip(got, [w for w, n in zip(want, needs) if n]):
-            assert _rel(a, b) <= bar, (needs, a.shape)
+            assert _rel(a, b) <= bar and a.is_contiguous(memory_format=fmt), (needs, a.shape)
