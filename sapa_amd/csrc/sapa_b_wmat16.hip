@@ -97,11 +97,11 @@ __device__ __forceinline__ int swz(int ch, int r) { return ((ch & 7) << 1) | ((r
 // low-res windows, which neighbouring tiles re-read, out of the caches (fused FPN-large bf16, 860 MB:
 // 271 -> 213 us; at a quarter of the size, where everything fits the memory-side cache, 50 -> 58 us:
 // the launcher decides by size)
-template <typename T, int NSW, bool STREAM>
-__global__ __launch_bounds__(64 * NSW) void
+template <typename T, int NSW, bool STREAM, bool ODD>
+__global__ __launch_bounds__(64 * NSW, 4) void
 sapa_b_wmat16_kernel(const T *__restrict__ q, const T *__restrict__ key, const T *__restrict__ value,
                      T *__restrict__ out, int d, int C, int H, int W, int tiles_x, int tiles_y, int ns,
-                     int nblocks, int per_xcd) {
+                     int nslices, int slice_chunks, int nblocks, int per_xcd) {
     constexpr int NT = 64 * NSW;
     constexpr int LROW = (4 * NSW + 4 + 7) / 8 * 4;          // dwords per staged window row: whole pieces of 8 cells
     constexpr int LOWBUF = WROWS * CHK * LROW;               // dwords per low-res buffer
@@ -123,7 +123,8 @@ sapa_b_wmat16_kernel(const T *__restrict__ q, const T *__restrict__ key, const T
 
     const int logical = (int)(blockIdx.x % 8) * per_xcd + (int)(blockIdx.x / 8);
     if (logical >= nblocks) return;
-    const int tx = logical % tiles_x, ty = (logical / tiles_x) % tiles_y, n = logical / (tiles_x * tiles_y);
+    const int tile = logical / nslices, vbase = (logical % nslices) * slice_chunks;      // first value chunk
+    const int tx = tile % tiles_x, ty = (tile / tiles_x) % tiles_y, n = tile / (tiles_x * tiles_y);
     const int X0 = tx * 4 * ns, Y0 = ty * 4;                 // first parent of the tile
     const int nsx = (W + 3) / 4;
     const int ns_here = nsx - tx * ns < ns ? nsx - tx * ns : ns;
@@ -141,7 +142,8 @@ sapa_b_wmat16_kernel(const T *__restrict__ q, const T *__restrict__ key, const T
     // that starts 2 cells before the image's first has no address: it reads as zeros and its 6
     // cells are fetched apart (patch_low).
     u32 off_low[NLI], off_hi[NHI];
-    bool half_piece[NHI];      // W % 4 == 2: a row's last 16-byte piece holds 4 of its children and 4 of the next row's
+    bool low_odd[NLI];         // ODD: the piece starts in the middle of a dword
+    int tail_children[NHI];    // children of its row in a row's last 16-byte piece (the rest is the next row's), else 8
     int patch_slot = -1;
 #pragma unroll
     for (int i = 0; i < NLI; ++i) {
@@ -149,7 +151,8 @@ sapa_b_wmat16_kernel(const T *__restrict__ q, const T *__restrict__ key, const T
         const int r = rc / CHK, ch = rc % CHK;
         const int y = Y0 - 2 + r, x = X0 - 2 + 8 * pc;
         const bool ok = slot < NLP && 8 * pc < 4 * ns_here + 4 && y >= 0 && y < H && x < W;
-        off_low[i] = ok ? (u32)(ch * lpix + (long)y * W + x) * (u32)sizeof(T) : OUTSIDE;
+        low_odd[i] = ODD && ((ch * lpix + (long)y * W) & 1);
+        off_low[i] = ok ? (u32)(ch * lpix + (long)y * W + x - low_odd[i]) * (u32)sizeof(T) : OUTSIDE;
         if (ok && x < 0 && y == 0 && ch == 0) patch_slot = slot;
     }
 #pragma unroll
@@ -159,16 +162,17 @@ sapa_b_wmat16_kernel(const T *__restrict__ q, const T *__restrict__ key, const T
         const int cy = 2 * Y0 + r, cx = 2 * X0 + 8 * pc;
         const bool ok = pc < ns_here && cy < 2 * H && cx < 2 * W;
         off_hi[i] = ok ? (u32)(ch * 4 * lpix + (long)cy * 2 * W + cx) * (u32)sizeof(T) : OUTSIDE;
-        half_piece[i] = ok && cx + 8 > 2 * W;
+        tail_children[i] = ok && cx + 8 > 2 * W ? 2 * W - cx : 8;
     }
 
-    const int nKc = (d + CHK - 1) / CHK, nVc = (C + CHK - 1) / CHK, ntot = nKc + nVc;
+    const int nKc = (d + CHK - 1) / CHK, allV = (C + CHK - 1) / CHK;
+    const int nVc = allV - vbase < slice_chunks ? allV - vbase : slice_chunks, ntot = nKc + nVc;
     const __amdgpu_buffer_rsrc_t rq = __builtin_amdgcn_make_buffer_rsrc(
         (void *)(q + (long)n * d * 4 * lpix), 0, (int)(d * hplane), 0x00020000);
     const __amdgpu_buffer_rsrc_t rk = __builtin_amdgcn_make_buffer_rsrc(
-        (void *)(key + (long)n * d * lpix), 0, (int)(d * lplane), 0x00020000);
+        (void *)(key + (long)n * d * lpix), 0, (int)((d * lplane + 3u) & ~3u), 0x00020000);
     const __amdgpu_buffer_rsrc_t rv = __builtin_amdgcn_make_buffer_rsrc(
-        (void *)(value + (long)n * C * lpix), 0, (int)(C * lplane), 0x00020000);
+        (void *)(value + (long)n * C * lpix), 0, (int)((C * lplane + 3u) & ~3u), 0x00020000);
     const __amdgpu_buffer_rsrc_t ro = __builtin_amdgcn_make_buffer_rsrc(
         (void *)(out + (long)n * C * 4 * lpix), 0, (int)(C * hplane), 0x00020000);
 
@@ -197,10 +201,38 @@ sapa_b_wmat16_kernel(const T *__restrict__ q, const T *__restrict__ key, const T
     };
     auto stage = [&](int j) __attribute__((always_inline)) {
         if (j < nKc) {
-            stage_low(rk, (u32)(j * CHK), j & 1);
+            if (!ODD) stage_low(rk, (u32)(j * CHK), j & 1);
             stage_q((u32)(j * CHK), j & 1);
-        } else if (j < ntot) {
-            stage_low(rv, (u32)((j - nKc) * CHK), j & 1);
+        } else if (!ODD && j < ntot) {
+            stage_low(rv, (u32)((j - nKc + vbase) * CHK), j & 1);
+        }
+    };
+    // ODD: an odd W puts every other row of a low-res plane in the middle of a dword, where direct loads
+    // cannot start.  The pieces of chunk j come through registers instead, from the dword before, and are
+    // moved by half a dword on their way into LDS: requested before chunk j - 1 is computed on, written
+    // behind it.
+    u32x4 low_reg[ODD ? NLI : 1];
+    u32 low_next[ODD ? NLI : 1];
+    auto low_load = [&](int j) __attribute__((always_inline)) {
+        if (!ODD || j >= ntot) return;
+        const u32 c0 = (u32)((j < nKc ? j : j - nKc + vbase) * CHK);
+        const __amdgpu_buffer_rsrc_t r = j < nKc ? rk : rv;
+#pragma unroll
+        for (int i = 0; i < NLI; ++i) {
+            low_reg[i] = __builtin_amdgcn_raw_buffer_load_b128(r, off_low[i] + c0 * lplane, 0, 0);
+            low_next[i] = __builtin_amdgcn_raw_buffer_load_b32(r, off_low[i] + c0 * lplane + 16, 0, 0);
+        }
+    };
+    auto low_commit = [&](int j) __attribute__((always_inline)) {
+        if (!ODD || j >= ntot) return;
+#pragma unroll
+        for (int i = 0; i < NLI; ++i) {
+            const u32x4 v = low_reg[i];
+            u32x4 m = v;
+            if (low_odd[i])
+                m = u32x4{__builtin_amdgcn_alignbyte(v[1], v[0], 2), __builtin_amdgcn_alignbyte(v[2], v[1], 2),
+                          __builtin_amdgcn_alignbyte(v[3], v[2], 2), __builtin_amdgcn_alignbyte(low_next[i], v[3], 2)};
+            if (i * NT + tid < NLP) *(u32x4 *)(lowbuf + (j & 1) * LOWBUF + (i * NT + tid) * 4) = m;
         }
     };
     // Waits are counted: the counter of vector-memory operations retires in issue order, so
@@ -220,7 +252,7 @@ sapa_b_wmat16_kernel(const T *__restrict__ q, const T *__restrict__ key, const T
     // cells of the piece that has no address (first row of the image's first channel, tile at the
     // left edge)
     auto patch_low = [&](int jn) __attribute__((always_inline)) {
-        if (tx == 0 && ty == 0 && patch_slot >= 0) {
+        if (tx == 0 && ty == 0 && patch_slot >= 0 && (jn < nKc || vbase == 0)) {
             const __amdgpu_buffer_rsrc_t r = jn < nKc ? rk : rv;
             u32 *dst = lowbuf + (jn & 1) * LOWBUF + patch_slot * 4;
 #pragma unroll
@@ -238,10 +270,12 @@ sapa_b_wmat16_kernel(const T *__restrict__ q, const T *__restrict__ key, const T
     const bool active = wave < ns_here;
     const int t = wave;                                       // this wave's block of the tile
 
+    low_load(0);
+    low_commit(0);
     stage(0);
     stage(1);
     // chunk 0: all but chunk 1's loads
-    wait_all_but(ntot < 2 ? 0 : (NLP - wave * 64 + NT - 1) / NT + (1 < nKc ? NHI : 0));
+    wait_all_but(ODD ? 0 : ntot < 2 ? 0 : (NLP - wave * 64 + NT - 1) / NT + (1 < nKc ? NHI : 0));
     patch_low(0);
     barrier();
 
@@ -257,6 +291,7 @@ sapa_b_wmat16_kernel(const T *__restrict__ q, const T *__restrict__ key, const T
     // L % 4 of the 16 (row (L % 4) / 2 of the pair, columns 4 (L % 2) ..)
     const int tch = 4 * g + (i16 >> 2), trow = (i16 & 3) >> 1, tcol = i16 & 1;
     for (int j = 0; j < nKc; ++j) {
+        low_load(j + 1);
         if (active) {
             const u32 *kb = lowbuf + (j & 1) * LOWBUF, *qb = hibuf + (j & 1) * HIBUF;
             u32x2 a[4], b[4];
@@ -273,6 +308,7 @@ sapa_b_wmat16_kernel(const T *__restrict__ q, const T *__restrict__ key, const T
 #pragma unroll
                 for (int nb = 0; nb < 4; ++nb) sim[mb][nb] = Mma<T>::k16(a[mb], b[nb], sim[mb][nb]);
         }
+        low_commit(j + 1);
         // chunk j + 1: nothing was issued after its loads
         wait_all_but(0);
         if (j + 1 == nKc) patch_low(nKc);
@@ -362,8 +398,9 @@ sapa_b_wmat16_kernel(const T *__restrict__ q, const T *__restrict__ key, const T
 
     // ---- aggregation: out[child][channel], per chunk of 16 channels ----
     for (int j = nKc; j < ntot; ++j) {
-        const u32 c0 = (u32)((j - nKc) * CHK);
+        const u32 c0 = (u32)((j - nKc + vbase) * CHK);
         u32 *ob = hibuf + (j & 1) * HIBUF;                      // no loads into this ring any more
+        low_load(j + 1);
         if (active) {
             const u32 *vb = lowbuf + (j & 1) * LOWBUF;
             // B operand of step s: lane (g, channel i16) holds the cells of rows 4 s + g / 2 and
@@ -389,6 +426,7 @@ sapa_b_wmat16_kernel(const T *__restrict__ q, const T *__restrict__ key, const T
                     u32x2{pack2<T>(acc[0], acc[1]), pack2<T>(acc[2], acc[3])};
             }
         }
+        low_commit(j + 1);
         // chunk j + 1: its loads were the last operations issued
 #if defined(__HIP_DEVICE_COMPILE__)
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
@@ -402,41 +440,56 @@ sapa_b_wmat16_kernel(const T *__restrict__ q, const T *__restrict__ key, const T
         for (int i = 0; i < NHI; ++i) {
             const u32x4 o = *(const u32x4 *)(ob + (i * NT + tid) * 4);
             u32 off = off_hi[i] + c0 * hplane;
-            if (row_tail && half_piece[i]) {
-                __builtin_amdgcn_raw_buffer_store_b64(u32x2{o[0], o[1]}, ro, off, 0, 0);
+            if (row_tail && tail_children[i] < 8) {
+                if (!ODD) {
+                    __builtin_amdgcn_raw_buffer_store_b64(u32x2{o[0], o[1]}, ro, off, 0, 0);
+                } else {
+#pragma unroll
+                    for (int k = 0; k < 3; ++k)
+                        if (2 * k < tail_children[i]) __builtin_amdgcn_raw_buffer_store_b32(o[k], ro, off + 4 * k, 0, 0);
+                }
                 off = OUTSIDE;
             }
             if constexpr (STREAM) __builtin_amdgcn_raw_buffer_store_b128(o, ro, off, 0, 2);
             else __builtin_amdgcn_raw_buffer_store_b128(o, ro, off, 0, 0);
         }
         // (the next request behind the stores: 208 us at FPN-large against 216 with the loads first)
-        if (j + 2 < ntot) stage_low(rv, (u32)((j + 2 - nKc) * CHK), j & 1);
+        if (!ODD && j + 2 < ntot) stage_low(rv, (u32)((j + 2 - nKc + vbase) * CHK), j & 1);
     }
 }
 
-template <typename T, int NSW, bool STREAM>
+template <typename T, int NSW, bool STREAM, bool ODD>
 static hipError_t launch_geom(const void *q, const void *key, const void *value, void *out, int B, int d,
                               int C, int H, int W, hipStream_t st) {
     const int nsx = (W + 3) / 4;
     const int tiles_x = (nsx + NSW - 1) / NSW, tiles_y = (H + 3) / 4;
     const int ns = (nsx + tiles_x - 1) / tiles_x;             // blocks per tile, balanced over the row
-    const long nb = (long)tiles_x * tiles_y * B;
+    const long tiles = (long)tiles_x * tiles_y * B;
+    // Fewer tiles than CUs: a workgroup's time is a chain of one step per 16 channels, so the value
+    // channels are split over several workgroups per tile, each forming the weights again, up to one
+    // workgroup per CU (B=8, C=256, d=32, bf16, 16x16: 12.5 us unsplit, 8.0 / 7.3 / 8.9 with up to 128 /
+    // 256 / 512 workgroups; 32x32: 16.6, 12.6 / 11.1 / 13.2; B=2, d=64, 50x84: 18.7, 18.4 / 13.6 / 14.8)
+    const int allV = (C + CHK - 1) / CHK;
+    long want = 256 / tiles;
+    want = want < 1 ? 1 : want > allV ? allV : want;
+    const int slice_chunks = (int)((allV + want - 1) / want), nslices = (allV + slice_chunks - 1) / slice_chunks;
+    const long nb = tiles * nslices;
     if (nb > (1L << 30)) return hipErrorNotSupported;
     const int per_xcd = (int)((nb + 7) / 8);
-    hipLaunchKernelGGL((sapa_b_wmat16_kernel<T, NSW, STREAM>), dim3(per_xcd * 8), dim3(64 * NSW), 0, st, (const T *)q,
-                       (const T *)key, (const T *)value, (T *)out, d, C, H, W, tiles_x, tiles_y, ns, (int)nb,
-                       per_xcd);
+    hipLaunchKernelGGL((sapa_b_wmat16_kernel<T, NSW, STREAM, ODD>), dim3(per_xcd * 8), dim3(64 * NSW), 0, st, (const T *)q,
+                       (const T *)key, (const T *)value, (T *)out, d, C, H, W, tiles_x, tiles_y, ns,
+                       nslices, slice_chunks, (int)nb, per_xcd);
     return hipGetLastError();
 }
 
 }  // namespace wm16
 
-// Fused forward only; f16 / bf16, K = 5, s = 2, W even (rows of whole dwords), low-res tensors 4-byte and
+// Fused forward only; f16 / bf16, K = 5, s = 2, W >= 4 (one block), low-res tensors 4-byte and
 // high-res tensors 16-byte aligned, every image of every tensor below 2 GiB (32-bit offsets
 // inside an image); hipErrorNotSupported otherwise.
 hipError_t sapa_b_wmat16_launch(int mode, const void *q, const void *key, const void *value, void *out, int B,
                                 int d, int C, int H, int W, int K, int s, int dtype, hipStream_t st) {
-    if (mode != TILED_FUSED || K != 5 || s != 2 || W % 2 != 0 || W < 16) return hipErrorNotSupported;
+    if (mode != TILED_FUSED || K != 5 || s != 2 || W < 4) return hipErrorNotSupported;
     if (dtype != 2 && dtype != 3) return hipErrorNotSupported;
     const long hplane = (long)H * W * 8;
     if ((long)(d > C ? d : C) * hplane >= (1L << 31)) return hipErrorNotSupported;
@@ -445,13 +498,19 @@ hipError_t sapa_b_wmat16_launch(int mode, const void *q, const void *key, const 
     // bytes read and written once; beyond the 256 MB memory-side cache they are streamed, in tiles of
     // up to 16 blocks (longer rows per store); what fits the cache takes tiles of 8 blocks, two
     // workgroups per CU (FPN 25x42 at B=16: 24 -> 19 us, SegFormer 64x64 at B=8: 25 -> 20 us).  The
-    // arithmetic of a child does not depend on the tiling: results are the same bit for bit.
+    // arithmetic of a child does not depend on the tiling: results are the same bit for bit.  An odd W
+    // (low-res rows through registers) has tiles of 8 blocks only: with 16 the registers do not suffice
+    // (B=16, C=256, d=64, 42x25: 24 us, by vector fmas 65; 100x167: 289 us against 451; rows below 16
+    // cells, 13x13 at B=8: 9 us against 19 on the one-block-per-parent matrix kernel).
     const bool stream = 2L * ((long)B * H * W * (5L * d + 5L * C)) > (256L << 20);
-    if (dtype == 2)
-        return stream ? wm16::launch_geom<f16_t, 16, true>(q, key, value, out, B, d, C, H, W, st)
-                      : wm16::launch_geom<f16_t, 8, false>(q, key, value, out, B, d, C, H, W, st);
-    return stream ? wm16::launch_geom<bf16_t, 16, true>(q, key, value, out, B, d, C, H, W, st)
-                  : wm16::launch_geom<bf16_t, 8, false>(q, key, value, out, B, d, C, H, W, st);
+    const bool odd = W % 2 != 0;
+#define SAPA_WM16_CASE(T)                                                                                       \
+    return odd      ? wm16::launch_geom<T, 8, false, true>(q, key, value, out, B, d, C, H, W, st)                \
+           : stream ? wm16::launch_geom<T, 16, true, false>(q, key, value, out, B, d, C, H, W, st)               \
+                    : wm16::launch_geom<T, 8, false, false>(q, key, value, out, B, d, C, H, W, st)
+    if (dtype == 2) SAPA_WM16_CASE(f16_t);
+    SAPA_WM16_CASE(bf16_t);
+#undef SAPA_WM16_CASE
 }
 
 }  // namespace sapa

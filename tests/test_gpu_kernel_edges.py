@@ -59,3 +59,26 @@ def test_fused_backward_from_operands(dtype, channels_last, B, d, C, H, W):
         got = torch.autograd.grad(sapa_amd.sapa_fused(*leaves, 5, 2), [t for t in leaves if t.requires_grad], go)
         for a, b in zip(got, [w for w, n in zip(want, needs) if n]):
             assert _rel(a, b) <= bar and a.is_contiguous(memory_format=fmt), (needs, a.shape)
+
+
+@pytest.mark.parametrize('dtype', [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize('B,d,C,H,W', [
+    (1, 16, 16, 4, 4),       # one block; the value channels cannot be split
+    (2, 24, 40, 5, 7),       # odd rows inside one tile, ragged channel chunks
+    (1, 17, 33, 3, 33),      # an odd number of channels and cells: the last dword of a tensor is half its own
+    (3, 32, 256, 9, 18),     # value channels split over workgroups
+    (2, 32, 72, 21, 67),     # three tiles of an odd row
+])
+def test_fused_dense_window_kernel_edges(dtype, B, d, C, H, W):
+    """The contiguous 16-bit dense-window forward where rows are odd or short and where its value
+    channels are split, against the fp64 operator; bar as above."""
+    import sapa_amd
+    from sapa_amd import _lib
+    g = torch.Generator(device='cuda').manual_seed(W)
+    shapes = ((B, d, 2 * H, 2 * W), (B, d, H, W), (B, C, H, W))
+    ops = [torch.randn(s, generator=g, device='cuda').mul(0.6).to(dtype) for s in shapes]
+    with torch.no_grad():
+        got = sapa_amd.sapa_fused(*ops, 5, 2)
+        assert _lib.last_kernel() == 'sapa_b_wmat16_kernel'
+        want = sapa_amd.sapa_fused(*[t.double() for t in ops], 5, 2)
+    assert _rel(got, want) <= torch.finfo(dtype).eps / 2 / 3 ** 0.5 * 1.2
