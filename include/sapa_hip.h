@@ -497,6 +497,17 @@ int sapa_project_nchw(const void *x, const void *weight, const void *bias, void 
                       int B, int C, int O, long long HW, int out_channels_last, int dtype,
                       void *stream);
 
+/* A plain 1x1 convolution, self.q(y) / self.k(x) / self.offset(x) of SAPADeform
+ * (deformsapa/deformsapa/sapa_deform.py:36-47): weight [O,C] and bias [O] (NULL: none)
+ * shared by all images, any O that is a multiple of 8, C in {64,128,256,512}; x [B,C,HW], or
+ * [B,HW,C] when x_channels_last != 0; out [B,O,HW], or [B,HW,O] when out_channels_last != 0
+ * (x channels-last only with out channels-last).  The types, the arithmetic and the
+ * conditions on HW and on alignment of the two entry points above; SAPA_ERR_UNSUPPORTED
+ * otherwise. */
+int sapa_project_shared(const void *x, const void *weight, const void *bias, void *out,
+                        int B, int C, int O, long long HW, int x_channels_last,
+                        int out_channels_last, int dtype, void *stream);
+
 /* self.q(self.norm_y(y)) / self.k(self.norm_x(x)) (sapa/sapa/sapa_base.py:27-35; GroupNorm and a
  * 1x1 Conv2d, ATen calls there) in one call: sapa_channel_moments, sapa_groupnorm_fold and
  * sapa_project_nhwc (x_channels_last != 0; the result is channels-last) or sapa_project_nchw

@@ -23,6 +23,7 @@ SIGNATURES = {
     'sapa_fused_forward_nhwc_qbias': [_vp, _vp, _vp, _vp, _vp, _i, _i, _i, _i, _i, _i, _i, _i, _vp],
     'sapa_project_nhwc': [_vp, _vp, _vp, _vp, _i, _i, _i, _ll, _i, _vp],
     'sapa_project_nchw': [_vp, _vp, _vp, _vp, _i, _i, _i, _ll, _i, _i, _vp],
+    'sapa_project_shared': [_vp, _vp, _vp, _vp, _i, _i, _i, _ll, _i, _i, _i, _vp],
     'sapa_norm_project': [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _i, _i, _i, _ll, _i, ctypes.c_float, _i, _i, _i,
                           _vp],
     'sapa_channel_moments': [_vp, _vp, _vp, _i, _i, _ll, _i, _i, _vp],
@@ -246,6 +247,7 @@ def call_nhwc(name, device, *args):
 
 
 UNSUPPORTED = -2   # SAPA_ERR_UNSUPPORTED: a valid request this build has no kernel for
+TOO_LARGE = -3     # SAPA_ERR_TOO_LARGE: beyond the kernels' index range
 
 
 def call_status(name, device, *args):
@@ -379,6 +381,38 @@ def project_nchw(x, weight, bias=None, channels_last_out=False):
     if status == UNSUPPORTED:
         return None
     check(status, 'sapa_project_nchw')
+    return out
+
+
+def project_shared(x, weight, bias=None, channels_last_out=False):
+    """F.conv2d(x, weight, bias) of a 1x1 weight [O, C, 1, 1] for a dense f16 / bf16 / fp32 CUDA
+    feature x [B, C, H, W] (contiguous, or in channels_last order with channels_last_out): a
+    tensor [B, O, H, W] in contiguous / channels_last order, or None if the kernel does not cover
+    the configuration (the caller then uses a library convolution).  No autograd."""
+    B, C, H, W = x.shape
+    O = weight.shape[0]
+    if (x.dtype not in (torch.float16, torch.bfloat16, torch.float32) or weight.dtype != x.dtype
+            or weight.device != x.device or x.numel() == 0 or weight.shape[1] != C
+            or (bias is not None and (bias.dtype != x.dtype or bias.device != x.device))):
+        return None
+    x_cl = not x.is_contiguous()
+    if x_cl and not (channels_last_out and x.is_contiguous(memory_format=torch.channels_last)):
+        return None
+    if O % 8 or (not x_cl and H * W % (8 if x.element_size() == 2 else 1 if channels_last_out else 4)):
+        return None
+    weight = weight.reshape(O, C).contiguous()
+    if bias is not None:
+        bias = bias.contiguous()
+    with torch.cuda.device(x.device):
+        out = torch.empty(B, O, H, W, dtype=x.dtype, device=x.device,
+                          memory_format=torch.channels_last if channels_last_out else torch.contiguous_format)
+        status = lib().sapa_project_shared(
+            x.data_ptr(), weight.data_ptr(), None if bias is None else bias.data_ptr(), out.data_ptr(),
+            B, C, O, H * W, 1 if x_cl else 0, 1 if channels_last_out else 0, DTYPES[x.dtype],
+            torch.cuda.current_stream(x.device).cuda_stream)
+    if status in (UNSUPPORTED, TOO_LARGE):
+        return None
+    check(status, 'sapa_project_shared')
     return out
 
 

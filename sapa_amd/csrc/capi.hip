@@ -794,6 +794,18 @@ int sapa_project_nchw(const void *x, const void *weight, const void *bias, void 
     return finish(e);
 }
 
+int sapa_project_shared(const void *x, const void *weight, const void *bias, void *out, int B, int C, int O,
+                        long long HW, int x_channels_last, int out_channels_last, int dtype, void *stream) {
+    if (!dtype_ok(dtype) || B < 0 || C <= 0 || O <= 0 || HW <= 0) return SAPA_ERR_INVALID_ARGUMENT;
+    if ((long long)B * HW * (C > O ? C : O) >= kMaxElems) return SAPA_ERR_TOO_LARGE;
+    if (B == 0) return SAPA_OK;
+    if (!x || !weight || !out) return SAPA_ERR_INVALID_ARGUMENT;
+    const hipError_t e = project_shared_launch(x, weight, bias, out, B, C, O, (long)HW, x_channels_last,
+                                               out_channels_last, dtype, (hipStream_t)stream);
+    if (e == hipErrorNotSupported) return SAPA_ERR_UNSUPPORTED;
+    return finish(e);
+}
+
 namespace {
 long long round256(long long n) { return (n + 255) / 256 * 256; }
 long long esize_of(int dtype) { return dtype == SAPA_F32 ? 4 : dtype == SAPA_F64 ? 8 : 2; }

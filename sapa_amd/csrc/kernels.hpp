@@ -97,6 +97,8 @@ hipError_t project_nhwc_launch(const void *x, const void *w, const void *bias, v
 hipError_t project_nchw_launch(const void *x, const void *w, const void *bias, void *out, int B,
                                int C, int O, long HW, int out_channels_last, int dtype, hipStream_t st);
 // whether one of the two has a kernel for the configuration (pointer alignment aside)
+hipError_t project_shared_launch(const void *x, const void *w, const void *bias, void *out, int B, int C, int O,
+                                 long HW, int x_channels_last, int out_channels_last, int dtype, hipStream_t st);
 bool project_supported(int C, int O, long HW, bool x_channels_last, bool out_channels_last, int dtype);
 
 // sapa_d_nhwc.hip: fused SAPA-D forward for tensors in channels-last memory

@@ -26,11 +26,31 @@
 // weights are taken apart once per workgroup into three bf16 planes in LDS; x goes
 // from global memory straight into the A-operand registers (a lane reads two 16-byte
 // pieces of its pixel's record per step of 32 channels) and is taken apart there.
+//
+// WIDE kernels: weights [OT][C] and bias [OT] shared by all images, any number OT of outputs (a
+// multiple of 8) in blocks of O, one per blockIdx.z -- the plain 1x1 convolutions of SAPADeform
+// (128 query and key channels, 72 .. 800 offset channels).  The feature is read once per block; the
+// blocks of one pixel range run at the same time, so all but one of those reads come from a cache.
+// (SAPA-D module, 256 channels: B=8, 64x64, 9 points, fp32 382 us with library convolutions and their
+// bias passes, 298 with these; 25 points 638, 492; bf16 channels-last 361, 239.  What is left there in
+// fp32 is the matrix work of the six piece products: 30 us per 8.6 GFLOP at the rate of a large product.)
 #include "kernels.hpp"
 
 namespace sapa {
 
 namespace project {
+
+// where a workgroup's block of outputs lies: OT outputs in all (the stride of a channels-last
+// record), o0 the first of this block, `left` its number
+struct Span {
+    int OT, o0, left;
+};
+template <int O, bool WIDE>
+__device__ __forceinline__ Span span_of(int outputs) {
+    if (!WIDE) return Span{O, 0, O};
+    const int o0 = blockIdx.z * O;
+    return Span{outputs, o0, outputs - o0 < O ? outputs - o0 : O};
+}
 
 typedef unsigned u32;
 typedef u32 u32x2 __attribute__((ext_vector_type(2)));
@@ -81,10 +101,10 @@ __device__ __forceinline__ u32 pack2(float a, float b) {
 }
 
 // C input channels, O outputs (both multiples of 16); tiles of 16 pixels
-template <typename T, int C, int O>
+template <typename T, int C, int O, bool WIDE>
 __global__ void __launch_bounds__(256)
 project_kernel(const T *__restrict__ x, const T *__restrict__ w, const T *__restrict__ bias,
-               T *__restrict__ out, long HW, int tiles_per_block) {
+               T *__restrict__ out, long HW, int tiles_per_block, int outputs) {
     constexpr int RW = C / 2 + 4;                 // dwords per padded row of C 16-bit values
     constexpr int NL = C / 32;                    // 16-byte loads per lane and tile (16 rows of 2 C bytes)
     constexpr int NT = O / 16;                    // output tiles of 16 columns
@@ -96,14 +116,18 @@ project_kernel(const T *__restrict__ x, const T *__restrict__ w, const T *__rest
     u32 *xt = sh + O * RW + wave * XT;            // this wave's tile
     const int b = blockIdx.y;
     const T *xb = x + (long)b * HW * C;
-    T *ob = out + (long)b * HW * O;
+    const Span sp = span_of<O, WIDE>(outputs);
+    T *ob = out + (long)b * HW * sp.OT;
 
     // the image's weights -> LDS (16 bytes per thread and step)
     {
-        const u32x4 *src = (const u32x4 *)(w + (long)b * O * C);
-        for (int i = threadIdx.x; i < O * C / 8; i += 256) {
-            const int row = i / (C / 8), col = i % (C / 8);
-            *(u32x4 *)(wl + row * RW + 4 * col) = src[i];
+        const __amdgpu_buffer_rsrc_t rw = __builtin_amdgcn_make_buffer_rsrc(
+            (void *)(w + (WIDE ? (long)sp.o0 : (long)b * O) * C), 0, sp.left * C * 2, 0x00020000);
+        static_assert(O * C / 8 % 256 == 0, "whole steps");
+#pragma unroll
+        for (int k = 0; k < O * C / 8 / 256; ++k) {
+            const int i = k * 256 + threadIdx.x, row = i / (C / 8), col = i % (C / 8);
+            *(u32x4 *)(wl + row * RW + 4 * col) = __builtin_amdgcn_raw_buffer_load_b128(rw, (u32)i * 16u, 0, 0);
         }
     }
     __syncthreads();
@@ -114,7 +138,8 @@ project_kernel(const T *__restrict__ x, const T *__restrict__ w, const T *__rest
     const int r16 = lane & 15, kg = lane >> 4;    // row / column of a 16 x 16 tile, k group
     float bv[NT];
 #pragma unroll
-    for (int nt = 0; nt < NT; ++nt) bv[nt] = bias ? (float)bias[(long)b * O + 16 * nt + r16] : 0.f;
+    for (int nt = 0; nt < NT; ++nt)
+        bv[nt] = bias && 16 * nt + r16 < sp.left ? (float)bias[(WIDE ? (long)sp.o0 : (long)b * O) + 16 * nt + r16] : 0.f;
 
     // a tile's 16 records are one run of 32 C bytes: lane l takes 16-byte piece
     // j * 64 + l (pieces past the image: zeros)
@@ -147,6 +172,7 @@ project_kernel(const T *__restrict__ x, const T *__restrict__ w, const T *__rest
             const u32x2 a = *(const u32x2 *)(xt + r16 * RW + 8 * ks + 2 * kg);
 #pragma unroll
             for (int nt = 0; nt < NT; ++nt) {
+                if (WIDE && 16 * nt >= sp.left) break;
                 const u32x2 bm = *(const u32x2 *)(wl + (16 * nt + r16) * RW + 8 * ks + 2 * kg);
                 acc[nt] = Mma<T>::run(a, bm, acc[nt]);
             }
@@ -161,6 +187,17 @@ project_kernel(const T *__restrict__ x, const T *__restrict__ w, const T *__rest
                 const u32 h = pack2<T>(acc[nt][i] + bv[nt], 0.f);
                 rt[(4 * kg + i) * (2 * OW) + 16 * nt + r16] = (unsigned short)h;
             }
+        if (WIDE) {
+            // 16 pieces of 2 O bytes, one per pixel's record
+#pragma unroll
+            for (int j = 0; j < (16 * O / 8 + 63) / 64; ++j) {
+                const int i = j * 64 + lane, row = i / (O / 8), col = i % (O / 8);
+                if (i < 16 * O / 8 && 8 * col < sp.left && t * 16 + row < HW)
+                    __builtin_nontemporal_store(*(const u32x4 *)(xt + row * OW + 4 * col),
+                                                (u32x4 *)(ob + (t * 16 + row) * sp.OT + sp.o0 + 8 * col));
+            }
+            continue;
+        }
         // 16 rows of 2 O bytes -> one contiguous run of 32 O bytes
         const long obase = t * 16 * (O / 8), olimit = HW * (O / 8);
 #pragma unroll
@@ -173,22 +210,23 @@ project_kernel(const T *__restrict__ x, const T *__restrict__ w, const T *__rest
     }
 }
 
-template <typename T, int C, int O>
+template <typename T, int C, int O, bool WIDE = false>
 static hipError_t launch_co(const void *x, const void *w, const void *bias, void *out, int B, long HW,
-                            hipStream_t st) {
+                            hipStream_t st, int outputs = O) {
     constexpr int RW = C / 2 + 4, OW = O / 2 + 4;
     constexpr int XT = 16 * RW > 16 * OW ? 16 * RW : 16 * OW;
     constexpr size_t lds = (size_t)(O * RW + 4 * XT) * 4;
     static_assert(lds <= 160 * 1024, "weights and tiles must fit LDS");
     const long ntiles = (HW + 15) / 16;
+    const int blocks_o = (outputs + O - 1) / O;
     // two workgroups are resident per CU (LDS) and the part has 256 CUs: one round of at most 512
     // workgroups, at least 2 tiles per wave (16 images of 100 x 168 pixels, 256 -> 64: 37 us against
     // 46 with a fixed 8 tiles per wave; 200 x 336 pixels: 141 against 146)
-    long per = (ntiles * B + 4L * 512 - 1) / (4L * 512);
+    long per = (ntiles * B * blocks_o + 4L * 512 - 1) / (4L * 512);
     if (per < 2) per = 2;
     const long blocks = (ntiles + 4 * per - 1) / (4 * per);
-    if (blocks > 65535 * 32L || B > 65535) return hipErrorNotSupported;
-    auto kern = project_kernel<T, C, O>;
+    if (blocks > 65535 * 32L || B > 65535 || blocks_o > 65535) return hipErrorNotSupported;
+    auto kern = project_kernel<T, C, O, WIDE>;
     if (lds > 64 * 1024) {
         // more than the default 64 KB per workgroup: ask for it; a device that
         // cannot give it is not served by this kernel
@@ -202,8 +240,8 @@ static hipError_t launch_co(const void *x, const void *w, const void *bias, void
             return hipErrorNotSupported;
         }
     }
-    hipLaunchKernelGGL(kern, dim3((unsigned)blocks, B), dim3(256), lds, st, (const T *)x, (const T *)w,
-                       (const T *)bias, (T *)out, HW, (int)per);
+    hipLaunchKernelGGL(kern, dim3((unsigned)blocks, B, blocks_o), dim3(256), lds, st, (const T *)x, (const T *)w,
+                       (const T *)bias, (T *)out, HW, (int)per, outputs);
     return hipGetLastError();
 }
 
@@ -215,10 +253,10 @@ static hipError_t launch_co(const void *x, const void *w, const void *bias, void
 // channels inside a step as in the fp32 kernel below; weights [O][C] in that order in LDS.
 // Tiles of 64 pixels (four blocks of 16 matrix rows).  OUT_CL: out [B, HW, O], else [B, O, HW].
 // HW a multiple of 8 (16-byte pieces never run from one plane into the next).
-template <typename T, int C, int O, bool OUT_CL>
+template <typename T, int C, int O, bool OUT_CL, bool WIDE>
 __global__ void __launch_bounds__(256)
 project16p_kernel(const T *__restrict__ x, const T *__restrict__ w, const T *__restrict__ bias,
-                  T *__restrict__ out, long HW, int tiles_per_wave) {
+                  T *__restrict__ out, long HW, int tiles_per_wave, int outputs) {
     typedef short s16x4 __attribute__((ext_vector_type(4)));
     constexpr int NW = 4;
     constexpr int RW = C / 2 + 4;                 // dwords per padded row of C 16-bit values
@@ -237,14 +275,18 @@ project16p_kernel(const T *__restrict__ x, const T *__restrict__ w, const T *__r
     u32 *xt = sh + O * RW + wave * WF;            // this wave's x tile / result tile
     const int b = blockIdx.y;
 
+    const Span sp = span_of<O, WIDE>(outputs);
     // the image's weights -> LDS, 8 channels per thread and step: two groups of 4, which lie 8
     // places apart in the step's order
     {
-        const u32x4 *src = (const u32x4 *)(w + (long)b * O * C);
-        for (int i = threadIdx.x; i < O * C / 8; i += 64 * NW) {
-            const int o = i / (C / 8), c = 8 * (i % (C / 8)), cs = c % 32;
+        const __amdgpu_buffer_rsrc_t rw = __builtin_amdgcn_make_buffer_rsrc(
+            (void *)(w + (WIDE ? (long)sp.o0 : (long)b * O) * C), 0, sp.left * C * 2, 0x00020000);
+        static_assert(O * C / 8 % (64 * NW) == 0, "whole steps");
+#pragma unroll
+        for (int k = 0; k < O * C / 8 / (64 * NW); ++k) {
+            const int i = k * 64 * NW + threadIdx.x, o = i / (C / 8), c = 8 * (i % (C / 8)), cs = c % 32;
             const int pos = 32 * (c / 32) + 8 * ((cs % 16) / 4) + 4 * (cs / 16);
-            const u32x4 v = src[i];
+            const u32x4 v = __builtin_amdgcn_raw_buffer_load_b128(rw, (u32)i * 16u, 0, 0);
             u32 *dst = wl + o * RW + pos / 2;
             *(u32x2 *)dst = u32x2{v[0], v[1]};
             *(u32x2 *)(dst + 4) = u32x2{v[2], v[3]};
@@ -259,12 +301,15 @@ project16p_kernel(const T *__restrict__ x, const T *__restrict__ w, const T *__r
     const int r16 = lane & 15, kg = lane >> 4;
     float bv[NT];
 #pragma unroll
-    for (int nt = 0; nt < NT; ++nt) bv[nt] = bias ? (float)bias[(long)b * O + 16 * nt + r16] : 0.f;
+    for (int nt = 0; nt < NT; ++nt)
+        bv[nt] = bias && 16 * nt + r16 < sp.left ? (float)bias[(WIDE ? (long)sp.o0 : (long)b * O) + 16 * nt + r16] : 0.f;
 
     const __amdgpu_buffer_rsrc_t rx = __builtin_amdgcn_make_buffer_rsrc(
         (void *)(x + (long)b * HW * C), 0, (int)(HW * C * 2), 0x00020000);
+    // (planes: from the block's first plane to the end of its last, so that the rest is dropped)
     const __amdgpu_buffer_rsrc_t ro = __builtin_amdgcn_make_buffer_rsrc(
-        (void *)(out + (long)b * HW * O), 0, (int)(HW * O * 2), 0x00020000);
+        (void *)(out + ((long)b * sp.OT + (OUT_CL ? 0 : sp.o0)) * HW), 0,
+        (int)(HW * (OUT_CL ? sp.OT : sp.left) * 2), 0x00020000);
     // step (t, ks) of x: piece j = pixels 8 (lane % 8) .. + 7 of channel 8 j + lane / 8 of the step
     const u32 xoff = (u32)((lane >> 3) * HW + 8 * (lane & 7)) * 2u, xstride = (u32)(8 * HW * 2);
     u32x4 raw[RING][4];
@@ -304,6 +349,7 @@ project16p_kernel(const T *__restrict__ x, const T *__restrict__ w, const T *__r
             }
 #pragma unroll
             for (int nt = 0; nt < NT; ++nt) {
+                if (WIDE && 16 * nt >= sp.left) break;
                 const u32x4 bm = *(const u32x4 *)(wl + (16 * nt + r16) * RW + 16 * ks + 4 * kg);
 #pragma unroll
                 for (int mb = 0; mb < 4; ++mb) acc[mb][nt] = Mma32<T>::run(a[mb], bm, acc[mb][nt]);
@@ -320,12 +366,13 @@ project16p_kernel(const T *__restrict__ x, const T *__restrict__ w, const T *__r
 #pragma unroll
                     for (int i = 0; i < 4; ++i)
                         rt[(4 * kg + i) * (2 * OW) + 16 * nt + r16] = (unsigned short)pack2<T>(acc[mb][nt][i] + bv[nt], 0.f);
-                const u32 obase = (u32)((t * 64 + 16 * mb) * O * 2);
+                const u32 obase = (u32)(((t * 64 + 16 * mb) * sp.OT + sp.o0) * 2);
 #pragma unroll
                 for (int j = 0; j < (16 * O / 8 + 63) / 64; ++j) {
                     const int i = j * 64 + lane, row = i / (O / 8), col = i % (O / 8);
-                    if (16 * O / 8 % 64 == 0 || i < 16 * O / 8)
-                        __builtin_amdgcn_raw_buffer_store_b128(*(const u32x4 *)(xt + row * OW + 4 * col), ro, (u32)(i * 16) + obase, 0, 2);
+                    const u32 off = WIDE ? (u32)((row * sp.OT + 8 * col) * 2) : (u32)(i * 16);
+                    if ((16 * O / 8 % 64 == 0 || i < 16 * O / 8) && (!WIDE || 8 * col < sp.left))
+                        __builtin_amdgcn_raw_buffer_store_b128(*(const u32x4 *)(xt + row * OW + 4 * col), ro, off + obase, 0, 2);
                 }
             }
         } else {
@@ -333,6 +380,7 @@ project16p_kernel(const T *__restrict__ x, const T *__restrict__ w, const T *__r
             // 128 bytes; pieces past the plane's end are dropped
 #pragma unroll
             for (int nt = 0; nt < NT; ++nt) {
+                if (WIDE && 16 * nt >= sp.left) break;
 #pragma unroll
                 for (int mb = 0; mb < 4; ++mb)
                     *(u32x2 *)(xt + r16 * PW + 8 * mb + 2 * kg) =
@@ -350,23 +398,24 @@ project16p_kernel(const T *__restrict__ x, const T *__restrict__ w, const T *__r
     }
 }
 
-template <typename T, int C, int O, bool OUT_CL>
+template <typename T, int C, int O, bool OUT_CL, bool WIDE = false>
 static hipError_t launch16p_co(const void *x, const void *w, const void *bias, void *out, int B, long HW,
-                               hipStream_t st) {
+                               hipStream_t st, int outputs = O) {
     constexpr int RT = OUT_CL ? 16 * (O / 2 + 4) : 16 * 36, XT = 32 * 40;
     constexpr size_t lds = (size_t)(O * (C / 2 + 4) + 4 * (RT > XT ? RT : XT)) * 4;
     static_assert(lds <= 64 * 1024, "weights and tiles within the default LDS of a workgroup");
-    if (HW % 8 != 0 || HW * (long)(C > O ? C : O) * 2 >= (1L << 31)) return hipErrorNotSupported;
+    if (HW % 8 != 0 || HW * (long)(C > outputs ? C : outputs) * 2 >= (1L << 31)) return hipErrorNotSupported;
     const long ntiles = (HW + 63) / 64;
+    const int blocks_o = (outputs + O - 1) / O;
     // two workgroups are resident per CU (their registers) and the part has 256 CUs: one round of
     // at most 512 workgroups, at least 2 tiles per wave (q projection at 16 x 200 x 336 pixels:
     // 140 us against 152 with 704 workgroups)
-    long per = (ntiles * B + 4L * 512 - 1) / (4L * 512);
+    long per = (ntiles * B * blocks_o + 4L * 512 - 1) / (4L * 512);
     if (per < 2) per = 2;
     const long blocks = (ntiles + 4 * per - 1) / (4 * per);
-    if (blocks > 65535 * 32L || B > 65535) return hipErrorNotSupported;
-    hipLaunchKernelGGL((project16p_kernel<T, C, O, OUT_CL>), dim3((unsigned)blocks, B), dim3(256), lds, st,
-                       (const T *)x, (const T *)w, (const T *)bias, (T *)out, HW, (int)per);
+    if (blocks > 65535 * 32L || B > 65535 || blocks_o > 65535) return hipErrorNotSupported;
+    hipLaunchKernelGGL((project16p_kernel<T, C, O, OUT_CL, WIDE>), dim3((unsigned)blocks, B, blocks_o), dim3(256), lds,
+                       st, (const T *)x, (const T *)w, (const T *)bias, (T *)out, HW, (int)per, outputs);
     return hipGetLastError();
 }
 
@@ -418,10 +467,10 @@ __device__ __forceinline__ f32x4 mma32(u32x4 a, u32x4 b, f32x4 c) {
 // that the two channel groups of a half-wave read disjoint banks).  OUT_CL = false: out is
 // [B, O, HW]; a block of 16 outputs x 32 pixels goes back through LDS and leaves as 128-byte rows
 // (HW a multiple of 4: a 16-byte piece never runs from one plane into the next).
-template <int C, int O, bool IN_CL, bool OUT_CL>
+template <int C, int O, bool IN_CL, bool OUT_CL, bool WIDE>
 __global__ void __launch_bounds__(512)
 project32_kernel(const float *__restrict__ x, const float *__restrict__ w, const float *__restrict__ bias,
-                 float *__restrict__ out, long HW, int tiles_per_wave) {
+                 float *__restrict__ out, long HW, int tiles_per_wave, int waves, int outputs) {
     static_assert(IN_CL ? OUT_CL : true, "channels-last features give channels-last projections");
     constexpr int NW = 8;
     constexpr int RW = C / 2 + 4;                 // dwords per padded row of C bf16 values
@@ -441,37 +490,23 @@ project32_kernel(const float *__restrict__ x, const float *__restrict__ w, const
     float *rt = (float *)(sh + 3 * PLANE) + wave * WF;          // this wave's x tile / result tile
     const int b = blockIdx.y;
 
-    // the image's weights, taken apart, -> LDS (two neighbouring channels per thread and step)
-    {
-        typedef float f32x2 __attribute__((ext_vector_type(2)));
-        const f32x2 *src = (const f32x2 *)(w + (long)b * O * C);
-        for (int i = threadIdx.x; i < O * C / 2; i += 64 * NW) {
-            const int o = i / (C / 2), c = 2 * (i % (C / 2)), cs = c % 32;
-            const int pos = 32 * (c / 32) + 8 * ((cs % 16) / 4) + 4 * (cs / 16) + cs % 4;
-            const f32x2 v = src[i];
-            const Pieces pc = split2(v[0], v[1]);
-            u32 *dst = wl + o * RW + pos / 2;
-            dst[0] = pc.hi;
-            dst[PLANE] = pc.mid;
-            dst[2 * PLANE] = pc.lo;
-        }
-    }
-    __syncthreads();
+    const Span sp = span_of<O, WIDE>(outputs);
 
     const long ntiles = (HW + 31) / 32;
-    const long t0 = ((long)blockIdx.x * NW + wave) * tiles_per_wave;
-    const long t1 = t0 + tiles_per_wave < ntiles ? t0 + tiles_per_wave : ntiles;
-    if (t0 >= t1) return;
+    const long t0 = ((long)blockIdx.x * waves + wave) * tiles_per_wave;       // waves past `waves` help with the weights only
+    const long t1 = wave >= waves ? t0 : t0 + tiles_per_wave < ntiles ? t0 + tiles_per_wave : ntiles;
     const int r16 = lane & 15, kg = lane >> 4;    // row / column of a 16 x 16 tile, k group
     float bv[NT];
 #pragma unroll
-    for (int nt = 0; nt < NT; ++nt) bv[nt] = bias ? bias[(long)b * O + 16 * nt + r16] : 0.f;
+    for (int nt = 0; nt < NT; ++nt)
+        bv[nt] = bias && 16 * nt + r16 < sp.left ? bias[(WIDE ? (long)sp.o0 : (long)b * O) + 16 * nt + r16] : 0.f;
 
     // byte offsets inside the image: out of range = past the last pixel = zeros / dropped
     const __amdgpu_buffer_rsrc_t rx = __builtin_amdgcn_make_buffer_rsrc(
         (void *)(x + (long)b * HW * C), 0, (int)(HW * C * 4), 0x00020000);
     const __amdgpu_buffer_rsrc_t ro = __builtin_amdgcn_make_buffer_rsrc(
-        (void *)(out + (long)b * HW * O), 0, (int)(HW * O * 4), 0x00020000);
+        (void *)(out + ((long)b * sp.OT + (OUT_CL ? 0 : sp.o0)) * HW), 0,
+        (int)(HW * (OUT_CL ? sp.OT : sp.left) * 4), 0x00020000);
     // step (t, ks) of x, 4 pieces of 16 bytes per lane.  Channels-last: blocks mb = 0, 1 x pieces
     // h = 0, 1 of pixel r16's record.  Planes: piece j = pixels 4 (lane % 8) .. + 3 of channel
     // 8 j + lane / 8 of the step
@@ -491,8 +526,35 @@ project32_kernel(const float *__restrict__ x, const float *__restrict__ w, const
     // reads channel 4 kg (+ 16) of pixel r16 (+ 16)
     float *const xw = rt + (lane >> 3) * 32 + (((lane & 7) ^ ((lane >> 5) << 2)) << 2);
     const float *const xr = rt + 4 * kg * 32 + ((((r16 >> 2)) ^ ((kg & 1) << 2)) << 2) + (r16 & 3);
+    // (x first: the weights come in behind its latency; a wave without a tile loads zeros or a
+    // neighbouring wave's pixels)
 #pragma unroll
     for (int k = 0; k < RING; ++k) load_step(k, t0, k);
+    // the image's weights, taken apart, -> LDS, four neighbouring channels per thread and step, all
+    // loads in flight together (outputs past the last: past the descriptor, zeros)
+    {
+        const __amdgpu_buffer_rsrc_t rw = __builtin_amdgcn_make_buffer_rsrc(
+            (void *)(w + (WIDE ? (long)sp.o0 : (long)b * O) * C), 0, sp.left * C * 4, 0x00020000);
+        constexpr int N = O * C / 4 / (64 * NW);
+        static_assert(O * C / 4 % (64 * NW) == 0, "whole steps");
+        u32x4 v[N];
+#pragma unroll
+        for (int k = 0; k < N; ++k)
+            v[k] = __builtin_amdgcn_raw_buffer_load_b128(rw, (u32)(k * 64 * NW + threadIdx.x) * 16u, 0, 0);
+#pragma unroll
+        for (int k = 0; k < N; ++k) {
+            const int i = k * 64 * NW + threadIdx.x, o = i / (C / 4), c = 4 * (i % (C / 4)), cs = c % 32;
+            const int pos = 32 * (c / 32) + 8 * ((cs % 16) / 4) + 4 * (cs / 16);
+            const f32x4 f = __builtin_bit_cast(f32x4, v[k]);
+            const Pieces p0 = split2(f[0], f[1]), p1 = split2(f[2], f[3]);
+            u32 *dst = wl + o * RW + pos / 2;
+            *(u32x2 *)dst = u32x2{p0.hi, p1.hi};
+            *(u32x2 *)(dst + PLANE) = u32x2{p0.mid, p1.mid};
+            *(u32x2 *)(dst + 2 * PLANE) = u32x2{p0.lo, p1.lo};
+        }
+    }
+    __syncthreads();
+    if (t0 >= t1) return;
     for (long t = t0; t < t1; ++t) {
         f32x4 acc[2][NT];
 #pragma unroll
@@ -531,6 +593,7 @@ project32_kernel(const float *__restrict__ x, const float *__restrict__ w, const
             else if (t + 1 < t1) load_step(ks % RING, t + 1, ks + RING - KS);
 #pragma unroll
             for (int nt = 0; nt < NT; ++nt) {
+                if (WIDE && 16 * nt >= sp.left) break;
                 const u32 *wp = wl + (16 * nt + r16) * RW + 16 * ks + 4 * kg;
                 const u32x4 bhi = *(const u32x4 *)wp, bmid = *(const u32x4 *)(wp + PLANE), blo = *(const u32x4 *)(wp + 2 * PLANE);
 #pragma unroll
@@ -551,6 +614,7 @@ project32_kernel(const float *__restrict__ x, const float *__restrict__ w, const
             // neighbouring pixels), then 16 rows of 128 bytes; pieces past the plane's end are dropped
 #pragma unroll
             for (int nt = 0; nt < NT; ++nt) {
+                if (WIDE && 16 * nt >= sp.left) break;
 #pragma unroll
                 for (int mb = 0; mb < 2; ++mb) {
                     const f32x4 v = {acc[mb][nt][0] + bv[nt], acc[mb][nt][1] + bv[nt], acc[mb][nt][2] + bv[nt],
@@ -575,41 +639,53 @@ project32_kernel(const float *__restrict__ x, const float *__restrict__ w, const
             for (int nt = 0; nt < NT; ++nt)
 #pragma unroll
                 for (int i = 0; i < 4; ++i) rt[(4 * kg + i) * OS + 16 * nt + r16] = acc[mb][nt][i] + bv[nt];
-            const u32 obase = (u32)((t * 32 + 16 * mb) * O * 4);
+            const u32 obase = (u32)(((t * 32 + 16 * mb) * sp.OT + sp.o0) * 4);
 #pragma unroll
             for (int j = 0; j < (16 * O / 4 + 63) / 64; ++j) {
                 const int i = j * 64 + lane, row = i / (O / 4), col = i % (O / 4);
-                if (16 * O / 4 % 64 == 0 || i < 16 * O / 4)
-                    __builtin_amdgcn_raw_buffer_store_b128(*(const u32x4 *)(rt + row * OS + 4 * col), ro, (u32)(i * 16) + obase, 0, 2);
+                const u32 off = WIDE ? (u32)((row * sp.OT + 4 * col) * 4) : (u32)(i * 16);
+                if ((16 * O / 4 % 64 == 0 || i < 16 * O / 4) && (!WIDE || 4 * col < sp.left))
+                    __builtin_amdgcn_raw_buffer_store_b128(*(const u32x4 *)(rt + row * OS + 4 * col), ro, off + obase, 0, 2);
             }
         }
     }
 }
 
-template <int C, int O, bool IN_CL, bool OUT_CL>
+template <int C, int O, bool IN_CL, bool OUT_CL, bool WIDE = false>
 static hipError_t launch32_co(const void *x, const void *w, const void *bias, void *out, int B, long HW,
-                              hipStream_t st) {
+                              hipStream_t st, int outputs = O) {
     constexpr int RT = OUT_CL ? 16 * (O + 4) : 16 * 36, XB = IN_CL ? 0 : 32 * 32;
     constexpr size_t lds = (size_t)(3 * O * (C / 2 + 4) + 8 * (RT > XB ? RT : XB)) * 4;
     if (!OUT_CL && HW % 4 != 0) return hipErrorNotSupported;
     static_assert(lds <= 160 * 1024, "weights and tiles must fit LDS");
     // 32-bit byte offsets inside an image
-    if (HW * (long)(C > O ? C : O) * 4 >= (1L << 31)) return hipErrorNotSupported;
+    if (HW * (long)(C > outputs ? C : outputs) * 4 >= (1L << 31)) return hipErrorNotSupported;
     const long ntiles = (HW + 31) / 32;
+    const int blocks_o = (outputs + O - 1) / O;
+    const long sets = (long)B * blocks_o;         // workgroups that share a pixel range's place
     // One workgroup is resident per CU (its weight planes fill most of the LDS) and the part has
     // 256 CUs: two full rounds of workgroups where that leaves a wave 8 tiles or more, else one
     // (16 images: 200x336 pixels 301 us in two rounds against 315 in one; 100x168 pixels 71 us in
     // one round against 98 in 272 workgroups)
     const long slots = 256;
-    long blocks = 2 * slots / B > 1 ? 2 * slots / B : 1;
+    long blocks = 2 * slots / sets > 1 ? 2 * slots / sets : 1;
     long per = (ntiles + 8 * blocks - 1) / (8 * blocks);
     if (per < 8) {
-        blocks = slots / B > 1 ? slots / B : 1;
+        blocks = slots / sets > 1 ? slots / sets : 1;
         per = (ntiles + 8 * blocks - 1) / (8 * blocks);
     }
-    blocks = (ntiles + 8 * per - 1) / (8 * per);
-    if (blocks > 65535 * 32L || B > 65535) return hipErrorNotSupported;
-    auto kern = project32_kernel<C, O, IN_CL, OUT_CL>;
+    // fewer tiles than the chip has room for: a tile per wave and as few waves per workgroup as fill it
+    // (its matrix instructions are then not queued behind a second wave's; 4 images of 33x20 pixels,
+    // 256 -> 128 / 288: SAPA-D module 113 -> 104 us)
+    int waves = 8;
+    if (per == 1) {
+        const long room = slots / sets > 1 ? slots / sets : 1;
+        waves = (int)((ntiles + room - 1) / room);
+        waves = waves < 1 ? 1 : waves > 8 ? 8 : waves;
+    }
+    blocks = (ntiles + waves * per - 1) / (waves * per);
+    if (blocks > 65535 * 32L || B > 65535 || blocks_o > 65535) return hipErrorNotSupported;
+    auto kern = project32_kernel<C, O, IN_CL, OUT_CL, WIDE>;
     if (lds > 64 * 1024) {
         int dev = 0, most = 0;
         if (hipGetDevice(&dev) != hipSuccess ||
@@ -621,8 +697,8 @@ static hipError_t launch32_co(const void *x, const void *w, const void *bias, vo
             return hipErrorNotSupported;
         }
     }
-    hipLaunchKernelGGL(kern, dim3((unsigned)blocks, B), dim3(512), lds, st, (const float *)x, (const float *)w,
-                       (const float *)bias, (float *)out, HW, (int)per);
+    hipLaunchKernelGGL(kern, dim3((unsigned)blocks, B, blocks_o), dim3(512), lds, st, (const float *)x, (const float *)w,
+                       (const float *)bias, (float *)out, HW, (int)per, waves, outputs);
     return hipGetLastError();
 }
 
@@ -652,7 +728,42 @@ static hipError_t launch_t(const void *x, const void *w, const void *bias, void 
     return hipErrorNotSupported;
 }
 
+// one output block per 64 outputs (32 where 512 channels' weights leave no room for more)
+template <typename T, bool IN_CL, bool OUT_CL>
+static hipError_t launch_shared(const void *x, const void *w, const void *bias, void *out, int B, int C, int O,
+                                long HW, hipStream_t st) {
+#define SAPA_SHARED_CASE(CV, OV)                                                                                     \
+    if (C == CV) {                                                                                                   \
+        if constexpr (sizeof(T) == 4) return launch32_co<CV, OV, IN_CL, OUT_CL, true>(x, w, bias, out, B, HW, st, O); \
+        else if constexpr (IN_CL) return launch_co<T, CV, OV, true>(x, w, bias, out, B, HW, st, O);                  \
+        else return launch16p_co<T, CV, OV, OUT_CL, true>(x, w, bias, out, B, HW, st, O);                            \
+    }
+    SAPA_SHARED_CASE(64, 64) SAPA_SHARED_CASE(128, 64) SAPA_SHARED_CASE(256, 64) SAPA_SHARED_CASE(512, 32)
+#undef SAPA_SHARED_CASE
+    return hipErrorNotSupported;
+}
+
 }  // namespace project
+
+// A plain 1x1 convolution: weights w [O, C] and bias [O] (or null) shared by all images, x and out
+// in contiguous or channels-last order; C in {64, 128, 256, 512}, O a multiple of 8; what
+// project_nhwc_launch / project_nchw_launch require of HW and of pointers holds here too.
+hipError_t project_shared_launch(const void *x, const void *w, const void *bias, void *out, int B, int C, int O,
+                                 long HW, int x_channels_last, int out_channels_last, int dtype, hipStream_t st) {
+    const void *ptrs[3] = {x, w, out};
+    for (const void *p : ptrs)
+        if ((uintptr_t)p % 16 != 0) return hipErrorNotSupported;
+    if (O % 8 != 0 || (x_channels_last && !out_channels_last)) return hipErrorNotSupported;
+#define SAPA_SHARED(TV)                                                                                       \
+    return x_channels_last ? project::launch_shared<TV, true, true>(x, w, bias, out, B, C, O, HW, st)         \
+           : out_channels_last ? project::launch_shared<TV, false, true>(x, w, bias, out, B, C, O, HW, st)    \
+                               : project::launch_shared<TV, false, false>(x, w, bias, out, B, C, O, HW, st)
+    if (dtype == 0) SAPA_SHARED(float);
+    if (dtype == 2) SAPA_SHARED(f16_t);
+    if (dtype == 3) SAPA_SHARED(bf16_t);
+#undef SAPA_SHARED
+    return hipErrorNotSupported;
+}
 
 // x [B, HW, C], w [B, O, C], bias [B, O] or null, out [B, HW, O]; f16 / bf16 / fp32;
 // (C, O) among the instantiated pairs (C in {64, 128, 256, 512}, O in {32, 64, 128}; fp32:

@@ -115,6 +115,11 @@ def norm_project(x, norm, *convs, channels_last=False, defer_bias=False):
     for conv in convs:
         assert conv.kernel_size == (1, 1) and conv.groups == 1
         O = conv.out_channels
+        if norm is None and channels_last and not defer_bias and x.is_cuda and not torch.is_grad_enabled():
+            out = _lib.project_shared(x, conv.weight, conv.bias, channels_last_out=True)
+            if out is not None:
+                outs.append(out)
+                continue
         folded = None
         if norm is not None and mom is not None and not _needs_grad(norm, conv):
             # the per-image weights and bias in one small kernel launch (the kernel
@@ -161,6 +166,31 @@ def norm_project(x, norm, *convs, channels_last=False, defer_bias=False):
                 out = out.view(B, O, H, W)
         outs.append((out, b_b) if defer_bias else out)
     return outs
+
+
+def _plain(t):
+    """A tensor whose memory a kernel may be given: no subclass, no functorch wrapper."""
+    return type(t) in (torch.Tensor, nn.Parameter) and not torch._C._functorch.is_functorch_wrapped_tensor(t)
+
+
+def _project(conv, x):
+    """conv(x) for a 1x1 convolution: at inference on a contiguous GPU feature the library's streaming
+    projection, which adds the bias in its epilogue (at B=8, 256 channels, 128x128 fp32 the library
+    GEMM and the pass that adds the bias took 120 us for 128 outputs); everything else -- gradients,
+    autocast, tracing, tensor subclasses, hooks, another kind of convolution in the module's place --
+    is the module's call."""
+    if (not torch.is_grad_enabled() and type(conv) is nn.Conv2d and conv.kernel_size == (1, 1)
+            and conv.stride == (1, 1) and conv.padding == (0, 0) and conv.groups == 1
+            and x.dim() == 4 and x.is_cuda and x.is_contiguous()
+            and not (conv._forward_hooks or conv._forward_pre_hooks or nn.modules.module._global_forward_hooks
+                     or nn.modules.module._global_forward_pre_hooks)
+            and not torch.is_autocast_enabled('cuda') and not torch.jit.is_tracing()
+            and torch.autograd.forward_ad._current_level < 0 and torch._C._len_torch_dispatch_stack() == 0
+            and all(_plain(t) for t in (x, conv.weight) + (() if conv.bias is None else (conv.bias,)))):
+        out = _lib.project_shared(x, conv.weight, conv.bias)
+        if out is not None:
+            return out
+    return conv(x)
 
 
 def _init_projection(m):
@@ -297,7 +327,7 @@ class SAPADeform(nn.Module):
             x_ = self.norm_x(x) if self.norm else x
             if self.norm:
                 y = self.norm_y(y)
-            q, k, offset_lo = self.q(y), self.k(x_), self.offset(x_)
+            q, k, offset_lo = _project(self.q, y), _project(self.k, x_), _project(self.offset, x_)
         if self.fused and (x.is_contiguous()
                            or not x.is_contiguous(memory_format=torch.channels_last)):
             # the kernel reads the offset convolution's output in place

@@ -82,3 +82,35 @@ def test_fused_dense_window_kernel_edges(dtype, B, d, C, H, W):
         assert _lib.last_kernel() == 'sapa_b_wmat16_kernel'
         want = sapa_amd.sapa_fused(*[t.double() for t in ops], 5, 2)
     assert _rel(got, want) <= torch.finfo(dtype).eps / 2 / 3 ** 0.5 * 1.2
+
+
+@pytest.mark.parametrize('dtype', [torch.float32, torch.bfloat16, torch.float16])
+@pytest.mark.parametrize('in_cl,out_cl', [(False, False), (False, True), (True, True)])
+@pytest.mark.parametrize('B,C,O,H,W', [
+    (1, 64, 8, 2, 4),        # a part of one block of outputs, a part of one tile of pixels
+    (2, 128, 72, 7, 8),      # one block and a remainder of 8
+    (3, 256, 288, 9, 40),    # several blocks, the last one half full
+    (1, 512, 40, 12, 34),    # blocks of 32 outputs
+    (16, 256, 128, 16, 16),  # more workgroups than CUs for the 16-bit kernels
+])
+def test_projection_with_shared_weights(dtype, in_cl, out_cl, B, C, O, H, W):
+    """sapa_project_shared against fp64 products of the same operands: fp32 within an error bound of
+    a C-term fp32 dot product (C + 8 roundings of 2^-24 of the sum of magnitudes), 16-bit results one
+    rounding further."""
+    from sapa_amd import _lib
+    g = torch.Generator(device='cuda').manual_seed(O)
+    x = torch.randn(B, C, H, W, generator=g, device='cuda').to(dtype)
+    if in_cl:
+        x = x.contiguous(memory_format=torch.channels_last)
+    w = torch.randn(O, C, 1, 1, generator=g, device='cuda').mul(0.05).to(dtype)
+    b = torch.randn(O, generator=g, device='cuda').to(dtype)
+    x64, w64 = x.double().contiguous().reshape(B, C, H * W), w.double().reshape(1, O, C).expand(B, O, C).contiguous()
+    for bias in (b, None):
+        got = _lib.project_shared(x, w, bias, channels_last_out=out_cl)
+        assert got.is_contiguous(memory_format=torch.channels_last if out_cl else torch.contiguous_format)
+        want = torch.bmm(w64, x64).view(B, O, H, W)
+        mag = torch.bmm(w64.abs(), x64.abs()).view(B, O, H, W)
+        if bias is not None:
+            want, mag = want + b.double().view(1, O, 1, 1), mag + b.double().abs().view(1, O, 1, 1)
+        bar = (C + 8) * 2.0 ** -24 * mag + (0.0 if dtype == torch.float32 else 0.5 * torch.finfo(dtype).eps * want.abs() + 1e-7)
+        assert int(((got.double() - want).abs() > bar).sum()) == 0
