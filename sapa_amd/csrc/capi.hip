@@ -45,7 +45,7 @@ const long kSmallFusedCells = 12288;
 hipError_t tiled_launch(int mode, const void *q, const void *key, const void *attn_in,
                         const void *value, void *out, int B, int d, int C, int H, int W, int K,
                         int s, int dtype, hipStream_t st) {
-    // 16-bit fused problems of the common window first: both products on the 16-bit matrix
+    // 16-bit fused problems of the common windows first: both products on the 16-bit matrix
     // instructions, whatever the size (B=8, d=32, C=256, bf16: 32x32 21 -> 16 us, 64x64 48 -> 20 us)
     hipError_t e = hipErrorNotSupported;
 #ifndef SAPA_WMAT16_OFF

@@ -1,5 +1,5 @@
 // Fused SAPA-B forward (qk -> softmax -> av) for contiguous (NCHW) f16 / bf16 tensors on the
-// 16-bit matrix instructions, K = 5, s = 2.
+// 16-bit matrix instructions; written out for K = 5, s = 2, other windows at the kernel.
 //
 // The 16 parents of a 4 x 4 block share one 8 x 8 window of low-res cells (block + halo of 2),
 // and their 64 children need, each, 25 of those 64 cells.  Written over the whole window the two
@@ -97,22 +97,40 @@ __device__ __forceinline__ int swz(int ch, int r) { return ((ch & 7) << 1) | ((r
 // low-res windows, which neighbouring tiles re-read, out of the caches (fused FPN-large bf16, 860 MB:
 // 271 -> 213 us; at a quarter of the size, where everything fits the memory-side cache, 50 -> 58 us:
 // the launcher decides by size)
-template <typename T, int NSW, bool STREAM, bool ODD>
+//
+// (K, S) other than (5, 2) take the same blocks of 8 x 8 children and 8 x 8 cells, of PB = 8 / S
+// parents a side: (7, 4) uses all 64 cells of a window, (5, 4) and (3, 2) 36.  Windows of
+// neighbouring blocks start PB cells apart, which the transposing reads (4 cells, 8-byte aligned)
+// cannot follow in a shared row, so every block has a piece of 8 cells of its own per row (OWN): a
+// low-res cell is staged 8 / PB times, out of the caches, for S * S outputs.  Measured in bf16 against
+// the one-parent-per-block matrix kernel on fp32 operands, which these windows took before: K=7, s=4,
+// B=4, C=512, d=64, 64x64 250 -> 69 us (4.7 TB/s: memory), B=16, C=256, 50x84 756 -> 309 us (rows
+// of 672 bytes: split cache lines); K=5, s=4 165 -> 66 and 480 -> 263 us; K=3, s=2 57 -> 27 and
+// 132 -> 52 us; one image 16x16 33 -> 12, 20 -> 15 and 15 -> 15 us.
+template <typename T, int K, int S, int NSW, bool STREAM, bool ODD>
 __global__ __launch_bounds__(64 * NSW, 4) void
 sapa_b_wmat16_kernel(const T *__restrict__ q, const T *__restrict__ key, const T *__restrict__ value,
                      T *__restrict__ out, int d, int C, int H, int W, int tiles_x, int tiles_y, int ns,
                      int nslices, int slice_chunks, int nblocks, int per_xcd) {
     constexpr int NT = 64 * NSW;
-    constexpr int LROW = (4 * NSW + 4 + 7) / 8 * 4;          // dwords per staged window row: whole pieces of 8 cells
+    constexpr int PB = 8 / S, R = (K - 1) / 2, SS = S * S;
+    constexpr bool OWN = !(K == 5 && S == 2);
+    static_assert(PB + K - 1 <= 8 && S * PB == 8, "a block's window");
+    static_assert(!OWN || ODD, "pieces of a block's own come through registers");
+    // dwords per staged window row: whole pieces of 8 cells (OWN: one per block; a piece of padding
+    // keeps the rows of the 16 channels on different banks)
+    constexpr int LROW = OWN ? 4 * NSW + 4 : (4 * NSW + 4 + 7) / 8 * 4;
+    constexpr int LPC = OWN ? NSW : LROW / 4;                // pieces per row
+    constexpr int BSTEP = OWN ? 4 : 2;                       // dwords from a block's window to the next one's
     constexpr int LOWBUF = WROWS * CHK * LROW;               // dwords per low-res buffer
-    constexpr int NLP = LOWBUF / 4;                          // 16-byte pieces per low-res buffer
+    constexpr int NLP = WROWS * CHK * LPC;                   // 16-byte pieces per low-res buffer
     constexpr int NLI = (NLP + NT - 1) / NT;                 // 16-byte direct loads per thread and window, at most
     constexpr int HIROW = 8 * NSW / 2;                       // dwords per q / output tile row
     constexpr int HICH = WROWS * HIROW;                      // dwords per channel of the tile
     constexpr int HIBUF = CHK * HICH;                        // dwords per q / output buffer
     constexpr int NHI = HIBUF / 4 / NT;                      // 16-byte pieces per thread and tile
     static_assert(HIBUF % (4 * NT) == 0 && NLP % 64 == 0, "whole direct loads");
-    static_assert(4 * NSW + 4 <= 2 * LROW, "window row");
+    static_assert(OWN || 4 * NSW + 4 <= 2 * LROW, "window row");
     static_assert(NSW == 16 || NSW == 8, "piece swizzle");
     constexpr int NPC = 2 * NSW / 2;                         // 16-byte pieces per tile row = NSW
 
@@ -125,15 +143,15 @@ sapa_b_wmat16_kernel(const T *__restrict__ q, const T *__restrict__ key, const T
     if (logical >= nblocks) return;
     const int tile = logical / nslices, vbase = (logical % nslices) * slice_chunks;      // first value chunk
     const int tx = tile % tiles_x, ty = (tile / tiles_x) % tiles_y, n = tile / (tiles_x * tiles_y);
-    const int X0 = tx * 4 * ns, Y0 = ty * 4;                 // first parent of the tile
-    const int nsx = (W + 3) / 4;
+    const int X0 = tx * PB * ns, Y0 = ty * PB;               // first parent of the tile
+    const int nsx = (W + PB - 1) / PB;
     const int ns_here = nsx - tx * ns < ns ? nsx - tx * ns : ns;
 
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int g = lane >> 4, i16 = lane & 15;
     const long lpix = (long)H * W;
-    const u32 lplane = (u32)(lpix * sizeof(T)), hplane = 4 * lplane;
+    const u32 lplane = (u32)(lpix * sizeof(T)), hplane = SS * lplane;
 
     // direct-load offsets inside one image, without the chunk's first channel.  A low-res piece is
     // 8 cells from x = X0 - 2 + 8 pc on: 4-byte aligned, and where it runs over an end of its row it
@@ -147,11 +165,11 @@ sapa_b_wmat16_kernel(const T *__restrict__ q, const T *__restrict__ key, const T
     int patch_slot = -1;
 #pragma unroll
     for (int i = 0; i < NLI; ++i) {
-        const int slot = i * NT + tid, rc = slot / (LROW / 4), pc = slot % (LROW / 4);
+        const int slot = i * NT + tid, rc = slot / LPC, pc = slot % LPC;
         const int r = rc / CHK, ch = rc % CHK;
-        const int y = Y0 - 2 + r, x = X0 - 2 + 8 * pc;
-        const bool ok = slot < NLP && 8 * pc < 4 * ns_here + 4 && y >= 0 && y < H && x < W;
-        low_odd[i] = ODD && ((ch * lpix + (long)y * W) & 1);
+        const int y = Y0 - R + r, x = X0 - R + (OWN ? PB : 8) * pc;
+        const bool ok = slot < NLP && (OWN ? pc < ns_here : 8 * pc < 4 * ns_here + 4) && y >= 0 && y < H && x < W;
+        low_odd[i] = ODD && ((ch * lpix + (long)y * W + x) & 1);
         off_low[i] = ok ? (u32)(ch * lpix + (long)y * W + x - low_odd[i]) * (u32)sizeof(T) : OUTSIDE;
         if (ok && x < 0 && y == 0 && ch == 0) patch_slot = slot;
     }
@@ -159,22 +177,22 @@ sapa_b_wmat16_kernel(const T *__restrict__ q, const T *__restrict__ key, const T
     for (int i = 0; i < NHI; ++i) {
         const int slot = i * NT + tid, ch = slot / (WROWS * NPC), r = (slot / NPC) % WROWS;
         const int pc = (slot % NPC) ^ (swz(ch, r) & (NPC - 1));
-        const int cy = 2 * Y0 + r, cx = 2 * X0 + 8 * pc;
-        const bool ok = pc < ns_here && cy < 2 * H && cx < 2 * W;
-        off_hi[i] = ok ? (u32)(ch * 4 * lpix + (long)cy * 2 * W + cx) * (u32)sizeof(T) : OUTSIDE;
-        tail_children[i] = ok && cx + 8 > 2 * W ? 2 * W - cx : 8;
+        const int cy = S * Y0 + r, cx = S * X0 + 8 * pc;
+        const bool ok = pc < ns_here && cy < S * H && cx < S * W;
+        off_hi[i] = ok ? (u32)(ch * SS * lpix + (long)cy * S * W + cx) * (u32)sizeof(T) : OUTSIDE;
+        tail_children[i] = ok && cx + 8 > S * W ? S * W - cx : 8;
     }
 
     const int nKc = (d + CHK - 1) / CHK, allV = (C + CHK - 1) / CHK;
     const int nVc = allV - vbase < slice_chunks ? allV - vbase : slice_chunks, ntot = nKc + nVc;
     const __amdgpu_buffer_rsrc_t rq = __builtin_amdgcn_make_buffer_rsrc(
-        (void *)(q + (long)n * d * 4 * lpix), 0, (int)(d * hplane), 0x00020000);
+        (void *)(q + (long)n * d * SS * lpix), 0, (int)(d * hplane), 0x00020000);
     const __amdgpu_buffer_rsrc_t rk = __builtin_amdgcn_make_buffer_rsrc(
         (void *)(key + (long)n * d * lpix), 0, (int)((d * lplane + 3u) & ~3u), 0x00020000);
     const __amdgpu_buffer_rsrc_t rv = __builtin_amdgcn_make_buffer_rsrc(
         (void *)(value + (long)n * C * lpix), 0, (int)((C * lplane + 3u) & ~3u), 0x00020000);
     const __amdgpu_buffer_rsrc_t ro = __builtin_amdgcn_make_buffer_rsrc(
-        (void *)(out + (long)n * C * 4 * lpix), 0, (int)(C * hplane), 0x00020000);
+        (void *)(out + (long)n * C * SS * lpix), 0, (int)(C * hplane), 0x00020000);
 
     (void)rq, (void)rk, (void)rv;
     // Chunk j is the key + q channels 16 j .. for j < nKc and the value channels 16 (j - nKc) ..
@@ -219,20 +237,33 @@ sapa_b_wmat16_kernel(const T *__restrict__ q, const T *__restrict__ key, const T
         const __amdgpu_buffer_rsrc_t r = j < nKc ? rk : rv;
 #pragma unroll
         for (int i = 0; i < NLI; ++i) {
-            low_reg[i] = __builtin_amdgcn_raw_buffer_load_b128(r, off_low[i] + c0 * lplane, 0, 0);
-            low_next[i] = __builtin_amdgcn_raw_buffer_load_b32(r, off_low[i] + c0 * lplane + 16, 0, 0);
+            u32 off = off_low[i] + c0 * lplane;
+            // (OWN: the piece without an address: the tensor's first cells, put in place by low_commit)
+            if (OWN && c0 == 0 && patch_slot == i * NT + tid) off = 0;
+            low_reg[i] = __builtin_amdgcn_raw_buffer_load_b128(r, off, 0, 0);
+            low_next[i] = __builtin_amdgcn_raw_buffer_load_b32(r, off + 16, 0, 0);
         }
     };
     auto low_commit = [&](int j) __attribute__((always_inline)) {
         if (!ODD || j >= ntot) return;
 #pragma unroll
         for (int i = 0; i < NLI; ++i) {
+            const int slot = i * NT + tid;
             const u32x4 v = low_reg[i];
             u32x4 m = v;
             if (low_odd[i])
                 m = u32x4{__builtin_amdgcn_alignbyte(v[1], v[0], 2), __builtin_amdgcn_alignbyte(v[2], v[1], 2),
                           __builtin_amdgcn_alignbyte(v[3], v[2], 2), __builtin_amdgcn_alignbyte(low_next[i], v[3], 2)};
-            if (i * NT + tid < NLP) *(u32x4 *)(lowbuf + (j & 1) * LOWBUF + (i * NT + tid) * 4) = m;
+            if (OWN && patch_slot == slot && (j == 0 || (j == nKc && vbase == 0)))
+                // moved up by R cells (R = 3: by 1 in the second block's piece)
+                m = R == 2 ? u32x4{0u, v[0], v[1], v[2]}
+                    : R == 1 || slot % LPC == 1
+                        ? u32x4{v[0] << 16, __builtin_amdgcn_alignbyte(v[1], v[0], 2),
+                                __builtin_amdgcn_alignbyte(v[2], v[1], 2), __builtin_amdgcn_alignbyte(v[3], v[2], 2)}
+                        : u32x4{0u, v[0] << 16, __builtin_amdgcn_alignbyte(v[1], v[0], 2),
+                                __builtin_amdgcn_alignbyte(v[2], v[1], 2)};
+            const int at = OWN ? slot / LPC * LROW + slot % LPC * 4 : slot * 4;
+            if (NLP % NT == 0 || slot < NLP) *(u32x4 *)(lowbuf + (j & 1) * LOWBUF + at) = m;
         }
     };
     // Waits are counted: the counter of vector-memory operations retires in issue order, so
@@ -252,7 +283,7 @@ sapa_b_wmat16_kernel(const T *__restrict__ q, const T *__restrict__ key, const T
     // cells of the piece that has no address (first row of the image's first channel, tile at the
     // left edge)
     auto patch_low = [&](int jn) __attribute__((always_inline)) {
-        if (tx == 0 && ty == 0 && patch_slot >= 0 && (jn < nKc || vbase == 0)) {
+        if (!OWN && tx == 0 && ty == 0 && patch_slot >= 0 && (jn < nKc || vbase == 0)) {
             const __amdgpu_buffer_rsrc_t r = jn < nKc ? rk : rv;
             u32 *dst = lowbuf + (jn & 1) * LOWBUF + patch_slot * 4;
 #pragma unroll
@@ -266,7 +297,7 @@ sapa_b_wmat16_kernel(const T *__restrict__ q, const T *__restrict__ key, const T
 #endif
     };
 
-    const bool row_tail = (W & 3) != 0 && X0 + 4 * ns_here > W;      // wave-uniform
+    const bool row_tail = W % PB != 0 && X0 + PB * ns_here > W;      // wave-uniform
     const bool active = wave < ns_here;
     const int t = wave;                                       // this wave's block of the tile
 
@@ -297,7 +328,7 @@ sapa_b_wmat16_kernel(const T *__restrict__ q, const T *__restrict__ key, const T
             u32x2 a[4], b[4];
 #pragma unroll
             for (int mb = 0; mb < 4; ++mb)
-                a[mb] = read_tr(kb + ((2 * mb + trow) * CHK + tch) * LROW + 2 * t + 2 * tcol);
+                a[mb] = read_tr(kb + ((2 * mb + trow) * CHK + tch) * LROW + BSTEP * t + 2 * tcol);
 #pragma unroll
             for (int nb = 0; nb < 4; ++nb) {
                 const int r = 2 * nb + trow;
@@ -326,8 +357,8 @@ sapa_b_wmat16_kernel(const T *__restrict__ q, const T *__restrict__ key, const T
         // ends have such columns.
         bool cell_outside[4];
 #pragma unroll
-        for (int v = 0; v < 4; ++v) cell_outside[v] = (u32)(X0 + 4 * t - 2 + 4 * (g & 1) + v) >= (u32)W;
-        const bool at_row_end = X0 + 4 * t - 2 < 0 || X0 + 4 * t + 5 >= W;      // wave-uniform
+        for (int v = 0; v < 4; ++v) cell_outside[v] = (u32)(X0 + PB * t - R + 4 * (g & 1) + v) >= (u32)W;
+        const bool at_row_end = X0 + PB * t - R < 0 || X0 + PB * t - R + 7 >= W;      // wave-uniform
         if (at_row_end) {
 #pragma unroll
             for (int mb = 0; mb < 4; ++mb)
@@ -337,20 +368,21 @@ sapa_b_wmat16_kernel(const T *__restrict__ q, const T *__restrict__ key, const T
                     for (int v = 0; v < 4; ++v)
                         if (cell_outside[v]) sim[mb][nb][v] = 0.f;
         }
-        // a child of parent column px takes window columns px .. px + 4: -inf added to the others
-        const int px = (i16 & 7) >> 1;
+        // a child of parent column px takes window columns px .. px + K - 1: -inf added to the others
+        const int px = (i16 & 7) / S;
         const float NEG_INF = -__builtin_inff(), LOG2E = 1.4426950408889634f;
         float col_bias[4];
 #pragma unroll
-        for (int v = 0; v < 4; ++v) col_bias[v] = (u32)(4 * (g & 1) + v - px) <= 4u ? 0.f : NEG_INF;
+        for (int v = 0; v < 4; ++v) col_bias[v] = (u32)(4 * (g & 1) + v - px) < (u32)K ? 0.f : NEG_INF;
 #pragma unroll
         for (int nb = 0; nb < 4; ++nb) {
-            // child row 2 nb + i16 / 8 -> parent row nb: window rows nb .. nb + 4.  Block mb holds
+            // child row 2 nb + i16 / 8 -> parent row pr: window rows pr .. pr + K - 1.  Block mb holds
             // rows 2 mb (lanes g < 2) and 2 mb + 1: all, some or none of its lanes take part
+            const int pr = 2 * nb / S;
             float x[4][4], m = NEG_INF;
 #pragma unroll
             for (int mb = 0; mb < 4; ++mb) {
-                const bool lo_in = 2 * mb >= nb && 2 * mb <= nb + 4, hi_in = 2 * mb + 1 >= nb && 2 * mb + 1 <= nb + 4;
+                const bool lo_in = 2 * mb >= pr && 2 * mb < pr + K, hi_in = 2 * mb + 1 >= pr && 2 * mb + 1 < pr + K;
                 if (!lo_in && !hi_in) continue;
                 const float row_bias = lo_in && hi_in ? 0.f : ((g >> 1) ? hi_in : lo_in) ? 0.f : NEG_INF;
 #pragma unroll
@@ -366,7 +398,7 @@ sapa_b_wmat16_kernel(const T *__restrict__ q, const T *__restrict__ key, const T
             float e[4][4], sum = 0.f;
 #pragma unroll
             for (int mb = 0; mb < 4; ++mb) {
-                const bool lo_in = 2 * mb >= nb && 2 * mb <= nb + 4, hi_in = 2 * mb + 1 >= nb && 2 * mb + 1 <= nb + 4;
+                const bool lo_in = 2 * mb >= pr && 2 * mb < pr + K, hi_in = 2 * mb + 1 >= pr && 2 * mb + 1 < pr + K;
 #pragma unroll
                 for (int v = 0; v < 4; ++v) {
                     e[mb][v] = lo_in || hi_in ? __builtin_amdgcn_exp2f(__builtin_fmaf(x[mb][v], LOG2E, mneg)) : 0.f;
@@ -408,7 +440,7 @@ sapa_b_wmat16_kernel(const T *__restrict__ q, const T *__restrict__ key, const T
             u32x4 b[2];
 #pragma unroll
             for (int s = 0; s < 2; ++s) {
-                const u32 *p = vb + ((4 * s + (g >> 1)) * CHK + i16) * LROW + 2 * t + 2 * (g & 1);
+                const u32 *p = vb + ((4 * s + (g >> 1)) * CHK + i16) * LROW + BSTEP * t + 2 * (g & 1);
                 const u32x2 lo = *(const u32x2 *)p, hi = *(const u32x2 *)(p + 2 * CHK * LROW);
                 b[s] = u32x4{lo[0], lo[1], hi[0], hi[1]};
             }
@@ -441,7 +473,7 @@ sapa_b_wmat16_kernel(const T *__restrict__ q, const T *__restrict__ key, const T
             const u32x4 o = *(const u32x4 *)(ob + (i * NT + tid) * 4);
             u32 off = off_hi[i] + c0 * hplane;
             if (row_tail && tail_children[i] < 8) {
-                if (!ODD) {
+                if (S == 4 || !ODD) {
                     __builtin_amdgcn_raw_buffer_store_b64(u32x2{o[0], o[1]}, ro, off, 0, 0);
                 } else {
 #pragma unroll
@@ -458,11 +490,12 @@ sapa_b_wmat16_kernel(const T *__restrict__ q, const T *__restrict__ key, const T
     }
 }
 
-template <typename T, int NSW, bool STREAM, bool ODD>
+template <typename T, int K, int S, int NSW, bool STREAM, bool ODD>
 static hipError_t launch_geom(const void *q, const void *key, const void *value, void *out, int B, int d,
                               int C, int H, int W, hipStream_t st) {
-    const int nsx = (W + 3) / 4;
-    const int tiles_x = (nsx + NSW - 1) / NSW, tiles_y = (H + 3) / 4;
+    constexpr int PB = 8 / S;
+    const int nsx = (W + PB - 1) / PB;
+    const int tiles_x = (nsx + NSW - 1) / NSW, tiles_y = (H + PB - 1) / PB;
     const int ns = (nsx + tiles_x - 1) / tiles_x;             // blocks per tile, balanced over the row
     const long tiles = (long)tiles_x * tiles_y * B;
     // Fewer tiles than CUs: a workgroup's time is a chain of one step per 16 channels, so the value
@@ -476,7 +509,7 @@ static hipError_t launch_geom(const void *q, const void *key, const void *value,
     const long nb = tiles * nslices;
     if (nb > (1L << 30)) return hipErrorNotSupported;
     const int per_xcd = (int)((nb + 7) / 8);
-    hipLaunchKernelGGL((sapa_b_wmat16_kernel<T, NSW, STREAM, ODD>), dim3(per_xcd * 8), dim3(64 * NSW), 0, st, (const T *)q,
+    hipLaunchKernelGGL((sapa_b_wmat16_kernel<T, K, S, NSW, STREAM, ODD>), dim3(per_xcd * 8), dim3(64 * NSW), 0, st, (const T *)q,
                        (const T *)key, (const T *)value, (T *)out, d, C, H, W, tiles_x, tiles_y, ns,
                        nslices, slice_chunks, (int)nb, per_xcd);
     return hipGetLastError();
@@ -484,14 +517,15 @@ static hipError_t launch_geom(const void *q, const void *key, const void *value,
 
 }  // namespace wm16
 
-// Fused forward only; f16 / bf16, K = 5, s = 2, W >= 4 (one block), low-res tensors 4-byte and
+// Fused forward only; f16 / bf16, (K, s) = (5, 2), (7, 4), (5, 4) or (3, 2), W >= 4, low-res tensors 4-byte and
 // high-res tensors 16-byte aligned, every image of every tensor below 2 GiB (32-bit offsets
 // inside an image); hipErrorNotSupported otherwise.
 hipError_t sapa_b_wmat16_launch(int mode, const void *q, const void *key, const void *value, void *out, int B,
                                 int d, int C, int H, int W, int K, int s, int dtype, hipStream_t st) {
-    if (mode != TILED_FUSED || K != 5 || s != 2 || W < 4) return hipErrorNotSupported;
+    const bool k5s2 = K == 5 && s == 2, k7s4 = K == 7 && s == 4, k5s4 = K == 5 && s == 4, k3s2 = K == 3 && s == 2;
+    if (mode != TILED_FUSED || !(k5s2 || k7s4 || k5s4 || k3s2) || W < 4) return hipErrorNotSupported;
     if (dtype != 2 && dtype != 3) return hipErrorNotSupported;
-    const long hplane = (long)H * W * 8;
+    const long hplane = (long)H * W * s * s * 2;
     if ((long)(d > C ? d : C) * hplane >= (1L << 31)) return hipErrorNotSupported;
     if (((uintptr_t)key | (uintptr_t)value) % 4 != 0 || ((uintptr_t)q | (uintptr_t)out) % 16 != 0)
         return hipErrorNotSupported;
@@ -502,15 +536,27 @@ hipError_t sapa_b_wmat16_launch(int mode, const void *q, const void *key, const 
     // (low-res rows through registers) has tiles of 8 blocks only: with 16 the registers do not suffice
     // (B=16, C=256, d=64, 42x25: 24 us, by vector fmas 65; 100x167: 289 us against 451; rows below 16
     // cells, 13x13 at B=8: 9 us against 19 on the one-block-per-parent matrix kernel).
-    const bool stream = 2L * ((long)B * H * W * (5L * d + 5L * C)) > (256L << 20);
+    const bool stream = 2L * ((long)B * H * W * (1L + s * s) * ((long)d + C)) > (256L << 20);
     const bool odd = W % 2 != 0;
+    // Other windows: streamed only where a tile's rows are whole 128-byte lines (s W a multiple of 64);
+    // else parts of a line are written by two workgroups, and the caches put them together
+    // (K=7, s=4, bf16: B=4, C=512, 64x64: 69 us streamed, 114 not; B=16, C=256, 50x84: 386 and 309)
+    const bool lines = stream && s * W % 64 == 0;
+#define SAPA_WM16_OWN(T, KV, SV)                                                                                 \
+    if (K == KV && s == SV)                                                                                      \
+        return lines ? wm16::launch_geom<T, KV, SV, 8, true, true>(q, key, value, out, B, d, C, H, W, st)       \
+                      : wm16::launch_geom<T, KV, SV, 8, false, true>(q, key, value, out, B, d, C, H, W, st);
 #define SAPA_WM16_CASE(T)                                                                                       \
-    return odd      ? wm16::launch_geom<T, 8, false, true>(q, key, value, out, B, d, C, H, W, st)                \
-           : stream ? wm16::launch_geom<T, 16, true, false>(q, key, value, out, B, d, C, H, W, st)               \
-                    : wm16::launch_geom<T, 8, false, false>(q, key, value, out, B, d, C, H, W, st)
-    if (dtype == 2) SAPA_WM16_CASE(f16_t);
+    SAPA_WM16_OWN(T, 7, 4) SAPA_WM16_OWN(T, 5, 4) SAPA_WM16_OWN(T, 3, 2)                                         \
+    return odd      ? wm16::launch_geom<T, 5, 2, 8, false, true>(q, key, value, out, B, d, C, H, W, st)          \
+           : stream ? wm16::launch_geom<T, 5, 2, 16, true, false>(q, key, value, out, B, d, C, H, W, st)         \
+                    : wm16::launch_geom<T, 5, 2, 8, false, false>(q, key, value, out, B, d, C, H, W, st)
+    if (dtype == 2) {
+        SAPA_WM16_CASE(f16_t);
+    }
     SAPA_WM16_CASE(bf16_t);
 #undef SAPA_WM16_CASE
+#undef SAPA_WM16_OWN
 }
 
 }  // namespace sapa

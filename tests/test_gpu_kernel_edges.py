@@ -67,6 +67,7 @@ def test_fused_backward_from_operands(dtype, channels_last, B, d, C, H, W):
     (2, 24, 40, 5, 7),       # odd rows inside one tile, ragged channel chunks
     (1, 17, 33, 3, 33),      # an odd number of channels and cells: the last dword of a tensor is half its own
     (3, 32, 256, 9, 18),     # value channels split over workgroups
+    (2, 17, 33, 3, 33),      # images of an odd number of elements: the second starts in the middle of a dword
     (2, 32, 72, 21, 67),     # three tiles of an odd row
 ])
 def test_fused_dense_window_kernel_edges(dtype, B, d, C, H, W):
@@ -114,3 +115,27 @@ def test_projection_with_shared_weights(dtype, in_cl, out_cl, B, C, O, H, W):
             want, mag = want + b.double().view(1, O, 1, 1), mag + b.double().abs().view(1, O, 1, 1)
         bar = (C + 8) * 2.0 ** -24 * mag + (0.0 if dtype == torch.float32 else 0.5 * torch.finfo(dtype).eps * want.abs() + 1e-7)
         assert int(((got.double() - want).abs() > bar).sum()) == 0
+
+
+@pytest.mark.parametrize('dtype', [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize('K,s', [(7, 4), (5, 4), (3, 2)])
+@pytest.mark.parametrize('B,d,C,H,W', [
+    (1, 16, 16, 1, 4),       # one row, the smallest width
+    (2, 24, 40, 5, 7),       # odd rows inside one tile, ragged channel chunks
+    (2, 17, 33, 3, 21),      # an odd number of channels and cells: images start in the middle of a dword
+    (3, 32, 136, 9, 18),     # several tiles of s = 4, a partial one; value channels split over workgroups
+    (1, 32, 72, 6, 67),      # tiles of an odd row
+    (16, 40, 64, 33, 64),    # more tiles than CUs
+])
+def test_fused_dense_window_kernel_other_windows(dtype, K, s, B, d, C, H, W):
+    """The dense-window forward with a window piece per block, against the fp64 operator; bar as above."""
+    import sapa_amd
+    from sapa_amd import _lib
+    g = torch.Generator(device='cuda').manual_seed(W)
+    shapes = ((B, d, s * H, s * W), (B, d, H, W), (B, C, H, W))
+    ops = [torch.randn(sh, generator=g, device='cuda').mul(0.6).to(dtype) for sh in shapes]
+    with torch.no_grad():
+        got = sapa_amd.sapa_fused(*ops, K, s)
+        assert _lib.last_kernel() == 'sapa_b_wmat16_kernel'
+        want = sapa_amd.sapa_fused(*[t.double() for t in ops], K, s)
+    assert _rel(got, want) <= torch.finfo(dtype).eps / 2 / 3 ** 0.5 * 1.2
