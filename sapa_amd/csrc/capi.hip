@@ -813,7 +813,7 @@ long long esize_of(int dtype) { return dtype == SAPA_F32 ? 4 : dtype == SAPA_F64
 
 long long sapa_norm_project_scratch(int B, int C, int O, long long HW, int x_channels_last, int dtype) {
     if (B <= 0 || C <= 0 || O <= 0 || HW <= 0 || !dtype_ok(dtype)) return 0;
-    return round256(channel_moments_workspace(B, C, (long)HW, x_channels_last != 0)) + round256((long long)B * C * 8) +
+    return round256(channel_moments_workspace(B, C, (long)HW, x_channels_last != 0)) +
            round256((long long)B * O * C * esize_of(dtype)) + round256((long long)B * O * esize_of(dtype));
 }
 
@@ -832,15 +832,15 @@ int sapa_norm_project(const void *x, const void *gamma, const void *beta, const 
     char *p = (char *)scratch;
     void *ws = p;
     p += round256(channel_moments_workspace(B, C, (long)HW, x_channels_last != 0));
-    float *mean_var = (float *)p;
-    p += round256((long long)B * C * 8);
     void *w_b = p;
     p += round256((long long)B * O * C * esize_of(dtype));
     void *b_b = bias_out ? bias_out : (void *)p;
     hipStream_t st = (hipStream_t)stream;
-    hipError_t e = channel_moments_launch(x, ws, mean_var, B, C, (long)HW, x_channels_last != 0, dtype, st);
+    // (the projections' channel counts end at 512: the final sums and the fold are one launch)
+    hipError_t e = channel_moments_launch(x, ws, nullptr, B, C, (long)HW, x_channels_last != 0, dtype, st);
     if (e == hipSuccess)
-        e = groupnorm_fold_launch(mean_var, gamma, beta, weight, bias, w_b, b_b, B, C, O, groups, eps, dtype, st);
+        e = moments_fold_launch(x, ws, gamma, beta, weight, bias, w_b, b_b, B, C, O, groups, eps, (long)HW,
+                                x_channels_last != 0, dtype, st);
     if (e == hipSuccess)
         e = x_channels_last ? project_nhwc_launch(x, w_b, bias_out ? nullptr : b_b, out, B, C, O, (long)HW, dtype, st)
                             : project_nchw_launch(x, w_b, bias_out ? nullptr : b_b, out, B, C, O, (long)HW,

@@ -220,6 +220,7 @@ static void chunking_for(long HW, int B, int C, bool cl, long &seg, int &chunks)
 template <typename T>
 static hipError_t launch_t(const T *x, float *ws, float *mean_var, int B, int C, long HW, bool cl,
                            hipStream_t st) {
+    // mean_var null: the partial sums only
     long seg;
     int chunks;
     if (cl) {
@@ -232,7 +233,8 @@ static hipError_t launch_t(const T *x, float *ws, float *mean_var, int B, int C,
         else
             hipLaunchKernelGGL((partial_nhwc_kernel<T, 4>), dim3(chunks, B), dim3(256), 0, st, x, ws, C,
                                HW, seg, chunks);
-        hipLaunchKernelGGL((finish_kernel<T, true>), dim3(((long)B * C + 255) / 256), dim3(256), 0, st, x,
+        if (mean_var)
+            hipLaunchKernelGGL((finish_kernel<T, true>), dim3(((long)B * C + 255) / 256), dim3(256), 0, st, x,
                            ws, mean_var, B, C, HW, chunks);
     } else {
         chunking_for(HW, B, C, false, seg, chunks);
@@ -242,7 +244,8 @@ static hipError_t launch_t(const T *x, float *ws, float *mean_var, int B, int C,
             hipLaunchKernelGGL((partial_nchw_kernel<T, VEC>), grid, dim3(256), 0, st, x, ws, HW, seg, chunks);
         else
             hipLaunchKernelGGL((partial_nchw_kernel<T, 1>), grid, dim3(256), 0, st, x, ws, HW, seg, chunks);
-        hipLaunchKernelGGL((finish_kernel<T, false>), dim3(((long)B * C + 255) / 256), dim3(256), 0, st, x,
+        if (mean_var)
+            hipLaunchKernelGGL((finish_kernel<T, false>), dim3(((long)B * C + 255) / 256), dim3(256), 0, st, x,
                            ws, mean_var, B, C, HW, chunks);
     }
     return hipGetLastError();
@@ -298,6 +301,132 @@ fold_kernel(const float *__restrict__ mean_var, const T *__restrict__ gamma,
     }
 }
 
+// finish_kernel and fold_kernel in one launch, for a caller that wants the weights only: every block
+// adds up the partial sums of its image's channels again (from the cache: C * chunks * 8 bytes per
+// `rows` output rows).  Bound by the latency of its loads: what depends on no other load is requested
+// at once, and where an image has many chunks (`parts` > 1) several threads share a channel's, so
+// that a thread waits for a few batches of 16 instead of for all of them in turn.  Per feature, 2.4 + 6.2
+// us for the two kernels and 5 for this one at B=8, C=256, 16x16 in bf16, 6 + 8 and 10 at
+// B=16, C=256, 200x336 in channels-last bf16 (128 chunks).
+constexpr int kFoldChannels = 2048;                // 4 floats of LDS each
+template <typename T, bool CL>
+__global__ void __launch_bounds__(1024)
+finish_fold_kernel(const T *__restrict__ x, const float *__restrict__ part, const T *__restrict__ gamma,
+                   const T *__restrict__ beta, const T *__restrict__ w, const T *__restrict__ bias,
+                   T *__restrict__ w_out, T *__restrict__ b_out, int C, int O, int G, float eps, long HW,
+                   int chunks, int parts, int rows) {
+    typedef float f32x2 __attribute__((ext_vector_type(2)));
+    extern __shared__ float sh[];                  // mean[C], var[C], scale[C], shift[C]; before: sums[parts][C][2]
+    float *mean = sh, *var = sh + C, *scale = sh + 2 * C, *shift = sh + 3 * C;
+    f32x2 *sums = (f32x2 *)(sh + 4 * C);
+    const int nt = blockDim.x, nw = nt / 64, b = blockIdx.x, per = C / G;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int o0 = blockIdx.y * rows + wave, o1 = (int)(blockIdx.y + 1) * rows < O ? (int)(blockIdx.y + 1) * rows : O;
+    float first[4];                                // the first 256 channels of the wave's first row
+#pragma unroll
+    for (int u = 0; u < 4; ++u) first[u] = o0 < o1 && lane + 64 * u < C ? (float)w[(long)o0 * C + lane + 64 * u] : 0.f;
+    // sums of a channel's chunks k0 .. k1 - 1, in their order
+    auto add_up = [&](int c, int k0, int k1) {
+        const long i = (long)b * C + c;
+        auto at = [&](int k) {
+            return *(const f32x2 *)(CL ? part + (((long)b * chunks + k) * C + c) * 2 : part + (i * chunks + k) * 2);
+        };
+        f32x2 s = {0.f, 0.f};
+        int k = k0;
+        for (; k + 16 <= k1; k += 16) {
+            f32x2 v[16];
+#pragma unroll
+            for (int u = 0; u < 16; ++u) v[u] = at(k + u);
+#pragma unroll
+            for (int u = 0; u < 16; ++u) s[0] += v[u][0], s[1] += v[u][1];
+        }
+        for (; k < k1; k += 4) {
+            f32x2 v[4];
+#pragma unroll
+            for (int u = 0; u < 4; ++u) v[u] = at(k + u < k1 ? k + u : k1 - 1);
+#pragma unroll
+            for (int u = 0; u < 4; ++u)
+                if (k + u < k1) s[0] += v[u][0], s[1] += v[u][1];
+        }
+        return s;
+    };
+    if (parts > 1) {
+        const int len = (chunks + parts - 1) / parts;
+        for (int i = threadIdx.x; i < parts * C; i += nt) {
+            const int k0 = i / C * len, k1 = k0 + len < chunks ? k0 + len : chunks;
+            sums[i] = add_up(i % C, k0, k1);
+        }
+        __syncthreads();
+    }
+    for (int c = threadIdx.x; c < C; c += nt) {
+        const float origin = (float)(CL ? x[(long)b * HW * C + c] : x[((long)b * C + c) * HW]);
+        f32x2 s;
+        if (parts > 1) {
+            s = sums[c];
+            for (int p = 1; p < parts; ++p) s[0] += sums[p * C + c][0], s[1] += sums[p * C + c][1];
+        } else {
+            s = add_up(c, 0, chunks);
+        }
+        const float m = s[0] / (float)HW;
+        mean[c] = origin + m;
+        var[c] = __builtin_fmaxf(s[1] / (float)HW - m * m, 0.f);
+    }
+    __syncthreads();
+    // every channel's thread forms its group's moments
+    for (int c = threadIdx.x; c < C; c += nt) {
+        const float ga = gamma ? (float)gamma[c] : 1.f, be = beta ? (float)beta[c] : 0.f;
+        const int g0 = c / per * per;
+        float m = 0.f;
+#pragma unroll 8
+        for (int k = 0; k < per; ++k) m += mean[g0 + k];
+        m /= (float)per;
+        float v = 0.f;
+#pragma unroll 8
+        for (int k = 0; k < per; ++k) {
+            const float dm = mean[g0 + k] - m;
+            v += var[g0 + k] + dm * dm;
+        }
+        const float rstd = 1.f / __builtin_sqrtf(v / (float)per + eps);
+        scale[c] = ga * rstd;
+        shift[c] = be - m * ga * rstd;
+    }
+    __syncthreads();
+    for (int o = o0; o < o1; o += nw) {
+        const T *wr = w + (long)o * C;
+        T *wo = w_out + ((long)b * O + o) * C;
+        float acc = 0.f;
+        for (int c = lane, u = 0; c < C; c += 64, ++u) {
+            const float v = o == o0 && u < 4 ? (u == 0 ? first[0] : u == 1 ? first[1] : u == 2 ? first[2] : first[3]) : (float)wr[c];
+            wo[c] = (T)(v * scale[c]);
+            acc = fma_(v, shift[c], acc);
+        }
+#pragma unroll
+        for (int d = 32; d > 0; d >>= 1) acc += __shfl_xor(acc, d);
+        if (lane == 0) b_out[(long)b * O + o] = (T)(acc + (bias ? (float)bias[o] : 0.f));
+    }
+}
+
+template <typename T>
+static hipError_t finish_fold_t(const void *x, const float *part, const void *gamma, const void *beta, const void *w,
+                                const void *bias, void *w_out, void *b_out, int B, int C, int O, int G, float eps,
+                                long HW, bool cl, hipStream_t st) {
+    long seg;
+    int chunks;
+    chunking_for(HW, B, C, cl, seg, chunks);
+    // few chunks: a thread per channel, a row per wave of 4; else up to 1024 threads that share a
+    // channel's chunks in runs of 16 or more, and 16 rows for what they fetch
+    const bool many = chunks > 16;
+    const int nt = many ? 1024 : 256, rows = many ? 16 : 4;
+    int parts = many && C < nt ? nt / C : 1;
+    if (parts > chunks / 16) parts = chunks / 16 < 1 ? 1 : chunks / 16;
+    const size_t lds = (size_t)(4 * C + (parts > 1 ? 2 * parts * C : 0)) * sizeof(float);
+    auto kern = cl ? finish_fold_kernel<T, true> : finish_fold_kernel<T, false>;
+    hipLaunchKernelGGL(kern, dim3(B, (O + rows - 1) / rows), dim3(nt), lds, st, (const T *)x, part,
+                       (const T *)gamma, (const T *)beta, (const T *)w, (const T *)bias, (T *)w_out, (T *)b_out, C, O,
+                       G, eps, HW, chunks, parts, rows);
+    return hipGetLastError();
+}
+
 template <typename T>
 static hipError_t fold_t(const float *mean_var, const void *gamma, const void *beta, const void *w,
                          const void *bias, void *w_out, void *b_out, int B, int C, int O, int G,
@@ -319,7 +448,8 @@ long channel_moments_workspace(int B, int C, long HW, bool channels_last) {
 }
 
 // x: [B, C, HW] contiguous or [B, HW, C] (channels_last), f32 / f16 / bf16;
-// mean_var: [B, C, 2] fp32.  Channels-last needs C % 4 == 0, C <= 1024 and x
+// mean_var: [B, C, 2] fp32 (null: the partial sums stay in the workspace, for
+// moments_fold_launch).  Channels-last needs C % 4 == 0, C <= 1024 and x
 // aligned to 4 elements; the contiguous layout B * C <= 65535.
 // hipErrorNotSupported otherwise.
 hipError_t channel_moments_launch(const void *x, void *workspace, float *mean_var, int B, int C,
@@ -408,6 +538,21 @@ hipError_t groupnorm_fold_launch(const float *mean_var, const void *gamma, const
         case 0: return moments::fold_t<float>(mean_var, gamma, beta, w, bias, w_out, b_out, B, C, O, G, eps, st);
         case 2: return moments::fold_t<f16_t>(mean_var, gamma, beta, w, bias, w_out, b_out, B, C, O, G, eps, st);
         case 3: return moments::fold_t<bf16_t>(mean_var, gamma, beta, w, bias, w_out, b_out, B, C, O, G, eps, st);
+        default: return hipErrorNotSupported;
+    }
+}
+
+// channel_moments_launch's finish and groupnorm_fold_launch in one: `partial` is the workspace of a
+// channel_moments_launch without mean_var on the same x.  C % G == 0, C <= 2048.
+hipError_t moments_fold_launch(const void *x, const void *partial, const void *gamma, const void *beta, const void *w,
+                               const void *bias, void *w_out, void *b_out, int B, int C, int O, int G, float eps,
+                               long HW, bool channels_last, int dtype, hipStream_t st) {
+    if (G < 1 || C % G != 0 || C > moments::kFoldChannels) return hipErrorNotSupported;
+    const float *p = (const float *)partial;
+    switch (dtype) {
+        case 0: return moments::finish_fold_t<float>(x, p, gamma, beta, w, bias, w_out, b_out, B, C, O, G, eps, HW, channels_last, st);
+        case 2: return moments::finish_fold_t<f16_t>(x, p, gamma, beta, w, bias, w_out, b_out, B, C, O, G, eps, HW, channels_last, st);
+        case 3: return moments::finish_fold_t<bf16_t>(x, p, gamma, beta, w, bias, w_out, b_out, B, C, O, G, eps, HW, channels_last, st);
         default: return hipErrorNotSupported;
     }
 }
