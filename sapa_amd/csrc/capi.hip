@@ -38,6 +38,8 @@ const long long kMaxElems = 1LL << 40;
 
 // fused K = 5, s = 2 problems of at most this many low-res cells go to the matrix-pipe kernel
 const long kSmallFusedCells = 12288;
+// ... and the separate operators of at most this many cells (logits) and cells x channels (aggregation)
+const long kSmallLogitCells = 40000, kSmallAggregation = 1L << 20;
 
 // LDS-tiled SAPA-B kernel for `mode`: the VALU kernel where it has an
 // instance (K = 5, s = 2, where it is the faster one), else the matrix-pipe
@@ -54,8 +56,15 @@ hipError_t tiled_launch(int mode, const void *q, const void *key, const void *at
     // small fused problems next: the matrix-pipe kernel's lane-per-child decomposition fills the
     // chip where the thread-per-parent kernels leave it latency-bound
     // (B=8, d=32, C=256, fp32: 16x16 32 -> 12 us, 32x32 32 -> 23 us)
-    if (e == hipErrorNotSupported && K == 5 && s == 2 && dtype != SAPA_F64 && mode == TILED_FUSED &&
-        (long)B * H * W <= kSmallFusedCells)
+    // The separate operators of small problems likewise, their sums in the same order (us, d / C = 64 /
+    // 256, fp32).  Logits: 957 cells 37 -> 13, 6400 25 -> 13, 32000 40 -> 27, 67200 35 -> 44; aggregation:
+    // 957 cells 16 -> 7.5, 5160 17.4 -> 16.4, 6400 17.4 -> 18.7, 12288 21 -> 31; bf16 crosses at the
+    // same sizes (logits 32000 33 -> 26, 67200 29 -> 45).
+    const long cells = (long)B * H * W;
+    const bool small = mode == TILED_FUSED ? cells <= kSmallFusedCells
+                       : mode == TILED_AV  ? cells * C <= kSmallAggregation
+                                           : cells <= kSmallLogitCells;
+    if (e == hipErrorNotSupported && K == 5 && s == 2 && dtype != SAPA_F64 && small)
         e = took("sapa_b_mfma_kernel",
                  sapa_b_mfma_launch(mode, q, key, attn_in, value, out, B, d, C, H, W, K, s, dtype, st));
     if (e == hipErrorNotSupported)

@@ -139,3 +139,25 @@ def test_fused_dense_window_kernel_other_windows(dtype, K, s, B, d, C, H, W):
         assert _lib.last_kernel() == 'sapa_b_wmat16_kernel'
         want = sapa_amd.sapa_fused(*[t.double() for t in ops], K, s)
     assert _rel(got, want) <= torch.finfo(dtype).eps / 2 / 3 ** 0.5 * 1.2
+
+
+@pytest.mark.parametrize('dtype', [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize('B,d,C,H,W', [
+    (1, 32, 64, 32, 32),      # one image
+    (3, 17, 5, 7, 19),        # ragged tiles, channels that fill no chunk
+    (1, 40, 256, 64, 64),     # the last size of the aggregation on this kernel
+    (10, 8, 4, 50, 80),       # the last size of the logits on this kernel
+    (1, 8, 260, 65, 63),      # the first size past the aggregation's
+])
+def test_small_separate_operators(dtype, B, d, C, H, W):
+    """qk and av around the sizes where they change kernels: fp32 bit for bit the reference order's
+    sums (the C oracle); 16-bit results within one rounding of the fp32 call on the same values."""
+    import sapa_amd
+    from oracle import c_oracle
+    g = torch.Generator().manual_seed(W)
+    q, k, v = (torch.randn(s, generator=g).to(dtype) for s in ((B, d, 2 * H, 2 * W), (B, d, H, W), (B, C, H, W)))
+    a = torch.softmax(torch.randn(B, 25, 2 * H, 2 * W, generator=g), dim=1).to(dtype)
+    got = sapa_amd.qk(q.cuda(), k.cuda(), 5, 2).cpu(), sapa_amd.av(a.cuda(), v.cuda(), 5, 2).cpu()
+    want = c_oracle.qk(q.float(), k.float(), 5, 2, 'f32'), c_oracle.av(a.float(), v.float(), 5, 2, 'f32')
+    for x, y in zip(got, want):
+        assert torch.equal(x, y) if dtype == torch.float32 else _rel(x, y.double()) <= torch.finfo(dtype).eps / 2 / 3 ** 0.5 * 1.2
