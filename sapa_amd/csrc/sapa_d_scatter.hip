@@ -45,35 +45,39 @@ typedef float f32x4 __attribute__((ext_vector_type(4)));
 
 constexpr int RCH = 4;          // window reach around the region's parents, in low-res cells
 
-// Tensor elements through a buffer descriptor, widened to float: an offset with
-// bit 31 set lies beyond every descriptor and returns 0 without touching memory,
-// so a load needs no branch around it (and the compiler can count the loads in
-// flight: with loads in branches it waits for all of them at every use).
+// Tensor elements through a buffer descriptor: an offset with bit 31 set lies beyond every
+// descriptor and returns 0 without touching memory, so a load needs no branch around it (and the
+// compiler can count the loads in flight: with loads in branches it waits for all of them at every
+// use).  They stay raw bits until they are used: a 16-bit value widened where it is loaded, inside
+// the branch between vector and single loads, makes the wave wait for it there -- a whole memory
+// latency per step (B=8, C=256, 25 points, 64x64 in bf16: 265 / 221 us for value / key, 215 / 180 without).
 typedef unsigned u32x2 __attribute__((ext_vector_type(2)));
 typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
 constexpr unsigned OOB = 0x80000000u;
 template <typename T> struct Ld;
 template <> struct Ld<float> {
-    static __device__ __forceinline__ float one(__amdgpu_buffer_rsrc_t r, unsigned off) {
-        return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(r, off, 0, 0));
+    static __device__ __forceinline__ u32 one(__amdgpu_buffer_rsrc_t r, unsigned off) {
+        return __builtin_amdgcn_raw_buffer_load_b32(r, off, 0, 0);
     }
-    static __device__ __forceinline__ void four(__amdgpu_buffer_rsrc_t r, unsigned off, float (&v)[4]) {
-        union { u32x4 u; float f[4]; } x;
-        x.u = __builtin_amdgcn_raw_buffer_load_b128(r, off, 0, 0);
+    static __device__ __forceinline__ void four(__amdgpu_buffer_rsrc_t r, unsigned off, u32 (&v)[4]) {
+        const u32x4 x = __builtin_amdgcn_raw_buffer_load_b128(r, off, 0, 0);
 #pragma unroll
-        for (int e = 0; e < 4; ++e) v[e] = x.f[e];
+        for (int e = 0; e < 4; ++e) v[e] = x[e];
     }
+    static __device__ __forceinline__ float wide(u32 v) { return __builtin_bit_cast(float, v); }
+    static __device__ __forceinline__ float of_four(const u32 (&v)[4], int e) { return wide(v[e]); }
 };
 template <typename H> struct Ld16 {
-    static __device__ __forceinline__ float one(__amdgpu_buffer_rsrc_t r, unsigned off) {
-        return (float)__builtin_bit_cast(H, (unsigned short)__builtin_amdgcn_raw_buffer_load_b16(r, off, 0, 0));
+    static __device__ __forceinline__ u32 one(__amdgpu_buffer_rsrc_t r, unsigned off) {
+        return (unsigned short)__builtin_amdgcn_raw_buffer_load_b16(r, off, 0, 0);
     }
-    static __device__ __forceinline__ void four(__amdgpu_buffer_rsrc_t r, unsigned off, float (&v)[4]) {
-        union { u32x2 u; H h[4]; } x;
-        x.u = __builtin_amdgcn_raw_buffer_load_b64(r, off, 0, 0);
-#pragma unroll
-        for (int e = 0; e < 4; ++e) v[e] = (float)x.h[e];
+    static __device__ __forceinline__ void four(__amdgpu_buffer_rsrc_t r, unsigned off, u32 (&v)[4]) {
+        const u32x2 x = __builtin_amdgcn_raw_buffer_load_b64(r, off, 0, 0);
+        v[0] = x[0];
+        v[1] = x[1];
     }
+    static __device__ __forceinline__ float wide(u32 v) { return (float)__builtin_bit_cast(H, (unsigned short)v); }
+    static __device__ __forceinline__ float of_four(const u32 (&v)[4], int e) { return wide(e & 1 ? v[e / 2] >> 16 : v[e / 2]); }
 };
 template <> struct Ld<f16_t> : Ld16<f16_t> {};
 template <> struct Ld<bf16_t> : Ld16<bf16_t> {};
@@ -87,7 +91,8 @@ constexpr int GS = CHK + 16;    // floats per pixel of the staged hi tile: 16 mo
 // CLO: grad_low is a channels-last fp32 buffer [B, H, W, Cx] (a cell's channels in
 // one piece: the final atomics of a wave then fall on two cache lines instead of
 // one per window row and channel); else the contiguous [B, Cx, H, W] tensor.
-template <typename T, typename TS, int S, int RG, bool CLO>
+// VEC: rows of hi are whole aligned vectors of 4 elements.
+template <typename T, typename TS, int S, int RG, bool CLO, bool VEC>
 __global__ void __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4, 4)))
 deform_scatter_mat_kernel(const T *__restrict__ hi, const TS *__restrict__ sc,
                           const T *__restrict__ offset, float *__restrict__ grad_low, int Cx, int H,
@@ -153,7 +158,6 @@ deform_scatter_mat_kernel(const T *__restrict__ hi, const TS *__restrict__ sc,
     // values (lane = channel), their rows of Wm (zeroed, then filled by the wave's
     // own lanes: LDS operations of one wave execute in order, so no barrier sits
     // between the two) and their scales
-    const bool vec4 = hW % 4 == 0 && (uintptr_t)hi % (4 * sizeof(T)) == 0;
     // the chunk's planes of hi, the group's scalars and offsets (byte offsets below 2^31: the launcher checks)
     const __amdgpu_buffer_rsrc_t hrsrc = __builtin_amdgcn_make_buffer_rsrc(
         (void *)(hi + ch0 * hpl), 0, (int)(cvalid * hpl * (long)sizeof(T)), 0x00020000);
@@ -162,13 +166,13 @@ deform_scatter_mat_kernel(const T *__restrict__ hi, const TS *__restrict__ sc,
     const __amdgpu_buffer_rsrc_t orsrc = __builtin_amdgcn_make_buffer_rsrc(
         (void *)(offset + (k0 << 1) * hpl), 0, (int)(2 * P * hpl * (long)sizeof(T)), 0x00020000);
     // what a step needs from global memory, fetched two steps ahead (two sets in turn)
-    struct Pre { float greg[4], scr[2], oxr[2], oyr[2]; };
+    struct Pre { u32 greg[4], scr[2], oxr[2], oyr[2]; };
     auto load_hi = [&](int step, Pre &pre) __attribute__((always_inline)) {
         int qh, qw;
         step_pixel(step, 4 * wave, qh, qw);
-        const bool row_ok = lane < cvalid && qh < hH;
+        const bool row_ok = step < NSTEP && lane < cvalid && qh < hH;
         const unsigned off = (unsigned)(((long)lane * hpl + (long)qh * hW + qw) * (long)sizeof(T));
-        if (vec4) {     // (uniform) whole aligned vectors: inside the image or outside as a whole
+        if (VEC) {      // inside the image or outside as a whole
             Ld<T>::four(hrsrc, row_ok && qw < hW ? off : OOB, pre.greg);
         } else {
 #pragma unroll
@@ -190,7 +194,7 @@ deform_scatter_mat_kernel(const T *__restrict__ hi, const TS *__restrict__ sc,
         for (int ps = 0; ps < 2; ++ps) {
             int qh, qw;
             step_pixel(step, sample_pixel(ps), qh, qw);
-            const bool ok = ps < npass && pt < P && qh < hH && qw < hW;
+            const bool ok = step < NSTEP && ps < npass && pt < P && qh < hH && qw < hW;
             const long pp = (long)pt * hpl + (long)qh * hW + qw;        // the point's plane of sc
             const long po = pp + (long)pt * hpl;                        // its dx plane of the offsets
             pre.scr[ps] = Ld<TS>::one(srsrc, ok ? (unsigned)(pp * (long)sizeof(TS)) : OOB);
@@ -199,7 +203,6 @@ deform_scatter_mat_kernel(const T *__restrict__ hi, const TS *__restrict__ sc,
         }
     };
     auto produce = [&](int step, Pre &pre) __attribute__((always_inline)) {
-        const float (&scr)[2] = pre.scr, (&oxr)[2] = pre.oxr, (&oyr)[2] = pre.oyr;
         int *const Wl = Wl2 + (step & 1) * SPX * WSR;
         float *const Gl = Gl2 + (step & 1) * SPX * GS;
         float *const invl = invl2 + (step & 1) * SPX;
@@ -214,51 +217,82 @@ deform_scatter_mat_kernel(const T *__restrict__ hi, const TS *__restrict__ sc,
         u32 bad = 0;
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
-            const bool fin = __builtin_fabsf(pre.greg[e]) < __builtin_huge_valf();
+            const float gv = VEC ? Ld<T>::of_four(pre.greg, e) : Ld<T>::wide(pre.greg[e]);
+            const bool fin = __builtin_fabsf(gv) < __builtin_huge_valf();
             bad |= __builtin_amdgcn_ballot_w64(!fin) != 0 ? 1u << e : 0u;
-            Gl[(4 * wave + e) * GS + lane] = fin ? pre.greg[e] : 0.f;
+            Gl[(4 * wave + e) * GS + lane] = fin ? gv : 0.f;
         }
-        // ---- per (pixel, point): the corners' shares of sc into the pixel's row
-        auto sample = [&](auto nl, int ps) __attribute__((always_inline)) {
-            constexpr int NL = decltype(nl)::value;
-            const int t = sample_pixel(ps);
-            const bool isbad = bad >> (t & 3) & 1;
-            int qh, qw;
-            step_pixel(step, t, qh, qw);
-            const bool live = qh < hH && qw < hW && pt < P;
-            const float scv = scr[ps];
-            // the row's scale: |sum of any subset of its entries| <= L1 < 2^ex
-            const float l1 = reduce_lanes<false, NL>(live ? __builtin_fabsf(scv) : 0.f);
-            const bool finite = l1 < __builtin_huge_valf();
-            int ex = 0;
-            (void)__builtin_frexpf(l1, &ex);
-            const float scale = __builtin_ldexpf(1.f, 30 - ex);
-            if (pt == 0) invl[t] = (finite && l1 > 0.f) ? __builtin_ldexpf(1.f, ex - 30) : 0.f;
-            if (!live || (scv == 0.f && !isbad)) return;
-            const float kw = (float)(qw / S) + oxr[ps], kh = (float)(qh / S) + oyr[ps];
-            const WinTap<float> wt = win_tap<float>(kh, kw, H, W, wy0, wx0, WWR, WWR);
-            if (!wt.guard) return;
-            if (wt.inwin && wt.hl >= b0 && wt.hl < b1 && finite && !isbad) {
-                int *wp = Wl + t * WSR + wt.hl * WWR + wt.wl;
-                const float sv = scv * scale;
-                __hip_atomic_fetch_add(wp, (int)__builtin_rintf(sv * wt.w1), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-                __hip_atomic_fetch_add(wp + 1, (int)__builtin_rintf(sv * wt.w2), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-                __hip_atomic_fetch_add(wp + WWR, (int)__builtin_rintf(sv * wt.w3), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-                __hip_atomic_fetch_add(wp + WWR + 1, (int)__builtin_rintf(sv * wt.w4), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-            } else {
-                // the reference's own way: one float atomic per term (rare).  (The
-                // position is made opaque: its taps are set up in this branch only.)
-                float fkh = kh, fkw = kw;
-                asm volatile("" : "+v"(fkh), "+v"(fkw));
+        // ---- per (pixel, point): the corners' shares of sc into the pixel's row.  Straight-line code over
+        // both passes -- a producer wave's step is one chain of dependent instructions, and with
+        // the conditions as nested branches (the direct way of the rare samples between them)
+        // it took longer than the matrix instructions it feeds (B=8, C=256, 25 points, 64x64 in bf16: value /
+        // key 222 / 181 us with branches, 214 / 170 so)
+        auto samples = [&](auto nl, auto np) __attribute__((always_inline)) {
+            constexpr int NL = decltype(nl)::value, NP = decltype(np)::value;
+            int share[NP][4], *wp[NP];
+            float scv[NP], kh[NP], kw[NP];
+            bool fast[NP], slow[NP];
+#pragma unroll
+            for (int ps = 0; ps < NP; ++ps) {
+                const int t = sample_pixel(ps);
+                const bool isbad = bad >> (t & 3) & 1;
+                int qh, qw;
+                step_pixel(step, t, qh, qw);
+                const bool live = (qh < hH) & (qw < hW) & (pt < P);
+                scv[ps] = Ld<TS>::wide(pre.scr[ps]);
+                // the row's scale: |sum of any subset of its entries| <= L1 < 2^ex
+                const float l1 = reduce_lanes<false, NL>(live ? __builtin_fabsf(scv[ps]) : 0.f);
+                const bool finite = l1 < __builtin_huge_valf();
+                int ex = 0;
+                (void)__builtin_frexpf(l1, &ex);
+                const float scale = __builtin_ldexpf(1.f, 30 - ex);
+                const float inv = (finite & (l1 > 0.f)) ? __builtin_ldexpf(1.f, ex - 30) : 0.f;
+                if (pt == 0) invl[t] = inv;
+                kw[ps] = (float)(qw / S) + Ld<T>::wide(pre.oxr[ps]);
+                kh[ps] = (float)(qh / S) + Ld<T>::wide(pre.oyr[ps]);
+                // (win_tap's expressions)
+                const bool guard = (kh[ps] > -1.f) & (kh[ps] < (float)H) & (kw[ps] > -1.f) & (kw[ps] < (float)W);
+                const float fh = floor_(kh[ps]), fw = floor_(kw[ps]);
+                const int hl = (int)fh - wy0, wl = (int)fw - wx0;
+                const bool inwin = ((u32)hl <= (u32)(WWR - 2)) & ((u32)wl <= (u32)(WWR - 2)) & (hl >= b0) & (hl < b1);
+                const bool counts = live & ((scv[ps] != 0.f) | isbad) & guard;
+                fast[ps] = counts & inwin & finite & !isbad;
+                slow[ps] = counts & !fast[ps];
+                const float lh = kh[ps] - fh, lw = kw[ps] - fw, hh = 1.f - lh, hw = 1.f - lw;
+                const float sv = scv[ps] * scale;
+                wp[ps] = Wl + t * WSR + hl * WWR + wl;
+                share[ps][0] = (int)__builtin_rintf(sv * (hh * hw));
+                share[ps][1] = (int)__builtin_rintf(sv * (hh * lw));
+                share[ps][2] = (int)__builtin_rintf(sv * (lh * hw));
+                share[ps][3] = (int)__builtin_rintf(sv * (lh * lw));
+            }
+#pragma unroll
+            for (int ps = 0; ps < NP; ++ps)
+                if (fast[ps]) {
+                    __hip_atomic_fetch_add(wp[ps], share[ps][0], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+                    __hip_atomic_fetch_add(wp[ps] + 1, share[ps][1], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+                    __hip_atomic_fetch_add(wp[ps] + WWR, share[ps][2], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+                    __hip_atomic_fetch_add(wp[ps] + WWR + 1, share[ps][3], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+                }
+            bool any = slow[0];
+#pragma unroll
+            for (int ps = 1; ps < NP; ++ps) any |= slow[ps];
+            if (__builtin_amdgcn_ballot_w64(any) == 0) return;
+#pragma unroll
+            for (int ps = 0; ps < NP; ++ps) {
+                if (!slow[ps]) continue;
+                // the reference's own way: one float atomic per term (rare)
+                int qh, qw;
+                step_pixel(step, sample_pixel(ps), qh, qw);
                 Tap<float> tp = {};
-                tap_setup(fkh, fkw, H, W, tp);
+                tap_setup(kh[ps], kw[ps], H, W, tp);
                 const T *hp = hi + ch0 * hpl + (long)qh * hW + qw;
                 // element (cell i, channel c of the chunk) of grad_low
                 const long cstep = CLO ? Cx : 1, chstep = CLO ? 1 : lpix;
                 float *const g0 = grad_low + (CLO ? (long)n * lpix * Cx + (long)g * cg + c0 : ch0 * lpix);
                 for (int c = 0; c < cvalid; ++c) {
                     float *gp = g0 + c * chstep;
-                    const float tv = (float)hp[c * hpl] * scv;
+                    const float tv = (float)hp[c * hpl] * scv[ps];
                     if (tp.m1) unsafeAtomicAdd(gp + tp.i1 * cstep, tp.w1 * tv);
                     if (tp.m2) unsafeAtomicAdd(gp + tp.i2 * cstep, tp.w2 * tv);
                     if (tp.m3) unsafeAtomicAdd(gp + tp.i3 * cstep, tp.w3 * tv);
@@ -266,17 +300,13 @@ deform_scatter_mat_kernel(const T *__restrict__ hi, const TS *__restrict__ sc,
                 }
             }
         };
-        if (narrow) {
-            sample(std::integral_constant<int, 16>{}, 0);
-        } else {
-            sample(std::integral_constant<int, 32>{}, 0);
-            sample(std::integral_constant<int, 32>{}, 1);
-        }
+        if (narrow) samples(std::integral_constant<int, 16>{}, std::integral_constant<int, 1>{});
+        else samples(std::integral_constant<int, 32>{}, std::integral_constant<int, 2>{});
         // the loads of the step after the next go out (into the set this step has used up)
-        if (step + 2 < NSTEP) {
-            load_hi(step + 2, pre);
-            load_samples(step + 2, pre);
-        }
+        // (past the last step too, from nowhere: on a path without them the compiler would have to
+        // assume fewer loads in flight and wait for the other set's as well)
+        load_hi(step + 2, pre);
+        load_samples(step + 2, pre);
     };
 
     // ---- the region's sums into grad_low.  D[cbi][nb][r] = cell 16 cb + 4 mk + r,
@@ -335,12 +365,14 @@ deform_scatter_mat_kernel(const T *__restrict__ hi, const TS *__restrict__ sc,
         load_samples(0, pre0);
         load_hi(1, pre1);
         load_samples(1, pre1);
-        for (int i = 0; i <= NSTEP; i += 2) {
-            if (i < NSTEP) produce(i, pre0);
+        for (int i = 0; i < NSTEP; i += 2) {
+            produce(i, pre0);
             __syncthreads();
-            if (i + 1 < NSTEP) produce(i + 1, pre1);
+            produce(i + 1, pre1);
             __syncthreads();
         }
+        __syncthreads();        // (the last step is consumed)
+        __syncthreads();
         for (int cbi = 0; cbi < CBI; ++cbi) {
             __syncthreads();
             flush(cbi);
@@ -353,6 +385,10 @@ deform_scatter_mat_kernel(const T *__restrict__ hi, const TS *__restrict__ sc,
         for (int cbi = 0; cbi < CBI; ++cbi)
 #pragma unroll
             for (int nb = 0; nb < CHK / 16; ++nb) D[cbi][nb] = f32x4{0.f, 0.f, 0.f, 0.f};
+        // (a cell block's operands of two reduction steps are read together: with one read and one
+        // wait between two uniform branches the matrix pipe stood still)
+        constexpr int KU = 2;
+        const bool half = cvalid <= CHK / 2;         // (uniform) a short chunk skips its empty half
         auto consume = [&](int step) __attribute__((always_inline)) {
             const int *const Wl = Wl2 + (step & 1) * SPX * WSR;
             const float *const Gl = Gl2 + (step & 1) * SPX * GS;
@@ -360,20 +396,30 @@ deform_scatter_mat_kernel(const T *__restrict__ hi, const TS *__restrict__ sc,
             int b0, b1, cb0, cb1;
             band(step, b0, b1, cb0, cb1);
 #pragma unroll
-            for (int ks = 0; ks < SPX / 4; ++ks) {
-                const float inv = invl[4 * ks + mk];
-                float b[CHK / 16];
+            for (int k0 = 0; k0 < SPX / 4; k0 += KU) {
+                float inv[KU], b[KU][CHK / 16];
 #pragma unroll
-                for (int nb = 0; nb < CHK / 16; ++nb) b[nb] = Gl[(4 * ks + mk) * GS + 16 * nb + mi];
+                for (int u = 0; u < KU; ++u) {
+                    const int row = 4 * (k0 + u) + mk;
+                    inv[u] = invl[row];
+#pragma unroll
+                    for (int nb = 0; nb < CHK / 16; ++nb) b[u][nb] = Gl[row * GS + 16 * nb + mi];
+                }
 #pragma unroll
                 for (int cbi = 0; cbi < CBI; ++cbi) {
                     const int cb = wave + 4 * cbi;
-                    if (cb >= cb0 && cb <= cb1) {
-                        const float a = (float)Wl[(4 * ks + mk) * WSR + 16 * cb + mi] * inv;
+                    if (cb < cb0 || cb > cb1) continue;
+                    float a[KU];
 #pragma unroll
-                        for (int nb = 0; nb < CHK / 16; ++nb)
-                            if (16 * nb < cvalid)       // (uniform) a short chunk skips its empty channel blocks
-                                D[cbi][nb] = __builtin_amdgcn_mfma_f32_16x16x4f32(a, b[nb], D[cbi][nb], 0, 0, 0);
+                    for (int u = 0; u < KU; ++u) a[u] = (float)Wl[(4 * (k0 + u) + mk) * WSR + 16 * cb + mi] * inv[u];
+#pragma unroll
+                    for (int h = 0; h < 2; ++h) {
+                        if (h == 1 && half) break;
+#pragma unroll
+                        for (int u = 0; u < KU; ++u)
+#pragma unroll
+                            for (int nb = h * CHK / 32; nb < (h + 1) * CHK / 32; ++nb)
+                                D[cbi][nb] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[u], b[u][nb], D[cbi][nb], 0, 0, 0);
                     }
                 }
             }
@@ -402,7 +448,9 @@ static hipError_t launch_geom(const void *hi, const void *sc, const void *offset
     const long nb = (long)regions_x * regions_y * nchunks * G * B;
     if (nb > (1L << 30)) return hipErrorNotSupported;
     const int per_xcd = (int)((nb + 7) / 8);
-    hipLaunchKernelGGL((deform_scatter_mat_kernel<T, TS, S, RG, CLO>), dim3(per_xcd * 8), dim3(NT), 0, st,
+    const bool vec = W * S % 4 == 0 && (uintptr_t)hi % (4 * sizeof(T)) == 0;
+    auto kern = vec ? deform_scatter_mat_kernel<T, TS, S, RG, CLO, true> : deform_scatter_mat_kernel<T, TS, S, RG, CLO, false>;
+    hipLaunchKernelGGL(kern, dim3(per_xcd * 8), dim3(NT), 0, st,
                        (const T *)hi, (const TS *)sc, (const T *)offset, (float *)grad_low, Cx, H, W, P, G,
                        regions_x, regions_y, nchunks, (int)nb, per_xcd);
     return hipGetLastError();
