@@ -167,13 +167,17 @@ def dtype_code(t):
 def require_cuda_contiguous(**tensors):
     """The reference's CHECK_INPUT (sapa/sapa/src/cuda/qk_cuda.cpp:34-39):
     device tensors, contiguous, and here also one device and one dtype."""
+    _require_alike(tensors, True)
+
+
+def _require_alike(tensors, contiguous):
     first = None
     for name, t in tensors.items():
         if t is None:
             continue
         if not t.is_cuda:
             raise RuntimeError(f'{name} must be a CUDA tensor')
-        if not t.is_contiguous():
+        if contiguous and not t.is_contiguous():
             raise RuntimeError(f'{name} must be contiguous')
         if first is None:
             first = (name, t)
@@ -191,12 +195,10 @@ def memory_layout(**tensors):
     points); anything else raises like the reference's CHECK_INPUT."""
     ts = [t for t in tensors.values() if t is not None]
     if all(t.is_contiguous() for t in ts):
-        require_cuda_contiguous(**tensors)
+        _require_alike(tensors, False)
         return 'contiguous'
     if all(t.dim() == 4 and t.is_contiguous(memory_format=torch.channels_last) for t in ts):
-        # same device / dtype checks, on views that are contiguous
-        require_cuda_contiguous(**{k: (None if t is None else t.permute(0, 2, 3, 1))
-                                   for k, t in tensors.items()})
+        _require_alike(tensors, False)
         return 'channels_last'
     bad = [k for k, t in tensors.items() if t is not None and not t.is_contiguous()]
     raise RuntimeError(f'{bad[0]} must be contiguous (or every tensor in torch.channels_last order)')
@@ -253,9 +255,7 @@ TOO_LARGE = -3     # SAPA_ERR_TOO_LARGE: beyond the kernels' index range
 def call_status(name, device, *args):
     """Like `call`, but hands back SAPA_ERR_UNSUPPORTED instead of raising on
     it, for entry points that have a composite fallback."""
-    with torch.cuda.device(device):
-        stream = torch.cuda.current_stream(device).cuda_stream
-        status = getattr(lib(), name)(*args, stream)
+    status = _run(name, device, args)
     if status != UNSUPPORTED:
         check(status, name)
     return status
@@ -263,9 +263,18 @@ def call_status(name, device, *args):
 
 def call(name, device, *args):
     """Run entry point `name` on `device`'s current torch stream."""
+    check(_run(name, device, args), name)
+
+
+def _run(name, device, args):
+    """The status of entry point `name` on `device`'s current torch stream, with `device` current: the
+    device is switched only where it is another one, and the stream is asked for as the bare handle
+    (the context manager and the Stream object took 4 us of the host's time per call)."""
+    fn = getattr(lib(), name)
+    if torch._C._cuda_getDevice() == device.index:
+        return fn(*args, torch._C._cuda_getCurrentRawStream(device.index))
     with torch.cuda.device(device):
-        stream = torch.cuda.current_stream(device).cuda_stream
-        check(getattr(lib(), name)(*args, stream), name)
+        return fn(*args, torch.cuda.current_stream(device).cuda_stream)
 
 
 def channel_moments(x):
@@ -339,22 +348,16 @@ def norm_project(x, norm, conv, channels_last_out=False, defer_bias=False):
     else:
         return None
     out_cl = 1 if (cl or channels_last_out) else 0
-    handle = lib()
-    ptr = lambda t: None if t is None else t.data_ptr()
-    with torch.cuda.device(x.device):
-        nbytes = handle.sapa_norm_project_scratch(B, C, O, H * W, cl, DTYPES[dtype])
-        scratch = torch.empty(max(nbytes, 16), dtype=torch.uint8, device=x.device)
-        out = torch.empty(B, O, H, W, dtype=dtype, device=x.device,
-                          memory_format=torch.channels_last if out_cl else torch.contiguous_format)
-        b_out = torch.empty(B, O, dtype=dtype, device=x.device) if defer_bias else None
-        status = handle.sapa_norm_project(
-            x.data_ptr(), ptr(norm.weight), ptr(norm.bias), conv.weight.data_ptr(), ptr(conv.bias),
-            scratch.data_ptr(), out.data_ptr(), ptr(b_out), B, C, O, H * W, norm.num_groups, float(norm.eps),
-            cl, out_cl, DTYPES[dtype], torch.cuda.current_stream(x.device).cuda_stream)
-    if status == UNSUPPORTED:
-        return None
-    check(status, 'sapa_norm_project')
-    return out, b_out
+    nbytes = lib().sapa_norm_project_scratch(B, C, O, H * W, cl, DTYPES[dtype])
+    scratch = torch.empty(max(nbytes, 16), dtype=torch.uint8, device=x.device)
+    out = torch.empty(B, O, H, W, dtype=dtype, device=x.device,
+                      memory_format=torch.channels_last if out_cl else torch.contiguous_format)
+    b_out = torch.empty(B, O, dtype=dtype, device=x.device) if defer_bias else None
+    status = call_status(
+        'sapa_norm_project', x.device, x.data_ptr(), ptr(norm.weight), ptr(norm.bias), conv.weight.data_ptr(),
+        ptr(conv.bias), scratch.data_ptr(), out.data_ptr(), ptr(b_out), B, C, O, H * W, norm.num_groups,
+        float(norm.eps), cl, out_cl, DTYPES[dtype])
+    return None if status == UNSUPPORTED else (out, b_out)
 
 
 def project_nchw(x, weight, bias=None, channels_last_out=False):
@@ -403,13 +406,11 @@ def project_shared(x, weight, bias=None, channels_last_out=False):
     weight = weight.reshape(O, C).contiguous()
     if bias is not None:
         bias = bias.contiguous()
-    with torch.cuda.device(x.device):
-        out = torch.empty(B, O, H, W, dtype=x.dtype, device=x.device,
-                          memory_format=torch.channels_last if channels_last_out else torch.contiguous_format)
-        status = lib().sapa_project_shared(
-            x.data_ptr(), weight.data_ptr(), None if bias is None else bias.data_ptr(), out.data_ptr(),
-            B, C, O, H * W, 1 if x_cl else 0, 1 if channels_last_out else 0, DTYPES[x.dtype],
-            torch.cuda.current_stream(x.device).cuda_stream)
+    out = torch.empty(B, O, H, W, dtype=x.dtype, device=x.device,
+                      memory_format=torch.channels_last if channels_last_out else torch.contiguous_format)
+    status = _run('sapa_project_shared', x.device, (
+        x.data_ptr(), weight.data_ptr(), ptr(bias), out.data_ptr(), B, C, O, H * W, 1 if x_cl else 0,
+        1 if channels_last_out else 0, DTYPES[x.dtype]))
     if status in (UNSUPPORTED, TOO_LARGE):
         return None
     check(status, 'sapa_project_shared')

@@ -822,7 +822,8 @@ long long esize_of(int dtype) { return dtype == SAPA_F32 ? 4 : dtype == SAPA_F64
 
 long long sapa_norm_project_scratch(int B, int C, int O, long long HW, int x_channels_last, int dtype) {
     if (B <= 0 || C <= 0 || O <= 0 || HW <= 0 || !dtype_ok(dtype)) return 0;
-    return round256(channel_moments_workspace(B, C, (long)HW, x_channels_last != 0)) +
+    // (with room for the moments [B, C, 2], which callers have counted on)
+    return round256(channel_moments_workspace(B, C, (long)HW, x_channels_last != 0)) + round256((long long)B * C * 8) +
            round256((long long)B * O * C * esize_of(dtype)) + round256((long long)B * O * esize_of(dtype));
 }
 
