@@ -526,6 +526,17 @@ int sapa_norm_project(const void *x, const void *gamma, const void *beta, const 
                       const void *bias, void *scratch, void *out, void *bias_out, int B, int C,
                       int O, long long HW, int groups, float eps, int x_channels_last,
                       int out_channels_last, int dtype, void *stream);
+/* The same for two features at once (a module's query and key feature: the same B, C, O, groups,
+ * eps, types and memory orders; HW and everything else their own): their moments are one launch and their
+ * folds another.  scratch: the sum of the two features' sapa_norm_project_scratch.  Nothing
+ * is launched and SAPA_ERR_UNSUPPORTED returned unless both are served. */
+int sapa_norm_project_pair(const void *x0, const void *gamma0, const void *beta0,
+                           const void *weight0, const void *bias0, void *out0, void *bias_out0,
+                           long long HW0, const void *x1, const void *gamma1, const void *beta1,
+                           const void *weight1, const void *bias1, void *out1, void *bias_out1,
+                           long long HW1, void *scratch, int B, int C, int O, int groups, float eps,
+                           int x_channels_last, int out_channels_last, int dtype, void *stream);
+
 
 /* ------------------------------------------------------------ calibration */
 

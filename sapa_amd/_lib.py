@@ -26,6 +26,7 @@ SIGNATURES = {
     'sapa_project_shared': [_vp, _vp, _vp, _vp, _i, _i, _i, _ll, _i, _i, _i, _vp],
     'sapa_norm_project': [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _i, _i, _i, _ll, _i, ctypes.c_float, _i, _i, _i,
                           _vp],
+    'sapa_norm_project_pair': ([_vp] * 7 + [_ll]) * 2 + [_vp, _i, _i, _i, _i, ctypes.c_float, _i, _i, _i, _vp],
     'sapa_channel_moments': [_vp, _vp, _vp, _i, _i, _ll, _i, _i, _vp],
     'sapa_channel_moments_static': [_vp, _vp, _i, _i, _ll, _i, _i, _vp],
     'sapa_groupnorm_fold': [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _i, _i, _i, _i, ctypes.c_float, _i, _vp],
@@ -334,30 +335,67 @@ def norm_project(x, norm, conv, channels_last_out=False, defer_bias=False):
     per-image bias [B, O]); out is channels_last for a channels_last x or with
     channels_last_out.  None if some step has no kernel for the configuration (nothing was
     launched then; the caller takes the steps one by one)."""
+    order = _norm_project_order(x, norm, conv)
+    if order is None:
+        return None
     B, C, H, W = x.shape
-    O = conv.out_channels
-    dtype = x.dtype
+    out_cl = order or bool(channels_last_out)
+    out, b_out, args = _norm_project_args(x, norm, conv, out_cl, defer_bias)
+    scratch = _norm_project_scratch(((x, conv),), order)
+    *pointers, HW = args
+    status = call_status('sapa_norm_project', x.device, *pointers[:5], scratch.data_ptr(), *pointers[5:], B, C,
+                         conv.out_channels, HW, norm.num_groups, float(norm.eps), int(order), int(out_cl), DTYPES[x.dtype])
+    return None if status == UNSUPPORTED else (out, b_out)
+
+
+def _norm_project_order(x, norm, conv):
+    """Whether x is in channels_last order, or None if sapa_norm_project does not take the operands."""
+    C = x.shape[1]
     params = [norm.weight, norm.bias, conv.weight, conv.bias]
-    if (dtype not in DTYPES or x.numel() == 0 or conv.weight.numel() != O * C
-            or any(p is not None and (p.dtype != dtype or not p.is_contiguous()) for p in params)):
+    if (x.dtype not in DTYPES or x.numel() == 0 or conv.weight.numel() != conv.out_channels * C
+            or any(p is not None and (p.dtype != x.dtype or not p.is_contiguous()) for p in params)):
         return None
     if x.is_contiguous():
-        cl = 0
-    elif x.is_contiguous(memory_format=torch.channels_last):
-        cl = 1
-    else:
-        return None
-    out_cl = 1 if (cl or channels_last_out) else 0
-    nbytes = lib().sapa_norm_project_scratch(B, C, O, H * W, cl, DTYPES[dtype])
-    scratch = torch.empty(max(nbytes, 16), dtype=torch.uint8, device=x.device)
-    out = torch.empty(B, O, H, W, dtype=dtype, device=x.device,
+        return False
+    return True if x.is_contiguous(memory_format=torch.channels_last) else None
+
+
+def _norm_project_args(x, norm, conv, out_cl, defer_bias):
+    """(out, per-image bias or None, the feature's arguments)"""
+    B, _, H, W = x.shape
+    O = conv.out_channels
+    out = torch.empty(B, O, H, W, dtype=x.dtype, device=x.device,
                       memory_format=torch.channels_last if out_cl else torch.contiguous_format)
-    b_out = torch.empty(B, O, dtype=dtype, device=x.device) if defer_bias else None
-    status = call_status(
-        'sapa_norm_project', x.device, x.data_ptr(), ptr(norm.weight), ptr(norm.bias), conv.weight.data_ptr(),
-        ptr(conv.bias), scratch.data_ptr(), out.data_ptr(), ptr(b_out), B, C, O, H * W, norm.num_groups,
-        float(norm.eps), cl, out_cl, DTYPES[dtype])
-    return None if status == UNSUPPORTED else (out, b_out)
+    b_out = torch.empty(B, O, dtype=x.dtype, device=x.device) if defer_bias else None
+    return out, b_out, (x.data_ptr(), ptr(norm.weight), ptr(norm.bias), conv.weight.data_ptr(), ptr(conv.bias),
+                        out.data_ptr(), ptr(b_out), H * W)
+
+
+def _norm_project_scratch(features, order):
+    nbytes = 0
+    for x, conv in features:
+        B, C, H, W = x.shape
+        nbytes += lib().sapa_norm_project_scratch(B, C, conv.out_channels, H * W, int(order), DTYPES[x.dtype])
+    return torch.empty(max(nbytes, 16), dtype=torch.uint8, device=features[0][0].device)
+
+
+def norm_project_pair(y, norm_y, conv_y, x, norm_x, conv_x, channels_last_out=False, defer_bias_y=False):
+    """norm_project of two features whose norms and convolutions are alike, with their moments and
+    their folds in one launch each: ((out, bias or None), out), or None (nothing launched)."""
+    order = _norm_project_order(y, norm_y, conv_y)
+    if (order is None or order != _norm_project_order(x, norm_x, conv_x) or y.dtype != x.dtype or y.device != x.device
+            or y.shape[:2] != x.shape[:2] or conv_y.out_channels != conv_x.out_channels
+            or norm_y.num_groups != norm_x.num_groups or norm_y.eps != norm_x.eps):
+        return None
+    out_cl = order or bool(channels_last_out)
+    out_y, bias_y, args_y = _norm_project_args(y, norm_y, conv_y, out_cl, defer_bias_y)
+    out_x, _, args_x = _norm_project_args(x, norm_x, conv_x, out_cl, False)
+    scratch = _norm_project_scratch(((y, conv_y), (x, conv_x)), order)
+    B, C = y.shape[:2]
+    status = call_status('sapa_norm_project_pair', y.device, *args_y, *args_x, scratch.data_ptr(), B, C,
+                         conv_y.out_channels, norm_y.num_groups, float(norm_y.eps), int(order), int(out_cl),
+                         DTYPES[y.dtype])
+    return None if status == UNSUPPORTED else ((out_y, bias_y), out_x)
 
 
 def project_nchw(x, weight, bias=None, channels_last_out=False):

@@ -827,36 +827,67 @@ long long sapa_norm_project_scratch(int B, int C, int O, long long HW, int x_cha
            round256((long long)B * O * C * esize_of(dtype)) + round256((long long)B * O * esize_of(dtype));
 }
 
+namespace {
+// one feature of a norm_project call
+struct NormProject {
+    const void *x, *gamma, *beta, *weight, *bias;
+    void *out, *bias_out;
+    long long HW;
+};
+
+int norm_project(const NormProject *f, int n, void *scratch, int B, int C, int O, int groups, float eps,
+                 int x_channels_last, int out_channels_last, int dtype, hipStream_t st) {
+    if (!dtype_ok(dtype) || B < 0 || C <= 0 || O <= 0 || groups <= 0) return SAPA_ERR_INVALID_ARGUMENT;
+    for (int i = 0; i < n; ++i) {
+        if (f[i].HW <= 0) return SAPA_ERR_INVALID_ARGUMENT;
+        if ((long long)B * f[i].HW * (C > O ? C : O) >= kMaxElems) return SAPA_ERR_TOO_LARGE;
+    }
+    if (B == 0) return SAPA_OK;
+    for (int i = 0; i < n; ++i)
+        if (!f[i].x || !f[i].weight || !scratch || !f[i].out) return SAPA_ERR_INVALID_ARGUMENT;
+    // nothing is launched unless every step has a kernel for the configuration
+    if (dtype == SAPA_F64 || C % groups != 0 || C > 8192 || (uintptr_t)scratch % 16 != 0) return SAPA_ERR_UNSUPPORTED;
+    NormFold nf[2] = {};
+    char *p = (char *)scratch;
+    for (int i = 0; i < n; ++i) {
+        if (!project_supported(C, O, (long)f[i].HW, x_channels_last != 0, out_channels_last != 0, dtype) ||
+            ((uintptr_t)f[i].x | (uintptr_t)f[i].out) % 16 != 0)
+            return SAPA_ERR_UNSUPPORTED;
+        char *next = p + sapa_norm_project_scratch(B, C, O, f[i].HW, x_channels_last, dtype);
+        nf[i] = NormFold{f[i].x, p, f[i].gamma, f[i].beta, f[i].weight, f[i].bias, nullptr, nullptr, (long)f[i].HW};
+        p += round256(channel_moments_workspace(B, C, (long)f[i].HW, x_channels_last != 0));
+        nf[i].w_out = p;
+        p += round256((long long)B * O * C * esize_of(dtype));
+        nf[i].b_out = f[i].bias_out ? f[i].bias_out : (void *)p;
+        p = next;
+    }
+    hipError_t e = norm_fold_launch(nf, n, B, C, O, groups, eps, x_channels_last != 0, dtype, st);
+    for (int i = 0; i < n && e == hipSuccess; ++i) {
+        const void *b_b = f[i].bias_out ? nullptr : nf[i].b_out;
+        e = x_channels_last ? project_nhwc_launch(f[i].x, nf[i].w_out, b_b, f[i].out, B, C, O, (long)f[i].HW, dtype, st)
+                            : project_nchw_launch(f[i].x, nf[i].w_out, b_b, f[i].out, B, C, O, (long)f[i].HW,
+                                                  out_channels_last, dtype, st);
+    }
+    if (e == hipErrorNotSupported) return SAPA_ERR_UNSUPPORTED;
+    return finish(e);
+}
+}  // namespace
+
 int sapa_norm_project(const void *x, const void *gamma, const void *beta, const void *weight, const void *bias,
                       void *scratch, void *out, void *bias_out, int B, int C, int O, long long HW, int groups,
                       float eps, int x_channels_last, int out_channels_last, int dtype, void *stream) {
-    if (!dtype_ok(dtype) || B < 0 || C <= 0 || O <= 0 || HW <= 0 || groups <= 0) return SAPA_ERR_INVALID_ARGUMENT;
-    if ((long long)B * HW * (C > O ? C : O) >= kMaxElems) return SAPA_ERR_TOO_LARGE;
-    if (B == 0) return SAPA_OK;
-    if (!x || !weight || !scratch || !out) return SAPA_ERR_INVALID_ARGUMENT;
-    // nothing is launched unless every step has a kernel for the configuration
-    if (dtype == SAPA_F64 || C % groups != 0 || C > 8192 ||
-        !project_supported(C, O, (long)HW, x_channels_last != 0, out_channels_last != 0, dtype) ||
-        ((uintptr_t)x | (uintptr_t)out | (uintptr_t)scratch) % 16 != 0)
-        return SAPA_ERR_UNSUPPORTED;
-    char *p = (char *)scratch;
-    void *ws = p;
-    p += round256(channel_moments_workspace(B, C, (long)HW, x_channels_last != 0));
-    void *w_b = p;
-    p += round256((long long)B * O * C * esize_of(dtype));
-    void *b_b = bias_out ? bias_out : (void *)p;
-    hipStream_t st = (hipStream_t)stream;
-    // (the projections' channel counts end at 512: the final sums and the fold are one launch)
-    hipError_t e = channel_moments_launch(x, ws, nullptr, B, C, (long)HW, x_channels_last != 0, dtype, st);
-    if (e == hipSuccess)
-        e = moments_fold_launch(x, ws, gamma, beta, weight, bias, w_b, b_b, B, C, O, groups, eps, (long)HW,
-                                x_channels_last != 0, dtype, st);
-    if (e == hipSuccess)
-        e = x_channels_last ? project_nhwc_launch(x, w_b, bias_out ? nullptr : b_b, out, B, C, O, (long)HW, dtype, st)
-                            : project_nchw_launch(x, w_b, bias_out ? nullptr : b_b, out, B, C, O, (long)HW,
-                                                  out_channels_last, dtype, st);
-    if (e == hipErrorNotSupported) return SAPA_ERR_UNSUPPORTED;
-    return finish(e);
+    const NormProject f{x, gamma, beta, weight, bias, out, bias_out, HW};
+    return norm_project(&f, 1, scratch, B, C, O, groups, eps, x_channels_last, out_channels_last, dtype, (hipStream_t)stream);
+}
+
+int sapa_norm_project_pair(const void *x0, const void *gamma0, const void *beta0, const void *weight0, const void *bias0,
+                           void *out0, void *bias_out0, long long HW0, const void *x1, const void *gamma1,
+                           const void *beta1, const void *weight1, const void *bias1, void *out1, void *bias_out1,
+                           long long HW1, void *scratch, int B, int C, int O, int groups, float eps,
+                           int x_channels_last, int out_channels_last, int dtype, void *stream) {
+    const NormProject f[2] = {{x0, gamma0, beta0, weight0, bias0, out0, bias_out0, HW0},
+                              {x1, gamma1, beta1, weight1, bias1, out1, bias_out1, HW1}};
+    return norm_project(f, 2, scratch, B, C, O, groups, eps, x_channels_last, out_channels_last, dtype, (hipStream_t)stream);
 }
 
 int sapa_layout_copy(const void *src, void *dst, int B, int C, long long HW, int to_channels_last,

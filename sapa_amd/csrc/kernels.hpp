@@ -79,9 +79,15 @@ hipError_t channel_moments_static_launch(const void *x, float *mean_var, int B, 
 hipError_t groupnorm_fold_launch(const float *mean_var, const void *gamma, const void *beta,
                                  const void *w, const void *bias, void *w_out, void *b_out, int B,
                                  int C, int O, int G, float eps, int dtype, hipStream_t st);
-hipError_t moments_fold_launch(const void *x, const void *partial, const void *gamma, const void *beta, const void *w,
-                               const void *bias, void *w_out, void *b_out, int B, int C, int O, int G, float eps,
-                               long HW, bool channels_last, int dtype, hipStream_t st);
+struct NormFold {
+    const void *x;
+    void *workspace;
+    const void *gamma, *beta, *w, *bias;
+    void *w_out, *b_out;
+    long HW;
+};
+hipError_t norm_fold_launch(const NormFold *f, int n, int B, int C, int O, int G, float eps, bool channels_last,
+                            int dtype, hipStream_t st);
 
 // sapa_stream.hip: a kernel that only moves bytes, `units` units that each read one
 // contiguous run of reads * 4 KiB and write one of writes * 4 KiB, `reps` consecutive units per

@@ -672,9 +672,12 @@ hipError_t sapa_b_bwd16_launch(const void *q, const void *key, const void *value
     if (((uintptr_t)key | (uintptr_t)value | (uintptr_t)grad_key | (uintptr_t)grad_value) % 4 != 0 ||
         ((uintptr_t)q | (uintptr_t)grad_out | (uintptr_t)grad_q | (uintptr_t)stats) % 16 != 0)
         return hipErrorNotSupported;
-    // beyond the 256 MB memory-side cache the pixel kernel's hi-res traffic is non-temporal, as the
-    // forward kernel's
-    const bool stream = 2L * ((long)B * H * W * (5L * d + 5L * C)) > (256L << 20);
+    // Beyond the 256 MB memory-side cache the pixel kernel's hi-res traffic is non-temporal, as the
+    // forward kernel's -- where the rows of a tile of 8 blocks are whole 128-byte lines (W a multiple
+    // of 32); else two workgroups use parts of a line and the caches serve the second (both gradient
+    // kernels, B=16, C=256, d=64, bf16: 96x160 621 us streamed, 643 not; 100x168 728 and 710; 168x100
+    // 802 and 765).
+    const bool stream = W % 32 == 0 && 2L * ((long)B * H * W * (5L * d + 5L * C)) > (256L << 20);
     float *f = (float *)stats;
     if (dtype == 2)
         return stream ? bwm16::launch<f16_t, true>(q, key, value, grad_out, f, grad_q, grad_key, grad_value, B, d, C, H, W, st)

@@ -69,15 +69,35 @@ __device__ __forceinline__ void block_sum2(float &a, float &b, float (*red)[2]) 
     }
 }
 
+// One feature of a launch; a launch takes one or two (of the same B and C: a module's query and key
+// features), the second's chunks behind the first's along blockIdx.x (chunks = 0: none).
+template <typename T> struct Feature {
+    const T *x;
+    float *part;
+    long HW, seg;
+    int chunks;
+};
+template <typename F>
+__device__ __forceinline__ F feature_of(const F &f0, const F &f1, int &chunk) {
+    chunk = blockIdx.x;
+    if (chunk < f0.chunks) return f0;
+    chunk -= f0.chunks;
+    return f1;
+}
+
 // contiguous layout: block = (chunk, image * C + channel); VEC elements per load
 // (1: any alignment)
 template <typename T, int VEC>
 __global__ void __launch_bounds__(256)
-partial_nchw_kernel(const T *__restrict__ x, float *__restrict__ part, long HW, long seg, int chunks) {
+partial_nchw_kernel(Feature<T> f0, Feature<T> f1) {
     __shared__ float red[4][2];
     const long bc = blockIdx.y;
-    const int chunk = blockIdx.x;
-    const T *xc = x + bc * HW;
+    int chunk;
+    const Feature<T> f = feature_of(f0, f1, chunk);
+    const long HW = f.HW, seg = f.seg;
+    const int chunks = f.chunks;
+    float *const part = f.part;
+    const T *xc = f.x + bc * HW;
     const float shift = (float)xc[0];
     const long lo = chunk * seg, hi = lo + seg < HW ? lo + seg : HW;
     float s1 = 0.f, s2 = 0.f;
@@ -113,10 +133,15 @@ partial_nchw_kernel(const T *__restrict__ x, float *__restrict__ part, long HW, 
 // CPT channels); SAPA_MOMENTS_UNROLL pixels per thread are in flight at a time
 template <typename T, int CPT>
 __global__ void __launch_bounds__(256)
-partial_nhwc_kernel(const T *__restrict__ x, float *__restrict__ part, int C, long HW, long seg,
-                    int chunks) {
+partial_nhwc_kernel(Feature<T> f0, Feature<T> f1, int C) {
     __shared__ float red[256][2 * CPT];
-    const int b = blockIdx.y, chunk = blockIdx.x;
+    const int b = blockIdx.y;
+    int chunk;
+    const Feature<T> f = feature_of(f0, f1, chunk);
+    const long HW = f.HW, seg = f.seg;
+    const int chunks = f.chunks;
+    const T *const x = f.x;
+    float *const part = f.part;
     const int nq = C / CPT, npl = 256 / nq;            // channel groups, pixel lanes
     const int quad = threadIdx.x % nq, pl = threadIdx.x / nq;
     const T *xb = x + (long)b * HW * C + CPT * quad;
@@ -217,37 +242,41 @@ static void chunking_for(long HW, int B, int C, bool cl, long &seg, int &chunks)
     else chunking(HW, (long)B * C, 4096, 512, seg, chunks);
 }
 
+// the partial sums of one or two features (x1 null: one)
+template <typename T>
+static void launch_partial(const T *x0, float *ws0, long HW0, const T *x1, float *ws1, long HW1, int B, int C, bool cl,
+                           hipStream_t st) {
+    Feature<T> f0{x0, ws0, HW0, 0, 0}, f1{x1, ws1, HW1, 0, 0};
+    chunking_for(HW0, B, C, cl, f0.seg, f0.chunks);
+    if (x1) chunking_for(HW1, B, C, cl, f1.seg, f1.chunks);
+    const int chunks = f0.chunks + f1.chunks;
+    const bool aligned = ((uintptr_t)x0 | (uintptr_t)x1) % 16 == 0;
+    if (cl) {
+        // 16 bytes per lane where the channel count and the alignment allow it
+        constexpr int WIDE = 16 / (int)sizeof(T);
+        if (WIDE == 8 && C % 8 == 0 && aligned)
+            hipLaunchKernelGGL((partial_nhwc_kernel<T, WIDE>), dim3(chunks, B), dim3(256), 0, st, f0, f1, C);
+        else
+            hipLaunchKernelGGL((partial_nhwc_kernel<T, 4>), dim3(chunks, B), dim3(256), 0, st, f0, f1, C);
+    } else {
+        constexpr int VEC = 16 / (int)sizeof(T);
+        const dim3 grid(chunks, B * C);
+        if (HW0 % VEC == 0 && (!x1 || HW1 % VEC == 0) && aligned)
+            hipLaunchKernelGGL((partial_nchw_kernel<T, VEC>), grid, dim3(256), 0, st, f0, f1);
+        else
+            hipLaunchKernelGGL((partial_nchw_kernel<T, 1>), grid, dim3(256), 0, st, f0, f1);
+    }
+}
+
 template <typename T>
 static hipError_t launch_t(const T *x, float *ws, float *mean_var, int B, int C, long HW, bool cl,
                            hipStream_t st) {
-    // mean_var null: the partial sums only
+    launch_partial<T>(x, ws, HW, nullptr, nullptr, 0, B, C, cl, st);
     long seg;
     int chunks;
-    if (cl) {
-        chunking_for(HW, B, C, true, seg, chunks);
-        // 16 bytes per lane where the channel count and the alignment allow it
-        constexpr int WIDE = 16 / (int)sizeof(T);
-        if (WIDE == 8 && C % 8 == 0 && (uintptr_t)x % 16 == 0)
-            hipLaunchKernelGGL((partial_nhwc_kernel<T, WIDE>), dim3(chunks, B), dim3(256), 0, st, x, ws, C,
-                               HW, seg, chunks);
-        else
-            hipLaunchKernelGGL((partial_nhwc_kernel<T, 4>), dim3(chunks, B), dim3(256), 0, st, x, ws, C,
-                               HW, seg, chunks);
-        if (mean_var)
-            hipLaunchKernelGGL((finish_kernel<T, true>), dim3(((long)B * C + 255) / 256), dim3(256), 0, st, x,
-                           ws, mean_var, B, C, HW, chunks);
-    } else {
-        chunking_for(HW, B, C, false, seg, chunks);
-        constexpr int VEC = 16 / (int)sizeof(T);
-        const dim3 grid(chunks, B * C);
-        if (HW % VEC == 0 && (uintptr_t)x % 16 == 0)
-            hipLaunchKernelGGL((partial_nchw_kernel<T, VEC>), grid, dim3(256), 0, st, x, ws, HW, seg, chunks);
-        else
-            hipLaunchKernelGGL((partial_nchw_kernel<T, 1>), grid, dim3(256), 0, st, x, ws, HW, seg, chunks);
-        if (mean_var)
-            hipLaunchKernelGGL((finish_kernel<T, false>), dim3(((long)B * C + 255) / 256), dim3(256), 0, st, x,
-                           ws, mean_var, B, C, HW, chunks);
-    }
+    chunking_for(HW, B, C, cl, seg, chunks);
+    auto kern = cl ? finish_kernel<T, true> : finish_kernel<T, false>;
+    hipLaunchKernelGGL(kern, dim3(((long)B * C + 255) / 256), dim3(256), 0, st, x, ws, mean_var, B, C, HW, chunks);
     return hipGetLastError();
 }
 
@@ -309,19 +338,35 @@ fold_kernel(const float *__restrict__ mean_var, const T *__restrict__ gamma,
 // us for the two kernels and 5 for this one at B=8, C=256, 16x16 in bf16, 6 + 8 and 10 at
 // B=16, C=256, 200x336 in channels-last bf16 (128 chunks).
 constexpr int kFoldChannels = 2048;                // 4 floats of LDS each
+// One or two features and their projections per launch: the second's blocks of rows behind the
+// first's `blocks0` along blockIdx.y.  (Two at once: the smaller feature's latencies lie beside the
+// other's; module forward B=8, C=256, 16x16 in bf16 57 -> 47 us, B=16, 100x168 channels-last 492 -> 474.)
+template <typename T> struct Fold {
+    const T *x;
+    const float *part;
+    const T *gamma, *beta, *w, *bias;
+    T *w_out, *b_out;
+    long HW;
+    int chunks, parts;
+};
 template <typename T, bool CL>
 __global__ void __launch_bounds__(1024)
-finish_fold_kernel(const T *__restrict__ x, const float *__restrict__ part, const T *__restrict__ gamma,
-                   const T *__restrict__ beta, const T *__restrict__ w, const T *__restrict__ bias,
-                   T *__restrict__ w_out, T *__restrict__ b_out, int C, int O, int G, float eps, long HW,
-                   int chunks, int parts, int rows) {
+finish_fold_kernel(Fold<T> f0, Fold<T> f1, int blocks0, int C, int O, int G, float eps, int rows) {
+    const bool second = (int)blockIdx.y >= blocks0;
+    const Fold<T> f = second ? f1 : f0;
+    const int block = (int)blockIdx.y - (second ? blocks0 : 0), chunks = f.chunks, parts = f.parts;
+    const long HW = f.HW;
+    const T *__restrict__ x = f.x, *__restrict__ gamma = f.gamma, *__restrict__ beta = f.beta, *__restrict__ w = f.w,
+            *__restrict__ bias = f.bias;
+    const float *__restrict__ part = f.part;
+    T *__restrict__ w_out = f.w_out, *__restrict__ b_out = f.b_out;
     typedef float f32x2 __attribute__((ext_vector_type(2)));
     extern __shared__ float sh[];                  // mean[C], var[C], scale[C], shift[C]; before: sums[parts][C][2]
     float *mean = sh, *var = sh + C, *scale = sh + 2 * C, *shift = sh + 3 * C;
     f32x2 *sums = (f32x2 *)(sh + 4 * C);
     const int nt = blockDim.x, nw = nt / 64, b = blockIdx.x, per = C / G;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int o0 = blockIdx.y * rows + wave, o1 = (int)(blockIdx.y + 1) * rows < O ? (int)(blockIdx.y + 1) * rows : O;
+    const int o0 = block * rows + wave, o1 = (block + 1) * rows < O ? (block + 1) * rows : O;
     float first[4];                                // the first 256 channels of the wave's first row
 #pragma unroll
     for (int u = 0; u < 4; ++u) first[u] = o0 < o1 && lane + 64 * u < C ? (float)w[(long)o0 * C + lane + 64 * u] : 0.f;
@@ -407,23 +452,31 @@ finish_fold_kernel(const T *__restrict__ x, const float *__restrict__ part, cons
 }
 
 template <typename T>
-static hipError_t finish_fold_t(const void *x, const float *part, const void *gamma, const void *beta, const void *w,
-                                const void *bias, void *w_out, void *b_out, int B, int C, int O, int G, float eps,
-                                long HW, bool cl, hipStream_t st) {
-    long seg;
-    int chunks;
-    chunking_for(HW, B, C, cl, seg, chunks);
+static hipError_t norm_fold_t(const NormFold *f, int n, int B, int C, int O, int G, float eps, bool cl, hipStream_t st) {
+    const bool two = n == 2;
+    launch_partial<T>((const T *)f[0].x, (float *)f[0].workspace, f[0].HW, two ? (const T *)f[1].x : nullptr,
+                      two ? (float *)f[1].workspace : nullptr, two ? f[1].HW : 0, B, C, cl, st);
+    Fold<T> a[2] = {};
+    bool many = false;
+    for (int i = 0; i < n; ++i) {
+        long seg;
+        a[i] = Fold<T>{(const T *)f[i].x, (const float *)f[i].workspace, (const T *)f[i].gamma, (const T *)f[i].beta,
+                       (const T *)f[i].w, (const T *)f[i].bias, (T *)f[i].w_out, (T *)f[i].b_out, f[i].HW, 0, 1};
+        chunking_for(f[i].HW, B, C, cl, seg, a[i].chunks);
+        many |= a[i].chunks > 16;
+    }
     // few chunks: a thread per channel, a row per wave of 4; else up to 1024 threads that share a
     // channel's chunks in runs of 16 or more, and 16 rows for what they fetch
-    const bool many = chunks > 16;
-    const int nt = many ? 1024 : 256, rows = many ? 16 : 4;
-    int parts = many && C < nt ? nt / C : 1;
-    if (parts > chunks / 16) parts = chunks / 16 < 1 ? 1 : chunks / 16;
+    const int nt = many ? 1024 : 256, rows = many ? 16 : 4, blocks = (O + rows - 1) / rows;
+    int parts = 1;
+    for (int i = 0; i < n; ++i) {
+        if (many && C < nt) a[i].parts = nt / C;
+        if (a[i].parts > a[i].chunks / 16) a[i].parts = a[i].chunks / 16 < 1 ? 1 : a[i].chunks / 16;
+        if (a[i].parts > parts) parts = a[i].parts;
+    }
     const size_t lds = (size_t)(4 * C + (parts > 1 ? 2 * parts * C : 0)) * sizeof(float);
     auto kern = cl ? finish_fold_kernel<T, true> : finish_fold_kernel<T, false>;
-    hipLaunchKernelGGL(kern, dim3(B, (O + rows - 1) / rows), dim3(nt), lds, st, (const T *)x, part,
-                       (const T *)gamma, (const T *)beta, (const T *)w, (const T *)bias, (T *)w_out, (T *)b_out, C, O,
-                       G, eps, HW, chunks, parts, rows);
+    hipLaunchKernelGGL(kern, dim3(B, n * blocks), dim3(nt), lds, st, a[0], a[1], blocks, C, O, G, eps, rows);
     return hipGetLastError();
 }
 
@@ -447,20 +500,19 @@ long channel_moments_workspace(int B, int C, long HW, bool channels_last) {
     return (long)B * C * chunks * 2 * (long)sizeof(float);
 }
 
+static bool channel_moments_served(const void *x, int B, int C, bool channels_last, int dtype) {
+    if (!channels_last) return (long)B * C <= 65535;
+    const int esize = dtype == 0 ? 4 : 2;
+    return C % 4 == 0 && C <= 1024 && (uintptr_t)x % (4 * esize) == 0 && B <= 65535;
+}
+
 // x: [B, C, HW] contiguous or [B, HW, C] (channels_last), f32 / f16 / bf16;
-// mean_var: [B, C, 2] fp32 (null: the partial sums stay in the workspace, for
-// moments_fold_launch).  Channels-last needs C % 4 == 0, C <= 1024 and x
+// mean_var: [B, C, 2] fp32.  Channels-last needs C % 4 == 0, C <= 1024 and x
 // aligned to 4 elements; the contiguous layout B * C <= 65535.
 // hipErrorNotSupported otherwise.
 hipError_t channel_moments_launch(const void *x, void *workspace, float *mean_var, int B, int C,
                                   long HW, bool channels_last, int dtype, hipStream_t st) {
-    if (channels_last) {
-        const int esize = dtype == 0 ? 4 : 2;
-        if (C % 4 != 0 || C > 1024 || (uintptr_t)x % (4 * esize) != 0 || B > 65535)
-            return hipErrorNotSupported;
-    } else if ((long)B * C > 65535) {
-        return hipErrorNotSupported;
-    }
+    if (!channel_moments_served(x, B, C, channels_last, dtype)) return hipErrorNotSupported;
     float *ws = (float *)workspace;
     switch (dtype) {
         case 0: return moments::launch_t((const float *)x, ws, mean_var, B, C, HW, channels_last, st);
@@ -542,17 +594,19 @@ hipError_t groupnorm_fold_launch(const float *mean_var, const void *gamma, const
     }
 }
 
-// channel_moments_launch's finish and groupnorm_fold_launch in one: `partial` is the workspace of a
-// channel_moments_launch without mean_var on the same x.  C % G == 0, C <= 2048.
-hipError_t moments_fold_launch(const void *x, const void *partial, const void *gamma, const void *beta, const void *w,
-                               const void *bias, void *w_out, void *b_out, int B, int C, int O, int G, float eps,
-                               long HW, bool channels_last, int dtype, hipStream_t st) {
-    if (G < 1 || C % G != 0 || C > moments::kFoldChannels) return hipErrorNotSupported;
-    const float *p = (const float *)partial;
+// Moments and folded projection weights of one feature, or of two with the same B, C, O, G and eps,
+// in two launches; f[i].workspace: channel_moments_workspace bytes each.  What
+// channel_moments_launch and groupnorm_fold_launch require holds for each; C <= 2048.
+// hipErrorNotSupported otherwise, nothing launched.
+hipError_t norm_fold_launch(const NormFold *f, int n, int B, int C, int O, int G, float eps, bool channels_last,
+                            int dtype, hipStream_t st) {
+    if (n < 1 || n > 2 || G < 1 || C % G != 0 || C > moments::kFoldChannels) return hipErrorNotSupported;
+    for (int i = 0; i < n; ++i)
+        if (!channel_moments_served(f[i].x, B, C, channels_last, dtype)) return hipErrorNotSupported;
     switch (dtype) {
-        case 0: return moments::finish_fold_t<float>(x, p, gamma, beta, w, bias, w_out, b_out, B, C, O, G, eps, HW, channels_last, st);
-        case 2: return moments::finish_fold_t<f16_t>(x, p, gamma, beta, w, bias, w_out, b_out, B, C, O, G, eps, HW, channels_last, st);
-        case 3: return moments::finish_fold_t<bf16_t>(x, p, gamma, beta, w, bias, w_out, b_out, B, C, O, G, eps, HW, channels_last, st);
+        case 0: return moments::norm_fold_t<float>(f, n, B, C, O, G, eps, channels_last, st);
+        case 2: return moments::norm_fold_t<f16_t>(f, n, B, C, O, G, eps, channels_last, st);
+        case 3: return moments::norm_fold_t<bf16_t>(f, n, B, C, O, G, eps, channels_last, st);
         default: return hipErrorNotSupported;
     }
 }

@@ -115,7 +115,8 @@ def norm_project(x, norm, *convs, channels_last=False, defer_bias=False):
     for conv in convs:
         assert conv.kernel_size == (1, 1) and conv.groups == 1
         O = conv.out_channels
-        if norm is None and channels_last and not defer_bias and x.is_cuda and not torch.is_grad_enabled():
+        if (norm is None and channels_last and not defer_bias and x.is_cuda and not torch.is_grad_enabled()
+                and not torch.is_autocast_enabled('cuda')):
             out = _lib.project_shared(x, conv.weight, conv.bias, channels_last_out=True)
             if out is not None:
                 outs.append(out)
@@ -168,6 +169,20 @@ def norm_project(x, norm, *convs, channels_last=False, defer_bias=False):
     return outs
 
 
+def norm_project_pair(y, norm_y, conv_y, x, norm_x, conv_x, channels_last=False, defer_bias=False):
+    """norm_project of the query and the key feature: at inference on the GPU, where both go the
+    same way, as one library call; else one after the other.  (q or (q, bias), k)."""
+    if (norm_y is not None and norm_x is not None and y.is_cuda and x.is_cuda and not torch.is_grad_enabled()
+            and all(c.kernel_size == (1, 1) and c.groups == 1 for c in (conv_y, conv_x))
+            and (channels_last or (y.is_contiguous() and x.is_contiguous()))):
+        res = _lib.norm_project_pair(y, norm_y, conv_y, x, norm_x, conv_x, channels_last, defer_bias)
+        if res is not None:
+            return (res[0] if defer_bias else res[0][0]), res[1]
+    (q,) = norm_project(y, norm_y, conv_y, channels_last=channels_last, defer_bias=defer_bias)
+    (k,) = norm_project(x, norm_x, conv_x, channels_last=channels_last)
+    return q, k
+
+
 def _plain(t):
     """A tensor whose memory a kernel may be given: no subclass, no functorch wrapper."""
     return type(t) in (torch.Tensor, nn.Parameter) and not torch._C._functorch.is_functorch_wrapped_tensor(t)
@@ -179,13 +194,15 @@ def _project(conv, x):
     GEMM and the pass that adds the bias took 120 us for 128 outputs); everything else -- gradients,
     autocast, tracing, tensor subclasses, hooks, another kind of convolution in the module's place --
     is the module's call."""
-    if (not torch.is_grad_enabled() and type(conv) is nn.Conv2d and conv.kernel_size == (1, 1)
+    if (not torch.is_grad_enabled() and not torch.compiler.is_compiling()
+            and type(conv) is nn.Conv2d and conv.kernel_size == (1, 1)
             and conv.stride == (1, 1) and conv.padding == (0, 0) and conv.groups == 1
             and x.dim() == 4 and x.is_cuda and x.is_contiguous()
             and not (conv._forward_hooks or conv._forward_pre_hooks or nn.modules.module._global_forward_hooks
                      or nn.modules.module._global_forward_pre_hooks)
             and not torch.is_autocast_enabled('cuda') and not torch.jit.is_tracing()
-            and torch.autograd.forward_ad._current_level < 0 and torch._C._len_torch_dispatch_stack() == 0
+            and torch.autograd.forward_ad._current_level < 0
+            and torch._C._len_torch_dispatch_stack() == 0 and torch._C._len_torch_function_stack() == 0
             and all(_plain(t) for t in (x, conv.weight) + (() if conv.bias is None else (conv.bias,)))):
         out = _lib.project_shared(x, conv.weight, conv.bias)
         if out is not None:
@@ -231,13 +248,12 @@ class SAPA(nn.Module):
             ny, nx = (self.norm_y, self.norm_x) if self.norm else (None, None)
             # the query's bias goes into the fused operator instead of a pass of its
             # own over the hi-res query tensor
-            ((q, q_bias),) = norm_project(y, ny, self.q, channels_last=True, defer_bias=True)
+            (q, q_bias), k = norm_project_pair(y, ny, self.q, x, nx, self.k, channels_last=True, defer_bias=True)
             if not self.fused:
                 q, q_bias = q.add_(q_bias[:, :, None, None]), None
-            (k,) = norm_project(x, nx, self.k, channels_last=True)
             return self.attention(q, k, in_memory_order(x, torch.channels_last), q_bias)
         if self.norm and self.fold_norm:
-            (q,), (k,) = norm_project(y, self.norm_y, self.q), norm_project(x, self.norm_x, self.k)
+            q, k = norm_project_pair(y, self.norm_y, self.q, x, self.norm_x, self.k)
             return self.attention(q, k, x)
         x_ = self.norm_x(x) if self.norm else x
         if self.norm:

@@ -161,3 +161,31 @@ def test_small_separate_operators(dtype, B, d, C, H, W):
     want = c_oracle.qk(q.float(), k.float(), 5, 2, 'f32'), c_oracle.av(a.float(), v.float(), 5, 2, 'f32')
     for x, y in zip(got, want):
         assert torch.equal(x, y) if dtype == torch.float32 else _rel(x, y.double()) <= torch.finfo(dtype).eps / 2 / 3 ** 0.5 * 1.2
+
+
+@pytest.mark.parametrize('dtype', [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize('channels_last', [False, True])
+@pytest.mark.parametrize('B,C,O,h,w', [
+    (1, 64, 32, 2, 4),         # one chunk per feature
+    (2, 256, 64, 100, 168),    # chunks shared by several threads in one feature, a thread per channel in the other
+    (3, 512, 32, 24, 20),      # more channels than the threads of a block of few chunks
+])
+def test_norm_project_of_two_features(dtype, channels_last, B, C, O, h, w):
+    """sapa_norm_project_pair gives what sapa_norm_project gives for each feature.  (Where one feature
+    has many chunks the other's few are added by the same thread either way: bit for bit.)"""
+    from sapa_amd import _lib
+    g = torch.Generator(device='cuda').manual_seed(C)
+    fmt = torch.channels_last if channels_last else torch.contiguous_format
+    y, x = (torch.randn(B, C, a, b, generator=g, device='cuda').add_(0.3).to(dtype).contiguous(memory_format=fmt)
+            for a, b in ((2 * h, 2 * w), (h, w)))
+    norms = [torch.nn.GroupNorm(32, C).cuda().to(dtype) for _ in 'yx']
+    convs = [torch.nn.Conv2d(C, O, 1).cuda().to(dtype) for _ in 'yx']
+    with torch.no_grad():
+        for m in norms:
+            m.weight.add_(torch.randn(C, generator=g, device='cuda').to(dtype) * 0.1)
+        for defer in (False, True):
+            (q, qb), k = _lib.norm_project_pair(y, norms[0], convs[0], x, norms[1], convs[1], channels_last, defer)
+            want_q, want_qb = _lib.norm_project(y, norms[0], convs[0], channels_last, defer)
+            want_k, _ = _lib.norm_project(x, norms[1], convs[1], channels_last)
+            assert torch.equal(q, want_q) and torch.equal(k, want_k)
+            assert qb is None and want_qb is None if not defer else torch.equal(qb, want_qb)
