@@ -12,7 +12,7 @@
 //     contiguous run of memory, fetched as 16 bytes per lane with the next
 //     tile's loads in flight during the current tile's arithmetic, and passed
 //     through a wave-private LDS tile (rows padded the same way) into the A
-//     operand layout of v_mfma_f32_16x16x16 (row = pixel);
+//     operand layout of v_mfma_f32_16x16x32 (row = pixel);
 //   * the 16 x 16 results per output tile go back through LDS, so that a lane
 //     stores 16 contiguous bytes and the wave one contiguous run of 32 O bytes.
 //
@@ -62,22 +62,6 @@ typedef float f32x4 __attribute__((ext_vector_type(4)));
 // and an instruction that overwrites its data registers, and the first dword of a piece was then
 // now and then stored with the overwriting value (once a second workgroup on the CU kept the store
 // waiting: 16-bit planes, 16 images of 200 x 336 pixels, 5000 of 69 M results).
-
-template <typename T> struct Mma;
-template <> struct Mma<f16_t> {
-    typedef _Float16 v4 __attribute__((ext_vector_type(4)));
-    static __device__ __forceinline__ f32x4 run(u32x2 a, u32x2 b, f32x4 c) {
-        return __builtin_amdgcn_mfma_f32_16x16x16f16(__builtin_bit_cast(v4, a), __builtin_bit_cast(v4, b),
-                                                     c, 0, 0, 0);
-    }
-};
-template <> struct Mma<bf16_t> {
-    typedef short v4 __attribute__((ext_vector_type(4)));
-    static __device__ __forceinline__ f32x4 run(u32x2 a, u32x2 b, f32x4 c) {
-        return __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(__builtin_bit_cast(v4, a),
-                                                         __builtin_bit_cast(v4, b), c, 0, 0, 0);
-    }
-};
 
 template <typename T> struct Mma32;
 template <> struct Mma32<f16_t> {
@@ -167,14 +151,16 @@ project_kernel(const T *__restrict__ x, const T *__restrict__ w, const T *__rest
 #pragma unroll
         for (int nt = 0; nt < NT; ++nt) acc[nt] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-        for (int ks = 0; ks < C / 16; ++ks) {
-            // A: pixel r16, channels 16 ks + 4 kg .. +3; B: output 16 nt + r16, same channels
-            const u32x2 a = *(const u32x2 *)(xt + r16 * RW + 8 * ks + 2 * kg);
+        for (int ks = 0; ks < C / 32; ++ks) {
+            // A: pixel r16, channels 32 ks + 8 kg .. +7; B: output 16 nt + r16, same channels.  (16-byte
+            // reads: the 16 rows of a lane group lie on different bank quads, which they do not with 8
+            // bytes and v_mfma_f32_16x16x16: 16 images of 200 x 336 and 100 x 168 pixels, 256 -> 64, 187 -> 176 us)
+            const u32x4 a = *(const u32x4 *)(xt + r16 * RW + 16 * ks + 4 * kg);
 #pragma unroll
             for (int nt = 0; nt < NT; ++nt) {
                 if (WIDE && 16 * nt >= sp.left) break;
-                const u32x2 bm = *(const u32x2 *)(wl + (16 * nt + r16) * RW + 8 * ks + 2 * kg);
-                acc[nt] = Mma<T>::run(a, bm, acc[nt]);
+                const u32x4 bm = *(const u32x4 *)(wl + (16 * nt + r16) * RW + 16 * ks + 4 * kg);
+                acc[nt] = Mma32<T>::run(a, bm, acc[nt]);
             }
         }
         // acc[nt][i]: pixel 4 kg + i, output 16 nt + r16 -> the tile again, as 16-bit
