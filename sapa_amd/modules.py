@@ -115,8 +115,7 @@ def norm_project(x, norm, *convs, channels_last=False, defer_bias=False):
     for conv in convs:
         assert conv.kernel_size == (1, 1) and conv.groups == 1
         O = conv.out_channels
-        if (norm is None and channels_last and not defer_bias and x.is_cuda and not torch.is_grad_enabled()
-                and not torch.is_autocast_enabled('cuda')):
+        if norm is None and channels_last and not defer_bias and _kernel_reads(conv, x):
             out = _lib.project_shared(x, conv.weight, conv.bias, channels_last_out=True)
             if out is not None:
                 outs.append(out)
@@ -188,22 +187,28 @@ def _plain(t):
     return type(t) in (torch.Tensor, nn.Parameter) and not torch._C._functorch.is_functorch_wrapped_tensor(t)
 
 
+def _kernel_reads(conv, x):
+    """Whether a kernel may read x and conv's parameters in the place of torch's operators: at
+    inference on the GPU, outside autocast, tracing and tensor subclasses, modes or transforms."""
+    return (x.is_cuda and not torch.is_grad_enabled() and not torch.compiler.is_compiling()
+            and not torch.is_autocast_enabled('cuda') and not torch.jit.is_tracing()
+            and torch.autograd.forward_ad._current_level < 0
+            and torch._C._len_torch_dispatch_stack() == 0 and torch._C._len_torch_function_stack() == 0
+            and all(_plain(t) for t in (x, conv.weight) + (() if conv.bias is None else (conv.bias,))))
+
+
 def _project(conv, x):
     """conv(x) for a 1x1 convolution: at inference on a contiguous GPU feature the library's streaming
     projection, which adds the bias in its epilogue (at B=8, 256 channels, 128x128 fp32 the library
     GEMM and the pass that adds the bias took 120 us for 128 outputs); everything else -- gradients,
     autocast, tracing, tensor subclasses, hooks, another kind of convolution in the module's place --
     is the module's call."""
-    if (not torch.is_grad_enabled() and not torch.compiler.is_compiling()
-            and type(conv) is nn.Conv2d and conv.kernel_size == (1, 1)
+    if (type(conv) is nn.Conv2d and conv.kernel_size == (1, 1)
             and conv.stride == (1, 1) and conv.padding == (0, 0) and conv.groups == 1
-            and x.dim() == 4 and x.is_cuda and x.is_contiguous()
+            and x.dim() == 4 and x.is_contiguous()
             and not (conv._forward_hooks or conv._forward_pre_hooks or nn.modules.module._global_forward_hooks
                      or nn.modules.module._global_forward_pre_hooks)
-            and not torch.is_autocast_enabled('cuda') and not torch.jit.is_tracing()
-            and torch.autograd.forward_ad._current_level < 0
-            and torch._C._len_torch_dispatch_stack() == 0 and torch._C._len_torch_function_stack() == 0
-            and all(_plain(t) for t in (x, conv.weight) + (() if conv.bias is None else (conv.bias,)))):
+            and _kernel_reads(conv, x)):
         out = _lib.project_shared(x, conv.weight, conv.bias)
         if out is not None:
             return out

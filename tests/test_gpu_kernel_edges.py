@@ -189,3 +189,24 @@ def test_norm_project_of_two_features(dtype, channels_last, B, C, O, h, w):
             want_k, _ = _lib.norm_project(x, norms[1], convs[1], channels_last)
             assert torch.equal(q, want_q) and torch.equal(k, want_k)
             assert qb is None and want_qb is None if not defer else torch.equal(qb, want_qb)
+
+
+@pytest.mark.parametrize('channels_last', [False, True])
+def test_plain_projection_keeps_forward_mode_tangents(channels_last):
+    """A plain projection in channels_last order of a dual feature under no_grad: the tangent is the
+    projection of the feature's tangent (linear up to the bias), within an error bound of a C-term
+    fp32 dot product."""
+    from torch.autograd import forward_ad
+    from sapa_amd.modules import norm_project
+    g = torch.Generator(device='cuda').manual_seed(0)
+    fmt = torch.channels_last if channels_last else torch.contiguous_format
+    x, t = (torch.randn(2, 64, 8, 12, generator=g, device='cuda').contiguous(memory_format=fmt) for _ in 'xt')
+    conv = torch.nn.Conv2d(64, 128, 1).cuda()
+    with torch.no_grad(), forward_ad.dual_level():
+        (out,) = norm_project(forward_ad.make_dual(x, t), None, conv, channels_last=True)
+        got = forward_ad.unpack_dual(out).tangent
+    assert got is not None
+    w = conv.weight.detach().double().reshape(128, 64)
+    want = (t.double().permute(0, 2, 3, 1) @ w.T).permute(0, 3, 1, 2)
+    mag = (t.double().abs().permute(0, 2, 3, 1) @ w.abs().T).permute(0, 3, 1, 2)
+    assert bool(((got.double() - want).abs() <= (64 + 8) * 2.0 ** -24 * mag).all())
