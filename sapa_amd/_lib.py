@@ -335,7 +335,7 @@ def norm_project(x, norm, conv, channels_last_out=False, defer_bias=False):
     per-image bias [B, O]); out is channels_last for a channels_last x or with
     channels_last_out.  None if some step has no kernel for the configuration (nothing was
     launched then; the caller takes the steps one by one)."""
-    order = _norm_project_order(x, norm, conv)
+    order = _norm_project_order(x, norm, conv, channels_last_out)
     if order is None:
         return None
     B, C, H, W = x.shape
@@ -348,16 +348,23 @@ def norm_project(x, norm, conv, channels_last_out=False, defer_bias=False):
     return None if status == UNSUPPORTED else (out, b_out)
 
 
-def _norm_project_order(x, norm, conv):
+def _norm_project_order(x, norm, conv, channels_last_out):
     """Whether x is in channels_last order, or None if sapa_norm_project does not take the operands."""
-    C = x.shape[1]
+    _, C, H, W = x.shape
     params = [norm.weight, norm.bias, conv.weight, conv.bias]
     if (x.dtype not in DTYPES or x.numel() == 0 or conv.weight.numel() != conv.out_channels * C
             or any(p is not None and (p.dtype != x.dtype or not p.is_contiguous()) for p in params)):
         return None
     if x.is_contiguous():
-        return False
+        # rows of pixels that the kernels' loads do not divide: refused there too, but only after
+        # results and scratch have been allocated here (12 us of a forward whose key feature is refused)
+        return None if H * W % _plane_step(x, channels_last_out) else False
     return True if x.is_contiguous(memory_format=torch.channels_last) else None
+
+
+def _plane_step(x, channels_last_out):
+    """What the extent of a contiguous feature's planes has to be a multiple of in the projection kernels."""
+    return 8 if x.element_size() == 2 else 1 if channels_last_out else 4
 
 
 def _norm_project_args(x, norm, conv, out_cl, defer_bias):
@@ -382,8 +389,8 @@ def _norm_project_scratch(features, order):
 def norm_project_pair(y, norm_y, conv_y, x, norm_x, conv_x, channels_last_out=False, defer_bias_y=False):
     """norm_project of two features whose norms and convolutions are alike, with their moments and
     their folds in one launch each: ((out, bias or None), out), or None (nothing launched)."""
-    order = _norm_project_order(y, norm_y, conv_y)
-    if (order is None or order != _norm_project_order(x, norm_x, conv_x) or y.dtype != x.dtype or y.device != x.device
+    order = _norm_project_order(y, norm_y, conv_y, channels_last_out)
+    if (order is None or order != _norm_project_order(x, norm_x, conv_x, channels_last_out) or y.dtype != x.dtype or y.device != x.device
             or y.shape[:2] != x.shape[:2] or conv_y.out_channels != conv_x.out_channels
             or norm_y.num_groups != norm_x.num_groups or norm_y.eps != norm_x.eps):
         return None
@@ -439,7 +446,7 @@ def project_shared(x, weight, bias=None, channels_last_out=False):
     x_cl = not x.is_contiguous()
     if x_cl and not (channels_last_out and x.is_contiguous(memory_format=torch.channels_last)):
         return None
-    if O % 8 or (not x_cl and H * W % (8 if x.element_size() == 2 else 1 if channels_last_out else 4)):
+    if O % 8 or (not x_cl and H * W % _plane_step(x, channels_last_out)):
         return None
     weight = weight.reshape(O, C).contiguous()
     if bias is not None:
