@@ -69,7 +69,7 @@ MEASURED_TRAFFIC = {
     ('fpn_small', 'fp32', 'nchw'): (137685860, 'profiles/sapa_b_fused_fpn_small_fp32.md', 'sapa_b_tiled_kernel'),
     ('segformer_16', 'fp32', 'nchw'): (11936679, 'profiles/sapa_b_mfma_fused_segformer_16_fp32.md',
                                        'sapa_b_mfma_kernel'),
-    ('stress', 'bf16', 'nchw'): (371333608, 'profiles/sapa_b_mfma_fused_stress_bf16.md', 'sapa_b_mfma_kernel'),
+    ('stress', 'bf16', 'nchw'): (355665437, 'profiles/sapa_b_wmat16_fused_stress_bf16.md', 'sapa_b_wmat16_kernel'),
     ('stress', 'fp32', 'channels_last'): (647422060, 'profiles/sapa_b_nhwc_mm_fused_stress_fp32.md',
                                           'sapa_b_nhwc_mm_kernel'),
     ('stress', 'bf16', 'channels_last'): (323264189, 'profiles/sapa_b_nhwc16_fused_stress_bf16.md',
@@ -462,7 +462,7 @@ def main():
                 torch.autograd.grad(y, leaves, go)
         else:
             def step():
-                y = sapa_amd.sapa_fused(q, key, v, K, s, save_attention=not args.recompute_attention)
+                y = sapa_amd.sapa_fused(q, key, v, K, s, save_attention=False if args.recompute_attention else None)
                 torch.autograd.grad(y, leaves, go)
 
     settle = {'ms': args.settle_ms, 'launches': 0}
