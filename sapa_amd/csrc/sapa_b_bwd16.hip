@@ -519,14 +519,11 @@ bwd_cell_kernel(const T *__restrict__ q, const T *__restrict__ key, const T *__r
         stage(j + CBUF);
     };
 
-#pragma unroll
-    for (int j = 0; j < CBUF - 1; ++j) stage(j);
-    next(-1, 0);
-
     // The three stats planes of the staged children, [16 rows][72] each, loaded straight into LDS in
     // front of everything else (fetched into registers between the products they cost a memory latency
-    // each, with nothing else to run meanwhile); zeros outside the image, so that children there have
-    // weight 0.  The first two planes lie where results will go later.
+    // each, with nothing else to run meanwhile): the wait for chunk 0 covers them, however few chunks
+    // there are.  Zeros outside the image, so that children there have weight 0.  The first two planes
+    // lie where results will go later.
     if (wave < 15) {
         const int k = wave / 5, slot = wave % 5 * 64 + lane, r = slot / (2 * CPC);
         const int cy = 8 * (J - 1) + r, cx = 8 * (I0 - 1) + slot % (2 * CPC) * 4;
@@ -534,6 +531,10 @@ bwd_cell_kernel(const T *__restrict__ q, const T *__restrict__ key, const T *__r
         load_lds(dma_rsrc(stats + ((long)((k + 2) % 3) * B + n) * 4 * lpix, (u32)(16 * lpix)), stat_at + (k * CSTAT + wave % 5 * 256) * 4,
                  ok ? (u32)(cy * 2 * W + cx) * 4u : OUTSIDE);
     }
+#pragma unroll
+    for (int j = 0; j < CBUF - 1; ++j) stage(j);
+    next(-1, 0);
+
     // this lane's 4 children of block (qx, nb)
     auto child_stats = [&](int k, int qx, int nb) __attribute__((always_inline)) {
         return *(const f32x4 *)(statbuf + k * CSTAT + (8 * (1 - qy) + 2 * nb + (g >> 1)) * 8 * CPC + 8 * (bi + 1 - qx) + 4 * (g & 1));
