@@ -522,8 +522,7 @@ bwd_cell_kernel(const T *__restrict__ q, const T *__restrict__ key, const T *__r
     // The three stats planes of the staged children, [16 rows][72] each, loaded straight into LDS in
     // front of everything else (fetched into registers between the products they cost a memory latency
     // each, with nothing else to run meanwhile): the wait for chunk 0 covers them, however few chunks
-    // there are.  Zeros outside the image, so that children there have weight 0.  The first two planes
-    // lie where results will go later.
+    // there are.  Zeros outside the image.  The first two planes lie where results will go later.
     if (wave < 15) {
         const int k = wave / 5, slot = wave % 5 * 64 + lane, r = slot / (2 * CPC);
         const int cy = 8 * (J - 1) + r, cx = 8 * (I0 - 1) + slot % (2 * CPC) * 4;
@@ -565,8 +564,10 @@ bwd_cell_kernel(const T *__restrict__ q, const T *__restrict__ key, const T *__r
                     const bool row_ok = qy ? cr <= nb : cr >= nb;
 #pragma unroll
                     for (int v = 0; v < 4; ++v) {
+                        // (a child right of the image is one of the next row's, whose product with this
+                        // cell no maximum bounds: it must not count, whatever it is)
                         const int px = 2 * (g & 1) + (v >> 1);
-                        const bool ok = row_ok & (qx ? cc <= px : cc >= px);
+                        const bool ok = row_ok & (qx ? cc <= px : cc >= px) & (4 * (I0 + bi - qx) + px < W);
                         const float e = __builtin_amdgcn_exp2f(__builtin_fmaf(acc[qx][nb][v], LOG2E, -mlog[v]));
                         w[4 * k + v] = ok ? e * inv[v] : 0.f;
                     }

@@ -449,8 +449,10 @@ bwd_cell_kernel(const T *__restrict__ q, const T *__restrict__ key, const T *__r
         __builtin_amdgcn_raw_buffer_store_b128(v, ro, ok ? (cell * (u32)cx + (u32)c) * (u32)sizeof(T) : OUTSIDE, 0, 0);
     };
 
-    // the three stats planes of the staged children, straight into LDS; zeros outside the image: children
-    // there have weight 0
+    // the three stats planes of the staged children, straight into LDS.  Zeros outside the image -- and, for
+    // an odd W, the statistics of the next row's first two children in a row's last piece: their weights are
+    // finite (a child at the row's left end has zeros among its logits: its maximum is not negative) and
+    // meet the zeros that are staged as such a child's q and grad_out
     if (wave < 12) {
         const int k = wave / 4, c = (wave % 4 * 64 + lane) * 4, cy = 8 * (J0 - 1) + c / XC, cx = 8 * (I0 - 1) + c % XC;
         const bool ok = (c < XR * XC) & ((u32)cy < (u32)hH) & ((u32)cx < (u32)hW);

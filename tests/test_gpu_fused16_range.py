@@ -51,3 +51,22 @@ def test_backward_of_one_chunk_of_keys(dtype, channels_last, d):
         assert rel(got, want) <= one_rounding(dtype)
     for _ in range(4):
         assert all(torch.equal(a, b) for a, b in zip(gradients(ops, go), first))
+
+
+@pytest.mark.parametrize('dtype', [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize('channels_last', [False, True])
+@pytest.mark.parametrize('W', [18, 20, 22, 23])
+def test_backward_with_logits_in_the_hundreds(dtype, channels_last, W):
+    """Softmaxes that are almost one cell, and rows whose last 16-byte piece of children (W = 18, 22; of
+    their statistics: W = 23) runs over into the next row: the products of those children with this
+    row's cells are beyond what the exponential holds and must not count.  Bar: one rounding, and the fp32 logits' own error (64 * 2^-24 * 500 = 2e-3 at most, a
+    tenth of that in the norm)."""
+    g = torch.Generator(device='cuda').manual_seed(W)
+    B, d, C, H = 2, 64, 24, 9
+    q, k, v, go = ((B, d, 2 * H, 2 * W), (B, d, H, W), (B, C, H, W), (B, C, 2 * H, 2 * W))
+    ops = [draw(g, q, dtype, 5.0, channels_last), draw(g, k, dtype, 5.0, channels_last), draw(g, v, dtype, 1.0, channels_last)]
+    go = draw(g, go, dtype, 1.0, channels_last)
+    want = exact_gradients(ops, go)[1:]
+    for got, w in zip(gradients(ops, go), want):
+        assert bool(torch.isfinite(got).all())
+        assert rel(got, w) <= one_rounding(dtype) + 2e-4
