@@ -22,8 +22,8 @@
 // and E written by the first kernel and read by the second, moves 2 x 100 values per parent
 // (430 MB each way at B=16, 100x168 in fp32) for the 2 x 29 % more matrix work that this costs.
 //
-// Operands: A and E enter the products as a 16-bit value plus a 16-bit remainder, everything
-// else is exact in 16 bits; sums are fp32.
+// Operands: A and E enter the products as a 16-bit value plus a 16-bit remainder (f16: of values brought
+// into its range, see Fit), everything else is exact in 16 bits; sums are fp32.
 //
 // Measured (B=16, C=256, d=64, 100x168, bf16): pixel kernel 310 us, cell kernel 454 us, a training step
 // 996 us against 1211 for the chain over K * K tensors (similarity and its softmax backward 274 us,
@@ -53,6 +53,7 @@ bwd_pixel_kernel(const T *__restrict__ q, const T *__restrict__ key, const T *__
                  const T *__restrict__ grad_out, T *__restrict__ grad_q, float *__restrict__ stats, int B, int d, int C,
                  int H, int W, int tiles_x, int tiles_y, int ns, int nblocks, int per_xcd) {
     constexpr int NT = 128 * NSW;
+    constexpr bool SCALED = __is_same(T, f16_t);             // E is brought into the type's range (Fit)
     constexpr int NBUF = 3;
     constexpr int LROW = (4 * NSW + 4 + 7) / 8 * 4;          // dwords per staged window row: whole pieces of 8 cells
     constexpr int LOWBUF = WROWS * CHK * LROW;               // dwords per low-res buffer
@@ -262,6 +263,7 @@ bwd_pixel_kernel(const T *__restrict__ q, const T *__restrict__ key, const T *__
 
     // ---- gradient of the logits; what the cell kernel needs to form it again ----
     u32x4 whi[2][2], wlo[2][2];
+    float down[2][4];           // f16: what the results of child 4 g + v of block nb are multiplied by
     if (active) {
         clear_outside(acc);
 #pragma unroll
@@ -280,13 +282,23 @@ bwd_pixel_kernel(const T *__restrict__ q, const T *__restrict__ key, const T *__
                 stats[g * plane + (long)n * 4 * lpix + (long)cy * 2 * W + cx] = g == 0 ? mlog[nb] : g == 1 ? inv[nb] : dsum;
             }
             // reduction step s of the last product covers the cells of blocks mb = 2 s, 2 s + 1
+            float e[2][8], m = 0.f;
 #pragma unroll
-            for (int s = 0; s < 2; ++s) {
-                float e[8];
+            for (int s = 0; s < 2; ++s)
 #pragma unroll
-                for (int k = 0; k < 8; ++k) e[k] = p[2 * s + k / 4][nb][k % 4] * (acc[2 * s + k / 4][nb][k % 4] - dsum);
-                split8<T>(e, whi[nb][s], wlo[nb][s]);
+                for (int k = 0; k < 8; ++k) {
+                    e[s][k] = p[2 * s + k / 4][nb][k % 4] * (acc[2 * s + k / 4][nb][k % 4] - dsum);
+                    if (SCALED) m = fmaxf(m, __builtin_fabsf(e[s][k]));
+                }
+            if (SCALED) {
+                const Fit f = fit<T>(over_groups(m));
+#pragma unroll
+                for (int v = 0; v < 4; ++v) down[nb][v] = __shfl(f.down, 4 * g + v);
+#pragma unroll
+                for (int k = 0; k < 16; ++k) e[k / 8][k % 8] *= f.up;
             }
+#pragma unroll
+            for (int s = 0; s < 2; ++s) split8<T>(e[s], whi[nb][s], wlo[nb][s]);
         }
     }
     if (!grad_q) return;
@@ -313,6 +325,10 @@ bwd_pixel_kernel(const T *__restrict__ q, const T *__restrict__ key, const T *__
                 for (int s = 0; s < 2; ++s) {
                     o = Mma<T>::k32(whi[nb][s], b[s], o);
                     o = Mma<T>::k32(wlo[nb][s], b[s], o);
+                }
+                if (SCALED) {
+#pragma unroll
+                    for (int v = 0; v < 4; ++v) o[v] *= down[nb][v];
                 }
                 // element v: child (row 2 (2 half + nb) + g / 2, column 4 (g % 2) + v), channel c0 + i16
                 const int r = 2 * (2 * half + nb) + (g >> 1);
@@ -382,6 +398,7 @@ bwd_cell_kernel(const T *__restrict__ q, const T *__restrict__ key, const T *__r
                 const T *__restrict__ grad_out, const float *__restrict__ stats, T *__restrict__ grad_key,
                 T *__restrict__ grad_value, int B, int d, int C, int H, int W, int tiles_x, int tiles_y, int nblocks,
                 int per_xcd) {
+    constexpr bool SCALED = __is_same(T, f16_t);             // A and E are brought into the type's range (Fit)
     __shared__ __attribute__((aligned(16))) u32 lds[CBUF * (CHI + CLOW) + CSTAT + 4 * COUT];
     u32 *const hibuf = lds, *const lowbuf = lds + CBUF * CHI;
     const u32 hi_base = lds_address((const __attribute__((address_space(3))) u32 *)lds), low_at = hi_base + CBUF * CHI * 4;
@@ -470,6 +487,24 @@ bwd_cell_kernel(const T *__restrict__ q, const T *__restrict__ key, const T *__r
     // rows 2 s and 2 s + 1 of the quadrant, in the order the weights are held in; element v of the
     // result: cell (row g, column v), channel i16
     u32x4 whi[2][2], wlo[2][2];
+    Fit f = {1.f, 1.f};         // f16: the factors of this lane's cell, the results' of cells (g, v)
+    float down[4];
+    auto hold = [&](float (&w)[2][2][8]) __attribute__((always_inline)) {
+        if (SCALED) {
+            float m = 0.f;
+#pragma unroll
+            for (int k = 0; k < 32; ++k) m = fmaxf(m, __builtin_fabsf(w[k / 16][k / 8 % 2][k % 8]));
+            f = fit<T>(over_groups(m));
+#pragma unroll
+            for (int v = 0; v < 4; ++v) down[v] = __shfl(f.down, 4 * g + v);
+#pragma unroll
+            for (int k = 0; k < 32; ++k) w[k / 16][k / 8 % 2][k % 8] *= f.up;
+        }
+#pragma unroll
+        for (int qx = 0; qx < 2; ++qx)
+#pragma unroll
+            for (int s = 0; s < 2; ++s) split8<T>(w[qx][s], whi[qx][s], wlo[qx][s]);
+    };
     auto gather = [&](int j) __attribute__((always_inline)) {
         const u32 *hb = hibuf + j % CBUF * CHI;
         f32x4 o = f32x4{0.f, 0.f, 0.f, 0.f};
@@ -482,6 +517,10 @@ bwd_cell_kernel(const T *__restrict__ q, const T *__restrict__ key, const T *__r
                 o = Mma<T>::k32(whi[qx][s], b, o);
                 o = Mma<T>::k32(wlo[qx][s], b, o);
             }
+        if (SCALED) {
+#pragma unroll
+            for (int v = 0; v < 4; ++v) o[v] *= down[v];
+        }
         *(f32x4 *)(outbuf + (2 * (j & 1) + qy) * COUT + out_at(i16, g, bi)) = o;
     };
     // the chunk's results, complete after the barrier
@@ -552,11 +591,11 @@ bwd_cell_kernel(const T *__restrict__ q, const T *__restrict__ key, const T *__r
 
     // ---- the weights of the wave's cells: A = exp2(S log2 e - max) / sum inside a child's window ----
     if (active) {
+        float w[2][2][8];
 #pragma unroll
         for (int qx = 0; qx < 2; ++qx)
 #pragma unroll
-            for (int s = 0; s < 2; ++s) {
-                float w[8];
+            for (int s = 0; s < 2; ++s)
 #pragma unroll
                 for (int k = 0; k < 2; ++k) {
                     const int nb = 2 * s + k;
@@ -569,11 +608,10 @@ bwd_cell_kernel(const T *__restrict__ q, const T *__restrict__ key, const T *__r
                         const int px = 2 * (g & 1) + (v >> 1);
                         const bool ok = row_ok & (qx ? cc <= px : cc >= px) & (4 * (I0 + bi - qx) + px < W);
                         const float e = __builtin_amdgcn_exp2f(__builtin_fmaf(acc[qx][nb][v], LOG2E, -mlog[v]));
-                        w[4 * k + v] = ok ? e * inv[v] : 0.f;
+                        w[qx][s][4 * k + v] = ok ? e * inv[v] : 0.f;
                     }
                 }
-                split8<T>(w, whi[qx][s], wlo[qx][s]);
-            }
+        hold(w);
     }
 
     lds_barrier();         // (the results of the first chunk overwrite the stats)
@@ -600,21 +638,20 @@ bwd_cell_kernel(const T *__restrict__ q, const T *__restrict__ key, const T *__r
 
     // ---- E = A (G - D), grad_key ----
     if (active) {
+        float w[2][2][8];
 #pragma unroll
         for (int qx = 0; qx < 2; ++qx)
 #pragma unroll
-            for (int s = 0; s < 2; ++s) {
-                float w[8];
+            for (int s = 0; s < 2; ++s)
 #pragma unroll
                 for (int k = 0; k < 2; ++k) {
                     const int nb = 2 * s + k;
                     const f32x4 dsum = child_stats(0, qx, nb);
 #pragma unroll
                     for (int v = 0; v < 4; ++v)
-                        w[4 * k + v] = joined<T>(whi[qx][s], wlo[qx][s], 4 * k + v) * (acc[qx][nb][v] - dsum[v]);
+                        w[qx][s][4 * k + v] = joined<T>(whi[qx][s], wlo[qx][s], 4 * k + v) * f.down * (acc[qx][nb][v] - dsum[v]);
                 }
-                split8<T>(w, whi[qx][s], wlo[qx][s]);
-            }
+        hold(w);
     }
     const __amdgpu_buffer_rsrc_t ro = __builtin_amdgcn_make_buffer_rsrc(
         (void *)(grad_key + (long)n * d * lpix), 0, (int)(d * lplane), 0x00020000);

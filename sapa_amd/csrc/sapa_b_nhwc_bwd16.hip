@@ -55,6 +55,7 @@ bwd_pixel_kernel(const T *__restrict__ q, const T *__restrict__ key, const T *__
     constexpr int NLI = (NLP + NT - 1) / NT;                 // direct loads per thread and window, at most
     static_assert(NLP % 64 == 0, "whole direct loads");
     constexpr int STREAM_AUX = STREAM ? 2 : 0;
+    constexpr bool SCALED = __is_same(T, f16_t);             // E is brought into the type's range (Fit)
     __shared__ __attribute__((aligned(16))) u32 lds[2 * LOWBUF + 2 * NSW * OSLOT];
     const u32 low_at = lds_address((const __attribute__((address_space(3))) u32 *)lds);
 
@@ -230,6 +231,7 @@ bwd_pixel_kernel(const T *__restrict__ q, const T *__restrict__ key, const T *__
 
     // ---- gradient of the logits; what the cell kernel needs to form it again ----
     u32x4 whi[2][2], wlo[2][2];
+    float down[2];              // f16: what the results of this lane's child of block nb are multiplied by
     if (active) {
 #pragma unroll
         for (int nb = 0; nb < 2; ++nb) {
@@ -244,13 +246,22 @@ bwd_pixel_kernel(const T *__restrict__ q, const T *__restrict__ key, const T *__
                 // planes [3][B, 2H, 2W]: maximum (times log2 e), 1 / sum, D; lanes g = 0, 1, 2 one each
                 stats[((long)g * B + n) * 4 * lpix + child[nb]] = g == 0 ? mlog[nb] : g == 1 ? inv[nb] : dsum;
             // reduction step s of the last product covers the cells of blocks mb = 2 s, 2 s + 1
+            float e[2][8], m = 0.f;
 #pragma unroll
-            for (int s = 0; s < 2; ++s) {
-                float e[8];
+            for (int s = 0; s < 2; ++s)
 #pragma unroll
-                for (int k = 0; k < 8; ++k) e[k] = p[2 * s + k / 4][nb][k % 4] * (acc[2 * s + k / 4][nb][k % 4] - dsum);
-                split8<T>(e, whi[nb][s], wlo[nb][s]);
+                for (int k = 0; k < 8; ++k) {
+                    e[s][k] = p[2 * s + k / 4][nb][k % 4] * (acc[2 * s + k / 4][nb][k % 4] - dsum);
+                    if (SCALED) m = fmaxf(m, __builtin_fabsf(e[s][k]));
+                }
+            if (SCALED) {
+                const Fit f = fit<T>(over_groups(m));
+                down[nb] = f.down;
+#pragma unroll
+                for (int k = 0; k < 16; ++k) e[k / 8][k % 8] *= f.up;
             }
+#pragma unroll
+            for (int s = 0; s < 2; ++s) split8<T>(e[s], whi[nb][s], wlo[nb][s]);
         }
     }
     if (!grad_q) return;
@@ -284,6 +295,7 @@ bwd_pixel_kernel(const T *__restrict__ q, const T *__restrict__ key, const T *__
                         o = Mma<T>::k32(va[mk][s], whi[nb][s], o);
                         o = Mma<T>::k32(va[mk][s], wlo[nb][s], o);
                     }
+                    if (SCALED) o *= down[nb];
                     *(u32x2 *)(oslot + piece_at(i16, 2 * mk + (g >> 1)) + 2 * (g & 1)) =
                         u32x2{pack2<T>(o[0], o[1]), pack2<T>(o[2], o[3])};
                 }
@@ -328,6 +340,7 @@ bwd_cell_kernel(const T *__restrict__ q, const T *__restrict__ key, const T *__r
                 const T *__restrict__ grad_out, const float *__restrict__ stats, T *__restrict__ grad_key,
                 T *__restrict__ grad_value, int B, int d, int C, int H, int W, int tiles_x, int tiles_y, int nblocks,
                 int per_xcd) {
+    constexpr bool SCALED = __is_same(T, f16_t);             // A and E are brought into the type's range (Fit)
     __shared__ __attribute__((aligned(16))) u32 lds[2 * CHI + CSTAT + 2 * CPART];
     float *const statbuf = (float *)(lds + 2 * CHI), *const part = statbuf + CSTAT;   // (D; the other planes over `part`)
     const u32 hi_base = lds_address((const __attribute__((address_space(3))) u32 *)lds);
@@ -419,6 +432,21 @@ bwd_cell_kernel(const T *__restrict__ q, const T *__restrict__ key, const T *__r
     // L of a 16-lane block addresses child L / 4 of the 4, channels 8 (L % 4) + 4 h .. + 3; so element v of
     // result h: channel 8 g + 4 h + v of cell i16
     u32x4 whi[2][2], wlo[2][2];
+    Fit f = {1.f, 1.f};         // f16: the factors of this lane's cell
+    auto hold = [&](float (&w)[2][2][8]) __attribute__((always_inline)) {
+        if (SCALED) {
+            float m = 0.f;
+#pragma unroll
+            for (int k = 0; k < 32; ++k) m = fmaxf(m, __builtin_fabsf(w[k / 16][k / 8 % 2][k % 8]));
+            f = fit<T>(over_groups(m));
+#pragma unroll
+            for (int k = 0; k < 32; ++k) w[k / 16][k / 8 % 2][k % 8] *= f.up;
+        }
+#pragma unroll
+        for (int qx = 0; qx < 2; ++qx)
+#pragma unroll
+            for (int s = 0; s < 2; ++s) split8<T>(w[qx][s], whi[qx][s], wlo[qx][s]);
+    };
     auto gather = [&](int j, f32x4 (&o)[2]) __attribute__((always_inline)) {
         const u32 *hb = lds + (j & 1) * CHI;
 #pragma unroll
@@ -433,6 +461,7 @@ bwd_cell_kernel(const T *__restrict__ q, const T *__restrict__ key, const T *__r
                     o[h] = Mma<T>::k32(a, whi[qx][s], o[h]);
                     o[h] = Mma<T>::k32(a, wlo[qx][s], o[h]);
                 }
+            if (SCALED) o[h] *= f.down;
         }
         if (qy) {
             float *p = part + (j & 1) * CPART + blk * 512 + lane * 4;
@@ -496,11 +525,11 @@ bwd_cell_kernel(const T *__restrict__ q, const T *__restrict__ key, const T *__r
 
     // ---- the weights of the wave's cells: A = exp2(S log2 e - max) / sum inside a child's window ----
     if (active) {
+        float w[2][2][8];
 #pragma unroll
         for (int qx = 0; qx < 2; ++qx)
 #pragma unroll
-            for (int s = 0; s < 2; ++s) {
-                float w[8];
+            for (int s = 0; s < 2; ++s)
 #pragma unroll
                 for (int k = 0; k < 2; ++k) {
                     const int nb = 2 * s + k;
@@ -511,11 +540,10 @@ bwd_cell_kernel(const T *__restrict__ q, const T *__restrict__ key, const T *__r
                         const int px = 2 * (g & 1) + (v >> 1);
                         const bool ok = row_ok & (qx ? cc <= px : cc >= px);
                         const float e = __builtin_amdgcn_exp2f(__builtin_fmaf(acc[qx][nb][v], LOG2E, -mlog[v]));
-                        w[4 * k + v] = ok ? e * inv[v] : 0.f;
+                        w[qx][s][4 * k + v] = ok ? e * inv[v] : 0.f;
                     }
                 }
-                split8<T>(w, whi[qx][s], wlo[qx][s]);
-            }
+        hold(w);
     }
     lds_barrier();         // (the sums handed over for the first chunks overwrite the stats)
 
@@ -539,21 +567,20 @@ bwd_cell_kernel(const T *__restrict__ q, const T *__restrict__ key, const T *__r
 
     // ---- E = A (G - D), grad_key ----
     if (active) {
+        float w[2][2][8];
 #pragma unroll
         for (int qx = 0; qx < 2; ++qx)
 #pragma unroll
-            for (int s = 0; s < 2; ++s) {
-                float w[8];
+            for (int s = 0; s < 2; ++s)
 #pragma unroll
                 for (int k = 0; k < 2; ++k) {
                     const int nb = 2 * s + k;
                     const f32x4 dsum = child_stats(0, qx, nb);
 #pragma unroll
                     for (int v = 0; v < 4; ++v)
-                        w[4 * k + v] = joined<T>(whi[qx][s], wlo[qx][s], 4 * k + v) * (acc[qx][nb][v] - dsum[v]);
+                        w[qx][s][4 * k + v] = joined<T>(whi[qx][s], wlo[qx][s], 4 * k + v) * f.down * (acc[qx][nb][v] - dsum[v]);
                 }
-                split8<T>(w, whi[qx][s], wlo[qx][s]);
-            }
+        hold(w);
     }
     const __amdgpu_buffer_rsrc_t ro = __builtin_amdgcn_make_buffer_rsrc(
         (void *)(grad_key + (long)n * d * lpix), 0, (int)(d * lpix * (long)sizeof(T)), 0x00020000);

@@ -56,6 +56,25 @@ __device__ __forceinline__ void split8(const float *p, u32x4 &hi, u32x4 &lo) {
     lo = u32x4{pack2<T>(r[0], r[1]), pack2<T>(r[2], r[3]), pack2<T>(r[4], r[5]), pack2<T>(r[6], r[7])};
 }
 
+// f16 holds a pair of operands to 2^-25 only and nothing beyond 65504, whatever its values' own size: a set
+// of values is multiplied by a power of two that takes its largest magnitude m to 2^14 .. 2^15 before
+// it is split, and sums of products by its inverse (exact: the pair then holds 23 bits of the largest
+// values and 2^-40 of it of the others).  bf16 has fp32's range: 1.
+struct Fit {
+    float up, down;
+};
+template <typename T>
+__device__ __forceinline__ Fit fit(float m) {
+    if constexpr (!__is_same(T, f16_t)) return Fit{1.f, 1.f};
+    const u32 b = __builtin_bit_cast(u32, m) >> 23, e = b < 27u ? 27u : b;    // (both factors normal numbers)
+    return Fit{__builtin_bit_cast(float, (268u - e) << 23), __builtin_bit_cast(float, (e - 14u) << 23)};
+}
+// the same in every lane: the largest of the four lane groups' m
+__device__ __forceinline__ float over_groups(float m) {
+    m = fmaxf(m, __shfl_xor(m, 16));
+    return fmaxf(m, __shfl_xor(m, 32));
+}
+
 // value k of a pair of operands made by split8
 template <typename T>
 __device__ __forceinline__ float joined(u32x4 hi, u32x4 lo, int k) {

@@ -70,3 +70,36 @@ def test_backward_with_logits_in_the_hundreds(dtype, channels_last, W):
     for got, w in zip(gradients(ops, go), want):
         assert bool(torch.isfinite(got).all())
         assert rel(got, w) <= one_rounding(dtype) + 2e-4
+
+
+@pytest.mark.parametrize('channels_last', [False, True])
+@pytest.mark.parametrize('scale_q,scale_k,scale_v,scale_go', [
+    (0.05, 0.05, 10.0, 3000.0),     # loss-scaled gradients of features that are not normalised: |E| beyond 65504
+    (0.0005, 100.0, 10.0, 0.2),     # large keys
+    (0.05, 8.0, 1.0, 2.0 ** -13),   # gradients of E below the smallest normal number, lifted by the keys
+    (4.0, 1e-2, 1.0, 2.0 ** -15),   # ... by the queries
+])
+def test_fp16_backward_at_the_ends_of_the_range(channels_last, scale_q, scale_k, scale_v, scale_go):
+    """The gradient of the logits leaves fp16's range in both directions while the gradients themselves
+    are within it.  Every gradient within one rounding of its own value (2^-11, and half the spacing of
+    the subnormals) and an fp32 error (2e-5) of the sum of the magnitudes that it adds up."""
+    import sapa_amd
+    g = torch.Generator(device='cuda').manual_seed(7)
+    B, d, C, H, W = 2, 32, 256, 14, 22
+    shapes = ((B, d, 2 * H, 2 * W), (B, d, H, W), (B, C, H, W), (B, C, 2 * H, 2 * W))
+    *ops, go = (draw(g, s, torch.float16, f, channels_last) for s, f in zip(shapes, (scale_q, scale_k, scale_v, scale_go)))
+    assert go.abs().max() < 20000
+    want = exact_gradients(ops, go)[1:]
+    # magnitudes: A, |E| and their products with |key|, |query|, |grad_out|
+    q, k, v, o = (t.double().contiguous() for t in (*ops, go))
+    a = torch.softmax(sapa_amd.qk(q, k, 5, 2), dim=1)
+    ga = sapa_amd.qk(o, v, 5, 2)
+    scale_e = a * (sapa_amd.qk(o.abs(), v.abs(), 5, 2) + (a * ga.abs()).sum(dim=1, keepdim=True))
+    leaves = [t.detach().clone().requires_grad_() for t in (q.abs(), k.abs())]
+    mags = list(torch.autograd.grad(sapa_amd.qk(*leaves, 5, 2), leaves, scale_e))
+    leaf = v.clone().requires_grad_()
+    mags += torch.autograd.grad(sapa_amd.av(a, leaf, 5, 2), leaf, o.abs())
+    for got, w, m in zip(gradients(ops, go), want, mags):
+        assert w.abs().max() < 65504 and bool(torch.isfinite(got).all())
+        bad = (got.double() - w).abs() > 2.0 ** -11 * w.abs() + 2.0 ** -25 + 2e-6 * m
+        assert int(bad.sum()) == 0, (int(bad.sum()), bad.numel())
