@@ -23,6 +23,7 @@
 // layout of the first product is the A-operand layout of the second, so the weights never leave
 // the registers.  They enter the product as a 16-bit value plus a 16-bit remainder (two
 // instructions), the sums are fp32: the result is within half a 16-bit spacing of the exact one.
+// (f16, which holds a pair to 2^-25 only, takes them times 2^15: small weights keep their bits.)
 // The 4 x 4 output blocks go back through LDS so that global stores are 16 bytes per lane along
 // whole tile rows.
 //
@@ -351,6 +352,7 @@ sapa_b_wmat16_kernel(const T *__restrict__ q, const T *__restrict__ key, const T
     // reduction step s of the aggregation covers the cells of blocks mb = 2 s, 2 s + 1; lane
     // (g, child) holds 4 + 4 of its 32
     u32x4 whi[4][2], wlo[4][2];
+    constexpr float UP = __is_same(T, f16_t) ? 32768.f : 1.f;
     if (active) {
         // element v of every block is window column 4 (g % 2) + v.  Outside the image the key is zero
         // (logit 0) and so is the value (the weight may as well be 0): only the waves at a row's
@@ -407,7 +409,7 @@ sapa_b_wmat16_kernel(const T *__restrict__ q, const T *__restrict__ key, const T
             }
             sum += __shfl_xor(sum, 16);
             sum += __shfl_xor(sum, 32);
-            const float inv = 1.f / sum;
+            const float inv = UP / sum;
 #pragma unroll
             for (int s = 0; s < 2; ++s) {
                 float p[8];
@@ -452,6 +454,7 @@ sapa_b_wmat16_kernel(const T *__restrict__ q, const T *__restrict__ key, const T
                     acc = Mma<T>::k32(whi[nb][s], b[s], acc);
                     acc = Mma<T>::k32(wlo[nb][s], b[s], acc);
                 }
+                if (UP != 1.f) acc *= 1.f / UP;
                 // element v: child (row 2 nb + g / 2, column 4 (g % 2) + v), channel c0 + i16
                 const int r = 2 * nb + (g >> 1);
                 *(u32x2 *)(ob + i16 * HICH + r * HIROW + ((t ^ (swz(i16, r) & (NPC - 1))) << 2) + 2 * (g & 1)) =

@@ -103,3 +103,23 @@ def test_fp16_backward_at_the_ends_of_the_range(channels_last, scale_q, scale_k,
         assert w.abs().max() < 65504 and bool(torch.isfinite(got).all())
         bad = (got.double() - w).abs() > 2.0 ** -11 * w.abs() + 2.0 ** -25 + 2e-6 * m
         assert int(bad.sum()) == 0, (int(bad.sum()), bad.numel())
+
+
+@pytest.mark.parametrize('K,s,W', [(5, 2, 24), (5, 2, 23), (5, 2, 6), (7, 4, 13), (5, 4, 12), (3, 2, 21)])
+def test_fp16_forward_of_small_weights(K, s, W):
+    """Weights below fp16's smallest normal number on values in the thousands, next to large weights on
+    small values: every result within one rounding and an fp32 error of the sum of its terms'
+    magnitudes."""
+    import sapa_amd
+    g = torch.Generator(device='cuda').manual_seed(W)
+    B, d, C, H = 2, 32, 16, 9
+    q, k = draw(g, (B, d, s * H, s * W), torch.float16, 1.5), draw(g, (B, d, H, W), torch.float16, 1.5)
+    v = draw(g, (B, C, H, W), torch.float16, 1.0)
+    v = v * torch.where(torch.rand(v.shape, generator=g, device='cuda') < 0.2, 8192.0, 2.0 ** -4).half()
+    with torch.no_grad():
+        got = sapa_amd.sapa_fused(q, k, v, K, s)
+        want = sapa_amd.sapa_fused(q.double(), k.double(), v.double(), K, s)
+        mag = sapa_amd.sapa_fused(q.double(), k.double(), v.double().abs(), K, s)
+    # (fp32 logits of magnitude 100 are off by 1e-5: so are the weights, relative to themselves)
+    bad = (got.double() - want).abs() > 2.0 ** -11 * want.abs() + 2.0 ** -25 + 1e-5 * mag
+    assert int(bad.sum()) == 0, (int(bad.sum()), bad.numel())
