@@ -108,7 +108,10 @@ __device__ __forceinline__ int swz(int ch, int r) { return ((ch & 7) << 1) | ((r
 // B=4, C=512, d=64, 64x64 250 -> 69 us (4.7 TB/s: memory), B=16, C=256, 50x84 756 -> 309 us (rows
 // of 672 bytes: split cache lines); K=5, s=4 165 -> 66 and 480 -> 263 us; K=3, s=2 57 -> 27 and
 // 132 -> 52 us; one image 16x16 33 -> 12, 20 -> 15 and 15 -> 15 us.
-template <typename T, int K, int S, int NSW, bool STREAM, bool ODD>
+//
+// HALF: images of the key or of the value of an odd number of elements (a kernel of its own: what it
+// takes in registers costs the others up to 10 % -- K=3, s=2, B=16, C=256, 50x84 in bf16 83 -> 91 us)
+template <typename T, int K, int S, int NSW, bool STREAM, bool ODD, bool HALF>
 __global__ __launch_bounds__(64 * NSW, 4) void
 sapa_b_wmat16_kernel(const T *__restrict__ q, const T *__restrict__ key, const T *__restrict__ value,
                      T *__restrict__ out, int d, int C, int H, int W, int tiles_x, int tiles_y, int ns,
@@ -118,6 +121,7 @@ sapa_b_wmat16_kernel(const T *__restrict__ q, const T *__restrict__ key, const T
     constexpr bool OWN = !(K == 5 && S == 2);
     static_assert(PB + K - 1 <= 8 && S * PB == 8, "a block's window");
     static_assert(!OWN || ODD, "pieces of a block's own come through registers");
+    static_assert(!HALF || ODD, "half a dword comes through registers");
     // dwords per staged window row: whole pieces of 8 cells (OWN: one per block; a piece of padding
     // keeps the rows of the 16 channels on different banks)
     constexpr int LROW = OWN ? 4 * NSW + 4 : (4 * NSW + 4 + 7) / 8 * 4;
@@ -188,10 +192,12 @@ sapa_b_wmat16_kernel(const T *__restrict__ q, const T *__restrict__ key, const T
     const int nVc = allV - vbase < slice_chunks ? allV - vbase : slice_chunks, ntot = nKc + nVc;
     const __amdgpu_buffer_rsrc_t rq = __builtin_amdgcn_make_buffer_rsrc(
         (void *)(q + (long)n * d * SS * lpix), 0, (int)(d * hplane), 0x00020000);
+    // (HALF: an image ends with half a dword, which lies outside: nothing behind a tensor is read, and
+    // low_end puts that element in its place)
     const __amdgpu_buffer_rsrc_t rk = __builtin_amdgcn_make_buffer_rsrc(
-        (void *)(key + (long)n * d * lpix), 0, (int)((d * lplane + 3u) & ~3u), 0x00020000);
+        (void *)(key + (long)n * d * lpix), 0, (int)(HALF ? d * lplane & ~3u : d * lplane), 0x00020000);
     const __amdgpu_buffer_rsrc_t rv = __builtin_amdgcn_make_buffer_rsrc(
-        (void *)(value + (long)n * C * lpix), 0, (int)((C * lplane + 3u) & ~3u), 0x00020000);
+        (void *)(value + (long)n * C * lpix), 0, (int)(HALF ? C * lplane & ~3u : C * lplane), 0x00020000);
     const __amdgpu_buffer_rsrc_t ro = __builtin_amdgcn_make_buffer_rsrc(
         (void *)(out + (long)n * C * SS * lpix), 0, (int)(C * hplane), 0x00020000);
 
@@ -267,6 +273,18 @@ sapa_b_wmat16_kernel(const T *__restrict__ q, const T *__restrict__ key, const T
             if (NLP % NT == 0 || slot < NLP) *(u32x4 *)(lowbuf + (j & 1) * LOWBUF + at) = m;
         }
     };
+    // behind low_commit(j), by the wave that wrote the piece: the last element of an image of an odd number
+    auto low_end = [&](int j) __attribute__((always_inline)) {
+        const int c0 = (j < nKc ? j : j - nKc + vbase) * CHK, nch = j < nKc ? d : C;
+        if (!HALF || j >= ntot || c0 + CHK < nch || !(nch & lpix & 1)) return;
+        const T last = (j < nKc ? key : value)[((long)n + 1) * nch * lpix - 1];
+#pragma unroll
+        for (int i = 0; i < NLI; ++i) {
+            const int slot = i * NT + tid, at = OWN ? slot / LPC * LROW + slot % LPC * 4 : slot * 4;
+            const u32 e = (u32)((long)(nch - c0) * lpix) - 1u - (u32)(((int)off_low[i] >> 1) + (low_odd[i] ? 1 : 0));
+            if (e < 8u) ((T *)(lowbuf + (j & 1) * LOWBUF + at))[e] = last;
+        }
+    };
     // Waits are counted: the counter of vector-memory operations retires in issue order, so
     // "at most N outstanding" means that everything but the last N issued is complete.  Written out
     // because the compiler does not track a direct load's LDS write.
@@ -304,6 +322,7 @@ sapa_b_wmat16_kernel(const T *__restrict__ q, const T *__restrict__ key, const T
 
     low_load(0);
     low_commit(0);
+    low_end(0);
     stage(0);
     stage(1);
     // chunk 0: all but chunk 1's loads
@@ -341,6 +360,7 @@ sapa_b_wmat16_kernel(const T *__restrict__ q, const T *__restrict__ key, const T
                 for (int nb = 0; nb < 4; ++nb) sim[mb][nb] = Mma<T>::k16(a[mb], b[nb], sim[mb][nb]);
         }
         low_commit(j + 1);
+        low_end(j + 1);
         // chunk j + 1: nothing was issued after its loads
         wait_all_but(0);
         if (j + 1 == nKc) patch_low(nKc);
@@ -459,9 +479,13 @@ sapa_b_wmat16_kernel(const T *__restrict__ q, const T *__restrict__ key, const T
                 const int r = 2 * nb + (g >> 1);
                 *(u32x2 *)(ob + i16 * HICH + r * HIROW + ((t ^ (swz(i16, r) & (NPC - 1))) << 2) + 2 * (g & 1)) =
                     u32x2{pack2<T>(acc[0], acc[1]), pack2<T>(acc[2], acc[3])};
+                // (no register to spare: with the products of several nb in flight the loop went through scratch
+                // memory, 68 -> 78 us at B=4, C=512, 64x64)
+                if (K == 7 && UP != 1.f) __builtin_amdgcn_sched_barrier(0);
             }
         }
         low_commit(j + 1);
+        low_end(j + 1);
         // chunk j + 1: its loads were the last operations issued
 #if defined(__HIP_DEVICE_COMPILE__)
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
@@ -493,7 +517,7 @@ sapa_b_wmat16_kernel(const T *__restrict__ q, const T *__restrict__ key, const T
     }
 }
 
-template <typename T, int K, int S, int NSW, bool STREAM, bool ODD>
+template <typename T, int K, int S, int NSW, bool STREAM, bool ODD, bool HALF = false>
 static hipError_t launch_geom(const void *q, const void *key, const void *value, void *out, int B, int d,
                               int C, int H, int W, hipStream_t st) {
     constexpr int PB = 8 / S;
@@ -512,7 +536,7 @@ static hipError_t launch_geom(const void *q, const void *key, const void *value,
     const long nb = tiles * nslices;
     if (nb > (1L << 30)) return hipErrorNotSupported;
     const int per_xcd = (int)((nb + 7) / 8);
-    hipLaunchKernelGGL((sapa_b_wmat16_kernel<T, K, S, NSW, STREAM, ODD>), dim3(per_xcd * 8), dim3(64 * NSW), 0, st, (const T *)q,
+    hipLaunchKernelGGL((sapa_b_wmat16_kernel<T, K, S, NSW, STREAM, ODD, HALF>), dim3(per_xcd * 8), dim3(64 * NSW), 0, st, (const T *)q,
                        (const T *)key, (const T *)value, (T *)out, d, C, H, W, tiles_x, tiles_y, ns,
                        nslices, slice_chunks, (int)nb, per_xcd);
     return hipGetLastError();
@@ -540,18 +564,20 @@ hipError_t sapa_b_wmat16_launch(int mode, const void *q, const void *key, const 
     // (B=16, C=256, d=64, 42x25: 24 us, by vector fmas 65; 100x167: 289 us against 451; rows below 16
     // cells, 13x13 at B=8: 9 us against 19 on the one-block-per-parent matrix kernel).
     const bool stream = 2L * ((long)B * H * W * (1L + s * s) * ((long)d + C)) > (256L << 20);
-    const bool odd = W % 2 != 0;
+    const bool odd = W % 2 != 0, half = ((d | C) & H & W & 1) != 0;
     // Other windows: streamed only where a tile's rows are whole 128-byte lines (s W a multiple of 64);
     // else parts of a line are written by two workgroups, and the caches put them together
     // (K=7, s=4, bf16: B=4, C=512, 64x64: 69 us streamed, 114 not; B=16, C=256, 50x84: 386 and 309)
     const bool lines = stream && s * W % 64 == 0;
 #define SAPA_WM16_OWN(T, KV, SV)                                                                                 \
     if (K == KV && s == SV)                                                                                      \
-        return lines ? wm16::launch_geom<T, KV, SV, 8, true, true>(q, key, value, out, B, d, C, H, W, st)       \
+        return half    ? wm16::launch_geom<T, KV, SV, 8, false, true, true>(q, key, value, out, B, d, C, H, W, st)  \
+               : lines ? wm16::launch_geom<T, KV, SV, 8, true, true>(q, key, value, out, B, d, C, H, W, st)       \
                       : wm16::launch_geom<T, KV, SV, 8, false, true>(q, key, value, out, B, d, C, H, W, st);
 #define SAPA_WM16_CASE(T)                                                                                       \
     SAPA_WM16_OWN(T, 7, 4) SAPA_WM16_OWN(T, 5, 4) SAPA_WM16_OWN(T, 3, 2)                                         \
-    return odd      ? wm16::launch_geom<T, 5, 2, 8, false, true>(q, key, value, out, B, d, C, H, W, st)          \
+    return half     ? wm16::launch_geom<T, 5, 2, 8, false, true, true>(q, key, value, out, B, d, C, H, W, st)    \
+           : odd    ? wm16::launch_geom<T, 5, 2, 8, false, true>(q, key, value, out, B, d, C, H, W, st)          \
            : stream ? wm16::launch_geom<T, 5, 2, 16, true, false>(q, key, value, out, B, d, C, H, W, st)         \
                     : wm16::launch_geom<T, 5, 2, 8, false, false>(q, key, value, out, B, d, C, H, W, st)
     if (dtype == 2) {

@@ -123,3 +123,25 @@ def test_fp16_forward_of_small_weights(K, s, W):
     # (fp32 logits of magnitude 100 are off by 1e-5: so are the weights, relative to themselves)
     bad = (got.double() - want).abs() > 2.0 ** -11 * want.abs() + 2.0 ** -25 + 1e-5 * mag
     assert int(bad.sum()) == 0, (int(bad.sum()), bad.numel())
+
+
+@pytest.mark.parametrize('dtype', [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize('K,s,H,W', [(5, 2, 3, 33), (5, 2, 5, 7), (7, 4, 3, 21), (5, 4, 5, 9), (3, 2, 3, 33)])
+@pytest.mark.parametrize('B', [1, 2, 3])
+def test_forward_reads_nothing_behind_a_tensor(K, s, H, W, B, dtype):
+    """Tensors of an odd number of elements that end in the middle of a dword, NaN behind them."""
+    import sapa_amd
+    g = torch.Generator(device='cuda').manual_seed(W)
+    d, C = 17, 33
+
+    def tail_nan(shape):
+        n = torch.Size(shape).numel()
+        buf = torch.full((n + 64,), float('nan'), dtype=dtype, device='cuda')
+        buf[:n] = (torch.randn(n, generator=g, device='cuda') * 0.5).to(dtype)
+        return buf[:n].view(shape)
+    ops = [tail_nan(sh) for sh in ((B, d, s * H, s * W), (B, d, H, W), (B, C, H, W))]
+    with torch.no_grad():
+        got = sapa_amd.sapa_fused(*ops, K, s)
+        again = sapa_amd.sapa_fused(*[t.clone() for t in ops], K, s)
+        want = sapa_amd.sapa_fused(*[t.double() for t in ops], K, s)
+    assert torch.equal(got, again) and rel(got, want) <= one_rounding(dtype)
