@@ -36,60 +36,18 @@
 // XOR-swizzled so that transposing reads, accumulator writes and the linear store pass are all
 // free of 4-way bank conflicts without padding.
 //
-// Masked cells still enter both products (a logit plus -inf, a weight of 0 times a value): a
-// non-finite key or value spreads to every child of the 4 x 4 block whose window holds it rather
-// than to the 25-cell neighbourhoods only.
-#include "kernels.hpp"
+// Masked cells still enter both products; what a non-finite value does there is mended behind the
+// aggregation (wm16_exact.hpp).
+#include "wm16_exact.hpp"
 
 namespace sapa {
 
 namespace wm16 {
 
-typedef unsigned u32;
-typedef float f32x4 __attribute__((ext_vector_type(4)));
-typedef u32 u32x2 __attribute__((ext_vector_type(2)));
-typedef u32 u32x4 __attribute__((ext_vector_type(4)));
-typedef short s16x4 __attribute__((ext_vector_type(4)));
+using namespace wm;
 
 constexpr int CHK = 16;            // channels per staged chunk
 constexpr int WROWS = 8;           // window rows = child rows of a block row
-constexpr u32 OUTSIDE = 0x80000000u;
-
-
-template <typename T> struct Mma;
-template <> struct Mma<f16_t> {
-    typedef _Float16 v4 __attribute__((ext_vector_type(4)));
-    typedef _Float16 v8 __attribute__((ext_vector_type(8)));
-    static __device__ __forceinline__ f32x4 k16(u32x2 a, u32x2 b, f32x4 c) {
-        return __builtin_amdgcn_mfma_f32_16x16x16f16(__builtin_bit_cast(v4, a), __builtin_bit_cast(v4, b), c, 0, 0, 0);
-    }
-    static __device__ __forceinline__ f32x4 k32(u32x4 a, u32x4 b, f32x4 c) {
-        return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(v8, a), __builtin_bit_cast(v8, b), c, 0, 0, 0);
-    }
-};
-template <> struct Mma<bf16_t> {
-    typedef __bf16 v8 __attribute__((ext_vector_type(8)));
-    static __device__ __forceinline__ f32x4 k16(u32x2 a, u32x2 b, f32x4 c) {
-        return __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(__builtin_bit_cast(s16x4, a), __builtin_bit_cast(s16x4, b), c, 0, 0, 0);
-    }
-    static __device__ __forceinline__ f32x4 k32(u32x4 a, u32x4 b, f32x4 c) {
-        return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(v8, a), __builtin_bit_cast(v8, b), c, 0, 0, 0);
-    }
-};
-
-template <typename T>
-__device__ __forceinline__ u32 pack2(float a, float b) {
-    typedef float f32x2 __attribute__((ext_vector_type(2)));
-    typedef T tx2 __attribute__((ext_vector_type(2)));
-    return __builtin_bit_cast(u32, __builtin_convertvector(f32x2{a, b}, tx2));
-}
-
-// 4 positions x 4 channels out of LDS, transposed: each lane of a 16-lane block addresses 4
-// consecutive positions of one channel and receives one position's 4 channels
-__device__ __forceinline__ u32x2 read_tr(const u32 *p) {
-    return __builtin_bit_cast(u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-                                         (s16x4 __attribute__((address_space(3))) *)p));
-}
 
 // position of the 16-byte piece `pc` of row r, channel ch in the swizzled q / output tile
 __device__ __forceinline__ int swz(int ch, int r) { return ((ch & 7) << 1) | ((r + (ch >> 3)) & 1); }
@@ -141,8 +99,11 @@ sapa_b_wmat16_kernel(const T *__restrict__ q, const T *__restrict__ key, const T
 
     // two buffers of each kind (three, i.e. requests two chunks ahead, measured slower: 208 against
     // 199 us at FPN-large)
-    __shared__ __attribute__((aligned(16))) u32 lds[2 * (LOWBUF + HIBUF)];
+    __shared__ __attribute__((aligned(16))) u32 lds[2 * (LOWBUF + HIBUF) + 4];
     u32 *const lowbuf = lds, *const hibuf = lds + 2 * LOWBUF;
+    // blocks of the tile with a non-finite result (in the same array: with a variable of its own the
+    // compiler waits for direct loads in other places, 258 -> 268 us at FPN-large)
+    u32 *const non_finite = lds + 2 * (LOWBUF + HIBUF);
 
     const int logical = (int)(blockIdx.x % 8) * per_xcd + (int)(blockIdx.x / 8);
     if (logical >= nblocks) return;
@@ -285,19 +246,6 @@ sapa_b_wmat16_kernel(const T *__restrict__ q, const T *__restrict__ key, const T
             if (e < 8u) ((T *)(lowbuf + (j & 1) * LOWBUF + at))[e] = last;
         }
     };
-    // Waits are counted: the counter of vector-memory operations retires in issue order, so
-    // "at most N outstanding" means that everything but the last N issued is complete.  Written out
-    // because the compiler does not track a direct load's LDS write.
-    auto wait_all_but = [&](int after) __attribute__((always_inline)) {
-#if defined(__HIP_DEVICE_COMPILE__)
-#define SAPA_WM16_WAIT(N) case N: asm volatile("s_waitcnt vmcnt(" #N ")" ::: "memory"); break;
-        switch (after) {
-            SAPA_WM16_WAIT(1) SAPA_WM16_WAIT(2) SAPA_WM16_WAIT(3) SAPA_WM16_WAIT(4)
-            default: asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); break;
-        }
-#undef SAPA_WM16_WAIT
-#endif
-    };
     // chunk jn (the first of the keys or of the values) has landed in this wave's slots: the 6
     // cells of the piece that has no address (first row of the image's first channel, tile at the
     // left edge)
@@ -309,17 +257,11 @@ sapa_b_wmat16_kernel(const T *__restrict__ q, const T *__restrict__ key, const T
             for (int k = 1; k < 4; ++k) dst[k] = __builtin_amdgcn_raw_buffer_load_b32(r, 4 * (k - 1), 0, 0);
         }
     };
-    // this wave's LDS writes are done; then every wave's (and every wave's landed loads)
-    auto barrier = [&]() __attribute__((always_inline)) {
-#if defined(__HIP_DEVICE_COMPILE__)
-        asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
-#endif
-    };
-
     const bool row_tail = W % PB != 0 && X0 + PB * ns_here > W;      // wave-uniform
     const bool active = wave < ns_here;
     const int t = wave;                                       // this wave's block of the tile
 
+    if (tid == 0) *non_finite = 0;
     low_load(0);
     low_commit(0);
     low_end(0);
@@ -328,7 +270,7 @@ sapa_b_wmat16_kernel(const T *__restrict__ q, const T *__restrict__ key, const T
     // chunk 0: all but chunk 1's loads
     wait_all_but(ODD ? 0 : ntot < 2 ? 0 : (NLP - wave * 64 + NT - 1) / NT + (1 < nKc ? NHI : 0));
     patch_low(0);
-    barrier();
+    lds_barrier();
 
     // ---- logits: Sim[cell][child], 4 x 4 accumulator blocks of 16 x 16 ----
     // block (mb, nb), lane (g, i16), element v: cell (row 2 mb + g / 2, column 4 (g % 2) + v) of the
@@ -364,7 +306,7 @@ sapa_b_wmat16_kernel(const T *__restrict__ q, const T *__restrict__ key, const T
         // chunk j + 1: nothing was issued after its loads
         wait_all_but(0);
         if (j + 1 == nKc) patch_low(nKc);
-        barrier();
+        lds_barrier();
         stage(j + 2);
     }
 
@@ -390,12 +332,12 @@ sapa_b_wmat16_kernel(const T *__restrict__ q, const T *__restrict__ key, const T
                     for (int v = 0; v < 4; ++v)
                         if (cell_outside[v]) sim[mb][nb][v] = 0.f;
         }
-        // a child of parent column px takes window columns px .. px + K - 1: -inf added to the others
+        // a child of parent column px takes window columns px .. px + K - 1: -inf for the others
         const int px = (i16 & 7) / S;
         const float NEG_INF = -__builtin_inff(), LOG2E = 1.4426950408889634f;
-        float col_bias[4];
+        bool col_in[4];
 #pragma unroll
-        for (int v = 0; v < 4; ++v) col_bias[v] = (u32)(4 * (g & 1) + v - px) < (u32)K ? 0.f : NEG_INF;
+        for (int v = 0; v < 4; ++v) col_in[v] = (u32)(4 * (g & 1) + v - px) < (u32)K;
 #pragma unroll
         for (int nb = 0; nb < 4; ++nb) {
             // child row 2 nb + i16 / 8 -> parent row pr: window rows pr .. pr + K - 1.  Block mb holds
@@ -406,10 +348,10 @@ sapa_b_wmat16_kernel(const T *__restrict__ q, const T *__restrict__ key, const T
             for (int mb = 0; mb < 4; ++mb) {
                 const bool lo_in = 2 * mb >= pr && 2 * mb < pr + K, hi_in = 2 * mb + 1 >= pr && 2 * mb + 1 < pr + K;
                 if (!lo_in && !hi_in) continue;
-                const float row_bias = lo_in && hi_in ? 0.f : ((g >> 1) ? hi_in : lo_in) ? 0.f : NEG_INF;
+                const bool row_in = (g >> 1) ? hi_in : lo_in;
 #pragma unroll
                 for (int v = 0; v < 4; ++v) {
-                    x[mb][v] = sim[mb][nb][v] + (lo_in && hi_in ? col_bias[v] : col_bias[v] + row_bias);
+                    x[mb][v] = (col_in[v] & row_in) ? sim[mb][nb][v] : NEG_INF;
                     m = fmaxf(m, x[mb][v]);
                 }
             }
@@ -451,6 +393,7 @@ sapa_b_wmat16_kernel(const T *__restrict__ q, const T *__restrict__ key, const T
     }
 
     // ---- aggregation: out[child][channel], per chunk of 16 channels ----
+    NonFinite seen;
     for (int j = nKc; j < ntot; ++j) {
         const u32 c0 = (u32)((j - nKc + vbase) * CHK);
         u32 *ob = hibuf + (j & 1) * HIBUF;                      // no loads into this ring any more
@@ -474,23 +417,22 @@ sapa_b_wmat16_kernel(const T *__restrict__ q, const T *__restrict__ key, const T
                     acc = Mma<T>::k32(whi[nb][s], b[s], acc);
                     acc = Mma<T>::k32(wlo[nb][s], b[s], acc);
                 }
+                seen.see(acc);
                 if (UP != 1.f) acc *= 1.f / UP;
                 // element v: child (row 2 nb + g / 2, column 4 (g % 2) + v), channel c0 + i16
                 const int r = 2 * nb + (g >> 1);
                 *(u32x2 *)(ob + i16 * HICH + r * HIROW + ((t ^ (swz(i16, r) & (NPC - 1))) << 2) + 2 * (g & 1)) =
                     u32x2{pack2<T>(acc[0], acc[1]), pack2<T>(acc[2], acc[3])};
-                // (no register to spare: with the products of several nb in flight the loop went through scratch
-                // memory, 68 -> 78 us at B=4, C=512, 64x64)
-                if (K == 7 && UP != 1.f) __builtin_amdgcn_sched_barrier(0);
+                // (no register to spare: with the products of several nb in flight the loop goes through scratch
+                // memory; K=7, s=4, B=4, C=512, 64x64 in bf16 71.2 us, 69.1 so)
+                if (OWN) __builtin_amdgcn_sched_barrier(0);
             }
         }
         low_commit(j + 1);
         low_end(j + 1);
         // chunk j + 1: its loads were the last operations issued
-#if defined(__HIP_DEVICE_COMPILE__)
-        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-#endif
-        barrier();
+        wait_all_but(0);
+        lds_barrier();
         // the tile's 16 channels x 8 rows, 16 bytes per lane, right after the barrier that completes
         // them (sending them behind the next chunk's matrix instructions measured slower); a piece
         // outside the tensor (ragged tile, channel past the last) lies outside the descriptor and
@@ -514,6 +456,20 @@ sapa_b_wmat16_kernel(const T *__restrict__ q, const T *__restrict__ key, const T
         }
         // (the next request behind the stores: 208 us at FPN-large against 216 with the loads first)
         if (!ODD && j + 2 < ntot) stage_low(rv, (u32)((j + 2 - nKc + vbase) * CHK), j & 1);
+    }
+
+    // ---- blocks with a non-finite result: again, term by term ----
+    if (seen.any()) atomicOr(non_finite, 1u << t);
+    lds_barrier();
+    const u32 blocks = __builtin_amdgcn_readfirstlane(*non_finite);
+    if (__builtin_expect(blocks != 0, 0)) {
+        settled();
+        const int c_hi = (vbase + nVc) * CHK < C ? (vbase + nVc) * CHK : C;
+        for (int b = 0; b < ns_here; ++b)
+            if (blocks >> b & 1)
+                exact_children<T, K, S, NT>((float *)lds, plane_of<false>(q, n, d, SS * lpix), plane_of<false>(key, n, d, lpix),
+                                            plane_of<false>(value, n, C, lpix), plane_of<false>(out, n, C, SS * lpix), d,
+                                            vbase * CHK, c_hi, H, W, S * Y0, S * X0 + 8 * b);
     }
 }
 

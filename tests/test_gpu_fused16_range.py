@@ -145,3 +145,30 @@ def test_forward_reads_nothing_behind_a_tensor(K, s, H, W, B, dtype):
         again = sapa_amd.sapa_fused(*[t.clone() for t in ops], K, s)
         want = sapa_amd.sapa_fused(*[t.double() for t in ops], K, s)
     assert torch.equal(got, again) and rel(got, want) <= one_rounding(dtype)
+
+
+def same_non_finite(got, want):
+    return (torch.equal(got.isnan(), want.isnan())
+            and torch.equal(got == float('inf'), want == float('inf')) and torch.equal(got == -float('inf'), want == -float('inf')))
+
+
+@pytest.mark.parametrize('dtype', [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize('value', [float('nan'), float('inf')])
+@pytest.mark.parametrize('which', [0, 1, 2])
+@pytest.mark.parametrize('K,s,W', [(5, 2, 24), (5, 2, 39), (5, 2, 9), (7, 4, 13), (5, 4, 22), (3, 2, 21)])
+def test_forward_keeps_non_finite_values_where_they_belong(K, s, W, which, value, dtype):
+    """One non-finite element of the query, the key or the value (inside the image and at both ends of a
+    row) reaches the results of the windows that hold it and no others."""
+    import sapa_amd
+    g = torch.Generator(device='cuda').manual_seed(W)
+    B, d, C, H = 2, 24, 40, 11
+    ops = [draw(g, sh, dtype, 0.5) for sh in ((B, d, s * H, s * W), (B, d, H, W), (B, C, H, W))]
+    ops[which][0, 3, 5, 0] = value
+    ops[which][1, 7, ops[which].shape[2] - 1, ops[which].shape[3] - 1] = value
+    ops[which][1, 2, 4, 7] = -value
+    with torch.no_grad():
+        got = sapa_amd.sapa_fused(*ops, K, s)
+        want = sapa_amd.sapa_fused(*[t.double() for t in ops], K, s)
+    assert same_non_finite(got, want)
+    ok = torch.isfinite(want)
+    assert rel(got[ok], want[ok]) <= one_rounding(dtype)
