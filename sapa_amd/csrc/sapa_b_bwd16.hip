@@ -25,10 +25,15 @@
 // Operands: A and E enter the products as a 16-bit value plus a 16-bit remainder (f16: of values brought
 // into its range, see Fit), everything else is exact in 16 bits; sums are fp32.
 //
-// Measured (B=16, C=256, d=64, 100x168, bf16): pixel kernel 310 us, cell kernel 454 us, a training step
-// 996 us against 1211 for the chain over K * K tensors (similarity and its softmax backward 274 us,
+// What a non-finite operand does to the products' cells and children outside a window is mended behind them
+// (wm16_exact.hpp): the masked logits are selected, so that the maximum and 1 / sum are the child's own
+// whatever lies around; D, the gradients of a block's queries and of its cells are formed again where
+// one of them is not finite.
+//
+// Measured (B=16, C=256, d=64, 100x168, bf16): pixel kernel 295 us, cell kernel 429 us, a training step
+// 970 us against 1211 for the chain over K * K tensors (similarity and its softmax backward 274 us,
 // grad_q 92, grad_value and grad_key by vector fmas 544, the weights 86).
-#include "wm16_common.hpp"
+#include "wm16_exact.hpp"
 
 namespace sapa {
 
@@ -39,8 +44,31 @@ using namespace wm;
 constexpr int CHK = 16;            // channels per staged chunk
 constexpr int WROWS = 8;           // window rows = child rows of a block row
 
+template <typename T> struct Args {
+    const T *q, *key, *value, *grad_out;
+    float *stats;
+    T *grad_q, *grad_key, *grad_value;
+    int B, d, C, H, W, tiles_x, tiles_y, ns, nblocks, per_xcd;
+};
+
 // position of the 16-byte piece of row r, channel ch in the swizzled tile of bwd_pixel_kernel
 __device__ __forceinline__ int swz(int ch, int r) { return ((ch & 7) << 1) | ((r + (ch >> 3)) & 1); }
+
+// the slow way of bwd_pixel_kernel for the blocks of its tile that are named
+template <typename T, int NT>
+__device__ __attribute__((noinline)) void children_again(Again again) {
+    settled();
+    const Args<T> a = again.arguments<Args<T>>();
+    const int at = (int)(again.workgroup() % 8) * a.per_xcd + (int)(again.workgroup() / 8), n = at / (a.tiles_x * a.tiles_y);
+    const int cy = 8 * (at / a.tiles_x % a.tiles_y), cx = 8 * a.ns * (at % a.tiles_x);
+    const long lpix = (long)a.H * a.W;
+    for (u32 b = 0, blocks = again.of_blocks(); blocks >> b; ++b)
+        if (blocks >> b & 1)
+            exact_grad_q<T, NT>(again.floats(), plane_of<false>(a.q, n, a.d, 4 * lpix), plane_of<false>(a.key, n, a.d, lpix),
+                                plane_of<false>(a.value, n, a.C, lpix), plane_of<false>(a.grad_out, n, a.C, 4 * lpix),
+                                plane_of<false>(a.grad_q, n, a.d, 4 * lpix), a.stats + (2L * a.B + n) * 4 * lpix, a.d, a.C, a.H, a.W,
+                                cy, cx + 8 * (int)b);
+}
 
 // ---- per-child gradients ----
 // A workgroup of 2 NSW waves owns up to NSW blocks side by side; waves t and t + NSW share block t,
@@ -49,9 +77,13 @@ __device__ __forceinline__ int swz(int ch, int r) { return ((ch & 7) << 1) | ((r
 // grad_out (G), key again (grad_q), in a ring of three buffers, the next two in flight.
 template <typename T, int NSW, bool STREAM>
 __global__ __launch_bounds__(128 * NSW) void
-bwd_pixel_kernel(const T *__restrict__ q, const T *__restrict__ key, const T *__restrict__ value,
-                 const T *__restrict__ grad_out, T *__restrict__ grad_q, float *__restrict__ stats, int B, int d, int C,
-                 int H, int W, int tiles_x, int tiles_y, int ns, int nblocks, int per_xcd) {
+bwd_pixel_kernel(const Args<T> args) {
+    const T *__restrict__ const q = args.q, *__restrict__ const key = args.key, *__restrict__ const value = args.value,
+            *__restrict__ const grad_out = args.grad_out;
+    T *__restrict__ const grad_q = args.grad_q;
+    float *__restrict__ const stats = args.stats;
+    const int B = args.B, d = args.d, C = args.C, H = args.H, W = args.W, tiles_x = args.tiles_x, tiles_y = args.tiles_y,
+              ns = args.ns, nblocks = args.nblocks, per_xcd = args.per_xcd;
     constexpr int NT = 128 * NSW;
     constexpr bool SCALED = __is_same(T, f16_t);             // E is brought into the type's range (Fit)
     constexpr int NBUF = 3;
@@ -64,8 +96,8 @@ bwd_pixel_kernel(const T *__restrict__ q, const T *__restrict__ key, const T *__
     constexpr int NPC = NSW;                                 // 16-byte pieces per tile row
     static_assert(HIBUF == 4 * NT && NLP % 64 == 0 && NLP <= NT, "one direct load per thread and buffer");
 
-    __shared__ __attribute__((aligned(16))) u32 lds[NBUF * (LOWBUF + HIBUF)];
-    u32 *const lowbuf = lds, *const hibuf = lds + NBUF * LOWBUF;
+    __shared__ __attribute__((aligned(16))) u32 lds[NBUF * (LOWBUF + HIBUF) + 4];
+    u32 *const lowbuf = lds, *const hibuf = lds + NBUF * LOWBUF, *const non_finite = lds + NBUF * (LOWBUF + HIBUF);
     const u32 low_at = lds_address((const __attribute__((address_space(3))) u32 *)lds), hi_base = low_at + NBUF * LOWBUF * 4;
 
     const int logical = (int)(blockIdx.x % 8) * per_xcd + (int)(blockIdx.x / 8);
@@ -145,6 +177,7 @@ bwd_pixel_kernel(const T *__restrict__ q, const T *__restrict__ key, const T *__
     const bool row_tail = (W & 3) != 0 && X0 + 4 * ns_here > W;      // workgroup-uniform
     const bool active = t < ns_here;
 
+    if (tid == 0) *non_finite = 0;          // blocks of the tile with a non-finite result
     stage(0);
     stage(1);
     for (int j = 2; j < NBUF; ++j) stage(j);
@@ -211,24 +244,23 @@ bwd_pixel_kernel(const T *__restrict__ q, const T *__restrict__ key, const T *__
     };
     f32x4 p[4][2];
     float mlog[2], inv[2];
+    // whether element v of block (mb, nb) lies in its child's window: parent row 2 half + nb and column px take
+    // window rows and columns from theirs on, 5 of each
+    const int px = (i16 & 7) >> 1;
+    auto inside = [&](int mb, int nb, int v) __attribute__((always_inline)) {
+        return ((u32)(4 * (g & 1) + v - px) <= 4u) & ((u32)(2 * mb + (g >> 1) - (2 * half + nb)) <= 4u);
+    };
     if (active) {
         clear_outside(acc);
-        const int px = (i16 & 7) >> 1;
         const float NEG_INF = -__builtin_inff();
-        float col_bias[4];
-#pragma unroll
-        for (int v = 0; v < 4; ++v) col_bias[v] = (u32)(4 * (g & 1) + v - px) <= 4u ? 0.f : NEG_INF;
 #pragma unroll
         for (int nb = 0; nb < 2; ++nb) {
-            // parent row 2 half + nb: window rows 2 half + nb .. + 4 take part
-            const int pr = 2 * half + nb;
             float m = NEG_INF;
 #pragma unroll
             for (int mb = 0; mb < 4; ++mb) {
-                const float row_bias = (u32)(2 * mb + (g >> 1) - pr) <= 4u ? 0.f : NEG_INF;
 #pragma unroll
                 for (int v = 0; v < 4; ++v) {
-                    p[mb][nb][v] = acc[mb][nb][v] + (col_bias[v] + row_bias);
+                    p[mb][nb][v] = inside(mb, nb, v) ? acc[mb][nb][v] : NEG_INF;
                     m = fmaxf(m, p[mb][nb][v]);
                 }
             }
@@ -263,6 +295,7 @@ bwd_pixel_kernel(const T *__restrict__ q, const T *__restrict__ key, const T *__
 
     // ---- gradient of the logits; what the cell kernel needs to form it again ----
     u32x4 whi[2][2], wlo[2][2];
+    NonFinite seen;
     float down[2][4];           // f16: what the results of child 4 g + v of block nb are multiplied by
     if (active) {
         clear_outside(acc);
@@ -275,6 +308,7 @@ bwd_pixel_kernel(const T *__restrict__ q, const T *__restrict__ key, const T *__
                 for (int v = 0; v < 4; ++v) dsum = __builtin_fmaf(p[mb][nb][v], acc[mb][nb][v], dsum);
             dsum += __shfl_xor(dsum, 16);
             dsum += __shfl_xor(dsum, 32);
+            seen.see(dsum);
             const int cy = 2 * Y0 + 2 * (2 * half + nb) + (i16 >> 3), cx = 2 * X0 + 8 * t + (i16 & 7);
             if (g < 3 && cy < 2 * H && cx < 2 * W) {
                 // planes [3][B, 2H, 2W]: maximum (times log2 e), 1 / sum, D; lanes g = 0, 1, 2 one each
@@ -301,7 +335,6 @@ bwd_pixel_kernel(const T *__restrict__ q, const T *__restrict__ key, const T *__
             for (int s = 0; s < 2; ++s) split8<T>(e[s], whi[nb][s], wlo[nb][s]);
         }
     }
-    if (!grad_q) return;
 
     // ---- grad_q[child][channel], per chunk of 16 channels, through the hi-res tile ----
     const __amdgpu_buffer_rsrc_t ro = __builtin_amdgcn_make_buffer_rsrc(
@@ -326,6 +359,7 @@ bwd_pixel_kernel(const T *__restrict__ q, const T *__restrict__ key, const T *__
                     o = Mma<T>::k32(whi[nb][s], b[s], o);
                     o = Mma<T>::k32(wlo[nb][s], b[s], o);
                 }
+                seen.see(o);
                 if (SCALED) {
 #pragma unroll
                     for (int v = 0; v < 4; ++v) o[v] *= down[nb][v];
@@ -349,6 +383,12 @@ bwd_pixel_kernel(const T *__restrict__ q, const T *__restrict__ key, const T *__
         __builtin_amdgcn_raw_buffer_store_b128(o, ro, off, 0, STREAM ? 2 : 0);
         stage(j + NBUF);
     }
+
+    // ---- blocks with a non-finite result: again, term by term ----
+    if (seen.any()) atomicOr(non_finite, 1u << t);
+    lds_barrier();
+    const u32 blocks = __builtin_amdgcn_readfirstlane(*non_finite);
+    if (__builtin_expect(blocks != 0, 0)) children_again<T, NT>(Again(lds, blocks));
 }
 
 // ---- per-cell gradients ----
@@ -377,7 +417,7 @@ constexpr int CNL = CLOW / 256;            // waves that a round over a chunk's 
 static_assert(CHI / 4 == CNH * CNT + 256 && CLOW % 256 == 0, "waves 0 .. 3 load the rest of the tile, waves 4 .. the cells");
 constexpr int CSTAT = 5 * 256;             // floats of one stats plane: 16 rows of 8 CPC, in whole loads of 5 waves
 static_assert(TBX == 8 && 16 * 8 * CPC <= CSTAT && 2 * CSTAT <= 4 * COUT, "stats planes");
-static_assert((CBUF * (CHI + CLOW) + CSTAT + 4 * COUT) * 4 <= 160 * 1024, "LDS");
+static_assert((CBUF * (CHI + CLOW) + CSTAT + 4 * COUT + 4) * 4 <= 160 * 1024, "LDS");
 
 // dword of piece `pc` of hi-res row r, channel ch
 __device__ __forceinline__ int hi_at(int ch, int r, int pc) {
@@ -392,19 +432,39 @@ __device__ __forceinline__ int out_at(int ch, int row, int bi) {
     return ((ch * 4 + row) ^ ((ch >> 3) & 1)) * 4 * TBX + 4 * (bi ^ (ch & 7));
 }
 
+// the slow way of bwd_cell_kernel for the cell blocks of its tile that are named
+template <typename T>
+__device__ __attribute__((noinline)) void cells_again(Again again) {
+    settled();
+    const Args<T> a = again.arguments<Args<T>>();
+    const int at = (int)(again.workgroup() % 8) * a.per_xcd + (int)(again.workgroup() / 8), n = at / (a.tiles_x * a.tiles_y);
+    const int cy = 4 * (at / a.tiles_x % a.tiles_y) - 2, cx = 4 * TBX * (at % a.tiles_x) - 2;
+    const long lpix = (long)a.H * a.W;
+    for (u32 b = 0, blocks = again.of_blocks(); blocks >> b; ++b)
+        if (blocks >> b & 1)
+            exact_grad_cells<T, CNT>(again.floats(), plane_of<false>(a.q, n, a.d, 4 * lpix), plane_of<false>(a.key, n, a.d, lpix),
+                                     plane_of<false>(a.value, n, a.C, lpix), plane_of<false>(a.grad_out, n, a.C, 4 * lpix),
+                                     a.stats + n * 4 * lpix, (long)a.B * 4 * lpix, plane_of<false>(a.grad_key, n, a.d, lpix),
+                                     plane_of<false>(a.grad_value, n, a.C, lpix), a.d, a.C, a.H, a.W, cy, cx + 4 * (int)b);
+}
+
 template <typename T>
 __global__ __launch_bounds__(CNT) void
-bwd_cell_kernel(const T *__restrict__ q, const T *__restrict__ key, const T *__restrict__ value,
-                const T *__restrict__ grad_out, const float *__restrict__ stats, T *__restrict__ grad_key,
-                T *__restrict__ grad_value, int B, int d, int C, int H, int W, int tiles_x, int tiles_y, int nblocks,
-                int per_xcd) {
+bwd_cell_kernel(const Args<T> args) {
+    const T *__restrict__ const q = args.q, *__restrict__ const key = args.key, *__restrict__ const value = args.value,
+            *__restrict__ const grad_out = args.grad_out;
+    T *__restrict__ const grad_key = args.grad_key, *__restrict__ const grad_value = args.grad_value;
+    const float *__restrict__ const stats = args.stats;
+    const int B = args.B, d = args.d, C = args.C, H = args.H, W = args.W, tiles_x = args.tiles_x, tiles_y = args.tiles_y,
+              nblocks = args.nblocks, per_xcd = args.per_xcd;
     constexpr bool SCALED = __is_same(T, f16_t);             // A and E are brought into the type's range (Fit)
-    __shared__ __attribute__((aligned(16))) u32 lds[CBUF * (CHI + CLOW) + CSTAT + 4 * COUT];
+    __shared__ __attribute__((aligned(16))) u32 lds[CBUF * (CHI + CLOW) + CSTAT + 4 * COUT + 4];
     u32 *const hibuf = lds, *const lowbuf = lds + CBUF * CHI;
     const u32 hi_base = lds_address((const __attribute__((address_space(3))) u32 *)lds), low_at = hi_base + CBUF * CHI * 4;
     // D in front, the other stats planes over the results [chunk % 2][half][16][4 rows][4 TBX cells]
     float *const statbuf = (float *)(lowbuf + CBUF * CLOW), *const outbuf = statbuf + CSTAT;
     const u32 stat_at = low_at + CBUF * CLOW * 4;
+    u32 *const non_finite = (u32 *)(outbuf + 4 * COUT);       // cell blocks with a non-finite result
 
     const int logical = (int)(blockIdx.x % 8) * per_xcd + (int)(blockIdx.x / 8);
     if (logical >= nblocks) return;
@@ -505,6 +565,7 @@ bwd_cell_kernel(const T *__restrict__ q, const T *__restrict__ key, const T *__r
 #pragma unroll
             for (int s = 0; s < 2; ++s) split8<T>(w[qx][s], whi[qx][s], wlo[qx][s]);
     };
+    NonFinite seen;
     auto gather = [&](int j) __attribute__((always_inline)) {
         const u32 *hb = hibuf + j % CBUF * CHI;
         f32x4 o = f32x4{0.f, 0.f, 0.f, 0.f};
@@ -517,6 +578,7 @@ bwd_cell_kernel(const T *__restrict__ q, const T *__restrict__ key, const T *__r
                 o = Mma<T>::k32(whi[qx][s], b, o);
                 o = Mma<T>::k32(wlo[qx][s], b, o);
             }
+        seen.see(o);
         if (SCALED) {
 #pragma unroll
             for (int v = 0; v < 4; ++v) o[v] *= down[v];
@@ -569,6 +631,7 @@ bwd_cell_kernel(const T *__restrict__ q, const T *__restrict__ key, const T *__r
         load_lds(dma_rsrc(stats + ((long)((k + 2) % 3) * B + n) * 4 * lpix, (u32)(16 * lpix)), stat_at + (k * CSTAT + wave % 5 * 256) * 4,
                  ok ? (u32)(cy * 2 * W + cx) * 4u : OUTSIDE);
     }
+    if (tid == 0) *non_finite = 0;
 #pragma unroll
     for (int j = 0; j < CBUF - 1; ++j) stage(j);
     next(-1, 0);
@@ -578,6 +641,7 @@ bwd_cell_kernel(const T *__restrict__ q, const T *__restrict__ key, const T *__r
         return *(const f32x4 *)(statbuf + k * CSTAT + (8 * (1 - qy) + 2 * nb + (g >> 1)) * 8 * CPC + 8 * (bi + 1 - qx) + 4 * (g & 1));
     };
     const int cr = i16 >> 2, cc = i16 & 3;
+    const bool cell_in = (u32)(4 * (I0 + bi) - 2 + cc) < (u32)W;
 
     f32x4 acc[2][4];
 #pragma unroll
@@ -603,10 +667,10 @@ bwd_cell_kernel(const T *__restrict__ q, const T *__restrict__ key, const T *__r
                     const bool row_ok = qy ? cr <= nb : cr >= nb;
 #pragma unroll
                     for (int v = 0; v < 4; ++v) {
-                        // (a child right of the image is one of the next row's, whose product with this
-                        // cell no maximum bounds: it must not count, whatever it is)
+                        // (a child or a cell beside the image is one of a neighbouring row's, whose products
+                        // no maximum bounds: it must not count, whatever it is)
                         const int px = 2 * (g & 1) + (v >> 1);
-                        const bool ok = row_ok & (qx ? cc <= px : cc >= px) & (4 * (I0 + bi - qx) + px < W);
+                        const bool ok = row_ok & (qx ? cc <= px : cc >= px) & (4 * (I0 + bi - qx) + px < W) & cell_in;
                         const float e = __builtin_amdgcn_exp2f(__builtin_fmaf(acc[qx][nb][v], LOG2E, -mlog[v]));
                         w[qx][s][4 * k + v] = ok ? e * inv[v] : 0.f;
                     }
@@ -634,32 +698,39 @@ bwd_cell_kernel(const T *__restrict__ q, const T *__restrict__ key, const T *__r
             store(j, ro, (u32)((j - nKc) * CHK));
         }
     }
-    if (!grad_key) return;
 
     // ---- E = A (G - D), grad_key ----
-    if (active) {
-        float w[2][2][8];
+    if (grad_key) {
+        if (active) {
+            float w[2][2][8];
 #pragma unroll
-        for (int qx = 0; qx < 2; ++qx)
+            for (int qx = 0; qx < 2; ++qx)
 #pragma unroll
-            for (int s = 0; s < 2; ++s)
+                for (int s = 0; s < 2; ++s)
 #pragma unroll
-                for (int k = 0; k < 2; ++k) {
-                    const int nb = 2 * s + k;
-                    const f32x4 dsum = child_stats(0, qx, nb);
+                    for (int k = 0; k < 2; ++k) {
+                        const int nb = 2 * s + k;
+                        const f32x4 dsum = child_stats(0, qx, nb);
 #pragma unroll
-                    for (int v = 0; v < 4; ++v)
-                        w[qx][s][4 * k + v] = joined<T>(whi[qx][s], wlo[qx][s], 4 * k + v) * f.down * (acc[qx][nb][v] - dsum[v]);
-                }
-        hold(w);
+                        for (int v = 0; v < 4; ++v)
+                            w[qx][s][4 * k + v] = joined<T>(whi[qx][s], wlo[qx][s], 4 * k + v) * f.down * (acc[qx][nb][v] - dsum[v]);
+                    }
+            hold(w);
+        }
+        const __amdgpu_buffer_rsrc_t ro = __builtin_amdgcn_make_buffer_rsrc(
+            (void *)(grad_key + (long)n * d * lpix), 0, (int)(d * lplane), 0x00020000);
+        for (int j = nKc + nVc; j < ntot; ++j) {
+            if (active) gather(j);
+            next(j, j - nKc);
+            store(j, ro, (u32)((j - nKc - nVc) * CHK));
+        }
     }
-    const __amdgpu_buffer_rsrc_t ro = __builtin_amdgcn_make_buffer_rsrc(
-        (void *)(grad_key + (long)n * d * lpix), 0, (int)(d * lplane), 0x00020000);
-    for (int j = nKc + nVc; j < ntot; ++j) {
-        if (active) gather(j);
-        next(j, j - nKc);
-        store(j, ro, (u32)((j - nKc - nVc) * CHK));
-    }
+
+    // ---- blocks with a non-finite result: again, term by term ----
+    if (seen.any()) atomicOr(non_finite, 1u << bi);
+    lds_barrier();
+    const u32 blocks = __builtin_amdgcn_readfirstlane(*non_finite);
+    if (__builtin_expect(blocks != 0, 0)) cells_again<T>(Again(lds, blocks));
 }
 
 template <typename T, bool STREAM>
@@ -667,29 +738,27 @@ static hipError_t launch(const void *q, const void *key, const void *value, cons
                          void *grad_q, void *grad_key, void *grad_value, int B, int d, int C, int H, int W,
                          hipStream_t st) {
     constexpr int NSW = 8;
+    Args<T> args{(const T *)q, (const T *)key, (const T *)value, (const T *)grad_out, stats, (T *)grad_q, (T *)grad_key,
+                 (T *)grad_value, B, d, C, H, W, 0, 0, 0, 0, 0};
+    // sets the tiles; false: too many
+    auto tile = [&](int tiles_x, int tiles_y) {
+        const long nb = (long)tiles_x * tiles_y * B;
+        args.tiles_x = tiles_x, args.tiles_y = tiles_y, args.nblocks = (int)nb, args.per_xcd = (int)((nb + 7) / 8);
+        return nb <= (1L << 30);
+    };
     {
         const int nsx = (W + 3) / 4;
-        const int tiles_x = (nsx + NSW - 1) / NSW, tiles_y = (H + 3) / 4;
-        const int ns = (nsx + tiles_x - 1) / tiles_x;         // blocks per tile, balanced over the row
-        const long nb = (long)tiles_x * tiles_y * B;
-        if (nb > (1L << 30)) return hipErrorNotSupported;
-        const int per_xcd = (int)((nb + 7) / 8);
-        hipLaunchKernelGGL((bwd_pixel_kernel<T, NSW, STREAM>), dim3(per_xcd * 8), dim3(128 * NSW), 0, st, (const T *)q,
-                           (const T *)key, (const T *)value, (const T *)grad_out, (T *)grad_q, stats, B, d, C, H, W,
-                           tiles_x, tiles_y, ns, (int)nb, per_xcd);
+        if (!tile((nsx + NSW - 1) / NSW, (H + 3) / 4)) return hipErrorNotSupported;
+        args.ns = (nsx + args.tiles_x - 1) / args.tiles_x;    // blocks per tile, balanced over the row
+        hipLaunchKernelGGL((bwd_pixel_kernel<T, NSW, STREAM>), dim3(args.per_xcd * 8), dim3(128 * NSW), 0, st, args);
         const hipError_t e = hipGetLastError();
         if (e != hipSuccess) return e;
     }
     if (!grad_key && !grad_value) return hipSuccess;
     // cell blocks 4 I - 2 .. 4 I + 1 that hold a cell of 0 .. W - 1
     const int nI = (W + 1) / 4 + 1, nJ = (H + 1) / 4 + 1;
-    const int tiles_x = (nI + TBX - 1) / TBX, tiles_y = nJ;
-    const long nb = (long)tiles_x * tiles_y * B;
-    if (nb > (1L << 30)) return hipErrorNotSupported;
-    const int per_xcd = (int)((nb + 7) / 8);
-    hipLaunchKernelGGL((bwd_cell_kernel<T>), dim3(per_xcd * 8), dim3(CNT), 0, st, (const T *)q, (const T *)key,
-                       (const T *)value, (const T *)grad_out, stats, (T *)grad_key, (T *)grad_value, B, d, C, H, W,
-                       tiles_x, tiles_y, (int)nb, per_xcd);
+    if (!tile((nI + TBX - 1) / TBX, nJ)) return hipErrorNotSupported;
+    hipLaunchKernelGGL((bwd_cell_kernel<T>), dim3(args.per_xcd * 8), dim3(CNT), 0, st, args);
     return hipGetLastError();
 }
 

@@ -10,11 +10,13 @@
 // through ds_read_tr16_b64 and leave 4 (8) consecutive channels in a lane; every position is a whole
 // unit of memory, so tiles have no edge cases, W may be odd, and a halo costs only its own bytes.
 //
-// Measured: a training step at B=16, C=256, d=64, 100x168 in bf16 0.72 ms (pixel kernel 241 us, cell
-// kernel 367) against 1.64 through copies into contiguous order and the chain over K * K tensors; at B=8,
+// Non-finite operands: as there.
+//
+// Measured: a training step at B=16, C=256, d=64, 100x168 in bf16 0.73 ms (pixel kernel 206 us, cell
+// kernel 342) against 1.64 through copies into contiguous order and the chain over K * K tensors; at B=8,
 // C=256, d=32, 64x64 in fp16 148 us against 271 (26 + 47 us).  The pixel kernel waits for memory (1.0 GB);
 // the cell kernel for LDS and L2: every hi-res value is staged 1.9 times and read by four blocks.
-#include "wm16_common.hpp"
+#include "wm16_exact.hpp"
 
 namespace sapa {
 
@@ -31,6 +33,13 @@ __device__ __forceinline__ void arrived(u32x4 &v) {
 #endif
 }
 
+template <typename T> struct Args {
+    const T *q, *key, *value, *grad_out;
+    float *stats;
+    T *grad_q, *grad_key, *grad_value;
+    int B, d, C, H, W, tiles_x, tiles_y, ns, nblocks, per_xcd;
+};
+
 // ---- per-child gradients ----
 // A workgroup of 2 NSW waves owns up to NSW blocks of 4 x 4 parents side by side; waves t and t + NSW
 // share block t, 32 of its children each.  Windows of 64 channels in two LDS buffers; q and grad_out go
@@ -45,18 +54,39 @@ constexpr int OSLOT = 16 * CELL;   // dwords of a wave's output slot: 16 childre
 // dword offset of the 16-byte piece `piece` (0..7) of cell / child `idx` in a [idx][64 channels] array
 __device__ __forceinline__ int piece_at(int idx, int piece) { return idx * CELL + ((piece ^ (idx & 7)) << 2); }
 
+// its slow way for the blocks of a tile that are named
+template <typename T>
+__device__ __attribute__((noinline)) void children_again(Again again) {
+    settled();
+    const Args<T> a = again.arguments<Args<T>>();
+    const int at = (int)(again.workgroup() % 8) * a.per_xcd + (int)(again.workgroup() / 8), n = at / (a.tiles_x * a.tiles_y);
+    const int cy = 8 * (at / a.tiles_x % a.tiles_y), cx = 8 * a.ns * (at % a.tiles_x);
+    const long lpix = (long)a.H * a.W;
+    for (u32 b = 0, blocks = again.of_blocks(); blocks >> b; ++b)
+        if (blocks >> b & 1)
+            exact_grad_q<T, 128 * NSW>(again.floats(), plane_of<true>(a.q, n, a.d, 4 * lpix), plane_of<true>(a.key, n, a.d, lpix),
+                                       plane_of<true>(a.value, n, a.C, lpix), plane_of<true>(a.grad_out, n, a.C, 4 * lpix),
+                                       plane_of<true>(a.grad_q, n, a.d, 4 * lpix), a.stats + (2L * a.B + n) * 4 * lpix, a.d, a.C,
+                                       a.H, a.W, cy, cx + 8 * (int)b);
+}
+
 template <typename T, bool STREAM>
 __global__ __launch_bounds__(128 * NSW, 4) void
-bwd_pixel_kernel(const T *__restrict__ q, const T *__restrict__ key, const T *__restrict__ value,
-                 const T *__restrict__ grad_out, T *__restrict__ grad_q, float *__restrict__ stats, int B, int d, int C,
-                 int H, int W, int tiles_x, int tiles_y, int ns, int nblocks, int per_xcd) {
+bwd_pixel_kernel(const Args<T> args) {
+    const T *__restrict__ const q = args.q, *__restrict__ const key = args.key, *__restrict__ const value = args.value,
+            *__restrict__ const grad_out = args.grad_out;
+    T *__restrict__ const grad_q = args.grad_q;
+    float *__restrict__ const stats = args.stats;
+    const int B = args.B, d = args.d, C = args.C, H = args.H, W = args.W, tiles_x = args.tiles_x, tiles_y = args.tiles_y,
+              ns = args.ns, nblocks = args.nblocks, per_xcd = args.per_xcd;
     constexpr int NT = 128 * NSW;
     constexpr int NLP = LOWBUF / 4;                          // 16-byte pieces per window buffer
     constexpr int NLI = (NLP + NT - 1) / NT;                 // direct loads per thread and window, at most
     static_assert(NLP % 64 == 0, "whole direct loads");
     constexpr int STREAM_AUX = STREAM ? 2 : 0;
     constexpr bool SCALED = __is_same(T, f16_t);             // E is brought into the type's range (Fit)
-    __shared__ __attribute__((aligned(16))) u32 lds[2 * LOWBUF + 2 * NSW * OSLOT];
+    __shared__ __attribute__((aligned(16))) u32 lds[2 * LOWBUF + 2 * NSW * OSLOT + 4];
+    u32 *const non_finite = lds + 2 * LOWBUF + 2 * NSW * OSLOT;          // blocks of the tile with a non-finite result
     const u32 low_at = lds_address((const __attribute__((address_space(3))) u32 *)lds);
 
     const int logical = (int)(blockIdx.x % 8) * per_xcd + (int)(blockIdx.x / 8);
@@ -161,6 +191,7 @@ bwd_pixel_kernel(const T *__restrict__ q, const T *__restrict__ key, const T *__
     };
     f32x4 acc[4][2];
     Hi h0, h1;
+    if (tid == 0) *non_finite = 0;
     stage(0);
     fetch(0, h0);
     fetch(1, h1);
@@ -181,22 +212,20 @@ bwd_pixel_kernel(const T *__restrict__ q, const T *__restrict__ key, const T *__
     // ---- softmax over each child's 5 x 5 cells ----
     f32x4 p[4][2];
     float mlog[2], inv[2];
+    const int px = (i16 & 7) >> 1;
+    auto inside = [&](int mb, int nb, int v) __attribute__((always_inline)) {
+        return ((u32)(4 * (g & 1) + v - px) <= 4u) & ((u32)(2 * mb + (g >> 1) - (2 * half + nb)) <= 4u);
+    };
     if (active) {
-        const int px = (i16 & 7) >> 1;
         const float NEG_INF = -__builtin_inff();
-        float col_bias[4];
-#pragma unroll
-        for (int v = 0; v < 4; ++v) col_bias[v] = (u32)(4 * (g & 1) + v - px) <= 4u ? 0.f : NEG_INF;
 #pragma unroll
         for (int nb = 0; nb < 2; ++nb) {
-            const int pr = 2 * half + nb;
             float m = NEG_INF;
 #pragma unroll
             for (int mb = 0; mb < 4; ++mb) {
-                const float row_bias = (u32)(2 * mb + (g >> 1) - pr) <= 4u ? 0.f : NEG_INF;
 #pragma unroll
                 for (int v = 0; v < 4; ++v) {
-                    p[mb][nb][v] = acc[mb][nb][v] + (col_bias[v] + row_bias);
+                    p[mb][nb][v] = inside(mb, nb, v) ? acc[mb][nb][v] : NEG_INF;
                     m = fmaxf(m, p[mb][nb][v]);
                 }
             }
@@ -231,6 +260,7 @@ bwd_pixel_kernel(const T *__restrict__ q, const T *__restrict__ key, const T *__
 
     // ---- gradient of the logits; what the cell kernel needs to form it again ----
     u32x4 whi[2][2], wlo[2][2];
+    NonFinite seen;
     float down[2];              // f16: what the results of this lane's child of block nb are multiplied by
     if (active) {
 #pragma unroll
@@ -239,7 +269,12 @@ bwd_pixel_kernel(const T *__restrict__ q, const T *__restrict__ key, const T *__
 #pragma unroll
             for (int mb = 0; mb < 4; ++mb)
 #pragma unroll
-                for (int v = 0; v < 4; ++v) dsum = __builtin_fmaf(p[mb][nb][v], acc[mb][nb][v], dsum);
+                for (int v = 0; v < 4; ++v) {
+                    // (as sapa_b_bwd16.hip has it, without this, the kernel needs 20 registers more than there are:
+                    // B=16, C=256, 100x168 in bf16 584 us for both kernels, 545 so)
+                    if (!inside(mb, nb, v)) acc[mb][nb][v] = 0.f;
+                    dsum = __builtin_fmaf(p[mb][nb][v], acc[mb][nb][v], dsum);
+                }
             dsum += __shfl_xor(dsum, 16);
             dsum += __shfl_xor(dsum, 32);
             if (g < 3 && child[nb] != OUTSIDE)
@@ -264,7 +299,6 @@ bwd_pixel_kernel(const T *__restrict__ q, const T *__restrict__ key, const T *__
             for (int s = 0; s < 2; ++s) split8<T>(e[s], whi[nb][s], wlo[nb][s]);
         }
     }
-    if (!grad_q) return;
 
     // ---- grad_q^T[channel][child], per chunk of 64 channels, through this wave's slot ----
     const __amdgpu_buffer_rsrc_t ro = __builtin_amdgcn_make_buffer_rsrc(
@@ -295,6 +329,7 @@ bwd_pixel_kernel(const T *__restrict__ q, const T *__restrict__ key, const T *__
                         o = Mma<T>::k32(va[mk][s], whi[nb][s], o);
                         o = Mma<T>::k32(va[mk][s], wlo[nb][s], o);
                     }
+                    seen.see(o);
                     if (SCALED) o *= down[nb];
                     *(u32x2 *)(oslot + piece_at(i16, 2 * mk + (g >> 1)) + 2 * (g & 1)) =
                         u32x2{pack2<T>(o[0], o[1]), pack2<T>(o[2], o[3])};
@@ -315,6 +350,12 @@ bwd_pixel_kernel(const T *__restrict__ q, const T *__restrict__ key, const T *__
             stage(j + 2);
         }
     }
+
+    // ---- blocks with a non-finite result: again, term by term ----
+    if (seen.any()) atomicOr(non_finite, 1u << t);
+    lds_barrier();
+    const u32 blocks = __builtin_amdgcn_readfirstlane(*non_finite);
+    if (__builtin_expect(blocks != 0, 0)) children_again<T>(Again(lds, blocks));
 }
 
 // ---- per-cell gradients ----
@@ -331,17 +372,38 @@ constexpr int CNH = (CHI / 4 + CNT - 1) / CNT;
 constexpr int CPART = 64 * TBX * TBY * 8;          // floats of a chunk's handed-over sums
 constexpr int CSTAT = 1024;                        // floats of one stats plane (24 x 40), in whole loads of 4 waves
 static_assert(XR * XC <= CSTAT && 2 * CSTAT <= 2 * CPART, "stats planes");
-static_assert((2 * CHI + CSTAT + 2 * CPART) * 4 <= 160 * 1024, "LDS");
+static_assert((2 * CHI + CSTAT + 2 * CPART + 4) * 4 <= 160 * 1024, "LDS");
 static_assert(XC % 8 == 0 && CNT % 64 == 0, "piece permutation");
+
+// the slow way of bwd_cell_kernel for the cell blocks of its tile that are named
+template <typename T>
+__device__ __attribute__((noinline)) void cells_again(Again again) {
+    settled();
+    const Args<T> a = again.arguments<Args<T>>();
+    const int at = (int)(again.workgroup() % 8) * a.per_xcd + (int)(again.workgroup() / 8), n = at / (a.tiles_x * a.tiles_y);
+    const int cy = 4 * TBY * (at / a.tiles_x % a.tiles_y) - 2, cx = 4 * TBX * (at % a.tiles_x) - 2;
+    const long lpix = (long)a.H * a.W;
+    for (u32 b = 0, blocks = again.of_blocks(); blocks >> b; ++b)
+        if (blocks >> b & 1)
+            exact_grad_cells<T, CNT>(again.floats(), plane_of<true>(a.q, n, a.d, 4 * lpix), plane_of<true>(a.key, n, a.d, lpix),
+                                     plane_of<true>(a.value, n, a.C, lpix), plane_of<true>(a.grad_out, n, a.C, 4 * lpix),
+                                     a.stats + n * 4 * lpix, (long)a.B * 4 * lpix, plane_of<true>(a.grad_key, n, a.d, lpix),
+                                     plane_of<true>(a.grad_value, n, a.C, lpix), a.d, a.C, a.H, a.W, cy + 4 * (int)(b / TBX),
+                                     cx + 4 * (int)(b % TBX));
+}
 
 template <typename T>
 __global__ __launch_bounds__(CNT) void
-bwd_cell_kernel(const T *__restrict__ q, const T *__restrict__ key, const T *__restrict__ value,
-                const T *__restrict__ grad_out, const float *__restrict__ stats, T *__restrict__ grad_key,
-                T *__restrict__ grad_value, int B, int d, int C, int H, int W, int tiles_x, int tiles_y, int nblocks,
-                int per_xcd) {
+bwd_cell_kernel(const Args<T> args) {
+    const T *__restrict__ const q = args.q, *__restrict__ const key = args.key, *__restrict__ const value = args.value,
+            *__restrict__ const grad_out = args.grad_out;
+    T *__restrict__ const grad_key = args.grad_key, *__restrict__ const grad_value = args.grad_value;
+    const float *__restrict__ const stats = args.stats;
+    const int B = args.B, d = args.d, C = args.C, H = args.H, W = args.W, tiles_x = args.tiles_x, tiles_y = args.tiles_y,
+              nblocks = args.nblocks, per_xcd = args.per_xcd;
     constexpr bool SCALED = __is_same(T, f16_t);             // A and E are brought into the type's range (Fit)
-    __shared__ __attribute__((aligned(16))) u32 lds[2 * CHI + CSTAT + 2 * CPART];
+    __shared__ __attribute__((aligned(16))) u32 lds[2 * CHI + CSTAT + 2 * CPART + 4];
+    u32 *const non_finite = lds + 2 * CHI + CSTAT + 2 * CPART;           // cell blocks with a non-finite result
     float *const statbuf = (float *)(lds + 2 * CHI), *const part = statbuf + CSTAT;   // (D; the other planes over `part`)
     const u32 hi_base = lds_address((const __attribute__((address_space(3))) u32 *)lds);
 
@@ -447,6 +509,7 @@ bwd_cell_kernel(const T *__restrict__ q, const T *__restrict__ key, const T *__r
 #pragma unroll
             for (int s = 0; s < 2; ++s) split8<T>(w[qx][s], whi[qx][s], wlo[qx][s]);
     };
+    NonFinite seen;
     auto gather = [&](int j, f32x4 (&o)[2]) __attribute__((always_inline)) {
         const u32 *hb = lds + (j & 1) * CHI;
 #pragma unroll
@@ -461,6 +524,7 @@ bwd_cell_kernel(const T *__restrict__ q, const T *__restrict__ key, const T *__r
                     o[h] = Mma<T>::k32(a, whi[qx][s], o[h]);
                     o[h] = Mma<T>::k32(a, wlo[qx][s], o[h]);
                 }
+            seen.see(o[h]);
             if (SCALED) o[h] *= f.down;
         }
         if (qy) {
@@ -500,6 +564,7 @@ bwd_cell_kernel(const T *__restrict__ q, const T *__restrict__ key, const T *__r
             for (int nb = 0; nb < 4; ++nb) acc[qx][nb] = f32x4{0.f, 0.f, 0.f, 0.f};
     };
     zero();
+    if (tid == 0) *non_finite = 0;
     stage(0);
     u32x4 l0 = fetch(0), l1 = fetch(1);
     wait_all_but(0);
@@ -563,61 +628,66 @@ bwd_cell_kernel(const T *__restrict__ q, const T *__restrict__ key, const T *__r
             if (active && !qy) store(j, o, ro, C, (j - nKc) * CCH);
         }
     }
-    if (!grad_key) return;
 
     // ---- E = A (G - D), grad_key ----
-    if (active) {
-        float w[2][2][8];
+    if (grad_key) {
+        if (active) {
+            float w[2][2][8];
 #pragma unroll
-        for (int qx = 0; qx < 2; ++qx)
+            for (int qx = 0; qx < 2; ++qx)
 #pragma unroll
-            for (int s = 0; s < 2; ++s)
+                for (int s = 0; s < 2; ++s)
 #pragma unroll
-                for (int k = 0; k < 2; ++k) {
-                    const int nb = 2 * s + k;
-                    const f32x4 dsum = child_stats(0, qx, nb);
+                    for (int k = 0; k < 2; ++k) {
+                        const int nb = 2 * s + k;
+                        const f32x4 dsum = child_stats(0, qx, nb);
 #pragma unroll
-                    for (int v = 0; v < 4; ++v)
-                        w[qx][s][4 * k + v] = joined<T>(whi[qx][s], wlo[qx][s], 4 * k + v) * f.down * (acc[qx][nb][v] - dsum[v]);
-                }
-        hold(w);
+                        for (int v = 0; v < 4; ++v)
+                            w[qx][s][4 * k + v] = joined<T>(whi[qx][s], wlo[qx][s], 4 * k + v) * f.down * (acc[qx][nb][v] - dsum[v]);
+                    }
+            hold(w);
+        }
+        const __amdgpu_buffer_rsrc_t ro = __builtin_amdgcn_make_buffer_rsrc(
+            (void *)(grad_key + (long)n * d * lpix), 0, (int)(d * lpix * (long)sizeof(T)), 0x00020000);
+        for (; j < ntot; ++j) {
+            if (active) gather(j, o);
+            next(j, active && !qy);
+            if (active && !qy) store(j, o, ro, d, (j - nKc - nVc) * CCH);
+        }
     }
-    const __amdgpu_buffer_rsrc_t ro = __builtin_amdgcn_make_buffer_rsrc(
-        (void *)(grad_key + (long)n * d * lpix), 0, (int)(d * lpix * (long)sizeof(T)), 0x00020000);
-    for (; j < ntot; ++j) {
-        if (active) gather(j, o);
-        next(j, active && !qy);
-        if (active && !qy) store(j, o, ro, d, (j - nKc - nVc) * CCH);
-    }
+
+    // ---- blocks with a non-finite result: again, term by term ----
+    if (seen.any()) atomicOr(non_finite, 1u << blk);
+    lds_barrier();
+    const u32 blocks = __builtin_amdgcn_readfirstlane(*non_finite);
+    if (__builtin_expect(blocks != 0, 0)) cells_again<T>(Again(lds, blocks));
 }
 
 template <typename T, bool STREAM>
 static hipError_t launch(const void *q, const void *key, const void *value, const void *grad_out, float *stats,
                          void *grad_q, void *grad_key, void *grad_value, int B, int d, int C, int H, int W,
                          hipStream_t st) {
+    Args<T> args{(const T *)q, (const T *)key, (const T *)value, (const T *)grad_out, stats, (T *)grad_q, (T *)grad_key,
+                 (T *)grad_value, B, d, C, H, W, 0, 0, 0, 0, 0};
+    // sets the tiles; false: too many
+    auto tile = [&](int tiles_x, int tiles_y) {
+        const long nb = (long)tiles_x * tiles_y * B;
+        args.tiles_x = tiles_x, args.tiles_y = tiles_y, args.nblocks = (int)nb, args.per_xcd = (int)((nb + 7) / 8);
+        return nb <= (1L << 30);
+    };
     {
         const int nsx = (W + 3) / 4;
-        const int tiles_x = (nsx + NSW - 1) / NSW, tiles_y = (H + 3) / 4;
-        const int ns = (nsx + tiles_x - 1) / tiles_x;         // blocks per tile, balanced over the row
-        const long nb = (long)tiles_x * tiles_y * B;
-        if (nb > (1L << 30)) return hipErrorNotSupported;
-        const int per_xcd = (int)((nb + 7) / 8);
-        hipLaunchKernelGGL((bwd_pixel_kernel<T, STREAM>), dim3(per_xcd * 8), dim3(128 * NSW), 0, st, (const T *)q,
-                           (const T *)key, (const T *)value, (const T *)grad_out, (T *)grad_q, stats, B, d, C, H, W,
-                           tiles_x, tiles_y, ns, (int)nb, per_xcd);
+        if (!tile((nsx + NSW - 1) / NSW, (H + 3) / 4)) return hipErrorNotSupported;
+        args.ns = (nsx + args.tiles_x - 1) / args.tiles_x;    // blocks per tile, balanced over the row
+        hipLaunchKernelGGL((bwd_pixel_kernel<T, STREAM>), dim3(args.per_xcd * 8), dim3(128 * NSW), 0, st, args);
         const hipError_t e = hipGetLastError();
         if (e != hipSuccess) return e;
     }
     if (!grad_key && !grad_value) return hipSuccess;
     // cell blocks 4 I - 2 .. 4 I + 1 that hold a cell of 0 .. W - 1
     const int nI = (W + 1) / 4 + 1, nJ = (H + 1) / 4 + 1;
-    const int tiles_x = (nI + TBX - 1) / TBX, tiles_y = (nJ + TBY - 1) / TBY;
-    const long nb = (long)tiles_x * tiles_y * B;
-    if (nb > (1L << 30)) return hipErrorNotSupported;
-    const int per_xcd = (int)((nb + 7) / 8);
-    hipLaunchKernelGGL((bwd_cell_kernel<T>), dim3(per_xcd * 8), dim3(CNT), 0, st, (const T *)q, (const T *)key,
-                       (const T *)value, (const T *)grad_out, stats, (T *)grad_key, (T *)grad_value, B, d, C, H, W,
-                       tiles_x, tiles_y, (int)nb, per_xcd);
+    if (!tile((nI + TBX - 1) / TBX, (nJ + TBY - 1) / TBY)) return hipErrorNotSupported;
+    hipLaunchKernelGGL((bwd_cell_kernel<T>), dim3(args.per_xcd * 8), dim3(CNT), 0, st, args);
     return hipGetLastError();
 }
 

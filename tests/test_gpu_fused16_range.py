@@ -172,3 +172,21 @@ def test_forward_keeps_non_finite_values_where_they_belong(K, s, W, which, value
     assert same_non_finite(got, want)
     ok = torch.isfinite(want)
     assert rel(got[ok], want[ok]) <= one_rounding(dtype)
+
+
+@pytest.mark.parametrize('dtype', [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize('value', [float('nan'), float('inf')])
+@pytest.mark.parametrize('which', [0, 1, 2, 3])
+@pytest.mark.parametrize('channels_last,W', [(False, 24), (False, 38), (True, 23)])
+def test_backward_keeps_non_finite_values_where_they_belong(channels_last, W, which, value, dtype):
+    g = torch.Generator(device='cuda').manual_seed(W)
+    B, d, C, H = 2, 24, 40, 11
+    shapes = ((B, d, 2 * H, 2 * W), (B, d, H, W), (B, C, H, W), (B, C, 2 * H, 2 * W))
+    ops = [draw(g, sh, dtype, 0.5, channels_last) for sh in shapes]
+    ops[which][0, 3, 5, 0] = value
+    ops[which][1, 7, ops[which].shape[2] - 1, ops[which].shape[3] - 1] = value
+    ops[which][1, 2, 4, 7] = -value
+    for got, want in zip(gradients(ops[:3], ops[3]), exact_gradients(ops[:3], ops[3])[1:]):
+        assert same_non_finite(got, want)
+        ok = torch.isfinite(want)
+        assert rel(got[ok], want[ok]) <= one_rounding(dtype)
