@@ -770,7 +770,7 @@ static hipError_t launch(const void *q, const void *key, const void *value, cons
 // hipErrorNotSupported otherwise (nothing is launched then).
 bool sapa_b_bwd16_serves(int d, int C, int H, int W, int K, int s, int dtype) {
     return K == 5 && s == 2 && W % 2 == 0 && W >= 16 && (dtype == 2 || dtype == 3) &&
-           (long)(d > C ? d : C) * H * W * 8 < (1L << 31);
+           wm::offsets_fit(d > C ? d : C, (long)H * W * 8);
 }
 
 hipError_t sapa_b_bwd16_launch(const void *q, const void *key, const void *value, const void *grad_out, void *stats,

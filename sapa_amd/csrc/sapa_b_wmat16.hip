@@ -508,8 +508,7 @@ hipError_t sapa_b_wmat16_launch(int mode, const void *q, const void *key, const 
     const bool k5s2 = K == 5 && s == 2, k7s4 = K == 7 && s == 4, k5s4 = K == 5 && s == 4, k3s2 = K == 3 && s == 2;
     if (mode != TILED_FUSED || !(k5s2 || k7s4 || k5s4 || k3s2) || W < 4) return hipErrorNotSupported;
     if (dtype != 2 && dtype != 3) return hipErrorNotSupported;
-    const long hplane = (long)H * W * s * s * 2;
-    if ((long)(d > C ? d : C) * hplane >= (1L << 31)) return hipErrorNotSupported;
+    if (!wm::offsets_fit(d > C ? d : C, (long)H * W * s * s * 2)) return hipErrorNotSupported;
     if (((uintptr_t)key | (uintptr_t)value) % 4 != 0 || ((uintptr_t)q | (uintptr_t)out) % 16 != 0)
         return hipErrorNotSupported;
     // bytes read and written once; beyond the 256 MB memory-side cache they are streamed, in tiles of

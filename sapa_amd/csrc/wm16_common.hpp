@@ -16,6 +16,13 @@ typedef short s16x4 __attribute__((ext_vector_type(4)));
 constexpr u32 OUTSIDE = 0x80000000u;      // past the end of every buffer descriptor: reads zero, stores nothing
 constexpr float LOG2E = 1.4426950408889634f;
 
+// Whether the byte offsets inside an image of up to `channels` planes of `plane` bytes are distinct 32-bit
+// numbers below OUTSIDE, and those of the last chunk's channels past the image (a chunk has 16), which
+// lie outside too, do not come round to its beginning
+inline bool offsets_fit(long channels, long plane) {
+    return channels * plane < (1L << 31) && (channels + 15) / 16 * 16 * plane <= (1L << 32);
+}
+
 template <typename T> struct Mma;
 template <> struct Mma<f16_t> {
     typedef _Float16 v4 __attribute__((ext_vector_type(4)));

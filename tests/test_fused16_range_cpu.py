@@ -1,0 +1,19 @@
+"""CPU: which sizes the two-kernel backward of 16-bit SAPA-B serves."""
+import pytest
+import torch
+
+from sapa_amd import _lib
+
+
+@pytest.mark.parametrize('dtype', [torch.float16, torch.bfloat16])
+def test_planes_whose_offsets_would_wrap_are_refused(dtype):
+    """The kernels stage 16 channels at a time with 32-bit offsets: with fewer channels than that the
+    ones past the tensor's last must not come round to its first."""
+    serves = _lib.lib().sapa_fused_backward_direct_serves
+    code = _lib.DTYPES[dtype]
+    # planes of 256 MiB: 16 of them are 2^32 bytes, 8 of them 2^31
+    for channels, H, W, contiguous in ((7, 4096, 8192, True), (8, 4096, 8192, False), (7, 4098, 8192, False),
+                                       (1, 4096, 8192, True), (1, 4098, 8192, False), (1, 16384, 16382, False),
+                                       (17, 1024, 8192, True), (31, 1024, 8192, True), (32, 1024, 8192, False)):
+        assert serves(channels, 1, H, W, 5, 2, 0, code) == contiguous, (channels, H, W)
+        assert serves(1, channels, H, W, 5, 2, 0, code) == contiguous, (channels, H, W)
