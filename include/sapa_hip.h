@@ -158,9 +158,11 @@ int sapa_fused_backward(const void *grad_out, const void *query, const void *key
  * nothing between the two products is rounded to 16 bits either way), and sapa_fused_backward_attn takes that
  * tensor instead of recomputing it; its workspace holds grad_logits only
  * (sapa_fused_backward_attn_workspace bytes, half of the other's).  Same results
- * as sapa_fused_backward on the same operands, one launch less per step and a
- * faster one in the forward pass of 16-bit tensors; the price is the attn tensor
- * kept alive.  Same SAPA_ERR_UNSUPPORTED cases. */
+ * as sapa_fused_backward on the same operands (to a rounding for the 16-bit tensors
+ * that sapa_fused_backward_direct below serves: sapa_fused_backward takes its way), one
+ * launch less per step and a faster one in the forward pass of 16-bit tensors; the
+ * price is the attn tensor kept alive.  out NULL: the weights alone (value is not read
+ * then).  Same SAPA_ERR_UNSUPPORTED cases. */
 int sapa_fused_forward_attn(const void *query, const void *key, const void *value,
                             void *attn, void *out, int B, int d, int C, int H, int W,
                             int K, int s, int dtype, void *stream);

@@ -385,7 +385,7 @@ int sapa_fused_forward_attn(const void *query, const void *key, const void *valu
     if (rc != SAPA_OK) return rc;
     if (dtype == SAPA_F64 || K != 5 || s != 2) return SAPA_ERR_UNSUPPORTED;
     if (B == 0) return SAPA_OK;
-    if (!query || !key || !value || !attn || !out) return SAPA_ERR_INVALID_ARGUMENT;
+    if (!query || !key || !attn || (out && !value)) return SAPA_ERR_INVALID_ARGUMENT;
     hipStream_t st = (hipStream_t)stream;
     // the weights once, in fp32, then the aggregation with them: the two launches of
     // the separate operators, without a 16-bit rounding between them
@@ -395,6 +395,7 @@ int sapa_fused_forward_attn(const void *query, const void *key, const void *valu
         e = sapa_b_tiled_launch(TILED_QK_SOFTMAX, query, key, nullptr, nullptr, attn, B, d, 0, H, W, K, s, dtype,
                                 st, true);
     SAPA_STAGE(e);
+    if (!out) return SAPA_OK;
     // the output of 16-bit tensors from the one-launch forward where it runs on the matrix
     // instructions (its weights are the same fp32 softmax of the same fp32 sums): 208 us against
     // 285 for the aggregation with the fp32 weights at B=16, C=256, 100x168

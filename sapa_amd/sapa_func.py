@@ -233,12 +233,13 @@ def _direct_backward(grad_output, query, key, value, K, s, needs):
     return None if status == _lib.UNSUPPORTED else tuple(grads)
 
 
-def _fused_backward(grad_output, query, key, value, K, s, needs=(True, True, True), attn=None):
-    """Gradients of av(softmax(qk(query, key)), value): the attention weights
+def _fused_backward(grad_output, query, key, value, K, s, needs=(True, True, True), attn=None, direct=True):
+    """Gradients of av(softmax(qk(query, key)), value): straight from the operands where
+    sapa_fused_backward_direct serves them (and `direct`); else the attention weights
     are recomputed (one launch) unless the forward pass kept them (`attn`, fp32),
     then the three operators' gradients chain."""
     need_q, need_k, need_v = needs
-    grads = _direct_backward(grad_output, query, key, value, K, s, needs)
+    grads = _direct_backward(grad_output, query, key, value, K, s, needs) if direct and attn is None else None
     if grads is not None:
         return grads
     cl = [_lib.is_channels_last(t) for t in (query, key, value)]
@@ -248,13 +249,20 @@ def _fused_backward(grad_output, query, key, value, K, s, needs=(True, True, Tru
         # of the tensor it belongs to
         grads = _fused_backward(_lib.layout_copy(grad_output, False), _lib.layout_copy(query, False),
                                 _lib.layout_copy(key, False), _lib.layout_copy(value, False), K, s, needs,
-                                None if attn is None else _lib.layout_copy(attn, False))
+                                None if attn is None else _lib.layout_copy(attn, False), direct)
         return tuple(_back(g, c) for g, c in zip(grads, cl))
     query, key, value = query.contiguous(), key.contiguous(), value.contiguous()
     grad_output = grad_output.contiguous()
     _lib.require_cuda_contiguous(grad_output=grad_output, query=query, key=key, value=value)
+    n, c, h, w = value.size()
+    if attn is None and not direct and _direct_serves(query, key, value, K, s, False):
+        # the weights that the forward pass would have kept (sapa_fused_backward takes the direct way)
+        attn = torch.empty((n, K * K, h * s, w * s), dtype=torch.float32, device=value.device)
+        status = _lib.call_status('sapa_fused_forward_attn', value.device, _lib.ptr(query), _lib.ptr(key), None,
+                                  _lib.ptr(attn), None, n, key.size(1), c, h, w, K, s, _lib.dtype_code(value))
+        if status == _lib.UNSUPPORTED:
+            attn = None
     if attn is not None:
-        n, c, h, w = value.size()
         nbytes = _lib.lib().sapa_fused_backward_attn_workspace(n, h, w, K, s)
         ws = torch.empty(max(nbytes // 4, 1), dtype=torch.float32, device=value.device)
         grads = [_lib.new_out(t) if need else None
@@ -313,21 +321,26 @@ def _fused_backward(grad_output, query, key, value, K, s, needs=(True, True, Tru
     return grad_query, grad_key, grad_value
 
 
-# Training steps of sapa_fused keep the fp32 attention weights between the forward and
-# the backward pass (faster: one launch less per step) unless this is False or the call
+# Training steps of sapa_fused whose gradients chain over the attention weights (fp32; 16-bit
+# tensors that sapa_fused_backward_direct does not serve) keep them between the forward and the
+# backward pass (faster: one launch less per step) unless this is False or the call
 # says save_attention=False (less memory: the weights are recomputed).
 SAVE_ATTENTION = True
 
 
 class SAPAFusedFunction(Function):
     """av(softmax(qk(query, key), dim=1), value) -- SAPA.attention
-    (sapa_base.py:38-40) -- as one launch in the forward pass.  When a gradient
-    is wanted and `save_attention` is set (the default, SAVE_ATTENTION), the
-    forward pass of operands that sapa_fused_backward_direct does not serve (fp32)
-    runs as two launches that leave the fp32 attention weights
+    (sapa_base.py:38-40) -- as one launch in the forward pass.  The gradients of
+    16-bit operands that sapa_fused_backward_direct serves come straight from them
+    (nothing kept, no K*K tensor at any time), unless the call says where its
+    attention weights are to come from: with save_attention=True the
+    forward pass runs as two launches that leave the fp32 weights
     [B,K*K,sH,sW] behind for the backward pass, as the reference's autograd graph
-    does; otherwise the backward pass recomputes them (one launch more, nothing
-    kept alive but the operands).  Then the three operators' gradients chain.
+    does; with save_attention=False the backward pass recomputes them (one launch
+    more, nothing kept alive but the operands).  Either way the three operators' gradients
+    then chain over them: the same gradients bit for bit.  Operands that are not served
+    chain in any case (save_attention=None: as SAVE_ATTENTION says).  Channels-last
+    operands keep no weights, whatever is asked for.
 
     query_bias [B, d] (optional): a per-image bias added to every query vector,
     i.e. the result for query + query_bias[:, :, None, None] -- what a 1x1
@@ -363,7 +376,8 @@ class SAPAFusedFunction(Function):
             query = query + query_bias[:, :, None, None]
             query_bias = None
         output = _lib.new_out(value, (n, c, h * scale_factor, w * scale_factor), nhwc)
-        # (where the gradients come straight from the operands the weights are kept on request only)
+        # (who says where the weights come from gets gradients that chain over them)
+        ctx.direct = save_attention is None or nhwc
         if save_attention is None:
             save_attention = SAVE_ATTENTION and not (
                 wants_grad and _direct_serves(query, key, value, kernel_size, scale_factor, nhwc))
@@ -403,7 +417,7 @@ class SAPAFusedFunction(Function):
         grad_query, grad_key, grad_value = _fused_backward(
             grad_output, query, key, value, ctx.kernel_size, ctx.scale_factor,
             (needs[0] or (ctx.has_bias and needs[5]), needs[1], needs[2]),
-            attn=ctx.saved_tensors[-1] if ctx.has_attn else None)
+            attn=ctx.saved_tensors[-1] if ctx.has_attn else None, direct=ctx.direct)
         if ctx.has_bias and needs[5]:
             wide = torch.float32 if grad_query.dtype in (torch.float16, torch.bfloat16) else None
             grad_bias = grad_query.sum(dim=(2, 3), dtype=wide).to(grad_query.dtype)

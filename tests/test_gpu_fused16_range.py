@@ -190,3 +190,22 @@ def test_backward_keeps_non_finite_values_where_they_belong(channels_last, W, wh
         assert same_non_finite(got, want)
         ok = torch.isfinite(want)
         assert rel(got[ok], want[ok]) <= one_rounding(dtype)
+
+
+@pytest.mark.parametrize('dtype', [torch.float32, torch.bfloat16, torch.float16])
+def test_kept_weights_are_the_ones_the_gradients_come_from(dtype):
+    """save_attention=True: the backward pass reads the weights that the forward pass kept (handed back
+    as zeros they leave no gradient), and without the option 16-bit tensors keep none."""
+    import sapa_amd
+    g = torch.Generator(device='cuda').manual_seed(0)
+    B, d, C, H, W = 2, 16, 24, 13, 22
+    shapes = ((B, d, 2 * H, 2 * W), (B, d, H, W), (B, C, H, W), (B, C, 2 * H, 2 * W))
+    *ops, go = (draw(g, sh, dtype, 0.5) for sh in shapes)
+    kept = (B, 25, 2 * H, 2 * W)
+    for save, expected in ((True, True), (False, False), (None, dtype == torch.float32)):
+        leaves, seen = [t.clone().requires_grad_() for t in ops], []
+        with torch.autograd.graph.saved_tensors_hooks(lambda t: t, lambda t: seen.append(tuple(t.shape)) or (t * 0 if tuple(t.shape) == kept else t)):
+            out = sapa_amd.sapa_fused(*leaves, 5, 2, save_attention=save)
+            grads = torch.autograd.grad(out, leaves, go)
+        assert (kept in seen) == expected
+        assert all(bool((t == 0).all()) for t in grads) == expected
