@@ -242,13 +242,20 @@ static void chunking_for(long HW, int B, int C, bool cl, long &seg, int &chunks)
     else chunking(HW, (long)B * C, 4096, 512, seg, chunks);
 }
 
-// the partial sums of one or two features (x1 null: one)
+// the partial sums of one or two features (x1 null: one).  Two planar features of which one cannot be read in
+// vectors take a launch each: the other one must not pay for it (fp32, a high-res feature beside a low-res
+// one of 13 x 13 cells)
 template <typename T>
 static void launch_partial(const T *x0, float *ws0, long HW0, const T *x1, float *ws1, long HW1, int B, int C, bool cl,
                            hipStream_t st) {
     Feature<T> f0{x0, ws0, HW0, 0, 0}, f1{x1, ws1, HW1, 0, 0};
     chunking_for(HW0, B, C, cl, f0.seg, f0.chunks);
     if (x1) chunking_for(HW1, B, C, cl, f1.seg, f1.chunks);
+    constexpr int VEC = 16 / (int)sizeof(T);
+    if (x1 && !cl && (HW0 % VEC == 0) != (HW1 % VEC == 0)) {
+        launch_partial<T>(x0, ws0, HW0, nullptr, nullptr, 0, B, C, cl, st);
+        return launch_partial<T>(x1, ws1, HW1, nullptr, nullptr, 0, B, C, cl, st);
+    }
     const int chunks = f0.chunks + f1.chunks;
     const bool aligned = ((uintptr_t)x0 | (uintptr_t)x1) % 16 == 0;
     if (cl) {
@@ -259,9 +266,8 @@ static void launch_partial(const T *x0, float *ws0, long HW0, const T *x1, float
         else
             hipLaunchKernelGGL((partial_nhwc_kernel<T, 4>), dim3(chunks, B), dim3(256), 0, st, f0, f1, C);
     } else {
-        constexpr int VEC = 16 / (int)sizeof(T);
         const dim3 grid(chunks, B * C);
-        if (HW0 % VEC == 0 && (!x1 || HW1 % VEC == 0) && aligned)
+        if (HW0 % VEC == 0 && aligned)
             hipLaunchKernelGGL((partial_nchw_kernel<T, VEC>), grid, dim3(256), 0, st, f0, f1);
         else
             hipLaunchKernelGGL((partial_nchw_kernel<T, 1>), grid, dim3(256), 0, st, f0, f1);

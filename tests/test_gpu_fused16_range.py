@@ -209,3 +209,19 @@ def test_kept_weights_are_the_ones_the_gradients_come_from(dtype):
             grads = torch.autograd.grad(out, leaves, go)
         assert (kept in seen) == expected
         assert all(bool((t == 0).all()) for t in grads) == expected
+
+
+@pytest.mark.parametrize('channels_last', [False, True])
+def test_moments_of_two_features_with_an_odd_low_res_plane(channels_last):
+    """fp32 features whose low-res planes are no multiple of a vector, into a channels-last module: the
+    high-res feature's moments are what they are by themselves, bit for bit."""
+    from sapa_amd import _lib
+    g = torch.Generator(device='cuda').manual_seed(0)
+    C = 64
+    y, x = (torch.randn(3, C, a, a, generator=g, device='cuda').contiguous(memory_format=ORDERS[channels_last]) for a in (26, 13))
+    norms = [torch.nn.GroupNorm(32, C).cuda() for _ in 'yx']
+    convs = [torch.nn.Conv2d(C, 32, 1).cuda() for _ in 'yx']
+    with torch.no_grad():
+        (q, _), k = _lib.norm_project_pair(y, norms[0], convs[0], x, norms[1], convs[1], True, False)
+        assert torch.equal(q, _lib.norm_project(y, norms[0], convs[0], True)[0])
+        assert torch.equal(k, _lib.norm_project(x, norms[1], convs[1], True)[0])
