@@ -225,3 +225,20 @@ def test_moments_of_two_features_with_an_odd_low_res_plane(channels_last):
         (q, _), k = _lib.norm_project_pair(y, norms[0], convs[0], x, norms[1], convs[1], True, False)
         assert torch.equal(q, _lib.norm_project(y, norms[0], convs[0], True)[0])
         assert torch.equal(k, _lib.norm_project(x, norms[1], convs[1], True)[0])
+
+
+@pytest.mark.parametrize('channels_last', [False, True])
+@pytest.mark.parametrize('C,O', [(64, 128), (128, 72), (256, 288), (512, 128)])
+@pytest.mark.parametrize('mean', [0.0, 1.0])
+def test_precision_of_the_plain_fp32_projections(C, O, mean, channels_last):
+    """sapa_project_shared in fp32: an error like that of one fp32 sum per 32 channels, C / 32 + 2
+    roundings that do not know of each other (a library's convolution is off by 0.9 to 2.8e-7 at these
+    sizes)."""
+    from sapa_amd import _lib
+    g = torch.Generator(device='cuda').manual_seed(C)
+    B, H, W = 2, 64, 64
+    x = (torch.randn(B, C, H, W, generator=g, device='cuda') + mean).contiguous(memory_format=ORDERS[channels_last])
+    w = torch.randn(O, C, 1, 1, generator=g, device='cuda').mul(0.02)
+    b = torch.randn(O, generator=g, device='cuda').mul(0.1)
+    want = torch.matmul(w.double().reshape(O, C), x.double().contiguous().reshape(B, C, H * W)).view(B, O, H, W) + b.double().view(1, O, 1, 1)
+    assert rel(_lib.project_shared(x, w, b, channels_last_out=channels_last), want) <= 2.0 ** -24 * (C / 32 + 2) ** 0.5
