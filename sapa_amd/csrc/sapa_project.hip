@@ -541,6 +541,25 @@ project32_kernel(const float *__restrict__ x, const float *__restrict__ w, const
     }
     __syncthreads();
     if (t0 >= t1) return;
+    // An infinite feature or weight has no three pieces (inf - inf), and inf times a piece that is zero is no
+    // number: a tile with a result that is not finite is formed again in plain fp32 products (a lane:
+    // a pixel, every other output), which are infinite or NaN where a convolution's are.
+    auto again = [&](long t, float largest) __attribute__((always_inline)) {
+        if (__builtin_expect(__builtin_amdgcn_ballot_w64(!(largest < __builtin_inff())) == 0, 1)) return;
+#if defined(__HIP_DEVICE_COMPILE__)
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");          // (the results below overwrite the tile's)
+#endif
+        const long p = t * 32 + (lane & 31);
+        if (p >= HW) return;
+        const float *xp = x + (long)b * HW * C + (IN_CL ? p * C : p);
+        for (int o = lane >> 5; o < sp.left; o += 2) {
+            const float *wp = w + ((WIDE ? (long)sp.o0 : (long)b * O) + o) * C;
+            float r = 0.f;
+            for (int c = 0; c < C; ++c) r = fmaf(xp[IN_CL ? (long)c : c * HW], wp[c], r);
+            if (bias) r += bias[(WIDE ? (long)sp.o0 : (long)b * O) + o];
+            out[OUT_CL ? ((long)b * HW + p) * sp.OT + sp.o0 + o : ((long)b * sp.OT + sp.o0 + o) * HW + p] = r;
+        }
+    };
     for (long t = t0; t < t1; ++t) {
         f32x4 acc[2][NT], low[2][NT];
 #pragma unroll
@@ -596,10 +615,15 @@ project32_kernel(const float *__restrict__ x, const float *__restrict__ w, const
                 }
             }
         }
+        float largest = 0.f;
 #pragma unroll
         for (int mb = 0; mb < 2; ++mb)
 #pragma unroll
-            for (int nt = 0; nt < NT; ++nt) acc[mb][nt] += low[mb][nt];
+            for (int nt = 0; nt < NT; ++nt) {
+                acc[mb][nt] += low[mb][nt];
+#pragma unroll
+                for (int i = 0; i < 4; ++i) largest = __builtin_elementwise_maximum(largest, __builtin_fabsf(acc[mb][nt][i]));
+            }
         // acc[mb][nt][i]: pixel 16 mb + 4 kg + i, output 16 nt + r16
         if (!OUT_CL) {
             // planes: a block of 16 outputs x 32 pixels -> the wave's tile (a lane holds 4
@@ -621,6 +645,7 @@ project32_kernel(const float *__restrict__ x, const float *__restrict__ w, const
                     __builtin_amdgcn_raw_buffer_store_b128(*(const u32x4 *)(rt + row * PS + 4 * col), ro, off + obase, 0, 2);
                 }
             }
+            again(t, largest);
             continue;
         }
         // channels-last: the wave's tile, then 16 rows of 4 O bytes -> one contiguous run of 64 O
@@ -640,6 +665,7 @@ project32_kernel(const float *__restrict__ x, const float *__restrict__ w, const
                     __builtin_amdgcn_raw_buffer_store_b128(*(const u32x4 *)(rt + row * OS + 4 * col), ro, off + obase, 0, 2);
             }
         }
+        again(t, largest);
     }
 }
 

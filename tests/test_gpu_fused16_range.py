@@ -227,6 +227,27 @@ def test_moments_of_two_features_with_an_odd_low_res_plane(channels_last):
         assert torch.equal(k, _lib.norm_project(x, norms[1], convs[1], True)[0])
 
 
+def test_an_infinite_feature_in_the_plain_projections():
+    """sapa_project_shared in fp32 with infinite and NaN features: infinite and NaN where a 1x1
+    convolution is, finite everywhere else."""
+    import torch.nn.functional as F
+    from sapa_amd import _lib
+    g = torch.Generator(device='cuda').manual_seed(0)
+    for C, O, H, W in ((64, 40, 9, 12), (256, 128, 16, 20)):
+        x = torch.randn(2, C, H, W, generator=g, device='cuda')
+        w = torch.randn(O, C, 1, 1, generator=g, device='cuda').mul(0.25)
+        w[::2] = w[::2].bfloat16().float()      # weights whose lower pieces are zeros
+        x[0, 3, 2, 5], x[0, 5, 8, 11], x[1, 7, 0, 0], x[1, 9, 4, 4], x[1, 10, 4, 4] = (float(t) for t in ('inf', '-inf', 'nan', 'inf', '-inf'))
+        x[1, 11, 6, 6] = 3.4e38
+        b = torch.randn(O, generator=g, device='cuda')
+        want = F.conv2d(x.double(), w.double(), b.double())
+        for fmt in ORDERS.values():
+            got = _lib.project_shared(x.contiguous(memory_format=fmt), w, b, channels_last_out=fmt == torch.channels_last)
+            assert same_non_finite(got, want)
+            ok = want.isfinite()
+            assert bool(((got[ok].double() - want[ok]).abs() <= 1e-5 + 1e-5 * want[ok].abs()).all())
+
+
 @pytest.mark.parametrize('channels_last', [False, True])
 @pytest.mark.parametrize('C,O', [(64, 128), (128, 72), (256, 288), (512, 128)])
 @pytest.mark.parametrize('mean', [0.0, 1.0])
