@@ -359,7 +359,8 @@ bwd_pixel_kernel(const Args<T> args) {
                     o = Mma<T>::k32(whi[nb][s], b[s], o);
                     o = Mma<T>::k32(wlo[nb][s], b[s], o);
                 }
-                seen.see(o);
+                // (a key that is not finite makes its channel's results so for every child of the block)
+                if (nb == 0) seen.see(o[0]);
                 if (SCALED) {
 #pragma unroll
                     for (int v = 0; v < 4; ++v) o[v] *= down[nb][v];
@@ -578,7 +579,8 @@ bwd_cell_kernel(const Args<T> args) {
                 o = Mma<T>::k32(whi[qx][s], b, o);
                 o = Mma<T>::k32(wlo[qx][s], b, o);
             }
-        seen.see(o);
+        // (what is not finite in a child makes its channel's results so for every cell of the block)
+        seen.see(o[0]);
         if (SCALED) {
 #pragma unroll
             for (int v = 0; v < 4; ++v) o[v] *= down[v];

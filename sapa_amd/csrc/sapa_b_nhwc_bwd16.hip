@@ -329,7 +329,7 @@ bwd_pixel_kernel(const Args<T> args) {
                         o = Mma<T>::k32(va[mk][s], whi[nb][s], o);
                         o = Mma<T>::k32(va[mk][s], wlo[nb][s], o);
                     }
-                    seen.see(o);
+                    if (nb == 0) seen.see(o);
                     if (SCALED) o *= down[nb];
                     *(u32x2 *)(oslot + piece_at(i16, 2 * mk + (g >> 1)) + 2 * (g & 1)) =
                         u32x2{pack2<T>(o[0], o[1]), pack2<T>(o[2], o[3])};

@@ -417,7 +417,8 @@ sapa_b_wmat16_kernel(const T *__restrict__ q, const T *__restrict__ key, const T
                     acc = Mma<T>::k32(whi[nb][s], b[s], acc);
                     acc = Mma<T>::k32(wlo[nb][s], b[s], acc);
                 }
-                seen.see(acc);
+                // (a value that is not finite makes its channel's results so for every child of the block)
+                if (nb == 0) seen.see(acc[0]);
                 if (UP != 1.f) acc *= 1.f / UP;
                 // element v: child (row 2 nb + g / 2, column 4 (g % 2) + v), channel c0 + i16
                 const int r = 2 * nb + (g >> 1);

@@ -15,8 +15,9 @@ namespace sapa {
 
 namespace wm {
 
-// whether a result among those shown to it is infinite or NaN: their largest magnitude (half an
-// instruction per value)
+// whether a result among those shown to it is infinite or NaN: their largest magnitude.  (What is not finite
+// and does not belong to a result meets a weight of zero there, and so for all children (cells) of a
+// block at once: one of them is looked at per channel.)
 struct NonFinite {
     float m = 0.f;
     __device__ __forceinline__ void see(f32x4 x) {
