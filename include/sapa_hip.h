@@ -524,6 +524,9 @@ int sapa_project_shared(const void *x, const void *weight, const void *bias, voi
  * of the projection entry points, x and out aligned to 16 bytes). */
 long long sapa_norm_project_scratch(int B, int C, int O, long long HW, int x_channels_last,
                                     int dtype);
+/* 1 where sapa_norm_project serves the configuration (alignment aside), else 0. */
+int sapa_norm_project_serves(int B, int C, int O, long long HW, int groups, int x_channels_last,
+                             int out_channels_last, int dtype);
 int sapa_norm_project(const void *x, const void *gamma, const void *beta, const void *weight,
                       const void *bias, void *scratch, void *out, void *bias_out, int B, int C,
                       int O, long long HW, int groups, float eps, int x_channels_last,

@@ -5,6 +5,7 @@ puts it.  There is no fallback: if the library is missing or a call fails,
 the operators raise.
 """
 import ctypes
+import functools
 import os
 
 import torch
@@ -26,6 +27,7 @@ SIGNATURES = {
     'sapa_project_shared': [_vp, _vp, _vp, _vp, _i, _i, _i, _ll, _i, _i, _i, _vp],
     'sapa_norm_project': [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _i, _i, _i, _ll, _i, ctypes.c_float, _i, _i, _i,
                           _vp],
+    'sapa_norm_project_serves': [_i, _i, _i, _ll, _i, _i, _i, _i],
     'sapa_norm_project_pair': ([_vp] * 7 + [_ll]) * 2 + [_vp, _i, _i, _i, _i, ctypes.c_float, _i, _i, _i, _vp],
     'sapa_channel_moments': [_vp, _vp, _vp, _i, _i, _ll, _i, _i, _vp],
     'sapa_channel_moments_static': [_vp, _vp, _i, _i, _ll, _i, _i, _vp],
@@ -348,18 +350,27 @@ def norm_project(x, norm, conv, channels_last_out=False, defer_bias=False):
     return None if status == UNSUPPORTED else (out, b_out)
 
 
+@functools.lru_cache(maxsize=1024)
+def _norm_project_serves(*sizes):
+    return bool(lib().sapa_norm_project_serves(*sizes))
+
+
 def _norm_project_order(x, norm, conv, channels_last_out):
-    """Whether x is in channels_last order, or None if sapa_norm_project does not take the operands."""
-    _, C, H, W = x.shape
+    """Whether x is in channels_last order, or None if sapa_norm_project does not take the operands.
+    (Asked before results and scratch are allocated: a call that is refused behind them costs a
+    forward pass 10 us for each of its features, which then go through the steps one by one.)"""
+    B, C, H, W = x.shape
+    O = conv.out_channels
     params = [norm.weight, norm.bias, conv.weight, conv.bias]
-    if (x.dtype not in DTYPES or x.numel() == 0 or conv.weight.numel() != conv.out_channels * C
+    if (x.dtype not in DTYPES or x.numel() == 0 or conv.weight.numel() != O * C
             or any(p is not None and (p.dtype != x.dtype or not p.is_contiguous()) for p in params)):
         return None
-    if x.is_contiguous():
-        # rows of pixels that the kernels' loads do not divide: refused there too, but only after
-        # results and scratch have been allocated here (12 us of a forward whose key feature is refused)
-        return None if H * W % _plane_step(x, channels_last_out) else False
-    return True if x.is_contiguous(memory_format=torch.channels_last) else None
+    order = not x.is_contiguous()
+    if order and not x.is_contiguous(memory_format=torch.channels_last):
+        return None
+    serves = _norm_project_serves(B, C, O, H * W, norm.num_groups, int(order), int(order or bool(channels_last_out)),
+                                  DTYPES[x.dtype])
+    return order if serves else None
 
 
 def _plane_step(x, channels_last_out):

@@ -828,6 +828,13 @@ long long sapa_norm_project_scratch(int B, int C, int O, long long HW, int x_cha
            round256((long long)B * O * C * esize_of(dtype)) + round256((long long)B * O * esize_of(dtype));
 }
 
+int sapa_norm_project_serves(int B, int C, int O, long long HW, int groups, int x_channels_last,
+                             int out_channels_last, int dtype) {
+    if (B <= 0 || C <= 0 || O <= 0 || HW <= 0 || (long long)B * HW * (C > O ? C : O) >= kMaxElems) return 0;
+    return norm_fold_supported(B, C, groups, x_channels_last != 0, dtype) &&
+           project_supported(C, O, (long)HW, x_channels_last != 0, out_channels_last != 0, dtype);
+}
+
 namespace {
 // one feature of a norm_project call
 struct NormProject {

@@ -86,6 +86,8 @@ struct NormFold {
     void *w_out, *b_out;
     long HW;
 };
+// whether norm_fold_launch serves a feature (alignment aside)
+bool norm_fold_supported(int B, int C, int G, bool channels_last, int dtype);
 hipError_t norm_fold_launch(const NormFold *f, int n, int B, int C, int O, int G, float eps, bool channels_last,
                             int dtype, hipStream_t st);
 

@@ -608,9 +608,14 @@ hipError_t groupnorm_fold_launch(const float *mean_var, const void *gamma, const
 // in two launches; f[i].workspace: channel_moments_workspace bytes each.  What
 // channel_moments_launch and groupnorm_fold_launch require holds for each; C <= 2048.
 // hipErrorNotSupported otherwise, nothing launched.
+bool norm_fold_supported(int B, int C, int G, bool channels_last, int dtype) {
+    return (dtype == 0 || dtype == 2 || dtype == 3) && G >= 1 && C % G == 0 && C <= moments::kFoldChannels &&
+           channel_moments_served(nullptr, B, C, channels_last, dtype);
+}
+
 hipError_t norm_fold_launch(const NormFold *f, int n, int B, int C, int O, int G, float eps, bool channels_last,
                             int dtype, hipStream_t st) {
-    if (n < 1 || n > 2 || G < 1 || C % G != 0 || C > moments::kFoldChannels) return hipErrorNotSupported;
+    if (n < 1 || n > 2 || !norm_fold_supported(B, C, G, channels_last, dtype)) return hipErrorNotSupported;
     for (int i = 0; i < n; ++i)
         if (!channel_moments_served(f[i].x, B, C, channels_last, dtype)) return hipErrorNotSupported;
     switch (dtype) {

@@ -17,3 +17,17 @@ def test_planes_whose_offsets_would_wrap_are_refused(dtype):
                                        (17, 1024, 8192, True), (31, 1024, 8192, True), (32, 1024, 8192, False)):
         assert serves(channels, 1, H, W, 5, 2, 0, code) == contiguous, (channels, H, W)
         assert serves(1, channels, H, W, 5, 2, 0, code) == contiguous, (channels, H, W)
+
+
+def test_norm_project_says_what_it_serves():
+    """Asked before anything is allocated: the configurations for which sapa_norm_project has every
+    step, by sizes, types and memory orders alone."""
+    serves = _lib.lib().sapa_norm_project_serves
+    f32, f16, f64 = (_lib.DTYPES[t] for t in (torch.float32, torch.float16, torch.float64))
+    for args, expected in (((16, 256, 64, 4200, 32, 0, 0, f32), 1), ((16, 256, 64, 4200, 32, 0, 0, f64), 0),
+                           ((1, 512, 64, 1680, 32, 0, 0, f16), 0), ((1, 512, 64, 1680, 32, 1, 1, f16), 1),
+                           ((8, 64, 32, 169, 32, 0, 0, f32), 0), ((8, 64, 32, 169, 32, 0, 1, f32), 1),
+                           ((8, 64, 32, 172, 32, 0, 1, f16), 0), ((8, 64, 32, 176, 32, 0, 1, f16), 1),
+                           ((8, 64, 32, 176, 24, 0, 1, f16), 0), ((1024, 64, 32, 176, 32, 0, 1, f16), 0),
+                           ((1024, 64, 32, 176, 32, 1, 1, f16), 1), ((0, 64, 32, 176, 32, 1, 1, f16), 0)):
+        assert serves(*args) == expected, args
