@@ -263,3 +263,20 @@ def test_precision_of_the_plain_fp32_projections(C, O, mean, channels_last):
     b = torch.randn(O, generator=g, device='cuda').mul(0.1)
     want = torch.matmul(w.double().reshape(O, C), x.double().contiguous().reshape(B, C, H * W)).view(B, O, H, W) + b.double().view(1, O, 1, 1)
     assert rel(_lib.project_shared(x, w, b, channels_last_out=channels_last), want) <= 2.0 ** -24 * (C / 32 + 2) ** 0.5
+
+
+@pytest.mark.parametrize('C,H,W,aggregated', [(512, 83, 85, False), (512, 85, 85, True), (512, 129, 133, True),
+                                              (512, 131, 133, False), (512, 85, 86, False)])
+def test_training_output_of_odd_rows_on_both_sides_of_the_rule(C, H, W, aggregated):
+    """The output of a training step that keeps its weights: with odd rows and a mid-sized value by the
+    aggregation with those weights, else by the one-launch forward, the same bits as without gradients."""
+    import sapa_amd
+    g = torch.Generator(device='cuda').manual_seed(W)
+    d = 16
+    ops = [draw(g, sh, torch.bfloat16, 0.5) for sh in ((1, d, 2 * H, 2 * W), (1, d, H, W), (1, C, H, W))]
+    got = sapa_amd.sapa_fused(*[t.clone().requires_grad_() for t in ops], 5, 2, save_attention=True).detach()
+    with torch.no_grad():
+        one_launch = sapa_amd.sapa_fused(*ops, 5, 2)
+        want = sapa_amd.sapa_fused(*[t.double() for t in ops], 5, 2)
+    assert torch.equal(got, one_launch) != aggregated
+    assert rel(got, want) <= one_rounding(torch.bfloat16)
