@@ -28,50 +28,17 @@
 // are fp32: the result is within half a 16-bit spacing of the exact one.  A masked cell still
 // enters both products (logit plus -inf, weight 0 times value): a non-finite key or value
 // reaches every child of the 4 x 4 block whose window holds it.
-#include "kernels.hpp"
+#include "wm16_common.hpp"
 
 namespace sapa {
 
 namespace cwm16 {
 
-typedef unsigned u32;
-typedef float f32x4 __attribute__((ext_vector_type(4)));
-typedef u32 u32x2 __attribute__((ext_vector_type(2)));
-typedef u32 u32x4 __attribute__((ext_vector_type(4)));
-typedef short s16x4 __attribute__((ext_vector_type(4)));
+using namespace wm;
 
 constexpr int CHK = 64;            // channels per staged chunk = 8 pieces of 16 bytes per cell
 constexpr int WROWS = 8;           // window rows
 constexpr int CELL = CHK / 2;      // dwords per cell
-constexpr u32 OUTSIDE = 0x80000000u;
-
-template <typename T> struct Mma;
-template <> struct Mma<f16_t> {
-    typedef _Float16 v8 __attribute__((ext_vector_type(8)));
-    static __device__ __forceinline__ f32x4 k32(u32x4 a, u32x4 b, f32x4 c) {
-        return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(v8, a), __builtin_bit_cast(v8, b), c, 0, 0, 0);
-    }
-};
-template <> struct Mma<bf16_t> {
-    typedef __bf16 v8 __attribute__((ext_vector_type(8)));
-    static __device__ __forceinline__ f32x4 k32(u32x4 a, u32x4 b, f32x4 c) {
-        return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(v8, a), __builtin_bit_cast(v8, b), c, 0, 0, 0);
-    }
-};
-
-template <typename T>
-__device__ __forceinline__ u32 pack2(float a, float b) {
-    typedef float f32x2 __attribute__((ext_vector_type(2)));
-    typedef T tx2 __attribute__((ext_vector_type(2)));
-    return __builtin_bit_cast(u32, __builtin_convertvector(f32x2{a, b}, tx2));
-}
-
-// 4 cells x 4 channels out of LDS, transposed: each lane of a 16-lane block addresses 4
-// consecutive channels of one cell and receives one channel of the 4 cells
-__device__ __forceinline__ u32x2 read_tr(const u32 *p) {
-    return __builtin_bit_cast(u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-                                         (s16x4 __attribute__((address_space(3))) *)p));
-}
 
 // dword offset of the 16-byte piece `piece` (0..7) of cell / child `idx` in a [idx][64 channels] array
 __device__ __forceinline__ int piece_at(int idx, int piece) { return idx * CELL + ((piece ^ (idx & 7)) << 2); }
