@@ -38,8 +38,9 @@ const long long kMaxElems = 1LL << 40;
 
 // fused K = 5, s = 2 problems of at most this many low-res cells go to the matrix-pipe kernel
 const long kSmallFusedCells = 12288;
-// ... and the separate operators of at most this many cells (logits) and cells x channels (aggregation)
-const long kSmallLogitCells = 40000, kSmallAggregation = 1L << 20;
+// ... and the separate operators of at most this many cells (logits: with rows that the other kernels do not
+// read in vectors of 4; with fp32 rows that they do) and cells x channels (aggregation)
+const long kSmallLogitCells = 40000, kSmallLogitCellsVec = 32768, kSmallAggregation = 1L << 20;
 
 // LDS-tiled SAPA-B kernel for `mode`: the VALU kernel where it has an
 // instance (K = 5, s = 2, where it is the faster one), else the matrix-pipe
@@ -58,12 +59,18 @@ hipError_t tiled_launch(int mode, const void *q, const void *key, const void *at
     // (B=8, d=32, C=256, fp32: 16x16 32 -> 12 us, 32x32 32 -> 23 us)
     // The separate operators of small problems likewise, their sums in the same order (us, d / C = 64 /
     // 256, fp32).  Logits: 957 cells 37 -> 13, 6400 25 -> 13, 32000 40 -> 27, 67200 35 -> 44; aggregation:
-    // 957 cells 16 -> 7.5, 5160 17.4 -> 16.4, 6400 17.4 -> 18.7, 12288 21 -> 31; bf16 crosses at the
-    // same sizes (logits 32000 33 -> 26, 67200 29 -> 45).
+    // 957 cells 16 -> 7.5, 5160 17.4 -> 16.4, 6400 17.4 -> 18.7, 12288 21 -> 31; bf16 with rows of no whole
+    // vectors crosses at the same sizes (logits 32000 33 -> 26, 67200 29 -> 45).  Where rows are whole vectors, by
+    // the time of qk, softmax and av (d / C = 64): fp32 logits up to 32768 cells 59.7, by the thread-per-parent
+    // kernel 62.3; 35360 cells 71.6 and 67.9; 16-bit ones by the dot-product kernel whatever the size
+    // (bf16, matrix-pipe / dot-product kernel: 1024 cells 45.5 / 39.4, 3200 45.7 / 44.6, 9984 53.4 / 50.3, 35360 69.7 / 62.5;
+    // d=32 39 / 33, 40 / 38, 45.3 / 46.7, 63 / 56)
     const long cells = (long)B * H * W;
+    const bool dot2 = W % 4 == 0 && W >= 32 && dtype != SAPA_F32;         // (rows that sapa_b_dot2_launch takes)
+    const long logit_cells = dot2 ? 0 : W % 4 == 0 && dtype == SAPA_F32 ? kSmallLogitCellsVec : kSmallLogitCells;
     const bool small = mode == TILED_FUSED ? cells <= kSmallFusedCells
                        : mode == TILED_AV  ? cells * C <= kSmallAggregation
-                                           : cells <= kSmallLogitCells;
+                                           : cells <= logit_cells;
     if (e == hipErrorNotSupported && K == 5 && s == 2 && dtype != SAPA_F64 && small)
         e = took("sapa_b_mfma_kernel",
                  sapa_b_mfma_launch(mode, q, key, attn_in, value, out, B, d, C, H, W, K, s, dtype, st));

@@ -280,3 +280,24 @@ def test_training_output_of_odd_rows_on_both_sides_of_the_rule(C, H, W, aggregat
         want = sapa_amd.sapa_fused(*[t.double() for t in ops], 5, 2)
     assert torch.equal(got, one_launch) != aggregated
     assert rel(got, want) <= one_rounding(torch.bfloat16)
+
+
+@pytest.mark.parametrize('dtype,B,H,W,kernel', [
+    (torch.bfloat16, 1, 8, 32, 'sapa_b_dot2_kernel'), (torch.float16, 4, 85, 104, 'sapa_b_dot2_kernel'),
+    (torch.bfloat16, 1, 8, 28, 'sapa_b_mfma_kernel'), (torch.float16, 4, 85, 102, 'sapa_b_mfma_kernel'),
+    (torch.float32, 8, 64, 64, 'sapa_b_mfma_kernel'), (torch.float32, 3, 110, 100, 'sapa_b_tiled_kernel'),
+    (torch.float32, 3, 110, 101, 'sapa_b_mfma_kernel')])
+def test_logits_on_both_sides_of_the_rule(dtype, B, H, W, kernel):
+    """qk by the matrix-pipe kernel where the thread-per-parent kernels do not read rows in vectors, and in
+    fp32 up to 32768 cells; by the dot-product kernel for 16-bit rows of whole vectors."""
+    import sapa_amd
+    from sapa_amd import _lib
+    g = torch.Generator(device='cuda').manual_seed(W)
+    d = 32
+    q, k = draw(g, (B, d, 2 * H, 2 * W), dtype, 0.5), draw(g, (B, d, H, W), dtype, 0.5)
+    with torch.no_grad():
+        got = sapa_amd.qk(q, k, 5, 2)
+        assert _lib.last_kernel().startswith(kernel)
+        want = sapa_amd.qk(q.double(), k.double(), 5, 2)
+    # (32 fp32 roundings that do not know of each other, or one to the result's type)
+    assert rel(got, want) <= (one_rounding(dtype) if dtype != torch.float32 else 32 ** 0.5 * 2.0 ** -24)
