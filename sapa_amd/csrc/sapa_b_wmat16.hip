@@ -107,7 +107,8 @@ sapa_b_wmat16_kernel(const T *__restrict__ q, const T *__restrict__ key, const T
 
     const int logical = (int)(blockIdx.x % 8) * per_xcd + (int)(blockIdx.x / 8);
     if (logical >= nblocks) return;
-    const int tile = logical / nslices, vbase = (logical % nslices) * slice_chunks;      // first value chunk
+    int tile = logical, vbase = 0;                           // first value chunk
+    if (nslices > 1) tile = logical / nslices, vbase = (logical - tile * nslices) * slice_chunks;
     const int tx = tile % tiles_x, ty = (tile / tiles_x) % tiles_y, n = tile / (tiles_x * tiles_y);
     const int X0 = tx * PB * ns, Y0 = ty * PB;               // first parent of the tile
     const int nsx = (W + PB - 1) / PB;
