@@ -443,6 +443,11 @@ def project_nchw(x, weight, bias=None, channels_last_out=False):
     return out
 
 
+def projects(x, O, channels_last_out):
+    """Whether project_shared takes x's extents and O outputs (asked first: it is what most often refuses)."""
+    return O % 8 == 0 and (x.shape[2] * x.shape[3] % _plane_step(x, channels_last_out) == 0 or not x.is_contiguous())
+
+
 def project_shared(x, weight, bias=None, channels_last_out=False):
     """F.conv2d(x, weight, bias) of a 1x1 weight [O, C, 1, 1] for a dense f16 / bf16 / fp32 CUDA
     feature x [B, C, H, W] (contiguous, or in channels_last order with channels_last_out): a
@@ -450,14 +455,12 @@ def project_shared(x, weight, bias=None, channels_last_out=False):
     the configuration (the caller then uses a library convolution).  No autograd."""
     B, C, H, W = x.shape
     O = weight.shape[0]
-    if (x.dtype not in (torch.float16, torch.bfloat16, torch.float32) or weight.dtype != x.dtype
-            or weight.device != x.device or x.numel() == 0 or weight.shape[1] != C
+    if (not projects(x, O, channels_last_out) or x.dtype not in (torch.float16, torch.bfloat16, torch.float32)
+            or weight.dtype != x.dtype or weight.device != x.device or x.numel() == 0 or weight.shape[1] != C
             or (bias is not None and (bias.dtype != x.dtype or bias.device != x.device))):
         return None
     x_cl = not x.is_contiguous()
     if x_cl and not (channels_last_out and x.is_contiguous(memory_format=torch.channels_last)):
-        return None
-    if O % 8 or (not x_cl and H * W % _plane_step(x, channels_last_out)):
         return None
     weight = weight.reshape(O, C).contiguous()
     if bias is not None:
