@@ -23,6 +23,8 @@
 // layout of the first product is the A-operand layout of the second, so the weights never leave
 // the registers.  They enter the product as a 16-bit value plus a 16-bit remainder (two
 // instructions), the sums are fp32: the result is within half a 16-bit spacing of the exact one.
+// (bf16: 16 significant bits of a weight.  Against 64 bits the results are off by 1.7e-3 in bf16 and 2.1e-4 in
+// fp16, one rounding, as with weights in fp32; a third piece needs 32 registers more than there are.)
 // (f16, which holds a pair to 2^-25 only, takes them times 2^15: small weights keep their bits.)
 // The 4 x 4 output blocks go back through LDS so that global stores are 16 bytes per lane along
 // whole tile rows.
