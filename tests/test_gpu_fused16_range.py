@@ -266,7 +266,7 @@ def test_precision_of_the_plain_fp32_projections(C, O, mean, channels_last):
 
 
 @pytest.mark.parametrize('C,H,W,aggregated', [(512, 83, 85, False), (512, 85, 85, True), (512, 129, 133, True),
-                                              (512, 131, 133, False), (512, 85, 86, False)])
+                                              (512, 131, 133, False), (512, 85, 86, False), (128, 190, 197, False)])
 def test_training_output_of_odd_rows_on_both_sides_of_the_rule(C, H, W, aggregated):
     """The output of a training step that keeps its weights: with odd rows and a mid-sized value by the
     aggregation with those weights, else by the one-launch forward, the same bits as without gradients."""
