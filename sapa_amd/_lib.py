@@ -366,6 +366,8 @@ def _norm_project_order(x, norm, conv, channels_last_out):
             or any(p is not None and (p.dtype != x.dtype or not p.is_contiguous()) for p in params)):
         return None
     order = not x.is_contiguous()
+    if not order and H * W % _plane_step(x, channels_last_out):     # (what most often refuses)
+        return None
     if order and not x.is_contiguous(memory_format=torch.channels_last):
         return None
     serves = _norm_project_serves(B, C, O, H * W, norm.num_groups, int(order), int(order or bool(channels_last_out)),
@@ -443,9 +445,10 @@ def project_nchw(x, weight, bias=None, channels_last_out=False):
     return out
 
 
-def projects(x, O, channels_last_out):
-    """Whether project_shared takes x's extents and O outputs (asked first: it is what most often refuses)."""
-    return O % 8 == 0 and (x.shape[2] * x.shape[3] % _plane_step(x, channels_last_out) == 0 or not x.is_contiguous())
+def projects_planes(x, O):
+    """Whether project_shared takes a contiguous feature of x's extents to O outputs in contiguous order."""
+    _, _, H, W = x.shape
+    return O % 8 == 0 and H * W % (8 if x.element_size() == 2 else 4) == 0
 
 
 def project_shared(x, weight, bias=None, channels_last_out=False):
@@ -455,12 +458,14 @@ def project_shared(x, weight, bias=None, channels_last_out=False):
     the configuration (the caller then uses a library convolution).  No autograd."""
     B, C, H, W = x.shape
     O = weight.shape[0]
-    if (not projects(x, O, channels_last_out) or x.dtype not in (torch.float16, torch.bfloat16, torch.float32)
-            or weight.dtype != x.dtype or weight.device != x.device or x.numel() == 0 or weight.shape[1] != C
+    if (x.dtype not in (torch.float16, torch.bfloat16, torch.float32) or weight.dtype != x.dtype
+            or weight.device != x.device or x.numel() == 0 or weight.shape[1] != C
             or (bias is not None and (bias.dtype != x.dtype or bias.device != x.device))):
         return None
     x_cl = not x.is_contiguous()
     if x_cl and not (channels_last_out and x.is_contiguous(memory_format=torch.channels_last)):
+        return None
+    if O % 8 or (not x_cl and H * W % _plane_step(x, channels_last_out)):
         return None
     weight = weight.reshape(O, C).contiguous()
     if bias is not None:

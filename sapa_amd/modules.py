@@ -115,7 +115,7 @@ def norm_project(x, norm, *convs, channels_last=False, defer_bias=False):
     for conv in convs:
         assert conv.kernel_size == (1, 1) and conv.groups == 1
         O = conv.out_channels
-        if norm is None and channels_last and not defer_bias and _kernel_reads(conv, x, True):
+        if norm is None and channels_last and not defer_bias and _kernel_reads(conv, x):
             out = _lib.project_shared(x, conv.weight, conv.bias, channels_last_out=True)
             if out is not None:
                 outs.append(out)
@@ -187,16 +187,13 @@ def _plain(t):
     return type(t) in (torch.Tensor, nn.Parameter) and not torch._C._functorch.is_functorch_wrapped_tensor(t)
 
 
-def _kernel_reads(conv, x, channels_last):
+def _kernel_reads(conv, x):
     """Whether a kernel may read x and conv's parameters in the place of torch's operators: at
-    inference on the GPU, outside autocast, tracing and tensor subclasses, modes or transforms, and
-    with extents that it serves (16-bit planes of no whole vectors came this far for nothing: SAPA-D
-    module, B=14, 256 channels, 21x13, 9 points in fp16 164 us, 149 with the extents asked here)."""
+    inference on the GPU, outside autocast, tracing and tensor subclasses, modes or transforms."""
     return (x.is_cuda and not torch.is_grad_enabled() and not torch.compiler.is_compiling()
             and not torch.is_autocast_enabled('cuda') and not torch.jit.is_tracing()
             and torch.autograd.forward_ad._current_level < 0
             and torch._C._len_torch_dispatch_stack() == 0 and torch._C._len_torch_function_stack() == 0
-            and _lib.projects(x, conv.out_channels, channels_last)
             and all(_plain(t) for t in (x, conv.weight) + (() if conv.bias is None else (conv.bias,))))
 
 
@@ -205,12 +202,16 @@ def _project(conv, x):
     projection, which adds the bias in its epilogue (at B=8, 256 channels, 128x128 fp32 the library
     GEMM and the pass that adds the bias took 120 us for 128 outputs); everything else -- gradients,
     autocast, tracing, tensor subclasses, hooks, another kind of convolution in the module's place --
-    is the module's call."""
-    if (type(conv) is nn.Conv2d and x.dim() == 4 and _kernel_reads(conv, x, False)
+    is the module's call.  (Extents that no kernel serves are asked first: SAPA-D module, B=14, 256 channels,
+    21x13, 9 points in fp16 164 us with them behind the other checks, 149 so.)"""
+    if (type(conv) is nn.Conv2d and x.is_cuda and not torch.is_grad_enabled() and x.dim() == 4
+            and not torch.compiler.is_compiling() and not torch.jit.is_tracing()
+            and _lib.projects_planes(x, conv.out_channels)
             and conv.kernel_size == (1, 1) and conv.stride == (1, 1) and conv.padding == (0, 0) and conv.groups == 1
             and x.is_contiguous()
             and not (conv._forward_hooks or conv._forward_pre_hooks or nn.modules.module._global_forward_hooks
-                     or nn.modules.module._global_forward_pre_hooks)):
+                     or nn.modules.module._global_forward_pre_hooks)
+            and _kernel_reads(conv, x)):
         out = _lib.project_shared(x, conv.weight, conv.bias)
         if out is not None:
             return out

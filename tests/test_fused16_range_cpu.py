@@ -35,9 +35,7 @@ def test_norm_project_says_what_it_serves():
 
 def test_plain_projections_say_what_extents_they_take():
     """Asked before anything else of a call that the projection kernels would refuse."""
-    for dtype, H, W, O, planes, cl in ((torch.bfloat16, 21, 13, 128, 0, 0), (torch.bfloat16, 42, 26, 128, 0, 0),
-                                       (torch.float16, 42, 28, 128, 1, 1), (torch.float16, 42, 28, 100, 0, 0),
-                                       (torch.float32, 42, 26, 128, 1, 1), (torch.float32, 21, 13, 128, 0, 1)):
-        x = torch.empty(2, 16, H, W, dtype=dtype)
-        assert _lib.projects(x, O, False) == bool(planes) and _lib.projects(x, O, True) == bool(cl), (dtype, H, W, O)
-        assert _lib.projects(x.contiguous(memory_format=torch.channels_last), O, True) == (O % 8 == 0)
+    for dtype, H, W, O, expected in ((torch.bfloat16, 21, 13, 128, False), (torch.bfloat16, 42, 26, 128, False),
+                                     (torch.float16, 42, 28, 128, True), (torch.float16, 42, 28, 100, False),
+                                     (torch.float32, 42, 26, 128, True), (torch.float32, 21, 13, 128, False)):
+        assert _lib.projects_planes(torch.empty(2, 16, H, W, dtype=dtype), O) == expected, (dtype, H, W, O)
