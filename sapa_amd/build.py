@@ -15,7 +15,7 @@ CSRC = os.path.join(HERE, 'csrc')
 OBJ = os.path.join(CSRC, '_obj')
 LIBDIR = os.path.join(HERE, 'lib')
 LIB = os.path.join(LIBDIR, 'libsapa_hip.so')
-SOURCES = ['capi.hip', 'sapa_b_generic.hip', 'sapa_b_tiled.hip', 'sapa_b_dot2.hip', 'sapa_b_wmat16.hip', 'sapa_b_nhwc.hip', 'sapa_b_nhwc_mm.hip', 'sapa_b_nhwc16.hip', 'sapa_b_nhwc_wm16.hip', 'sapa_b_mfma.hip', 'sapa_b_lowgrad.hip', 'sapa_b_bwd16.hip', 'sapa_b_nhwc_bwd16.hip', 'sapa_d.hip', 'sapa_d_lowgrad.hip', 'sapa_d_nhwc.hip', 'sapa_d_wmat16.hip', 'sapa_d_backward.hip', 'sapa_d_bwdmat.hip', 'sapa_d_scatter.hip', 'sapa_moments.hip', 'sapa_project.hip', 'sapa_layout.hip', 'sapa_stream.hip',
+SOURCES = ['capi.hip', 'sapa_b_generic.hip', 'sapa_b_tiled.hip', 'sapa_b_dot2.hip', 'sapa_b_wmat16.hip', 'sapa_b_nhwc.hip', 'sapa_b_nhwc_mm.hip', 'sapa_b_nhwc16.hip', 'sapa_b_nhwc_wm16.hip', 'sapa_b_mfma.hip', 'sapa_b_lowgrad.hip', 'sapa_b_bwd16.hip', 'sapa_b_nhwc_bwd16.hip', 'sapa_d.hip', 'sapa_d_lowgrad.hip', 'sapa_d_nhwc.hip', 'sapa_d_wmat16.hip', 'sapa_d_backward.hip', 'sapa_d_bwdmat.hip', 'sapa_d_region_bwd16.hip', 'sapa_d_scatter.hip', 'sapa_moments.hip', 'sapa_project.hip', 'sapa_layout.hip', 'sapa_stream.hip',
            'sapa_d_lds.hip']
 
 HIPCC = os.environ.get('HIPCC', '/opt/rocm/bin/hipcc')
@@ -35,6 +35,7 @@ SOURCE_FLAGS = {'sapa_b_bwd16.hip': ['-mllvm', '-amdgpu-mfma-vgpr-form'],
                 'sapa_b_nhwc16.hip': ['-mllvm', '-amdgpu-mfma-vgpr-form'],
                 'sapa_d_nhwc.hip': ['-mllvm', '-amdgpu-mfma-vgpr-form'],
                 'sapa_d_wmat16.hip': ['-mllvm', '-amdgpu-mfma-vgpr-form'],
+                'sapa_d_region_bwd16.hip': ['-mllvm', '-amdgpu-mfma-vgpr-form'],
                 'sapa_d_bwdmat.hip': ['-mllvm', '-amdgpu-mfma-vgpr-form'],
                 'sapa_d_scatter.hip': ['-mllvm', '-amdgpu-mfma-vgpr-form']}
 

@@ -194,6 +194,15 @@ hipError_t deform_fused_wmat16_launch(const void *q, const void *key, const void
                                       int W, int P, int s, int G, int dtype, hipStream_t st,
                                       bool nchw = false, int olayout = 0);
 
+// sapa_d_region_bwd16.hip: the fused operator's backward for f16 / bf16 and s = 2 in one kernel; key and value
+// as channels-last copies, grad_key / grad_value channels-last fp32 buffers that are accumulated into;
+// any gradient may be null.  hipErrorNotSupported where it does not serve the call.
+bool deform_bwd_region16_serves(int B, int Cq, int C, int H, int W, int P, int s, int G, int dtype);
+hipError_t deform_bwd_region16_launch(const void *grad_out, const void *q, const void *key_cl, const void *value_cl,
+                                      const void *offset, void *grad_q, void *grad_offset, float *grad_key,
+                                      float *grad_value, int B, int Cq, int C, int H, int W, int P, int s, int G,
+                                      int dtype, hipStream_t st);
+
 // sapa_b_dot2.hip: qk, qk+softmax and fused for f16 / bf16 tensors on the
 // two-term dot-product instructions (K = 5, s = 2); hipErrorNotSupported
 // otherwise.  wide: fp32 K*K-channel tensors next to the 16-bit features

@@ -1,0 +1,73 @@
+"""The one-kernel backward of fused SAPA-D for 16-bit tensors at up_factor 2: strips of parent rows that
+go round the window ring, ragged edges, far points, values that are not finite."""
+import pytest
+import torch
+
+import sapa_amd
+from helpers import deform_fused_backward_oracle, gen, randn
+from test_gpu_sapa_d import DEV, dev, make
+
+pytestmark = pytest.mark.gpu
+NAMES = ('grad_query', 'grad_key', 'grad_value', 'grad_offset')
+# B, G, dq, cg, H, W, P, offset scale: 37 rows go round the ring twice and a ragged strip beside a whole one;
+# rows of two pixels over a multiple of 4; one narrow strip, many segments; far points in both lane mappings
+SHAPES = [(1, 2, 32, 64, 37, 21, 25, 0.75), (2, 1, 24, 40, 20, 9, 16, 2.0), (1, 1, 8, 8, 50, 3, 2, 0.7),
+          (1, 2, 32, 64, 17, 13, 32, 6.0), (3, 2, 16, 24, 3, 5, 9, 1.0), (1, 1, 32, 48, 33, 16, 17, 1.5)]
+
+
+def _inputs(shape, dtype, seed=400):
+    B, G, dq, cg, H, W, P, oscale = shape
+    g = gen(seed)
+    q, key, v, off, _ = make(g, (B, G, dq, cg, H, W, P, 2), off_scale=oscale)
+    off = off.floor() + (off - off.floor()).clamp(0.2, 0.8)      # rounding must not cross a cell's edge
+    go = randn(g, B, G * cg, 2 * H, 2 * W)
+    return [t.to(dtype) for t in (q, key, v, off, go)]
+
+
+def _gradients(q, key, v, off, go, P, G):
+    t = [x.requires_grad_() for x in dev(q, key, v, off)]
+    out = sapa_amd.deform_sapa_fused(*t, P, 2, G)
+    return torch.autograd.grad(out, t, go.to(DEV))
+
+
+@pytest.mark.parametrize('dtype', [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize('shape', SHAPES, ids=['-'.join(map(str, s)) for s in SHAPES])
+def test_against_the_exact_chain(coracle, shape, dtype):
+    """One rounding of each gradient (half a spacing: 2^-8 / 2^-11 of the value at most), and the fp32 chain's
+    own errors, of some 1e-5 of what cancels in it (up to 40 rms over these sizes)."""
+    P, G = shape[6], shape[1]
+    q, key, v, off, go = _inputs(shape, dtype)
+    want = deform_fused_backward_oracle(coracle, go.float(), q.float(), key.float(), v.float(), off.float(), P, 2, G)
+    rel = 2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -11
+    for got, w, name in zip(_gradients(q, key, v, off, go, P, G), want, NAMES):
+        err, rms = (got.cpu().double() - w).abs(), w.pow(2).mean().sqrt()
+        worst = (err / (rel * w.abs() + 4e-4 * rms)).max().item()
+        assert worst <= 1, f'{name}: {worst}'
+
+
+@pytest.mark.parametrize('which', ['query', 'key', 'value', 'grad_out'])
+@pytest.mark.parametrize('bad', [float('inf'), float('nan')])
+def test_non_finite_values_reach_what_they_belong_to(coracle, which, bad):
+    """Gradients that the exact chain has as infinite or NaN, and no others, are not finite."""
+    shape = (1, 2, 16, 24, 19, 11, 9, 0.7)
+    q, key, v, off, go = _inputs(shape, torch.bfloat16, seed=401)
+    t = {'query': q, 'key': key, 'value': v, 'grad_out': go}[which]
+    t[0, 3, 6, 5] = bad
+    t[0, t.size(1) - 1, 12, 9] = bad
+    want = deform_fused_backward_oracle(coracle, go.float(), q.float(), key.float(), v.float(), off.float(), 9, 2, 2)
+    for got, w, name in zip(_gradients(q, key, v, off, go, 9, 2), want, NAMES):
+        assert torch.equal(torch.isfinite(got).cpu(), torch.isfinite(w)), name
+
+
+def test_gradients_of_any_size_in_fp16(coracle):
+    """fp16 gradients that are small or large as a whole (loss scales), and pixels 2^-12 apart."""
+    shape = (1, 1, 32, 64, 18, 17, 25, 0.75)
+    q, key, v, off, go = _inputs(shape, torch.float32, seed=402)
+    go[..., ::2] *= 2.0 ** -12
+    for scale in (2.0 ** -10, 2.0 ** 6):
+        a = [t.half() for t in (q, key, v, off, go * scale)]
+        want = deform_fused_backward_oracle(coracle, a[4].float(), *(t.float() for t in a[:4]), 25, 2, 1)
+        for got, w, name in zip(_gradients(*a, 25, 1), want, NAMES):
+            err, rms = (got.cpu().double() - w).abs(), w.pow(2).mean().sqrt()
+            # (2^-25: half the smallest spacing of the type)
+            assert bool((err <= 2.0 ** -11 * w.abs() + 4e-4 * rms + 2.0 ** -25).all()), (name, scale)
