@@ -187,6 +187,16 @@ int sapa_fused_backward_direct(const void *grad_out, const void *query, const vo
                                void *grad_key, void *grad_value, int B, int d, int C,
                                int H, int W, int K, int s, int channels_last, int dtype,
                                void *stream);
+/* The same with scratch of sapa_fused_backward_direct_workspace bytes (0: not served),
+ * which serves contiguous tensors of an odd W too (their key and value are copied
+ * into rows of an even number of cells there). */
+long long sapa_fused_backward_direct_workspace(int B, int d, int C, int H, int W, int K,
+                                               int s, int channels_last, int dtype);
+int sapa_fused_backward_direct_ws(const void *grad_out, const void *query, const void *key,
+                                  const void *value, void *workspace, void *grad_query,
+                                  void *grad_key, void *grad_value, int B, int d, int C,
+                                  int H, int W, int K, int s, int channels_last, int dtype,
+                                  void *stream);
 
 /* Softmax over the middle axis of x [N,R,M] -> y [N,R,M] (max-subtracted,
  * fp32 arithmetic for 16-bit types).  Covers the reference's

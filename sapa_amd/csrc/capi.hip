@@ -321,7 +321,7 @@ static int fused_backward_impl(const void *grad_out, const void *query, const vo
         // 16-bit tensors: two kernels from the four operands, no K*K tensors (they take 3 floats per
         // pixel of the workspace)
         const hipError_t e = sapa_b_bwd16_launch(query, key, value, grad_out, workspace, grad_query, grad_key,
-                                                 grad_value, B, d, C, H, W, K, s, dtype, st);
+                                                 grad_value, B, d, C, H, W, K, s, dtype, st, 12L * B * H * s * W * s);
         if (e != hipErrorNotSupported) return finish(e);
     }
     float *grad_logits = (float *)workspace + (attn_given ? 0LL : (long long)B * K * K * H * s * W * s);
@@ -366,23 +366,50 @@ int sapa_fused_backward(const void *grad_out, const void *query, const void *key
                                grad_value, B, d, C, H, W, K, s, dtype, stream);
 }
 
-int sapa_fused_backward_direct_serves(int d, int C, int H, int W, int K, int s, int channels_last, int dtype) {
-    if (d <= 0 || C <= 0 || H <= 0 || W <= 0) return 0;
-    return channels_last ? sapa_b_nhwc_bwd16_serves(d, C, H, W, K, s, dtype) : sapa_b_bwd16_serves(d, C, H, W, K, s, dtype);
-}
-
-int sapa_fused_backward_direct(const void *grad_out, const void *query, const void *key, const void *value,
-                               void *stats, void *grad_query, void *grad_key, void *grad_value, int B, int d,
-                               int C, int H, int W, int K, int s, int channels_last, int dtype, void *stream) {
+// scratch: bytes at `workspace`
+static int backward_direct(const void *grad_out, const void *query, const void *key, const void *value,
+                           void *workspace, long scratch, void *grad_query, void *grad_key, void *grad_value, int B,
+                           int d, int C, int H, int W, int K, int s, int channels_last, int dtype, void *stream) {
     const int rc = check_window_args(B, d, C, H, W, K, s, dtype);
     if (rc != SAPA_OK) return rc;
     if (B == 0) return SAPA_OK;
-    if (!grad_out || !query || !key || !value || !stats) return SAPA_ERR_INVALID_ARGUMENT;
-    const hipError_t e = (channels_last ? sapa_b_nhwc_bwd16_launch : sapa_b_bwd16_launch)(
-        query, key, value, grad_out, stats, grad_query, grad_key, grad_value, B, d, C, H, W, K, s, dtype,
-        (hipStream_t)stream);
+    if (!grad_out || !query || !key || !value || !workspace) return SAPA_ERR_INVALID_ARGUMENT;
+    hipStream_t st = (hipStream_t)stream;
+    const hipError_t e =
+        channels_last ? sapa_b_nhwc_bwd16_launch(query, key, value, grad_out, workspace, grad_query, grad_key, grad_value, B, d, C, H, W, K, s, dtype, st)
+                      : sapa_b_bwd16_launch(query, key, value, grad_out, workspace, grad_query, grad_key, grad_value, B, d, C, H, W, K, s, dtype, st, scratch);
     if (e == hipErrorNotSupported) return SAPA_ERR_UNSUPPORTED;
     return finish(e);
+}
+
+// (scratch of 3 floats per output pixel: contiguous rows of an odd number of cells need more)
+int sapa_fused_backward_direct_serves(int d, int C, int H, int W, int K, int s, int channels_last, int dtype) {
+    if (d <= 0 || C <= 0 || H <= 0 || W <= 0) return 0;
+    return channels_last ? sapa_b_nhwc_bwd16_serves(d, C, H, W, K, s, dtype)
+                         : W % 2 == 0 && sapa_b_bwd16_serves(d, C, H, W, K, s, dtype);
+}
+
+int sapa_fused_backward_direct(const void *grad_out, const void *query, const void *key, const void *value,
+                               void *stats, void *grad_query, void *grad_key, void *grad_value, int B, int d, int C,
+                               int H, int W, int K, int s, int channels_last, int dtype, void *stream) {
+    return backward_direct(grad_out, query, key, value, stats, 12L * B * H * s * W * s, grad_query, grad_key, grad_value, B,
+                           d, C, H, W, K, s, channels_last, dtype, stream);
+}
+
+long long sapa_fused_backward_direct_workspace(int B, int d, int C, int H, int W, int K, int s, int channels_last,
+                                               int dtype) {
+    if (B < 0 || d <= 0 || C <= 0 || H <= 0 || W <= 0) return 0;
+    if (B == 0) B = 1;      // (0 bytes: not served)
+    if (channels_last) return sapa_b_nhwc_bwd16_serves(d, C, H, W, K, s, dtype) ? 48LL * B * H * W : 0;
+    return sapa_b_bwd16_serves(d, C, H, W, K, s, dtype) ? sapa_b_bwd16_workspace(B, d, C, H, W) : 0;
+}
+
+int sapa_fused_backward_direct_ws(const void *grad_out, const void *query, const void *key, const void *value,
+                                  void *workspace, void *grad_query, void *grad_key, void *grad_value, int B, int d,
+                                  int C, int H, int W, int K, int s, int channels_last, int dtype, void *stream) {
+    return backward_direct(grad_out, query, key, value, workspace,
+                           sapa_fused_backward_direct_workspace(B, d, C, H, W, K, s, channels_last, dtype), grad_query,
+                           grad_key, grad_value, B, d, C, H, W, K, s, channels_last, dtype, stream);
 }
 
 int sapa_fused_forward_attn(const void *query, const void *key, const void *value, void *attn,

@@ -55,11 +55,13 @@ hipError_t sapa_b_nhwc_wm16_launch(int mode, const void *q, const void *key, con
 
 
 // sapa_b_bwd16.hip: the gradients of the fused operator (any may be NULL) for contiguous f16 / bf16 tensors,
-// K = 5, s = 2; stats: 3 floats per output pixel (scratch).  hipErrorNotSupported otherwise, nothing launched.
+// K = 5, s = 2; stats: scratch, of which sapa_b_bwd16_workspace bytes are needed.  hipErrorNotSupported otherwise,
+// nothing launched.
 bool sapa_b_bwd16_serves(int d, int C, int H, int W, int K, int s, int dtype);
+long sapa_b_bwd16_workspace(int B, int d, int C, int H, int W);
 hipError_t sapa_b_bwd16_launch(const void *q, const void *key, const void *value, const void *grad_out, void *stats,
                                void *grad_q, void *grad_key, void *grad_value, int B, int d, int C, int H, int W,
-                               int K, int s, int dtype, hipStream_t st);
+                               int K, int s, int dtype, hipStream_t st, long scratch);
 
 // sapa_b_nhwc_bwd16.hip: the same for channels-last tensors
 bool sapa_b_nhwc_bwd16_serves(int d, int C, int H, int W, int K, int s, int dtype);

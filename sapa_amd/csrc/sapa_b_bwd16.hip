@@ -32,7 +32,10 @@
 //
 // Measured (B=16, C=256, d=64, 100x168, bf16): pixel kernel 295 us, cell kernel 429 us, a training step
 // 970 us against 1211 for the chain over K * K tensors (similarity and its softmax backward 274 us,
-// grad_q 92, grad_value and grad_key by vector fmas 544, the weights 86).
+// grad_q 92, grad_value and grad_key by vector fmas 544, the weights 86).  Odd W: key and value are copied into rows
+// of an even number of cells first (direct loads begin on dwords); B=16, 100x167 1597 -> 1170 us for a step,
+// of which the copies 108 and the cell kernel 503 (hi-res pieces across cache lines, results moved by half
+// a dword; 560 with a 2-byte store per result); B=8, d=64, 51x83 441 -> 198, B=4, C=512, d=32, 97x165 916 -> 540.
 #include "wm16_exact.hpp"
 
 namespace sapa {
@@ -48,8 +51,42 @@ template <typename T> struct Args {
     const T *q, *key, *value, *grad_out;
     float *stats;
     T *grad_q, *grad_key, *grad_value;
-    int B, d, C, H, W, tiles_x, tiles_y, ns, nblocks, per_xcd;
+    // the key and value that the products read, in rows of `low_w` (even) cells: the tensors, or copies with a
+    // cell more per row where W is odd -- direct loads begin on dwords
+    const T *key_rows, *value_rows;
+    int B, d, C, H, W, low_w, tiles_x, tiles_y, ns, nblocks, per_xcd;
 };
+
+// Rows of w 16-bit cells -> rows of w + 1 (w odd), the added cell 0; two tensors in one launch.  A thread moves 4
+// dwords of a row, from the dword before where the row begins in the middle of one (B=16, d=64, C=256,
+// 100x167: 108 us = 3.2 TB/s; 131 with a thread per dword).
+__global__ __launch_bounds__(256) void
+pad_rows_kernel(const unsigned short *__restrict__ a, const unsigned short *__restrict__ b, u32 *__restrict__ pa,
+                u32 *__restrict__ pb, long rows_a, long rows_b, int w) {
+    const unsigned short *const src = blockIdx.y ? b : a;
+    u32 *const dst = blockIdx.y ? pb : pa;
+    const u32 per_row = (u32)(w + 1) / 2, pieces = (per_row + 3) / 4;
+    const long n = (blockIdx.y ? rows_b : rows_a) * pieces;
+    for (long i = blockIdx.x * 256L + threadIdx.x; i < n; i += gridDim.x * 256L) {
+        const long row = i < (1L << 31) ? (long)((u32)i / pieces) : i / pieces;
+        const u32 x = 4 * (u32)(i - row * pieces);           // first dword
+        const unsigned short *const p = src + row * w + 2 * x;
+        u32 *const o = dst + row * per_row + x;
+        if (x + 4 < per_row) {
+            // (cells 2 x .. 2 x + 7 and one more are the row's own)
+            typedef u32x4 __attribute__((aligned(4))) u32x4_a4;
+            const bool half = (uintptr_t)p % 4 != 0;
+            const u32 *const q = (const u32 *)(p - half);
+            const u32x4 v = *(const u32x4_a4 *)q;
+            const u32 next = half ? q[4] : 0u;
+            *(u32x4_a4 *)o = half ? u32x4{__builtin_amdgcn_alignbit(v[1], v[0], 16), __builtin_amdgcn_alignbit(v[2], v[1], 16),
+                                          __builtin_amdgcn_alignbit(v[3], v[2], 16), __builtin_amdgcn_alignbit(next, v[3], 16)}
+                                  : v;
+        } else {
+            for (u32 k = 0; k < per_row - x; ++k) o[k] = p[2 * k] | (2 * (x + k) + 1 < (u32)w ? (u32)p[2 * k + 1] << 16 : 0u);
+        }
+    }
+}
 
 // position of the 16-byte piece of row r, channel ch in the swizzled tile of bwd_pixel_kernel
 __device__ __forceinline__ int swz(int ch, int r) { return ((ch & 7) << 1) | ((r + (ch >> 3)) & 1); }
@@ -78,7 +115,7 @@ __device__ __attribute__((noinline)) void children_again(Again again) {
 template <typename T, int NSW, bool STREAM>
 __global__ __launch_bounds__(128 * NSW) void
 bwd_pixel_kernel(const Args<T> args) {
-    const T *__restrict__ const q = args.q, *__restrict__ const key = args.key, *__restrict__ const value = args.value,
+    const T *__restrict__ const q = args.q, *__restrict__ const key = args.key_rows, *__restrict__ const value = args.value_rows,
             *__restrict__ const grad_out = args.grad_out;
     T *__restrict__ const grad_q = args.grad_q;
     float *__restrict__ const stats = args.stats;
@@ -112,20 +149,22 @@ bwd_pixel_kernel(const Args<T> args) {
     const int t = wave % NSW, half = wave / NSW;              // block of the tile, half of its children
     const int g = lane >> 4, i16 = lane & 15;
     const long lpix = (long)H * W;
-    const u32 lplane = (u32)(lpix * sizeof(T)), hplane = 4 * lplane;
+    const int low_w = args.low_w;
+    const long lowpix = (long)H * low_w;
+    const u32 lplane = (u32)(lowpix * sizeof(T)), hplane = (u32)(4 * lpix * sizeof(T));
 
     // direct-load offsets inside one image, without the chunk's first channel; the low-res pieces as
     // in sapa_b_wmat16.hip (a piece that runs over an end of its row brings the neighbouring row's
     // cells; the one that starts before the image reads as zeros and is patched)
     u32 off_low, off_hi;
-    bool half_piece;           // W % 4 == 2: a row's last 16-byte piece holds 4 of its children and 4 of the next row's
+    int short_piece;           // W % 4 != 0: dwords of a row's last 16-byte piece (the rest is the next row's), else 0
     int patch_slot = -1;
     {
         const int slot = tid, rc = slot / (LROW / 4), pc = slot % (LROW / 4);
         const int r = rc / CHK, ch = rc % CHK;
         const int y = Y0 - 2 + r, x = X0 - 2 + 8 * pc;
         const bool ok = slot < NLP && 8 * pc < 4 * ns_here + 4 && y >= 0 && y < H && x < W;
-        off_low = ok ? (u32)(ch * lpix + (long)y * W + x) * (u32)sizeof(T) : OUTSIDE;
+        off_low = ok ? (u32)(ch * lowpix + (long)y * low_w + x) * (u32)sizeof(T) : OUTSIDE;
         if (ok && x < 0 && y == 0 && ch == 0) patch_slot = slot;
     }
     {
@@ -134,14 +173,14 @@ bwd_pixel_kernel(const Args<T> args) {
         const int cy = 2 * Y0 + r, cx = 2 * X0 + 8 * pc;
         const bool ok = pc < ns_here && cy < 2 * H && cx < 2 * W;
         off_hi = ok ? (u32)(ch * 4 * lpix + (long)cy * 2 * W + cx) * (u32)sizeof(T) : OUTSIDE;
-        half_piece = ok && cx + 8 > 2 * W;
+        short_piece = ok && cx + 8 > 2 * W ? W - cx / 2 : 0;
     }
 
     const int nKc = (d + CHK - 1) / CHK, nVc = (C + CHK - 1) / CHK;
     const int ntot = nKc + nVc + (grad_q ? nKc : 0);
     const u32x4 rq = dma_rsrc(q + (long)n * d * 4 * lpix, d * hplane);
-    const u32x4 rk = dma_rsrc(key + (long)n * d * lpix, d * lplane);
-    const u32x4 rv = dma_rsrc(value + (long)n * C * lpix, C * lplane);
+    const u32x4 rk = dma_rsrc(key + (long)n * d * lowpix, d * lplane);
+    const u32x4 rv = dma_rsrc(value + (long)n * C * lowpix, C * lplane);
     const u32x4 rg = dma_rsrc(grad_out + (long)n * C * 4 * lpix, C * hplane);
 
     // phase of chunk j: 0 = key + q, 1 = value + grad_out, 2 = key
@@ -167,7 +206,7 @@ bwd_pixel_kernel(const Args<T> args) {
     // upper left corner)
     auto patch_low = [&](int j) __attribute__((always_inline)) {
         if (tx == 0 && ty == 0 && patch_slot >= 0 && (j == 0 || j == nKc || j == nKc + nVc) && j < ntot) {
-            const u32 *src = (const u32 *)(j == nKc ? value + (long)n * C * lpix : key + (long)n * d * lpix);
+            const u32 *src = (const u32 *)(j == nKc ? value + (long)n * C * lowpix : key + (long)n * d * lowpix);
             u32 *dst = lowbuf + (j % NBUF) * LOWBUF + patch_slot * 4;
 #pragma unroll
             for (int k = 1; k < 4; ++k) dst[k] = src[k - 1];
@@ -377,8 +416,10 @@ bwd_pixel_kernel(const Args<T> args) {
         lds_barrier();
         const u32x4 o = *(const u32x4 *)(ob + tid * 4);
         u32 off = off_hi + c0 * hplane;
-        if (row_tail && half_piece) {
-            __builtin_amdgcn_raw_buffer_store_b64(u32x2{o[0], o[1]}, ro, off, 0, 0);
+        if (row_tail && short_piece) {
+#pragma unroll
+            for (int k = 0; k < 3; ++k)
+                if (k < short_piece) __builtin_amdgcn_raw_buffer_store_b32(o[k], ro, off + 4 * k, 0, 0);
             off = OUTSIDE;
         }
         __builtin_amdgcn_raw_buffer_store_b128(o, ro, off, 0, STREAM ? 2 : 0);
@@ -449,10 +490,11 @@ __device__ __attribute__((noinline)) void cells_again(Again again) {
                                      plane_of<false>(a.grad_value, n, a.C, lpix), a.d, a.C, a.H, a.W, cy, cx + 4 * (int)b);
 }
 
-template <typename T>
+// ODD: an odd W
+template <typename T, bool ODD>
 __global__ __launch_bounds__(CNT) void
 bwd_cell_kernel(const Args<T> args) {
-    const T *__restrict__ const q = args.q, *__restrict__ const key = args.key, *__restrict__ const value = args.value,
+    const T *__restrict__ const q = args.q, *__restrict__ const key = args.key_rows, *__restrict__ const value = args.value_rows,
             *__restrict__ const grad_out = args.grad_out;
     T *__restrict__ const grad_key = args.grad_key, *__restrict__ const grad_value = args.grad_value;
     const float *__restrict__ const stats = args.stats;
@@ -477,7 +519,9 @@ bwd_cell_kernel(const Args<T> args) {
     const int I0 = tx * TBX;
     const bool active = 4 * (I0 + bi) - 2 < W;
     const long lpix = (long)H * W;
-    const u32 lplane = (u32)(lpix * sizeof(T)), hplane = 4 * lplane;
+    const int low_w = ODD ? args.low_w : W;
+    const long lowpix = (long)H * low_w;
+    const u32 lplane = (u32)(lowpix * sizeof(T)), hplane = (u32)(4 * lpix * sizeof(T));
 
     // direct-load offsets inside one image, without the chunk's first channel
     u32 off_hi[CNH + 1];
@@ -495,15 +539,15 @@ bwd_cell_kernel(const Args<T> args) {
     // The piece 2 cells before the image's first has no address: zeros, and patched.
     const int lslot = tid & (64 * CNL - 1), lch = lslot / (2 * TBX), ly = 4 * J - 2 + (lslot / (TBX / 2)) % 4, lx = 4 * I0 - 2 + 8 * (lslot % (TBX / 2));
     const bool lrow = ((u32)ly < (u32)H) & (lx < W);
-    const u32 off_low = lrow ? (u32)(lch * lpix + (long)ly * W + lx) * (u32)sizeof(T) : OUTSIDE;
+    const u32 off_low = lrow ? (u32)(lch * lowpix + (long)ly * low_w + lx) * (u32)sizeof(T) : OUTSIDE;
     const bool patch = lx < 0 && ly == 0 && lch == 0 && wave >= 4 && wave < 4 + CNL;
     const bool ragged = I0 == 0 || 4 * I0 - 2 + 4 * TBX > W;  // workgroup-uniform
 
     const int nKc = (d + CHK - 1) / CHK, nVc = (C + CHK - 1) / CHK;
     const int ntot = nKc + nVc + (grad_key ? nKc : 0);
     const u32x4 rq = dma_rsrc(q + (long)n * d * 4 * lpix, d * hplane);
-    const u32x4 rk = dma_rsrc(key + (long)n * d * lpix, d * lplane);
-    const u32x4 rv = dma_rsrc(value + (long)n * C * lpix, C * lplane);
+    const u32x4 rk = dma_rsrc(key + (long)n * d * lowpix, d * lplane);
+    const u32x4 rv = dma_rsrc(value + (long)n * C * lowpix, C * lplane);
     const u32x4 rg = dma_rsrc(grad_out + (long)n * C * 4 * lpix, C * hplane);
 
     // chunk j: q + key (S), grad_out + value (G and grad_value), q again (grad_key)
@@ -595,7 +639,29 @@ bwd_cell_kernel(const Args<T> args) {
         const f32x4 a = *(const f32x4 *)p0 + *(const f32x4 *)(p0 + COUT), b = *(const f32x4 *)p1 + *(const f32x4 *)(p1 + COUT);
         const u32x4 o = {pack2<T>(a[0], a[1]), pack2<T>(a[2], a[3]), pack2<T>(b[0], b[1]), pack2<T>(b[2], b[3])};
         const u32 off = (u32)((c0 + (u32)lch) * (u32)lpix + ly * W + lx) * (u32)sizeof(T);
-        if (!ragged) {
+        if (ODD) {
+            // A row that begins in the middle of a dword takes its pieces half a dword to the left: the
+            // last cell of the piece before (the lane before's), then this one's first seven; the first cells
+            // of the tile's row and the last one before a piece that is not whole by themselves.  Pieces
+            // over an end of the image's row: cell by cell.
+            const int pc = lslot % (TBX / 2);
+            const u32 before = (u32)__shfl_up((int)o[3], 1);
+            const bool here = lrow & (lx >= 0) & (lx + 8 <= W), next_whole = (pc < TBX / 2 - 1) & (lx + 16 <= W);
+            const bool whole = here & ((pc > 0) | next_whole), half = ((((c0 + (u32)lch) & 1) * (u32)(lpix & 1) + (u32)(ly & 1)) & 1) != 0;
+            const u32x4 left = {__builtin_amdgcn_alignbit(o[0], before, 16), __builtin_amdgcn_alignbit(o[1], o[0], 16),
+                                __builtin_amdgcn_alignbit(o[2], o[1], 16), __builtin_amdgcn_alignbit(o[3], o[2], 16)};
+            const bool first = half & (pc == 0), last = half & !next_whole;
+            __builtin_amdgcn_raw_buffer_store_b128(half ? left : o, ro, whole & !first ? half ? off - 2 : off : OUTSIDE, 0, 0);
+            __builtin_amdgcn_raw_buffer_store_b96(u32x3{left[1], left[2], left[3]}, ro, whole & first ? off + 2 : OUTSIDE, 0, 0);
+            __builtin_amdgcn_raw_buffer_store_b16((unsigned short)(first ? o[0] : o[3] >> 16), ro,
+                                                  whole & first ? off : whole & last ? off + 14 : OUTSIDE, 0, 0);
+            if (ragged) {
+#pragma unroll
+                for (int k = 0; k < 8; ++k)
+                    __builtin_amdgcn_raw_buffer_store_b16((unsigned short)(o[k / 2] >> (16 * (k & 1))), ro,
+                                                          lrow & !whole & ((u32)(lx + k) < (u32)W) ? off + 2 * k : OUTSIDE, 0, 0);
+            }
+        } else if (!ragged) {
             __builtin_amdgcn_raw_buffer_store_b128(o, ro, lrow ? off : OUTSIDE, 0, 0);
         } else {
 #pragma unroll
@@ -608,12 +674,12 @@ bwd_cell_kernel(const Args<T> args) {
     // j + CBUF requested
     auto next = [&](int j, int outs) __attribute__((always_inline)) {
         if (outs > CBUF - 1) outs = CBUF - 1;
-        int after = wave < CNL ? outs * (ragged ? 4 : 1) : 0;
+        int after = wave < CNL ? outs * (ODD ? ragged ? 11 : 3 : ragged ? 4 : 1) : 0;
 #pragma unroll
         for (int i = 2; i < CBUF; ++i) after += loads_of(j + i);
         wait_all_but(after);
         if (patch && (j + 1 == 0 || j + 1 == nKc)) {
-            const u32 *src = (const u32 *)(j + 1 == 0 ? key + (long)n * d * lpix : value + (long)n * C * lpix);
+            const u32 *src = (const u32 *)(j + 1 == 0 ? key + (long)n * d * lowpix : value + (long)n * C * lowpix);
             u32 *dst = lowbuf + (j + 1) % CBUF * CLOW + lslot * 4;
 #pragma unroll
             for (int k = 1; k < 4; ++k) dst[k] = src[k - 1];
@@ -690,7 +756,7 @@ bwd_cell_kernel(const Args<T> args) {
     {
         // (a NULL grad_value: a descriptor of no bytes drops the stores)
         const __amdgpu_buffer_rsrc_t ro = __builtin_amdgcn_make_buffer_rsrc(
-            (void *)(grad_value + (long)n * C * lpix), 0, grad_value ? (int)(C * lplane) : 0, 0x00020000);
+            (void *)(grad_value + (long)n * C * lpix), 0, grad_value ? (int)(C * lpix * sizeof(T)) : 0, 0x00020000);
         for (int j = nKc; j < nKc + nVc; ++j) {
             if (active) {
                 if (grad_key) similarity(j, acc);
@@ -720,7 +786,7 @@ bwd_cell_kernel(const Args<T> args) {
             hold(w);
         }
         const __amdgpu_buffer_rsrc_t ro = __builtin_amdgcn_make_buffer_rsrc(
-            (void *)(grad_key + (long)n * d * lpix), 0, (int)(d * lplane), 0x00020000);
+            (void *)(grad_key + (long)n * d * lpix), 0, (int)(d * lpix * sizeof(T)), 0x00020000);
         for (int j = nKc + nVc; j < ntot; ++j) {
             if (active) gather(j);
             next(j, j - nKc);
@@ -735,13 +801,30 @@ bwd_cell_kernel(const Args<T> args) {
     if (__builtin_expect(blocks != 0, 0)) cells_again<T>(Again(lds, blocks));
 }
 
+static long align256(long x) { return (x + 255) / 256 * 256; }
+static long stats_bytes(int B, int H, int W) { return 48L * B * H * W; }
+static long padded_bytes(int B, int channels, int H, int W) { return 2L * B * channels * H * (W + 1); }
+
 template <typename T, bool STREAM>
 static hipError_t launch(const void *q, const void *key, const void *value, const void *grad_out, float *stats,
                          void *grad_q, void *grad_key, void *grad_value, int B, int d, int C, int H, int W,
                          hipStream_t st) {
     constexpr int NSW = 8;
+    const bool odd = W % 2 != 0;
+    const void *key_rows = key, *value_rows = value;
+    if (odd) {
+        u32 *const pk = (u32 *)((char *)stats + align256(stats_bytes(B, H, W)));
+        u32 *const pv = (u32 *)((char *)pk + align256(padded_bytes(B, d, H, W)));
+        const long most = (long)B * (d > C ? d : C) * H * (((W + 1) / 2 + 3) / 4);
+        const long blocks = (most + 255) / 256;
+        hipLaunchKernelGGL(pad_rows_kernel, dim3((unsigned)(blocks < 4096 ? blocks : 4096), 2), dim3(256), 0, st,
+                           (const unsigned short *)key, (const unsigned short *)value, pk, pv, (long)B * d * H, (long)B * C * H, W);
+        const hipError_t e = hipGetLastError();
+        if (e != hipSuccess) return e;
+        key_rows = pk, value_rows = pv;
+    }
     Args<T> args{(const T *)q, (const T *)key, (const T *)value, (const T *)grad_out, stats, (T *)grad_q, (T *)grad_key,
-                 (T *)grad_value, B, d, C, H, W, 0, 0, 0, 0, 0};
+                 (T *)grad_value, (const T *)key_rows, (const T *)value_rows, B, d, C, H, W, W + (odd ? 1 : 0), 0, 0, 0, 0, 0};
     // sets the tiles; false: too many
     auto tile = [&](int tiles_x, int tiles_y) {
         const long nb = (long)tiles_x * tiles_y * B;
@@ -760,26 +843,35 @@ static hipError_t launch(const void *q, const void *key, const void *value, cons
     // cell blocks 4 I - 2 .. 4 I + 1 that hold a cell of 0 .. W - 1
     const int nI = (W + 1) / 4 + 1, nJ = (H + 1) / 4 + 1;
     if (!tile((nI + TBX - 1) / TBX, nJ)) return hipErrorNotSupported;
-    hipLaunchKernelGGL((bwd_cell_kernel<T>), dim3(args.per_xcd * 8), dim3(CNT), 0, st, args);
+    if (odd) hipLaunchKernelGGL((bwd_cell_kernel<T, true>), dim3(args.per_xcd * 8), dim3(CNT), 0, st, args);
+    else hipLaunchKernelGGL((bwd_cell_kernel<T, false>), dim3(args.per_xcd * 8), dim3(CNT), 0, st, args);
     return hipGetLastError();
 }
 
 }  // namespace bwm16
 
-// Gradients of the fused operator (any of them may be NULL); f16 / bf16, K = 5, s = 2, W even (rows
-// of whole dwords) and >= 16, low-res tensors 4-byte and high-res tensors 16-byte aligned, every image
-// of every tensor below 2 GiB; stats: 3 floats per output pixel, 16-byte aligned.
+// Gradients of the fused operator (any of them may be NULL); f16 / bf16, K = 5, s = 2, W >= 16, low-res tensors
+// 4-byte (W odd: 2-byte) and high-res tensors 16-byte aligned, every image of every tensor below 2 GiB.
+// Scratch (`scratch` bytes at stats): 3 floats per output pixel and, where W is odd, padded copies of key and
+// value.
 // hipErrorNotSupported otherwise (nothing is launched then).
 bool sapa_b_bwd16_serves(int d, int C, int H, int W, int K, int s, int dtype) {
-    return K == 5 && s == 2 && W % 2 == 0 && W >= 16 && (dtype == 2 || dtype == 3) &&
-           wm::offsets_fit(d > C ? d : C, (long)H * W * 8);
+    return K == 5 && s == 2 && W >= 16 && (dtype == 2 || dtype == 3) &&
+           wm::offsets_fit(d > C ? d : C, (long)H * (W + W % 2) * 8);
+}
+
+long sapa_b_bwd16_workspace(int B, int d, int C, int H, int W) {
+    using namespace bwm16;
+    return W % 2 == 0 ? stats_bytes(B, H, W)
+                      : align256(stats_bytes(B, H, W)) + align256(padded_bytes(B, d, H, W)) + padded_bytes(B, C, H, W);
 }
 
 hipError_t sapa_b_bwd16_launch(const void *q, const void *key, const void *value, const void *grad_out, void *stats,
                                void *grad_q, void *grad_key, void *grad_value, int B, int d, int C, int H, int W,
-                               int K, int s, int dtype, hipStream_t st) {
-    if (!sapa_b_bwd16_serves(d, C, H, W, K, s, dtype)) return hipErrorNotSupported;
-    if (((uintptr_t)key | (uintptr_t)value | (uintptr_t)grad_key | (uintptr_t)grad_value) % 4 != 0 ||
+                               int K, int s, int dtype, hipStream_t st, long scratch) {
+    if (!sapa_b_bwd16_serves(d, C, H, W, K, s, dtype) || scratch < sapa_b_bwd16_workspace(B, d, C, H, W))
+        return hipErrorNotSupported;
+    if (((uintptr_t)key | (uintptr_t)value | (uintptr_t)grad_key | (uintptr_t)grad_value) % (W % 2 ? 2 : 4) != 0 ||
         ((uintptr_t)q | (uintptr_t)grad_out | (uintptr_t)grad_q | (uintptr_t)stats) % 16 != 0)
         return hipErrorNotSupported;
     // Beyond the 256 MB memory-side cache the pixel kernel's hi-res traffic is non-temporal, as the

@@ -10,6 +10,7 @@ namespace wm {
 typedef unsigned u32;
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef u32 u32x2 __attribute__((ext_vector_type(2)));
+typedef u32 u32x3 __attribute__((ext_vector_type(3)));
 typedef u32 u32x4 __attribute__((ext_vector_type(4)));
 typedef short s16x4 __attribute__((ext_vector_type(4)));
 
@@ -129,7 +130,8 @@ __device__ __forceinline__ void wait_all_but(int after) {
 #define SAPA_WAIT_CASE(N) case N: asm volatile("s_waitcnt vmcnt(" #N ")" ::: "memory"); break;
     switch (after) {
         SAPA_WAIT_CASE(1) SAPA_WAIT_CASE(2) SAPA_WAIT_CASE(3) SAPA_WAIT_CASE(4) SAPA_WAIT_CASE(5) SAPA_WAIT_CASE(6)
-        SAPA_WAIT_CASE(7) SAPA_WAIT_CASE(8) SAPA_WAIT_CASE(9) SAPA_WAIT_CASE(10) SAPA_WAIT_CASE(11)
+        SAPA_WAIT_CASE(7) SAPA_WAIT_CASE(8) SAPA_WAIT_CASE(9) SAPA_WAIT_CASE(10) SAPA_WAIT_CASE(11) SAPA_WAIT_CASE(13)
+        SAPA_WAIT_CASE(14) SAPA_WAIT_CASE(24) SAPA_WAIT_CASE(25)
         default: asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); break;
     }
 #undef SAPA_WAIT_CASE

@@ -206,28 +206,35 @@ def qk_softmax(query, key, kernel_size, scale_factor):
     return _qk_softmax_forward(query, key, kernel_size, scale_factor, nhwc)
 
 
+def _direct_scratch(query, key, value, K, s, nhwc):
+    """Bytes of scratch with which sapa_fused_backward_direct_ws serves these operands; 0: it does not."""
+    if not (value.dtype in (torch.float16, torch.bfloat16) and query.dtype == key.dtype == value.dtype):
+        return 0
+    n, c, h, w = value.size()
+    return _lib.lib().sapa_fused_backward_direct_workspace(n, key.size(1), c, h, w, K, s, int(nhwc), _lib.dtype_code(value))
+
+
 def _direct_serves(query, key, value, K, s, nhwc):
-    """Whether the gradients of these operands come from sapa_fused_backward_direct, which forms the
+    """Whether the gradients of these operands come from sapa_fused_backward_direct_ws, which forms the
     attention weights itself (nothing to keep from the forward pass)."""
-    return (value.dtype in (torch.float16, torch.bfloat16) and query.dtype == key.dtype == value.dtype
-            and bool(_lib.lib().sapa_fused_backward_direct_serves(key.size(1), value.size(1), key.size(2), key.size(3),
-                                                                  K, s, int(nhwc), _lib.dtype_code(value))))
+    return _direct_scratch(query, key, value, K, s, nhwc) > 0
 
 
 def _direct_backward(grad_output, query, key, value, K, s, needs):
-    """The gradients through sapa_fused_backward_direct (16-bit tensors in one memory order; the
+    """The gradients through sapa_fused_backward_direct_ws (16-bit tensors in one memory order; the
     output's gradient is brought into it); None where that entry point does not serve the call."""
     nhwc = all(_lib.is_channels_last(t) for t in (query, key, value))
     if not (nhwc or all(t.is_contiguous() for t in (query, key, value))):
         return None
-    if grad_output.dtype != value.dtype or not _direct_serves(query, key, value, K, s, nhwc):
+    nbytes = _direct_scratch(query, key, value, K, s, nhwc)
+    if grad_output.dtype != value.dtype or nbytes == 0:
         return None
     grad_output = _lib.layout_copy(grad_output, nhwc)
     n, c, h, w = value.size()
-    stats = torch.empty((3, n, h * s, w * s), dtype=torch.float32, device=value.device)
+    scratch = torch.empty(nbytes, dtype=torch.uint8, device=value.device)
     grads = [_lib.new_out(t, channels_last=nhwc) if need else None for t, need in zip((query, key, value), needs)]
-    status = _lib.call_status('sapa_fused_backward_direct', value.device, _lib.ptr(grad_output), _lib.ptr(query),
-                              _lib.ptr(key), _lib.ptr(value), _lib.ptr(stats), _lib.ptr(grads[0]),
+    status = _lib.call_status('sapa_fused_backward_direct_ws', value.device, _lib.ptr(grad_output), _lib.ptr(query),
+                              _lib.ptr(key), _lib.ptr(value), _lib.ptr(scratch), _lib.ptr(grads[0]),
                               _lib.ptr(grads[1]), _lib.ptr(grads[2]), n, key.size(1), c, h, w, K, s, int(nhwc),
                               _lib.dtype_code(value))
     return None if status == _lib.UNSUPPORTED else tuple(grads)
@@ -235,7 +242,7 @@ def _direct_backward(grad_output, query, key, value, K, s, needs):
 
 def _fused_backward(grad_output, query, key, value, K, s, needs=(True, True, True), attn=None, direct=True):
     """Gradients of av(softmax(qk(query, key)), value): straight from the operands where
-    sapa_fused_backward_direct serves them (and `direct`); else the attention weights
+    sapa_fused_backward_direct_ws serves them (and `direct`); else the attention weights
     are recomputed (one launch) unless the forward pass kept them (`attn`, fp32),
     then the three operators' gradients chain."""
     need_q, need_k, need_v = needs
@@ -322,7 +329,7 @@ def _fused_backward(grad_output, query, key, value, K, s, needs=(True, True, Tru
 
 
 # Training steps of sapa_fused whose gradients chain over the attention weights (fp32; 16-bit
-# tensors that sapa_fused_backward_direct does not serve) keep them between the forward and the
+# tensors that sapa_fused_backward_direct_ws does not serve) keep them between the forward and the
 # backward pass (faster: one launch less per step) unless this is False or the call
 # says save_attention=False (less memory: the weights are recomputed).
 SAVE_ATTENTION = True
@@ -331,7 +338,7 @@ SAVE_ATTENTION = True
 class SAPAFusedFunction(Function):
     """av(softmax(qk(query, key), dim=1), value) -- SAPA.attention
     (sapa_base.py:38-40) -- as one launch in the forward pass.  The gradients of
-    16-bit operands that sapa_fused_backward_direct serves come straight from them
+    16-bit operands that sapa_fused_backward_direct_ws serves come straight from them
     (nothing kept, no K*K tensor at any time), unless the call says where its
     attention weights are to come from: with save_attention=True the
     forward pass runs as two launches that leave the fp32 weights

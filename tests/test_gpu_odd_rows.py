@@ -1,0 +1,50 @@
+"""The two-kernel backward of contiguous 16-bit SAPA-B tensors whose rows have an odd number of cells."""
+import pytest
+import torch
+
+import sapa_amd
+from sapa_amd import _lib
+from sapa_amd.sapa_func import _direct_serves
+
+pytestmark = pytest.mark.gpu
+
+
+def _operands(dtype, B, d, C, H, W):
+    g = torch.Generator(device='cuda').manual_seed(H * W)
+    shapes = ((B, d, 2 * H, 2 * W), (B, d, H, W), (B, C, H, W), (B, C, 2 * H, 2 * W))
+    return [torch.randn(s, generator=g, device='cuda').mul(0.6).to(dtype) for s in shapes]
+
+
+@pytest.mark.parametrize('dtype', [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize('B,d,C,H,W', [
+    (1, 16, 16, 4, 17),      # the smallest width served; rows end two children into a piece
+    (2, 24, 40, 5, 19),      # ... six into one; ragged channel chunks, images of an odd number of cells
+    (2, 17, 33, 3, 33),      # an odd number of channels too: the last dword of a tensor is half its own
+    (1, 32, 64, 33, 31),     # one tile of cell blocks, its last one past the image
+    (1, 40, 24, 3, 67),      # several tiles, fewer rows than a block
+])
+def test_gradients_of_odd_rows(dtype, B, d, C, H, W):
+    """All gradients and one at a time against the fp64 operators.  Bar: one rounding of the result to its
+    type leaves a relative error of eps / 2 / sqrt(3) at most; weight pairs and fp32 sums are far below."""
+    *ops, go = _operands(dtype, B, d, C, H, W)
+    assert _direct_serves(*ops, 5, 2, False)
+    wide = [t.double().requires_grad_() for t in ops]
+    want = torch.autograd.grad(sapa_amd.sapa_fused(*wide, 5, 2), wide, go.double())
+    bar = torch.finfo(dtype).eps / 2 / 3 ** 0.5 * 1.2
+    for needs in ((True, True, True), (True, False, False), (False, True, False), (False, False, True)):
+        leaves = [t.clone().requires_grad_(n) for t, n in zip(ops, needs)]
+        got = torch.autograd.grad(sapa_amd.sapa_fused(*leaves, 5, 2), [t for t in leaves if t.requires_grad], go)
+        for a, b in zip(got, [w for w, n in zip(want, needs) if n]):
+            rel = ((a.double() - b).norm() / b.norm()).item()
+            assert rel <= bar and a.is_contiguous(), (needs, a.shape, rel)
+
+
+def test_scratch_of_three_floats_per_pixel_does_not_serve_odd_rows():
+    """The entry point whose scratch holds no padded copies refuses them and writes nothing."""
+    q, key, v, go = _operands(torch.bfloat16, 1, 16, 16, 4, 17)
+    scratch = torch.empty(3 * 8 * 34, dtype=torch.float32, device='cuda')
+    grads = [torch.full_like(t, 7.0) for t in (q, key, v)]
+    args = [_lib.ptr(t) for t in (go, q, key, v, scratch, *grads)]
+    status = _lib.call_status('sapa_fused_backward_direct', q.device, *args, 1, 16, 16, 4, 17, 5, 2, 0,
+                              _lib.dtype_code(q))
+    assert status == _lib.UNSUPPORTED and all(bool((t == 7.0).all()) for t in grads)
