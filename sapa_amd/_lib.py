@@ -43,6 +43,7 @@ SIGNATURES = {
     'sapa_fused_backward': [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _i, _i, _i, _i, _i, _i, _i, _i, _vp],
     'sapa_fused_backward_direct_serves': [_i] * 8,
     'sapa_fused_backward_direct': [_vp] * 8 + [_i] * 9 + [_vp],
+    'sapa_fused_backward_direct_workspace': [_i] * 9,       # (a size)
     'sapa_fused_backward_direct_ws': [_vp] * 8 + [_i] * 9 + [_vp],
     'sapa_fused_forward_attn': [_vp, _vp, _vp, _vp, _vp, _i, _i, _i, _i, _i, _i, _i, _i, _vp],
     'sapa_fused_backward_attn': [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _i, _i, _i, _i, _i, _i, _i, _i, _vp],
@@ -113,7 +114,6 @@ def lib():
         handle.sapa_fused_backward_attn_workspace.restype = _ll
         handle.sapa_fused_backward_attn_workspace.argtypes = [_i, _i, _i, _i, _i]
         handle.sapa_fused_backward_direct_workspace.restype = _ll
-        handle.sapa_fused_backward_direct_workspace.argtypes = [_i] * 9
         handle.sapa_deform_fused_forward_workspace.restype = _ll
         handle.sapa_deform_fused_forward_workspace.argtypes = [_i] * 9
         handle.sapa_deform_fused_backward_workspace.restype = _ll

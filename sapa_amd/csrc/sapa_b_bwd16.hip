@@ -112,7 +112,8 @@ __device__ __attribute__((noinline)) void children_again(Again again) {
 // the upper / lower 32 of its children each (with all 64 a wave would hold 128 accumulators and
 // weights, and half as many waves would be resident).  Chunks of 16 channels: key + q (S), value +
 // grad_out (G), key again (grad_q), in a ring of three buffers, the next two in flight.
-template <typename T, int NSW, bool STREAM>
+// ODD: an odd W
+template <typename T, int NSW, bool STREAM, bool ODD>
 __global__ __launch_bounds__(128 * NSW) void
 bwd_pixel_kernel(const Args<T> args) {
     const T *__restrict__ const q = args.q, *__restrict__ const key = args.key_rows, *__restrict__ const value = args.value_rows,
@@ -149,7 +150,7 @@ bwd_pixel_kernel(const Args<T> args) {
     const int t = wave % NSW, half = wave / NSW;              // block of the tile, half of its children
     const int g = lane >> 4, i16 = lane & 15;
     const long lpix = (long)H * W;
-    const int low_w = args.low_w;
+    const int low_w = ODD ? args.low_w : W;
     const long lowpix = (long)H * low_w;
     const u32 lplane = (u32)(lowpix * sizeof(T)), hplane = (u32)(4 * lpix * sizeof(T));
 
@@ -417,9 +418,13 @@ bwd_pixel_kernel(const Args<T> args) {
         const u32x4 o = *(const u32x4 *)(ob + tid * 4);
         u32 off = off_hi + c0 * hplane;
         if (row_tail && short_piece) {
+            if (ODD) {
 #pragma unroll
-            for (int k = 0; k < 3; ++k)
-                if (k < short_piece) __builtin_amdgcn_raw_buffer_store_b32(o[k], ro, off + 4 * k, 0, 0);
+                for (int k = 0; k < 3; ++k)
+                    if (k < short_piece) __builtin_amdgcn_raw_buffer_store_b32(o[k], ro, off + 4 * k, 0, 0);
+            } else {
+                __builtin_amdgcn_raw_buffer_store_b64(u32x2{o[0], o[1]}, ro, off, 0, 0);
+            }
             off = OUTSIDE;
         }
         __builtin_amdgcn_raw_buffer_store_b128(o, ro, off, 0, STREAM ? 2 : 0);
@@ -677,7 +682,10 @@ bwd_cell_kernel(const Args<T> args) {
         int after = wave < CNL ? outs * (ODD ? ragged ? 11 : 3 : ragged ? 4 : 1) : 0;
 #pragma unroll
         for (int i = 2; i < CBUF; ++i) after += loads_of(j + i);
-        wait_all_but(after);
+        // (odd rows store more often than wait_all_but counts, whose every further case costs all its callers:
+        // 1 us of 165; to wait for more than is needed is safe)
+        if (ODD && after > 11) asm volatile("s_waitcnt vmcnt(11)" ::: "memory");
+        else wait_all_but(after);
         if (patch && (j + 1 == 0 || j + 1 == nKc)) {
             const u32 *src = (const u32 *)(j + 1 == 0 ? key + (long)n * d * lowpix : value + (long)n * C * lowpix);
             u32 *dst = lowbuf + (j + 1) % CBUF * CLOW + lslot * 4;
@@ -835,7 +843,8 @@ static hipError_t launch(const void *q, const void *key, const void *value, cons
         const int nsx = (W + 3) / 4;
         if (!tile((nsx + NSW - 1) / NSW, (H + 3) / 4)) return hipErrorNotSupported;
         args.ns = (nsx + args.tiles_x - 1) / args.tiles_x;    // blocks per tile, balanced over the row
-        hipLaunchKernelGGL((bwd_pixel_kernel<T, NSW, STREAM>), dim3(args.per_xcd * 8), dim3(128 * NSW), 0, st, args);
+        if (odd) hipLaunchKernelGGL((bwd_pixel_kernel<T, NSW, false, true>), dim3(args.per_xcd * 8), dim3(128 * NSW), 0, st, args);
+        else hipLaunchKernelGGL((bwd_pixel_kernel<T, NSW, STREAM, false>), dim3(args.per_xcd * 8), dim3(128 * NSW), 0, st, args);
         const hipError_t e = hipGetLastError();
         if (e != hipSuccess) return e;
     }

@@ -130,8 +130,7 @@ __device__ __forceinline__ void wait_all_but(int after) {
 #define SAPA_WAIT_CASE(N) case N: asm volatile("s_waitcnt vmcnt(" #N ")" ::: "memory"); break;
     switch (after) {
         SAPA_WAIT_CASE(1) SAPA_WAIT_CASE(2) SAPA_WAIT_CASE(3) SAPA_WAIT_CASE(4) SAPA_WAIT_CASE(5) SAPA_WAIT_CASE(6)
-        SAPA_WAIT_CASE(7) SAPA_WAIT_CASE(8) SAPA_WAIT_CASE(9) SAPA_WAIT_CASE(10) SAPA_WAIT_CASE(11) SAPA_WAIT_CASE(13)
-        SAPA_WAIT_CASE(14) SAPA_WAIT_CASE(24) SAPA_WAIT_CASE(25)
+        SAPA_WAIT_CASE(7) SAPA_WAIT_CASE(8) SAPA_WAIT_CASE(9) SAPA_WAIT_CASE(10) SAPA_WAIT_CASE(11)
         default: asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); break;
     }
 #undef SAPA_WAIT_CASE
