@@ -440,8 +440,9 @@ __device__ __forceinline__ f32x4 mma32(u32x4 a, u32x4 b, f32x4 c) {
     return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(v8, a), __builtin_bit_cast(v8, b), c, 0, 0, 0);
 }
 
-// C input channels (a multiple of 32), O outputs (a multiple of 16); 8 waves, tiles of 32
-// pixels (two blocks of 16 matrix rows share every weight operand read from LDS).
+// C input channels (a multiple of 32), O outputs (a multiple of 16); 12 waves, tiles of 32
+// pixels (two blocks of 16 matrix rows share every weight operand read from LDS), the
+// workgroup's waves on neighbouring tiles.
 // Reduction step ks takes channels 32 ks ..; inside it lane group kg holds channels
 // 4 kg .. + 3 and 16 + 4 kg .. + 3 (two 16-byte pieces of memory; the 16 lanes of a piece
 // read 64 contiguous bytes per pixel) -- the weight planes are stored in that order.
@@ -453,12 +454,17 @@ __device__ __forceinline__ f32x4 mma32(u32x4 a, u32x4 b, f32x4 c) {
 // that the two channel groups of a half-wave read disjoint banks).  OUT_CL = false: out is
 // [B, O, HW]; a block of 16 outputs x 32 pixels goes back through LDS and leaves as 128-byte rows
 // (HW a multiple of 4: a 16-byte piece never runs from one plane into the next).
+// Twelve waves, as many as 168 registers and the LDS allow: what bounds the kernel is the chain of a step (tile
+// through LDS, pieces, matrix products), which three waves per SIMD hide better than two (two steps of
+// x in flight each instead of four); finer tiles per round besides (16 images, 256 -> 64: 100x168
+// pixels 81 -> 77 us, 50x84 35 -> 24, channels-last 86 -> 76 and 28 -> 22; 200x336 311 -> 300).
+constexpr int NW32 = 12;
 template <int C, int O, bool IN_CL, bool OUT_CL, bool WIDE>
-__global__ void __launch_bounds__(512)
+__global__ void __launch_bounds__(64 * NW32)
 project32_kernel(const float *__restrict__ x, const float *__restrict__ w, const float *__restrict__ bias,
                  float *__restrict__ out, long HW, int tiles_per_wave, int waves, int outputs) {
     static_assert(IN_CL ? OUT_CL : true, "channels-last features give channels-last projections");
-    constexpr int NW = 8;
+    constexpr int NW = NW32;
     constexpr int RW = C / 2 + 4;                 // dwords per padded row of C bf16 values
     constexpr int PLANE = O * RW;                 // dwords per piece plane
     constexpr int NT = O / 16;                    // output tiles of 16 columns
@@ -468,7 +474,7 @@ project32_kernel(const float *__restrict__ x, const float *__restrict__ w, const
     constexpr int RT = OUT_CL ? 16 * OS : 16 * PS;
     constexpr int WF = RT > XB ? RT : XB;         // floats of a wave's LDS (x tile, then results)
     constexpr int KS = C / 32;                    // reduction steps
-    constexpr int RING = KS < 4 ? KS : 4;         // steps of x in flight
+    constexpr int RING = KS < 4 || O == 64 ? 2 : 4;        // steps of x in flight
     static_assert(KS % RING == 0, "the ring of x registers is indexed by the step");
     extern __shared__ __attribute__((aligned(16))) u32 sh[];
     u32 *wl = sh;                                 // weights: 3 planes of O rows of RW dwords
@@ -479,8 +485,9 @@ project32_kernel(const float *__restrict__ x, const float *__restrict__ w, const
     const Span sp = span_of<O, WIDE>(outputs);
 
     const long ntiles = (HW + 31) / 32;
-    const long t0 = ((long)blockIdx.x * waves + wave) * tiles_per_wave;       // waves past `waves` help with the weights only
-    const long t1 = wave >= waves ? t0 : t0 + tiles_per_wave < ntiles ? t0 + tiles_per_wave : ntiles;
+    // tiles t0, t0 + waves ..: the waves read neighbouring pieces of a plane (waves past `waves` help with the weights only)
+    const long first = (long)blockIdx.x * waves * tiles_per_wave, last = first + (long)waves * tiles_per_wave;
+    const long t0 = first + wave, t1 = wave >= waves ? t0 : last < ntiles ? last : ntiles;
     const int r16 = lane & 15, kg = lane >> 4;    // row / column of a 16 x 16 tile, k group
     float bv[NT];
 #pragma unroll
@@ -521,8 +528,7 @@ project32_kernel(const float *__restrict__ x, const float *__restrict__ w, const
     {
         const __amdgpu_buffer_rsrc_t rw = __builtin_amdgcn_make_buffer_rsrc(
             (void *)(w + (WIDE ? (long)sp.o0 : (long)b * O) * C), 0, sp.left * C * 4, 0x00020000);
-        constexpr int N = O * C / 4 / (64 * NW);
-        static_assert(O * C / 4 % (64 * NW) == 0, "whole steps");
+        constexpr int PIECES = O * C / 4, N = (PIECES + 64 * NW - 1) / (64 * NW);
         u32x4 v[N];
 #pragma unroll
         for (int k = 0; k < N; ++k)
@@ -530,6 +536,7 @@ project32_kernel(const float *__restrict__ x, const float *__restrict__ w, const
 #pragma unroll
         for (int k = 0; k < N; ++k) {
             const int i = k * 64 * NW + threadIdx.x, o = i / (C / 4), c = 4 * (i % (C / 4)), cs = c % 32;
+            if (PIECES % (64 * NW) != 0 && i >= PIECES) break;
             const int pos = 32 * (c / 32) + 8 * ((cs % 16) / 4) + 4 * (cs / 16);
             const f32x4 f = __builtin_bit_cast(f32x4, v[k]);
             const Pieces p0 = split2(f[0], f[1]), p1 = split2(f[2], f[3]);
@@ -560,7 +567,7 @@ project32_kernel(const float *__restrict__ x, const float *__restrict__ w, const
             out[OUT_CL ? ((long)b * HW + p) * sp.OT + sp.o0 + o : ((long)b * sp.OT + sp.o0 + o) * HW + p] = r;
         }
     };
-    for (long t = t0; t < t1; ++t) {
+    for (long t = t0; t < t1; t += waves) {
         f32x4 acc[2][NT], low[2][NT];
 #pragma unroll
         for (int mb = 0; mb < 2; ++mb)
@@ -595,7 +602,7 @@ project32_kernel(const float *__restrict__ x, const float *__restrict__ w, const
             }
             // the ring slot is free: the step RING further on (of this tile or of the next)
             if (ks + RING < KS) load_step(ks % RING, t, ks + RING);
-            else if (t + 1 < t1) load_step(ks % RING, t + 1, ks + RING - KS);
+            else if (t + waves < t1) load_step(ks % RING, t + waves, ks + RING - KS);
 #pragma unroll
             for (int nt = 0; nt < NT; ++nt) {
                 if (WIDE && 16 * nt >= sp.left) break;
@@ -614,6 +621,8 @@ project32_kernel(const float *__restrict__ x, const float *__restrict__ w, const
                     acc[mb][nt] = mma32(ahi[mb], bhi, acc[mb][nt]);
                 }
             }
+            // (nothing of a later step moves up: it would not fit the registers of 12 waves)
+            __builtin_amdgcn_sched_barrier(0);
         }
         float largest = 0.f;
 #pragma unroll
@@ -673,7 +682,7 @@ template <int C, int O, bool IN_CL, bool OUT_CL, bool WIDE = false>
 static hipError_t launch32_co(const void *x, const void *w, const void *bias, void *out, int B, long HW,
                               hipStream_t st, int outputs = O) {
     constexpr int RT = OUT_CL ? 16 * (O + 4) : 16 * 36, XB = IN_CL ? 0 : 32 * 32;
-    constexpr size_t lds = (size_t)(3 * O * (C / 2 + 4) + 8 * (RT > XB ? RT : XB)) * 4;
+    constexpr size_t lds = (size_t)(3 * O * (C / 2 + 4) + NW32 * (RT > XB ? RT : XB)) * 4;
     if (!OUT_CL && HW % 4 != 0) return hipErrorNotSupported;
     static_assert(lds <= 160 * 1024, "weights and tiles must fit LDS");
     // 32-bit byte offsets inside an image
@@ -682,25 +691,22 @@ static hipError_t launch32_co(const void *x, const void *w, const void *bias, vo
     const int blocks_o = (outputs + O - 1) / O;
     const long sets = (long)B * blocks_o;         // workgroups that share a pixel range's place
     // One workgroup is resident per CU (its weight planes fill most of the LDS) and the part has
-    // 256 CUs: two full rounds of workgroups where that leaves a wave 8 tiles or more, else one
+    // 256 CUs: two full rounds of workgroups where that leaves a wave 6 tiles or more, else one
     // (16 images: 200x336 pixels 301 us in two rounds against 315 in one; 100x168 pixels 71 us in
     // one round against 98 in 272 workgroups)
     const long slots = 256;
     long blocks = 2 * slots / sets > 1 ? 2 * slots / sets : 1;
-    long per = (ntiles + 8 * blocks - 1) / (8 * blocks);
-    if (per < 8) {
+    long per = (ntiles + NW32 * blocks - 1) / (NW32 * blocks);
+    if (per < 6) {
         blocks = slots / sets > 1 ? slots / sets : 1;
-        per = (ntiles + 8 * blocks - 1) / (8 * blocks);
+        per = (ntiles + NW32 * blocks - 1) / (NW32 * blocks);
     }
-    // fewer tiles than the chip has room for: a tile per wave and as few waves per workgroup as fill it
-    // (its matrix instructions are then not queued behind a second wave's; 4 images of 33x20 pixels,
-    // 256 -> 128 / 288: SAPA-D module 113 -> 104 us)
-    int waves = 8;
-    if (per == 1) {
-        const long room = slots / sets > 1 ? slots / sets : 1;
-        waves = (int)((ntiles + room - 1) / room);
-        waves = waves < 1 ? 1 : waves > 8 ? 8 : waves;
-    }
+    // ... and as few waves per workgroup as cover the image in that many tiles each, so that no workgroup of the
+    // round is missing (8 images of 128x128 pixels, 256 -> 128: 240 workgroups of 12 waves else 256 of 11;
+    // fewer tiles than the chip has room for: a wave's matrix instructions are not queued behind a second
+    // wave's; 4 images of 33x20 pixels, 256 -> 128 / 288: SAPA-D module 113 -> 104 us)
+    int waves = (int)((ntiles + blocks * per - 1) / (blocks * per));
+    waves = waves < 1 ? 1 : waves > NW32 ? NW32 : waves;
     blocks = (ntiles + waves * per - 1) / (waves * per);
     if (blocks > 65535 * 32L || B > 65535 || blocks_o > 65535) return hipErrorNotSupported;
     auto kern = project32_kernel<C, O, IN_CL, OUT_CL, WIDE>;
@@ -715,7 +721,7 @@ static hipError_t launch32_co(const void *x, const void *w, const void *bias, vo
             return hipErrorNotSupported;
         }
     }
-    hipLaunchKernelGGL(kern, dim3((unsigned)blocks, B, blocks_o), dim3(512), lds, st, (const float *)x, (const float *)w,
+    hipLaunchKernelGGL(kern, dim3((unsigned)blocks, B, blocks_o), dim3(64 * NW32), lds, st, (const float *)x, (const float *)w,
                        (const float *)bias, (float *)out, HW, (int)per, waves, outputs);
     return hipGetLastError();
 }
