@@ -431,15 +431,19 @@ static hipError_t lowgrad_shift_launch(const void *hi, const void *w, void *out,
     constexpr int R = (K - 1) / 2, VX = RW - 2 * R, VY = 64 / RW * NW - 2 * R;
     const int tiles_x = (W + VX - 1) / VX, tiles_y = (H + VY - 1) / VY;
     const long tiles = (long)tiles_x * tiles_y * B;
-    // the channels of a tile over several workgroups until the grid fills the chip a
-    // few times over (each re-reads the tile's weights)
-#ifndef SAPA_LOWGRAD_SHIFT_MINWG
-#define SAPA_LOWGRAD_SHIFT_MINWG 2048
-#endif
-    int cgroups = 1;
-    const int max_groups = C / (4 * CH) > 0 ? C / (4 * CH) : 1;
-    while (cgroups * 2 <= max_groups && tiles * cgroups < SAPA_LOWGRAD_SHIFT_MINWG) cgroups *= 2;
-    const int cper = ((C + cgroups - 1) / cgroups + CH - 1) / CH * CH;
+    // Channels per workgroup, so that the rounds of workgroups (two are resident on each of 256 CUs) times what one
+    // costs are the fewest: its channels, and the tile's weights, which every workgroup of the tile reads
+    // again (as long as 6 channels take).  16 images, 256 channels, 50x84: 16 / 32 / 64 / 128 channels
+    // 164 / 153 / 148 / 145 us, the estimate 170 / 147 / 136 / 134; 64 channels, 8 / 16 / 32: 51 / 42 / 39
+    // and 54 / 43 / 38.
+    int cper = C < 8 ? (C + CH - 1) / CH * CH : 8;
+    double least = 0;
+    for (int c = cper; c < C + 4; c += 4) {
+        const double load = (double)tiles * ((C + c - 1) / c) / 512;
+        const double time = (load <= 1 ? 1 : 0.5 * (load + __builtin_ceil(load))) * (c + 6);
+        if (least == 0 || time < least) least = time, cper = c;
+    }
+    const int cgroups = (C + cper - 1) / cper;
     const long nb = tiles * cgroups;
     if (nb > (1L << 30)) return hipErrorNotSupported;
     const int per_xcd = (int)((nb + 7) / 8);
