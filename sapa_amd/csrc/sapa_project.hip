@@ -440,7 +440,7 @@ __device__ __forceinline__ f32x4 mma32(u32x4 a, u32x4 b, f32x4 c) {
     return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(v8, a), __builtin_bit_cast(v8, b), c, 0, 0, 0);
 }
 
-// C input channels (a multiple of 32), O outputs (a multiple of 16); 12 waves, tiles of 32
+// C input channels (a multiple of 32), O outputs (a multiple of 16); NW = 8 or 12 waves, tiles of 32
 // pixels (two blocks of 16 matrix rows share every weight operand read from LDS), the
 // workgroup's waves on neighbouring tiles.
 // Reduction step ks takes channels 32 ks ..; inside it lane group kg holds channels
@@ -454,17 +454,15 @@ __device__ __forceinline__ f32x4 mma32(u32x4 a, u32x4 b, f32x4 c) {
 // that the two channel groups of a half-wave read disjoint banks).  OUT_CL = false: out is
 // [B, O, HW]; a block of 16 outputs x 32 pixels goes back through LDS and leaves as 128-byte rows
 // (HW a multiple of 4: a 16-byte piece never runs from one plane into the next).
-// Twelve waves, as many as 168 registers and the LDS allow: what bounds the kernel is the chain of a step (tile
+// Twelve waves (of which launch32_co says where), as many as 168 registers and the LDS allow: what bounds the kernel is the chain of a step (tile
 // through LDS, pieces, matrix products), which three waves per SIMD hide better than two (two steps of
 // x in flight each instead of four); finer tiles per round besides (16 images, 256 -> 64: 100x168
 // pixels 81 -> 77 us, 50x84 35 -> 24, channels-last 86 -> 76 and 28 -> 22; 200x336 311 -> 300).
-constexpr int NW32 = 12;
-template <int C, int O, bool IN_CL, bool OUT_CL, bool WIDE>
-__global__ void __launch_bounds__(64 * NW32)
+template <int C, int O, bool IN_CL, bool OUT_CL, bool WIDE, int NW>
+__global__ void __launch_bounds__(64 * NW)
 project32_kernel(const float *__restrict__ x, const float *__restrict__ w, const float *__restrict__ bias,
                  float *__restrict__ out, long HW, int tiles_per_wave, int waves, int outputs) {
     static_assert(IN_CL ? OUT_CL : true, "channels-last features give channels-last projections");
-    constexpr int NW = NW32;
     constexpr int RW = C / 2 + 4;                 // dwords per padded row of C bf16 values
     constexpr int PLANE = O * RW;                 // dwords per piece plane
     constexpr int NT = O / 16;                    // output tiles of 16 columns
@@ -474,7 +472,7 @@ project32_kernel(const float *__restrict__ x, const float *__restrict__ w, const
     constexpr int RT = OUT_CL ? 16 * OS : 16 * PS;
     constexpr int WF = RT > XB ? RT : XB;         // floats of a wave's LDS (x tile, then results)
     constexpr int KS = C / 32;                    // reduction steps
-    constexpr int RING = KS < 4 || O == 64 ? 2 : 4;        // steps of x in flight
+    constexpr int RING = KS < 4 || (O == 64 && NW > 8) ? 2 : 4;        // steps of x in flight
     static_assert(KS % RING == 0, "the ring of x registers is indexed by the step");
     extern __shared__ __attribute__((aligned(16))) u32 sh[];
     u32 *wl = sh;                                 // weights: 3 planes of O rows of RW dwords
@@ -622,7 +620,7 @@ project32_kernel(const float *__restrict__ x, const float *__restrict__ w, const
                 }
             }
             // (nothing of a later step moves up: it would not fit the registers of 12 waves)
-            __builtin_amdgcn_sched_barrier(0);
+            if (NW > 8) __builtin_amdgcn_sched_barrier(0);
         }
         float largest = 0.f;
 #pragma unroll
@@ -678,38 +676,41 @@ project32_kernel(const float *__restrict__ x, const float *__restrict__ w, const
     }
 }
 
-template <int C, int O, bool IN_CL, bool OUT_CL, bool WIDE = false>
-static hipError_t launch32_co(const void *x, const void *w, const void *bias, void *out, int B, long HW,
-                              hipStream_t st, int outputs = O) {
-    constexpr int RT = OUT_CL ? 16 * (O + 4) : 16 * 36, XB = IN_CL ? 0 : 32 * 32;
-    constexpr size_t lds = (size_t)(3 * O * (C / 2 + 4) + NW32 * (RT > XB ? RT : XB)) * 4;
-    if (!OUT_CL && HW % 4 != 0) return hipErrorNotSupported;
-    static_assert(lds <= 160 * 1024, "weights and tiles must fit LDS");
-    // 32-bit byte offsets inside an image
-    if (HW * (long)(C > outputs ? C : outputs) * 4 >= (1L << 31)) return hipErrorNotSupported;
-    const long ntiles = (HW + 31) / 32;
-    const int blocks_o = (outputs + O - 1) / O;
-    const long sets = (long)B * blocks_o;         // workgroups that share a pixel range's place
-    // One workgroup is resident per CU (its weight planes fill most of the LDS) and the part has
-    // 256 CUs: two full rounds of workgroups where that leaves a wave 6 tiles or more, else one
-    // (16 images: 200x336 pixels 301 us in two rounds against 315 in one; 100x168 pixels 71 us in
-    // one round against 98 in 272 workgroups)
+// How a projection's tiles are spread: tiles per wave, waves per workgroup that have some, workgroups per image
+struct Spread {
+    long per, blocks;
+    int waves;
+};
+// One workgroup is resident per CU (its weight planes fill most of the LDS) and the part has
+// 256 CUs: two full rounds of workgroups where that leaves a wave 6 tiles or more, else one
+// (16 images: 200x336 pixels 301 us in two rounds against 315 in one; 100x168 pixels 71 us in
+// one round against 98 in 272 workgroups)
+static Spread spread32(long ntiles, long sets, int nw) {
     const long slots = 256;
     long blocks = 2 * slots / sets > 1 ? 2 * slots / sets : 1;
-    long per = (ntiles + NW32 * blocks - 1) / (NW32 * blocks);
+    long per = (ntiles + nw * blocks - 1) / (nw * blocks);
     if (per < 6) {
         blocks = slots / sets > 1 ? slots / sets : 1;
-        per = (ntiles + NW32 * blocks - 1) / (NW32 * blocks);
+        per = (ntiles + nw * blocks - 1) / (nw * blocks);
     }
     // ... and as few waves per workgroup as cover the image in that many tiles each, so that no workgroup of the
     // round is missing (8 images of 128x128 pixels, 256 -> 128: 240 workgroups of 12 waves else 256 of 11;
     // fewer tiles than the chip has room for: a wave's matrix instructions are not queued behind a second
     // wave's; 4 images of 33x20 pixels, 256 -> 128 / 288: SAPA-D module 113 -> 104 us)
     int waves = (int)((ntiles + blocks * per - 1) / (blocks * per));
-    waves = waves < 1 ? 1 : waves > NW32 ? NW32 : waves;
-    blocks = (ntiles + waves * per - 1) / (waves * per);
-    if (blocks > 65535 * 32L || B > 65535 || blocks_o > 65535) return hipErrorNotSupported;
-    auto kern = project32_kernel<C, O, IN_CL, OUT_CL, WIDE>;
+    waves = waves < 1 ? 1 : waves > nw ? nw : waves;
+    return Spread{per, (ntiles + waves * per - 1) / (waves * per), waves};
+}
+
+template <int C, int O, bool IN_CL, bool OUT_CL, bool WIDE, int NW>
+static hipError_t launch32_waves(const void *x, const void *w, const void *bias, void *out, int B, long HW,
+                                 hipStream_t st, int outputs, const Spread &s) {
+    constexpr int RT = OUT_CL ? 16 * (O + 4) : 16 * 36, XB = IN_CL ? 0 : 32 * 32;
+    constexpr size_t lds = (size_t)(3 * O * (C / 2 + 4) + NW * (RT > XB ? RT : XB)) * 4;
+    static_assert(lds <= 160 * 1024, "weights and tiles must fit LDS");
+    const int blocks_o = (outputs + O - 1) / O;
+    if (s.blocks > 65535 * 32L || B > 65535 || blocks_o > 65535) return hipErrorNotSupported;
+    auto kern = project32_kernel<C, O, IN_CL, OUT_CL, WIDE, NW>;
     if (lds > 64 * 1024) {
         int dev = 0, most = 0;
         if (hipGetDevice(&dev) != hipSuccess ||
@@ -721,9 +722,30 @@ static hipError_t launch32_co(const void *x, const void *w, const void *bias, vo
             return hipErrorNotSupported;
         }
     }
-    hipLaunchKernelGGL(kern, dim3((unsigned)blocks, B, blocks_o), dim3(64 * NW32), lds, st, (const float *)x, (const float *)w,
-                       (const float *)bias, (float *)out, HW, (int)per, waves, outputs);
+    hipLaunchKernelGGL(kern, dim3((unsigned)s.blocks, B, blocks_o), dim3(64 * NW), lds, st, (const float *)x, (const float *)w,
+                       (const float *)bias, (float *)out, HW, (int)s.per, s.waves, outputs);
     return hipGetLastError();
+}
+
+template <int C, int O, bool IN_CL, bool OUT_CL, bool WIDE = false>
+static hipError_t launch32_co(const void *x, const void *w, const void *bias, void *out, int B, long HW,
+                              hipStream_t st, int outputs = O) {
+    if (!OUT_CL && HW % 4 != 0) return hipErrorNotSupported;
+    // 32-bit byte offsets inside an image
+    if (HW * (long)(C > outputs ? C : outputs) * 4 >= (1L << 31)) return hipErrorNotSupported;
+    const long ntiles = (HW + 31) / 32, sets = (long)B * ((outputs + O - 1) / O);     // sets: workgroups that share a pixel range's place
+    const Spread s8 = spread32(ntiles, sets, 8), s12 = spread32(ntiles, sets, 12);
+    // Eight waves, with twice the steps of x in flight and no bar to moving work between steps, are faster over the
+    // same number of tiles each (us with 12 / 8 waves: 256 -> 32, 2 images 128x128 pixels 13.6 / 11.9, 8 images
+    // 27.5 / 26.0; 64 -> 32, 4 images 5.4 / 4.8), and throughout at 128 -> 32 (2 images 128x128 11.2 / 6.1, 16 of
+    // 50x84 14.0 / 12.0, of 100x168 30.1 / 29.2).  64 outputs (or 64 at a time): over one tile each (256 -> 128, 8
+    // images 64x64 18.5 / 17.0, 4 of 32x32 10.9 / 10.3; 256 -> 288, 8 of 64x64, 4 tiles, 38.6 / 40.3), from
+    // channels-last features where 7 or 8 of them have one (256 -> 64, 4 images 128x128 19.5 / 17.7; 2 images
+    // 12.1 / 13.3).
+    constexpr bool ALWAYS8 = C == 128 && O == 32;
+    if (ALWAYS8 || (O == 64 ? s8.per == 1 && (!IN_CL || s8.waves > 6) : s8.per <= s12.per))
+        return launch32_waves<C, O, IN_CL, OUT_CL, WIDE, 8>(x, w, bias, out, B, HW, st, outputs, s8);
+    return launch32_waves<C, O, IN_CL, OUT_CL, WIDE, ALWAYS8 ? 8 : 12>(x, w, bias, out, B, HW, st, outputs, s12);
 }
 
 template <bool IN_CL, bool OUT_CL>

@@ -24,3 +24,11 @@ def test_every_tile_of_every_wave(B, C, O, H, W):
         bar = (w[b].double().abs() @ x[b].double().abs().view(C, H * W)) * 2.0 ** -21
         assert bool(((planes[b].double().view(O, H * W) - want).abs() <= bar).all()), b
         assert torch.equal(records[b].reshape(O, H * W), planes[b].view(O, H * W)), b
+
+
+# (8 and 12 waves per workgroup on both sides of where one takes over: tiles for exactly 8 waves of 256 workgroups
+# and a few more, 256 -> 64 with 6 and 7 waves at work, two tiles for each of 8 waves; ragged last tiles)
+@pytest.mark.parametrize('B,C,O,H,W', [(2, 256, 32, 256, 128), (2, 256, 32, 256, 130), (2, 64, 32, 300, 170), (3, 128, 32, 50, 86),
+                                       (1, 256, 64, 224, 220), (1, 256, 64, 224, 212), (4, 512, 32, 256, 128), (1, 512, 32, 3, 4)])
+def test_both_numbers_of_waves(B, C, O, H, W):
+    test_every_tile_of_every_wave(B, C, O, H, W)
