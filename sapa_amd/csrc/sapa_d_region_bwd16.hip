@@ -46,7 +46,8 @@ namespace sapa {
 namespace dreg {
 
 constexpr int NTB = 1024;                   // threads: 16 waves
-// Window cells in LDS, by their number in the strip's window modulo RING.  A step's blocks reach up to two
+// Window cells in LDS, by their number in the column's whole window (parent row 0's first) modulo RING: the blocks of 16
+// cells that a pixel's sums are formed over are the same however the rows are split into segments.  A step's blocks reach up to two
 // rows beyond its band; while its products are formed the row behind those comes in: nothing is read
 // while it is written, and whether a row holds values that are not finite is known before a block reaches it.
 constexpr int RING = 256, AHEAD = BROWS + 2;
@@ -111,6 +112,7 @@ deform_bwd_region16_kernel(const BwdArgs<T> A) {
     const int hW = W * S, d = Cq / A.G, cg = C / A.G;
     const int p0 = seg * A.rows;                        // first row of parents
     const int nstep = H - p0 < A.rows ? H - p0 : A.rows;
+    const int c00 = p0 * WWX;                           // number of the segment's first window cell
     const int x0 = rx * RW, wy0 = p0 - RCH, wx0 = rx * RPX - RCH;
     const long hpl = (long)H * W * (S * S);
     const bool two_k = cg > 32;                                         // G' in two contraction steps
@@ -172,7 +174,7 @@ deform_bwd_region16_kernel(const BwdArgs<T> A) {
         return u32x4{a[0] | b[0], a[1] | b[1], a[2] | b[2], a[3] | b[3]};
     };
     auto put_piece = [&](int row, u32x4 v) __attribute__((always_inline)) {
-        const int at = (row * WWX + pwl) % RING;
+        const int at = (int)((u32)((p0 + row) * WWX + pwl) % RING);
         if (pu < 4) {
             *(u32x4 *)(Kl + at * KSB + pc8) = v;
             if (not_finite<T>(v)) kbad = 1;
@@ -218,8 +220,10 @@ deform_bwd_region16_kernel(const BwdArgs<T> A) {
         kbad = 0;
         fb_flag = 0;
     }
-    for (int i = AHEAD * WWX * KSB / 8 + t; i < RING * KSB / 8; i += NTB) ((u32x4 *)Kl)[i] = u32x4{0u, 0u, 0u, 0u};
-    for (int i = AHEAD * WWX * VSB / 8 + t; i < RING * VSB / 8; i += NTB) ((u32x4 *)Vl)[i] = u32x4{0u, 0u, 0u, 0u};
+    for (int i = AHEAD * WWX * (KSB / 8) + t; i < RING * (KSB / 8); i += NTB)
+        ((u32x4 *)Kl)[(c00 + i / (KSB / 8)) % RING * (KSB / 8) + i % (KSB / 8)] = u32x4{0u, 0u, 0u, 0u};
+    for (int i = AHEAD * WWX * (VSB / 8) + t; i < RING * (VSB / 8); i += NTB)
+        ((u32x4 *)Vl)[(c00 + i / (VSB / 8)) % RING * (VSB / 8) + i % (VSB / 8)] = u32x4{0u, 0u, 0u, 0u};
     {
         const __amdgpu_buffer_rsrc_t kr = rsrc(A.key + (long)n * H * W * Cq, (long)H * W * Cq * 2);
         const __amdgpu_buffer_rsrc_t vr = rsrc(A.value + (long)n * H * W * C, (long)H * W * C * 2);
@@ -246,12 +250,12 @@ deform_bwd_region16_kernel(const BwdArgs<T> A) {
         for (int i = 0; i < NK; ++i) {
             const int u = i * NTB + t;
             bad |= not_finite<T>(kw[i]);
-            if (u < NPC * 4) *(u32x4 *)(Kl + (u >> 2) * KSB + 8 * (u & 3)) = kw[i];
+            if (u < NPC * 4) *(u32x4 *)(Kl + (c00 + (u >> 2)) % RING * KSB + 8 * (u & 3)) = kw[i];
         }
 #pragma unroll
         for (int i = 0; i < NV; ++i) {
             const int u = i * NTB + t;
-            if (u < NPC * 8) *(u32x4 *)(Vl + (u >> 3) * VSB + 8 * (u & 7)) = vw[i];
+            if (u < NPC * 8) *(u32x4 *)(Vl + (c00 + (u >> 3)) % RING * VSB + 8 * (u & 7)) = vw[i];
         }
         if (bad) kbad = 1;
         if (hires) put(0);
@@ -274,7 +278,7 @@ deform_bwd_region16_kernel(const BwdArgs<T> A) {
     const int px_x = x0 + 4 * (pos >> 3) + (pos & 3);
     // the sums of this wave's cell block, which is `mine` until the band has passed it, then mine + 16
     f32x4 Dv[NVB], Dk[NKB];
-    int mine = wave;
+    int mine = band_base(p0) / 16 + ((wave - band_base(p0) / 16) & 15);
     auto clear = [&]() __attribute__((always_inline)) {
 #pragma unroll
         for (int nb = 0; nb < NVB; ++nb) Dv[nb] = f32x4{0.f, 0.f, 0.f, 0.f};
@@ -297,8 +301,8 @@ deform_bwd_region16_kernel(const BwdArgs<T> A) {
         const int ch = lane_o & 15;
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
-            const int cell = 16 * mine + 4 * (lane_o >> 4) + r;       // of the strip's window
-            const int gy = wy0 + cell / WWX, gx = wx0 + cell % WWX, pix = gy * W + gx;
+            const int cell = 16 * mine + 4 * (lane_o >> 4) + r;       // of the column's window
+            const int gy = cell / WWX - RCH, gx = wx0 + cell % WWX, pix = gy * W + gx;
             if (gy < 0 || gy >= H || gx < 0 || gx >= W) continue;
             if (want_v) {
 #pragma unroll
@@ -320,7 +324,7 @@ deform_bwd_region16_kernel(const BwdArgs<T> A) {
     for (int step = 0; step < nstep; ++step) {
         const int buf = step & 1;
         fetch(step + 1);
-        const int base = band_base(step), cb0 = base / 16;
+        const int base = band_base(p0 + step), cb0 = base / 16;
         const bool exact_q = kbad != 0;
 
         // ---- A: wave = (16 positions, blocks of cells)
@@ -341,7 +345,7 @@ deform_bwd_region16_kernel(const BwdArgs<T> A) {
             for (int i = 0; i < 2; ++i) {
                 const int cb = (wave >> 1) + 8 * i;
                 if (cb >= NBLK) break;
-                const int row = (base + 16 * cb) % RING + mi;
+                const int row = (int)((u32)(base + 16 * cb) % RING) + mi;
                 const T *kp = Kl + row * KSB + 8 * mk, *vp = Vl + row * VSB + 8 * mk;
                 const f32x4 sim = Mma<T>::k32(aq.u, *(const u32x4 *)kp, f32x4{0.f, 0.f, 0.f, 0.f});
                 f32x4 gp = Mma<T>::k32(ad[0].u, *(const u32x4 *)vp, f32x4{0.f, 0.f, 0.f, 0.f});
@@ -368,8 +372,8 @@ deform_bwd_region16_kernel(const BwdArgs<T> A) {
             kh = (float)(p0 + step) + (float)op[OFS];
             const bool guard = (kh > -1.f) & (kh < (float)H) & (kw > -1.f) & (kw < (float)W);
             const float fh = floor_(kh), fw = floor_(kw);
-            const int hl = (int)fh - wy0, wl = (int)fw - wx0;
-            const bool in = live & guard & ((u32)(hl - step) <= (u32)(BROWS - 2)) & ((u32)wl <= (u32)(WWX - 2));
+            const int hl = (int)fh + RCH, wl = (int)fw - wx0;       // of the column's window
+            const bool in = live & guard & ((u32)(hl - (p0 + step)) <= (u32)(BROWS - 2)) & ((u32)wl <= (u32)(WWX - 2));
             const bool out = live & guard & !in;
             const float lh = kh - fh, lw = kw - fw, hh = 1.f - lh, hw = 1.f - lw;
             const bool use = in | out;
@@ -606,7 +610,7 @@ deform_bwd_region16_kernel(const BwdArgs<T> A) {
                 for (int k = 0; k < 8; ++k) f[k] = (float)(int)(k < 4 ? w0[k] : w1[k - 4]) * WIN;
                 u32x4 a[PIECES<T>];
                 pieces8<T>(f, a);
-                const T *kt = Kl + ((base + 32 * ks + 8 * mk) % RING + (mi >> 2)) * KSB + 4 * (mi & 3);
+                const T *kt = Kl + ((u32)(base + 32 * ks + 8 * mk) % RING + (mi >> 2)) * KSB + 4 * (mi & 3);
 #pragma unroll
                 for (int nb = 0; nb < NKB; ++nb) {
                     union { u32x2 h[2]; u32x4 u; } b;
