@@ -593,7 +593,13 @@ static hipError_t launch_t(int mode, bool wide, const void *q, const void *key, 
         // allow it, 4 columns wider: those go straight into LDS.  25x42-class shapes measured
         // 59 -> 57 us, the 16 x 8 tiles 85 -> 73 us, the 16 x 16 tiles 66 -> 60 us.)
         constexpr bool F32 = std::is_same<T, float>::value;
-        if (mode == TILED_FUSED && !wide && (long)B * H * W <= SAPA_TILED_SMALL_PARENTS) {
+        // The similarity stages of the fp32 training step, whose channels no other workgroups share, likewise in one
+        // round of two workgroups per CU (with the softmax backward over 256 channels: 16 images 42x25 136 -> 71 us,
+        // 8 of 64x64 94 -> 68, 12 of 50x84, 504 tiles, 101 -> 88, but 14, 588 tiles, 108 -> 134 and 4 of 100x168
+        // 111 -> 143; 512 channels, 6 of 91x97 280 -> 177).
+        const bool similarity = mode == TILED_QK_SOFTMAX || mode == TILED_QK_SOFTMAX_BWD;
+        const bool one_round = (long)((W + 15) / 16) * ((H + 7) / 8) * B <= 512;
+        if ((mode == TILED_FUSED && !wide && (long)B * H * W <= SAPA_TILED_SMALL_PARENTS) || (F32 && similarity && one_round)) {
             if constexpr (F32)
                 if (aligned(4))
                     return launch_mode<T, 5, 2, 1, 1, 2, 16, 4, 16>(mode, wide, q, key, attn_in, value, out, B, d, C, H, W, st);
