@@ -25,7 +25,7 @@
 // per square in front of its first step, 115 us of 665 for the additions).
 //
 // Measured (B=8, C=256, 4 groups, d=32, 64x64 -> 128x128, bf16): this part of a training step 780 -> 470 us with
-// 25 points (step 1033 -> 713), 560 -> 330 with 9 (811 -> 574); C=128, 90x121, 9 points, channels-last
+// 25 points (step 1033 -> 718), 560 -> 330 with 9 (811 -> 574); C=128, 90x121, 9 points, channels-last
 // 1634 -> 1106 (whole step).  What bounds it is the chain of a step's three phases, each behind a barrier
 // with the 16 waves that one CU's LDS holds (of 470: A 35, B 150, C 175, memory 60, barriers 50): half
 // the vector instructions that it issues at the most, a tenth of the matrix rate, 1 TB/s.
