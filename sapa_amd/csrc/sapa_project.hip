@@ -441,8 +441,7 @@ __device__ __forceinline__ f32x4 mma32(u32x4 a, u32x4 b, f32x4 c) {
 }
 
 // C input channels (a multiple of 32), O outputs (a multiple of 16); NW = 8 or 12 waves, tiles of 32
-// pixels (two blocks of 16 matrix rows share every weight operand read from LDS), the
-// workgroup's waves on neighbouring tiles.
+// pixels (two blocks of 16 matrix rows share every weight operand read from LDS).
 // Reduction step ks takes channels 32 ks ..; inside it lane group kg holds channels
 // 4 kg .. + 3 and 16 + 4 kg .. + 3 (two 16-byte pieces of memory; the 16 lanes of a piece
 // read 64 contiguous bytes per pixel) -- the weight planes are stored in that order.
@@ -454,10 +453,15 @@ __device__ __forceinline__ f32x4 mma32(u32x4 a, u32x4 b, f32x4 c) {
 // that the two channel groups of a half-wave read disjoint banks).  OUT_CL = false: out is
 // [B, O, HW]; a block of 16 outputs x 32 pixels goes back through LDS and leaves as 128-byte rows
 // (HW a multiple of 4: a 16-byte piece never runs from one plane into the next).
-// Twelve waves (of which launch32_co says where), as many as 168 registers and the LDS allow: what bounds the kernel is the chain of a step (tile
-// through LDS, pieces, matrix products), which three waves per SIMD hide better than two (two steps of
-// x in flight each instead of four); finer tiles per round besides (16 images, 256 -> 64: 100x168
-// pixels 81 -> 77 us, 50x84 35 -> 24, channels-last 86 -> 76 and 28 -> 22; 200x336 311 -> 300).
+// Twelve waves (launch32_co says where): what bounds the kernel is the chain of a step (tile through LDS, pieces,
+// matrix products), which three waves per SIMD hide better than two, and a round's tiles divide more finely
+// (16 images, 256 -> 64: 100x168 pixels 81 -> 77 us, 50x84 35 -> 24, channels-last 86 -> 76 and 28 -> 22; 200x336
+// 311 -> 300).  Their 168 registers hold two steps of x in flight instead of four; 256 -> 64 still spills 3 (planes
+// to channels-last 8), 512 -> 32 2 to 5, 64 -> 64 2 to 11, 128 -> 64 from planes 11 and from channels-last
+// features 19 registers.
+// The tiles of a workgroup: wave after wave, so that the waves read neighbouring pieces of a plane (a plane of no whole
+// cache lines is otherwise read twice at every piece's end: 128 -> 128, 3 images 150x134 28.3 -> 22.1 us); eight waves
+// on channels-last features a run of them each (neighbouring tiles: 64 -> 32, one image 32x32 4.05 -> 4.6 us).
 template <int C, int O, bool IN_CL, bool OUT_CL, bool WIDE, int NW>
 __global__ void __launch_bounds__(64 * NW)
 project32_kernel(const float *__restrict__ x, const float *__restrict__ w, const float *__restrict__ bias,
@@ -483,9 +487,13 @@ project32_kernel(const float *__restrict__ x, const float *__restrict__ w, const
     const Span sp = span_of<O, WIDE>(outputs);
 
     const long ntiles = (HW + 31) / 32;
-    // tiles t0, t0 + waves ..: the waves read neighbouring pieces of a plane (waves past `waves` help with the weights only)
+    // tiles t0, t0 + stride .. below t1 (waves past `waves` help with the weights only)
+    constexpr bool NEIGHBOURS = !IN_CL || NW > 8;
     const long first = (long)blockIdx.x * waves * tiles_per_wave, last = first + (long)waves * tiles_per_wave;
-    const long t0 = first + wave, t1 = wave >= waves ? t0 : last < ntiles ? last : ntiles;
+    const long t0 = NEIGHBOURS ? first + wave : ((long)blockIdx.x * waves + wave) * tiles_per_wave;
+    const long t1 = wave >= waves ? t0 : NEIGHBOURS ? (last < ntiles ? last : ntiles)
+                                                    : (t0 + tiles_per_wave < ntiles ? t0 + tiles_per_wave : ntiles);
+    const long stride = NEIGHBOURS ? waves : 1;
     const int r16 = lane & 15, kg = lane >> 4;    // row / column of a 16 x 16 tile, k group
     float bv[NT];
 #pragma unroll
@@ -565,7 +573,7 @@ project32_kernel(const float *__restrict__ x, const float *__restrict__ w, const
             out[OUT_CL ? ((long)b * HW + p) * sp.OT + sp.o0 + o : ((long)b * sp.OT + sp.o0 + o) * HW + p] = r;
         }
     };
-    for (long t = t0; t < t1; t += waves) {
+    for (long t = t0; t < t1; t += stride) {
         f32x4 acc[2][NT], low[2][NT];
 #pragma unroll
         for (int mb = 0; mb < 2; ++mb)
@@ -600,7 +608,7 @@ project32_kernel(const float *__restrict__ x, const float *__restrict__ w, const
             }
             // the ring slot is free: the step RING further on (of this tile or of the next)
             if (ks + RING < KS) load_step(ks % RING, t, ks + RING);
-            else if (t + waves < t1) load_step(ks % RING, t + waves, ks + RING - KS);
+            else if (t + stride < t1) load_step(ks % RING, t + stride, ks + RING - KS);
 #pragma unroll
             for (int nt = 0; nt < NT; ++nt) {
                 if (WIDE && 16 * nt >= sp.left) break;
@@ -682,23 +690,25 @@ struct Spread {
     int waves;
 };
 // One workgroup is resident per CU (its weight planes fill most of the LDS) and the part has
-// 256 CUs: two full rounds of workgroups where that leaves a wave 6 tiles or more, else one
+// 256 CUs: two full rounds of workgroups where that leaves a wave 8 tiles or more (6 of 12 waves), else one
 // (16 images: 200x336 pixels 301 us in two rounds against 315 in one; 100x168 pixels 71 us in
-// one round against 98 in 272 workgroups)
+// one round against 98 in 272 workgroups; 256 -> 288, 8 images 128x128, 8 waves, 119 us in one against 130)
 static Spread spread32(long ntiles, long sets, int nw) {
     const long slots = 256;
     long blocks = 2 * slots / sets > 1 ? 2 * slots / sets : 1;
     long per = (ntiles + nw * blocks - 1) / (nw * blocks);
-    if (per < 6) {
+    if (per < (nw == 8 ? 8 : 6)) {
         blocks = slots / sets > 1 ? slots / sets : 1;
         per = (ntiles + nw * blocks - 1) / (nw * blocks);
     }
     // ... and as few waves per workgroup as cover the image in that many tiles each, so that no workgroup of the
-    // round is missing (8 images of 128x128 pixels, 256 -> 128: 240 workgroups of 12 waves else 256 of 11;
-    // fewer tiles than the chip has room for: a wave's matrix instructions are not queued behind a second
-    // wave's; 4 images of 33x20 pixels, 256 -> 128 / 288: SAPA-D module 113 -> 104 us)
+    // round is missing (240 workgroups of 12 waves else 256 of 11; 512 -> 72, 2 images 100x168, 8 waves in 198
+    // workgroups 35.8 us, 7 in 228 31.3; fewer tiles than the chip has room for: a wave's matrix instructions are not
+    // queued behind a second wave's; 4 images of 33x20 pixels, 256 -> 128 / 288: SAPA-D module 113 -> 104 us), but over
+    // several tiles each not with less than 6 of 8 (128 -> 32, 16 images 50x84: 5 waves 12.4 us, 8 11.7)
     int waves = (int)((ntiles + blocks * per - 1) / (blocks * per));
     waves = waves < 1 ? 1 : waves > nw ? nw : waves;
+    if (nw == 8 && per > 1 && waves < 6) waves = nw;
     return Spread{per, (ntiles + waves * per - 1) / (waves * per), waves};
 }
 
@@ -735,17 +745,17 @@ static hipError_t launch32_co(const void *x, const void *w, const void *bias, vo
     if (HW * (long)(C > outputs ? C : outputs) * 4 >= (1L << 31)) return hipErrorNotSupported;
     const long ntiles = (HW + 31) / 32, sets = (long)B * ((outputs + O - 1) / O);     // sets: workgroups that share a pixel range's place
     const Spread s8 = spread32(ntiles, sets, 8), s12 = spread32(ntiles, sets, 12);
-    // Eight waves, with twice the steps of x in flight and no bar to moving work between steps, are faster over the
-    // same number of tiles each (us with 12 / 8 waves: 256 -> 32, 2 images 128x128 pixels 13.6 / 11.9, 8 images
-    // 27.5 / 26.0; 64 -> 32, 4 images 5.4 / 4.8), and throughout at 128 -> 32 (2 images 128x128 11.2 / 6.1, 16 of
-    // 50x84 14.0 / 12.0, of 100x168 30.1 / 29.2).  64 outputs (or 64 at a time): over one tile each (256 -> 128, 8
-    // images 64x64 18.5 / 17.0, 4 of 32x32 10.9 / 10.3; 256 -> 288, 8 of 64x64, 4 tiles, 38.6 / 40.3), from
-    // channels-last features where 7 or 8 of them have one (256 -> 64, 4 images 128x128 19.5 / 17.7; 2 images
-    // 12.1 / 13.3).
-    constexpr bool ALWAYS8 = C == 128 && O == 32;
-    if (ALWAYS8 || (O == 64 ? s8.per == 1 && (!IN_CL || s8.waves > 6) : s8.per <= s12.per))
-        return launch32_waves<C, O, IN_CL, OUT_CL, WIDE, 8>(x, w, bias, out, B, HW, st, outputs, s8);
-    return launch32_waves<C, O, IN_CL, OUT_CL, WIDE, ALWAYS8 ? 8 : 12>(x, w, bias, out, B, HW, st, outputs, s12);
+    // Twelve waves where they shorten a wave's chain of tiles to what is asked for below (eight have twice the steps of
+    // x in flight and no bar to moving work between steps).  us with 8 / 12 waves, from planes: 5 tiles to 3 each
+    // (256 -> 64, 16 images 100x168) 66 / 60, 7 to 5 (128 -> 144, 8 images 128x128) 42.7 / 40.5, but 4 to 3
+    // (256 -> 400, 8 images 64x64) 45.3 / 46.5; from channels-last features 5 to 3 (256 -> 64) 64.9 / 61.9, but 7 to 5
+    // (256 -> 288, 14 images 72x68) 70 / 74 and, spilling, 5 to 3 at 128 -> 64 37 / 38.5 .. 42; 128 -> 32 with 2 tiles
+    // to 1 (16 images 50x84) 11.7 / 14.1.  Tenths of eight waves' tiles per tile of twelve waves:
+    constexpr int ASKED = C == 128 && O == 32 ? 1 << 20 : !IN_CL ? 14 : C == 128 ? 20 : 15;
+    // (and 256 -> 64 from channels-last features over one tile each for 3 to 6 waves: 8 images 64x64 13.9 / 12.5)
+    if (10 * s8.per >= ASKED * s12.per || (IN_CL && C == 256 && O == 64 && s8.per == 1 && s8.waves > 2 && s8.waves <= 6))
+        return launch32_waves<C, O, IN_CL, OUT_CL, WIDE, C == 128 && O == 32 ? 8 : 12>(x, w, bias, out, B, HW, st, outputs, s12);
+    return launch32_waves<C, O, IN_CL, OUT_CL, WIDE, 8>(x, w, bias, out, B, HW, st, outputs, s8);
 }
 
 template <bool IN_CL, bool OUT_CL>
