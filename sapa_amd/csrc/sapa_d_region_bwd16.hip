@@ -289,8 +289,10 @@ deform_bwd_region16_kernel(const BwdArgs<T> A) {
     // a power of two
     auto pow2 = [](int e) __attribute__((always_inline)) { return __builtin_ldexpf(1.f, e); };
     constexpr bool F16 = __is_same(T, f16_t);
-    constexpr int WEXP = F16 ? 15 : 30;                 // Wv (and a row of Wg) enters its products times 2^WEXP
-    constexpr float WIN = F16 ? 1.f / 32768.f : 1.f;
+    // Wv (and a row of Wg) enters its products times 2^WEXP: in fp16 as large as the type holds; bf16 has fp32's
+    // range, and sums times 2^30 would leave it above 2^97
+    constexpr int WEXP = F16 ? 15 : 0;
+    constexpr float WIN = F16 ? 1.f / 32768.f : 1.f / 1073741824.f;
 
     // ... added to the gradients: lanes along 16 channels of a cell
     auto flush = [&]() __attribute__((always_inline)) {

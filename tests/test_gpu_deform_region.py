@@ -71,3 +71,19 @@ def test_gradients_of_any_size_in_fp16(coracle):
             err, rms = (got.cpu().double() - w).abs(), w.pow(2).mean().sqrt()
             # (2^-25: half the smallest spacing of the type)
             assert bool((err <= 2.0 ** -11 * w.abs() + 4e-4 * rms + 2.0 ** -25).all()), (name, scale)
+
+
+@pytest.mark.parametrize('which', ['grad_out', 'key'])
+@pytest.mark.parametrize('big', [2.0 ** 98, 2.0 ** -98])
+def test_bf16_operands_near_the_types_ends(coracle, which, big):
+    """bf16 values of some 2^98 or 2^-98, whose gradients fp32 holds: the same as of ordinary ones but for the scale."""
+    shape = (1, 1, 32, 64, 18, 17, 25, 0.75)
+    q, key, v, off, go = _inputs(shape, torch.bfloat16, seed=403)
+    want = deform_fused_backward_oracle(coracle, go.float(), q.float(), key.float(), v.float(), off.float(), 25, 2, 1)
+    if which == 'grad_out':
+        got, scale = _gradients(q, key, v, off, go * big, 25, 1), (big, big, big, big)
+    else:
+        got, scale = _gradients(q / big, key * big, v, off, go, 25, 1), (big, 1 / big, 1.0, 1.0)
+    for a, w, f, name in zip(got, want, scale, NAMES):
+        err, rms = (a.cpu().double() / f - w).abs(), w.pow(2).mean().sqrt()
+        assert bool((err <= 2.0 ** -8 * w.abs() + 4e-4 * rms).all()), name
