@@ -31,9 +31,9 @@
 // the vector instructions that it issues at the most, a tenth of the matrix rate, 1 TB/s.
 //
 // Numerics: products of 16-bit values are exact in fp32, sums are fp32.  The integers (30 bits of a row's
-// largest possible sum; Wg's scaled by a power of two per pixel) enter the products as three bf16
-// operands (24 bits), in fp16 as two (22 bits and the type's subnormals below: for grad_key's sum over pixels
-// they are scaled to the step's largest pixel).  Points outside the band, every point of a pixel with operands or
+// largest possible sum; Wg's scaled by a power of two per pixel) enter the products as three 16-bit
+// operands, which hold all 24 bits of an fp32 number (in fp16 down to 2^-40 of the largest: for grad_key's sum over
+// pixels a cell's weights are scaled to the largest of the step).  Points outside the band, every point of a pixel with operands or
 // gradients that are not finite, and grad_query's terms where the key window holds a non-finite
 // value are added one by one: a dense product would spread 0 * inf.
 #include <utility>
@@ -71,15 +71,15 @@ struct BwdArgs {
     int Cq, C, H, W, P, G, strips_x, segments, rows, nblocks, per_xcd;
 };
 
-// 8 fp32 values as 16-bit operands that sum up to them: 3 of bf16, 2 of fp16
-template <typename T> constexpr int PIECES = __is_same(T, f16_t) ? 2 : 3;
+// 8 fp32 values as 16-bit operands that sum up to them
+constexpr int PIECES = 3;
 template <typename T>
-__device__ __forceinline__ void pieces8(float (&f)[8], u32x4 (&p)[PIECES<T>]) {
+__device__ __forceinline__ void pieces8(float (&f)[8], u32x4 (&p)[PIECES]) {
     typedef T tx8 __attribute__((ext_vector_type(8)));
 #pragma unroll
-    for (int i = 0; i < PIECES<T>; ++i) {
+    for (int i = 0; i < PIECES; ++i) {
         p[i] = u32x4{wm::pack2<T>(f[0], f[1]), wm::pack2<T>(f[2], f[3]), wm::pack2<T>(f[4], f[5]), wm::pack2<T>(f[6], f[7])};
-        if (i + 1 < PIECES<T>) {
+        if (i + 1 < PIECES) {
             const tx8 h = __builtin_bit_cast(tx8, p[i]);
 #pragma unroll
             for (int k = 0; k < 8; ++k) f[k] -= (float)h[k];
@@ -546,51 +546,49 @@ deform_bwd_region16_kernel(const BwdArgs<T> A) {
                     float f[8];
 #pragma unroll
                     for (int k = 0; k < 8; ++k) f[k] = (float)sp[k * RS] * WIN;
-                    u32x4 a[PIECES<T>];
+                    u32x4 a[PIECES];
                     pieces8<T>(f, a);
-                    u32x4 b[NVB];
+                    // (two blocks of channels at a time: four do not fit the registers)
 #pragma unroll
-                    for (int nb = 0; nb < NVB; ++nb) {
+                    for (int nb = 0; nb < NVB; nb += 2) {
                         if (16 * nb >= cg) break;
-                        b[nb] = operand(Dl[buf] + (16 * nb + mi) * PXS + 8 * mk);
-                    }
+                        const u32x4 b0 = operand(Dl[buf] + (16 * nb + mi) * PXS + 8 * mk);
+                        const u32x4 b1 = operand(Dl[buf] + (16 * nb + 16 + mi) * PXS + 8 * mk);
 #pragma unroll
-                    for (int i = PIECES<T> - 1; i >= 0; --i)
-#pragma unroll
-                        for (int nb = 0; nb < NVB; ++nb) {
-                            if (16 * nb >= cg) break;
-                            Dv[nb] = Mma<T>::k32(a[i], b[nb], Dv[nb]);
+                        for (int i = PIECES - 1; i >= 0; --i) {
+                            Dv[nb] = Mma<T>::k32(a[i], b0, Dv[nb]);
+                            Dv[nb + 1] = Mma<T>::k32(a[i], b1, Dv[nb + 1]);
                         }
+                    }
                 }
                 if (want_k) {
                     const int *gp = (const int *)Gl + 8 * mk * RS + 16 * role + mi;
-                    int e8[8], top = -126;
+                    float f[8], down[4];
 #pragma unroll
-                    for (int k = 0; k < 8; ++k) e8[k] = ex[8 * mk + k];
+                    for (int k = 0; k < 8; ++k) f[k] = __builtin_ldexpf((float)gp[k * RS], ex[8 * mk + k] - 30);
                     if (F16) {
+                        // (lanes of one mi hold the cell's 32 weights)
+                        float m = 0.f;
 #pragma unroll
-                        for (int k = 0; k < 8; ++k) top = e8[k] > top ? e8[k] : top;
-                        const int o = __shfl_xor(top, 16);
-                        top = o > top ? o : top;
-                        const int o2 = __shfl_xor(top, 32);
-                        top = o2 > top ? o2 : top;
+                        for (int k = 0; k < 8; ++k) m = fmaxf(m, __builtin_fabsf(f[k]));
+                        const wm::Fit fit = wm::fit<T>(wm::over_groups(m));
+#pragma unroll
+                        for (int k = 0; k < 8; ++k) f[k] *= fit.up;
+#pragma unroll
+                        for (int r = 0; r < 4; ++r) down[r] = __shfl(fit.down, 4 * mk + r);
                     }
-                    float f[8];
-#pragma unroll
-                    for (int k = 0; k < 8; ++k) f[k] = __builtin_ldexpf((float)gp[k * RS], e8[k] - 30 + (F16 ? 15 - top : 0));
-                    u32x4 a[PIECES<T>];
+                    u32x4 a[PIECES];
                     pieces8<T>(f, a);
-                    const float down = pow2(top - 15);
 #pragma unroll
                     for (int nb = 0; nb < NKB; ++nb) {
                         if (16 * nb >= d) break;
                         const u32x4 b = operand(Ql[buf] + (16 * nb + mi) * PXS + 8 * mk);
                         f32x4 acc = F16 ? f32x4{0.f, 0.f, 0.f, 0.f} : Dk[nb];
 #pragma unroll
-                        for (int i = PIECES<T> - 1; i >= 0; --i) acc = Mma<T>::k32(a[i], b, acc);
+                        for (int i = PIECES - 1; i >= 0; --i) acc = Mma<T>::k32(a[i], b, acc);
                         if (F16) {
 #pragma unroll
-                            for (int r = 0; r < 4; ++r) acc[r] = fma_(acc[r], down, Dk[nb][r]);
+                            for (int r = 0; r < 4; ++r) acc[r] = fma_(acc[r], down[r], Dk[nb][r]);
                         }
                         Dk[nb] = acc;
                     }
@@ -610,7 +608,7 @@ deform_bwd_region16_kernel(const BwdArgs<T> A) {
                 float f[8];
 #pragma unroll
                 for (int k = 0; k < 8; ++k) f[k] = (float)(int)(k < 4 ? w0[k] : w1[k - 4]) * WIN;
-                u32x4 a[PIECES<T>];
+                u32x4 a[PIECES];
                 pieces8<T>(f, a);
                 const T *kt = Kl + ((u32)(base + 32 * ks + 8 * mk) % RING + (mi >> 2)) * KSB + 4 * (mi & 3);
 #pragma unroll
@@ -619,7 +617,7 @@ deform_bwd_region16_kernel(const BwdArgs<T> A) {
                     b.h[0] = read_tr((const u32 *)(kt + 16 * nb));
                     b.h[1] = read_tr((const u32 *)(kt + 16 * nb + 4 * KSB));
 #pragma unroll
-                    for (int j = PIECES<T> - 1; j >= 0; --j) acc[nb] = Mma<T>::k32(a[j], b.u, acc[nb]);
+                    for (int j = PIECES - 1; j >= 0; --j) acc[nb] = Mma<T>::k32(a[j], b.u, acc[nb]);
                 }
             }
 #pragma unroll

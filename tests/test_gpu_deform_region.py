@@ -87,3 +87,32 @@ def test_bf16_operands_near_the_types_ends(coracle, which, big):
     for a, w, f, name in zip(got, want, scale, NAMES):
         err, rms = (a.cpu().double() / f - w).abs(), w.pow(2).mean().sqrt()
         assert bool((err <= 2.0 ** -8 * w.abs() + 4e-4 * rms).all()), name
+
+
+def test_corner_weights_hold_24_bits_in_fp16():
+    """Cells that one sample of one pixel reaches, with a gradient of the output of 1: grad_value is the corner's weight,
+    rounded once.  Equal logits of 3 points, two of them outside the image: weights of fl(1/3) times a corner's
+    share, in fixed point of 2^-30 (half a million of them: some would round the other way with a bit less)."""
+    B, G, H, W, P = 16, 8, 64, 64, 3
+    g = torch.Generator(device='cuda').manual_seed(404)
+    q = torch.zeros(B, 8 * G, 2 * H, 2 * W, device='cuda')
+    key, v = (torch.randn(B, 8 * G, H, W, generator=g, device='cuda') for _ in range(2))
+    off = torch.full((B, G, P, 2, 2 * H, 2 * W), 1000.0, device='cuda')
+    # (x, y) of every second parent, of all sizes below 1
+    steps = torch.exp2(-4 * torch.rand(B, G, 2, 32, 32, generator=g, device='cuda') - 0.1).half().float()
+    off[:, :, 0, :, ::4, ::4] = steps
+    go = torch.zeros_like(q)
+    go[..., ::4, ::4] = 1
+    at = 2.0 * torch.arange(32, device='cuda')
+    kw, kh = steps[:, :, 0] + at, steps[:, :, 1] + at[:, None]
+    low_w, low_h = kw.floor(), kh.floor()
+    lw, lh = kw - low_w, kh - low_h
+    want = torch.zeros(B, G, H + 1, W + 1, device='cuda')
+    n, grp = (torch.arange(k, device='cuda').view(s) for k, s in ((B, (B, 1, 1, 1)), (G, (1, G, 1, 1))))
+    third = torch.tensor(1.0, device='cuda') / 3 * 2.0 ** 30
+    for dy, dx, share in ((0, 0, (1 - lh) * (1 - lw)), (0, 1, (1 - lh) * lw), (1, 0, lh * (1 - lw)), (1, 1, lh * lw)):
+        want[n, grp, low_h.long() + dy, low_w.long() + dx] = (third * share).round() * 2.0 ** -30
+    want = want[:, :, :H, :W].half().unsqueeze(2).expand(B, G, 8, H, W).reshape(B, 8 * G, H, W)
+    t = [x.half().requires_grad_() for x in (q, key, v, off.view(B, 2 * G * P, 2 * H, 2 * W))]
+    got = torch.autograd.grad(sapa_amd.deform_sapa_fused(*t, P, 2, G), t, go.half())
+    assert torch.equal(got[2], want)
