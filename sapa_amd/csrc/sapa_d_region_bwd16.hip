@@ -169,8 +169,9 @@ deform_bwd_region16_kernel(const BwdArgs<T> A) {
     // (both loads of the window row: one of them is out of range; a branch would wait for what is in flight)
     auto load_row = [&](int gy) __attribute__((always_inline)) {
         const bool ok = gy >= 0 && gy < H;
-        const u32x4 a = __builtin_amdgcn_raw_buffer_load_b128(rsa, ok ? offa : OUTSIDE, (u32)(gy * W * Cq * 2), 0);
-        const u32x4 b = __builtin_amdgcn_raw_buffer_load_b128(rsb, ok ? offb : OUTSIDE, (u32)(gy * W * C * 2), 0);
+        const u32 row = ok ? (u32)(gy * W) * 2u : 0u;           // (no row beside the image is ever an offset)
+        const u32x4 a = __builtin_amdgcn_raw_buffer_load_b128(rsa, ok ? offa : OUTSIDE, row * (u32)Cq, 0);
+        const u32x4 b = __builtin_amdgcn_raw_buffer_load_b128(rsb, ok ? offb : OUTSIDE, row * (u32)C, 0);
         return u32x4{a[0] | b[0], a[1] | b[1], a[2] | b[2], a[3] | b[3]};
     };
     auto put_piece = [&](int row, u32x4 v) __attribute__((always_inline)) {
@@ -184,10 +185,12 @@ deform_bwd_region16_kernel(const BwdArgs<T> A) {
     };
     auto fetch = [&](int step) __attribute__((always_inline)) {
         if (hires) {
+            // (all of the offset in the lane's part, which the descriptor's check is made for dword by dword: where
+            // a row ends two pixels into a piece, the tensor's last one runs over its end)
             const u32 so = (u32)(step * 4 * hW);
             const bool ok = step < nstep;
-            const u32x2 v = __builtin_amdgcn_raw_buffer_load_b64(rsa, ok ? offa : OUTSIDE, so, 0);
-            ofr = __builtin_amdgcn_raw_buffer_load_b64(rsb, ok ? offb : OUTSIDE, so, 0);
+            const u32x2 v = __builtin_amdgcn_raw_buffer_load_b64(rsa, ok ? offa + so : OUTSIDE, 0, 0);
+            ofr = __builtin_amdgcn_raw_buffer_load_b64(rsb, ok ? offb + so : OUTSIDE, 0, 0);
             hr[0] = v[0], hr[1] = v[1];
         } else {
             hr = load_row(step + AHEAD - 1 < nstep + 2 * RCH + 1 ? wy0 + step + AHEAD - 1 : -1);

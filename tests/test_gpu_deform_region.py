@@ -116,3 +116,23 @@ def test_corner_weights_hold_24_bits_in_fp16():
     t = [x.half().requires_grad_() for x in (q, key, v, off.view(B, 2 * G * P, 2 * H, 2 * W))]
     got = torch.autograd.grad(sapa_amd.deform_sapa_fused(*t, P, 2, G), t, go.half())
     assert torch.equal(got[2], want)
+
+
+@pytest.mark.parametrize('dtype', [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize('shape', [(1, 1, 24, 40, 20, 9, 16, 1.0), (2, 2, 32, 64, 7, 21, 9, 1.0)], ids=['18-wide', '42-wide'])
+def test_last_pixels_of_rows_that_end_inside_a_piece(shape, dtype):
+    """Rows of 4 n + 2 pixels, the tensors' last ones with NaN right behind them: the piece that runs over the end brings
+    the two pixels in front of it and nothing that counts."""
+    P, G = shape[6], shape[1]
+    plain = [t.to(DEV) for t in _inputs(shape, dtype, seed=405)]
+
+    def before_nan(t):
+        room = torch.full((t.numel() + 64,), float('nan'), dtype=dtype, device=DEV)
+        return room[:t.numel()].copy_(t.detach().reshape(-1)).view_as(t)
+    want = _gradients(*plain, P, G)
+    got = _gradients(*(before_nan(t) for t in plain), P, G)
+    assert torch.equal(got[0], want[0]) and torch.equal(got[3], want[3])
+    for a, b in zip(got[1:3], want[1:3]):           # (atomic sums, in any order)
+        torch.testing.assert_close(a, b, rtol=torch.finfo(dtype).eps, atol=1e-5)
+    for t, grads in ((plain[0], got[0]), (plain[3], got[3])):
+        assert bool(torch.isfinite(grads).all()) and grads[..., -1, -2:].abs().max() > 0
