@@ -1,5 +1,5 @@
-"""The one-kernel backward of fused SAPA-D for 16-bit tensors at up_factor 2: strips of parent rows that
-go round the window ring, ragged edges, far points, values that are not finite."""
+"""The one-kernel backward of fused SAPA-D for 16-bit tensors at up_factor 2: strips of parent rows in one and in many
+steps round the window ring, ragged edges, far points, values that are not finite."""
 import pytest
 import torch
 
@@ -9,8 +9,9 @@ from test_gpu_sapa_d import DEV, dev, make
 
 pytestmark = pytest.mark.gpu
 NAMES = ('grad_query', 'grad_key', 'grad_value', 'grad_offset')
-# B, G, dq, cg, H, W, P, offset scale: 37 rows go round the ring twice and a ragged strip beside a whole one;
-# rows of two pixels over a multiple of 4; one narrow strip, many segments; far points in both lane mappings
+# B, G, dq, cg, H, W, P, offset scale: so few strips are split into segments of one row each (one step);
+# a ragged strip beside a whole one; rows of two pixels over a multiple of 4; one narrow strip; far points in both
+# lane mappings
 SHAPES = [(1, 2, 32, 64, 37, 21, 25, 0.75), (2, 1, 24, 40, 20, 9, 16, 2.0), (1, 1, 8, 8, 50, 3, 2, 0.7),
           (1, 2, 32, 64, 17, 13, 32, 6.0), (3, 2, 16, 24, 3, 5, 9, 1.0), (1, 1, 32, 48, 33, 16, 17, 1.5)]
 
@@ -43,6 +44,62 @@ def test_against_the_exact_chain(coracle, shape, dtype):
         err, rms = (got.cpu().double() - w).abs(), w.pow(2).mean().sqrt()
         worst = (err / (rel * w.abs() + 4e-4 * rms)).max().item()
         assert worst <= 1, f'{name}: {worst}'
+
+
+def _steps(B, G, H, W):
+    """Rows of parents per workgroup: the launcher's rule (the shortest of rounds of 256 workgroups times rows + 4)."""
+    columns, best = (W + 7) // 8 * G * B, None
+    for k in range(1, H + 1):
+        if k > 1 and columns * (k - 1) >= 4 * 256:
+            break
+        rows = -(-H // k)
+        time = -(-(columns * -(-H // rows)) // 256) * (rows + 4)
+        if best is None or time < best[0]:
+            best = time, rows
+    return best[1]
+
+
+# 256 strips, whole: 37 steps go round the ring of 15 window rows twice and more; a strip of 8 parents and a ragged one,
+# rows of 26 pixels; both lane mappings, samples far from their parents and near
+MANY = [(32, 4, 8, 8, 37, 13, 9, 0.9), (32, 4, 24, 40, 37, 13, 25, 2.5), (64, 2, 32, 64, 33, 9, 16, 0.75)]
+
+
+@pytest.mark.parametrize('dtype', [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize('shape', MANY, ids=['-'.join(map(str, s)) for s in MANY])
+def test_many_steps(coracle, shape, dtype):
+    """As above, the first and the last image."""
+    B, G, dq, cg, H, W, P, _ = shape
+    assert _steps(B, G, H, W) > 2 * 15
+    ops = _inputs(shape, dtype, seed=406)
+    got = _gradients(*ops, P, G)
+    rel = 2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -11
+    for n in (0, B - 1):
+        q, key, v, off, go = (t[n:n + 1].float() for t in ops)
+        want = deform_fused_backward_oracle(coracle, go, q, key, v, off, P, 2, G)
+        for a, w, name in zip(got, want, NAMES):
+            err, rms = (a[n:n + 1].cpu().double() - w).abs(), w.pow(2).mean().sqrt()
+            worst = (err / (rel * w.abs() + 4e-4 * rms)).max().item()
+            assert worst <= 1, f'{name} of image {n}: {worst}'
+
+
+@pytest.mark.parametrize('which', ['query', 'key', 'value', 'grad_out'])
+@pytest.mark.parametrize('row', [2, 31])
+def test_non_finite_values_in_one_of_many_steps(coracle, which, row):
+    """A value that is not finite in an early or late step: its image's gradients are not finite where the exact chain's are
+    not, and right elsewhere; its neighbour in the batch has none."""
+    shape = (32, 4, 8, 8, 37, 13, 9, 0.9)
+    ops = dict(zip(('query', 'key', 'value', 'offset', 'grad_out'), _inputs(shape, torch.float16, seed=407)))
+    t = ops[which]
+    t[5, 3, row * t.size(2) // 37 + 1, 5] = float('inf')
+    got = _gradients(*ops.values(), 9, 4)
+    for n in (5, 6):
+        q, key, v, off, go = (x[n:n + 1].float() for x in ops.values())
+        want = deform_fused_backward_oracle(coracle, go, q, key, v, off, 9, 2, 4)
+        for a, w, name in zip(got, want, NAMES):
+            a, fine = a[n:n + 1].cpu().double(), torch.isfinite(w)
+            assert torch.equal(torch.isfinite(a), fine), (name, n)
+            err, rms = (a - w)[fine].abs(), w[fine].pow(2).mean().sqrt()
+            assert bool((err <= 2.0 ** -11 * w[fine].abs() + 4e-4 * rms).all()), (name, n)
 
 
 @pytest.mark.parametrize('which', ['query', 'key', 'value', 'grad_out'])
