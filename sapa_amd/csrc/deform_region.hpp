@@ -1,11 +1,10 @@
-// Geometry and helpers shared by the region forms of the 16-bit SAPA-D kernels (s = 2): a workgroup
-// owns a region of 16 hi-res pixels by 2 * RPY rows of one (image, group), keeps the key and value
-// window of the whole region in LDS and walks over its pixels in steps.
+// Geometry and helpers of the 16-bit SAPA-D backward (s = 2, sapa_d_region_bwd16.hip): a workgroup owns a
+// strip of RPX parents (RW hi-res pixels) of one (image, group) and walks down it by one row of parents a step.
 //
-// The samples of a step's pixels -- one row of 8 parents -- lie within RCH cells of their parents (those
-// that do not are handled apart), i.e. in a band of 2 RCH + 2 window rows.  A step's dense products
-// run over the 16-cell blocks of the window that hold the band: 12 blocks from the one its
-// first cell is in, and a pixel's row of Sim / Wm has an entry per cell of those blocks.
+// A step's samples lie within RCH cells of their parents (those that do not are handled apart), i.e. in a band of
+// BROWS rows of the strip's window of WWX cells per row.  Its dense products run over the blocks of 16 window cells
+// that hold the band: NBLK from the one its first cell is in, and a pixel's row of Sim / Wm has an entry per
+// cell of those blocks.
 #pragma once
 #include "deform_tap.hpp"
 #include "wm16_common.hpp"
@@ -18,15 +17,13 @@ using wm::f32x4;
 using wm::Mma;
 using wm::OUTSIDE;
 using wm::read_tr;
-using wm::s16x4;
 using wm::u32;
 using wm::u32x2;
 using wm::u32x4;
-typedef float f32x2 __attribute__((ext_vector_type(2)));
 
 constexpr int S = 2;                        // up_factor
 constexpr int RCH = 4;                      // window reach around a parent, in low-res cells
-constexpr int RPX = 8, RW = RPX * S;        // parents / pixels of a region along x
+constexpr int RPX = 8, RW = RPX * S;        // parents / pixels of a strip along x
 constexpr int WWX = RPX + 2 * RCH + 1;      // window cells along x
 constexpr int BROWS = 2 * RCH + 2;          // window rows of a step's band
 constexpr int NBLK = (BROWS * WWX + 15 + 15) / 16, BC = 16 * NBLK;     // blocks of 16 cells that hold a band, their cells
@@ -38,8 +35,6 @@ constexpr float WSCALE = 1073741824.f;      // 2^30: fixed-point scale of Wm
 
 // first cell of the blocks of parent row pr
 __device__ __forceinline__ int band_base(int pr) { return pr * WWX / 16 * 16; }
-// window cells a region of RPY rows of parents keeps in LDS (its last rows belong to blocks only)
-constexpr int window_rows(int rpy) { return (rpy - 1) * WWX / 16 * 16 + BC; }
 
 // Whether a 32-bit word holds a 16-bit value that is not finite (its exponent bits are all set)
 template <typename T>
@@ -51,16 +46,6 @@ __device__ __forceinline__ bool not_finite(u32 x) {
 template <typename T>
 __device__ __forceinline__ bool not_finite(u32x4 x) {
     return not_finite<T>(x[0]) | not_finite<T>(x[1]) | not_finite<T>(x[2]) | not_finite<T>(x[3]);
-}
-
-// 4 consecutive 16-bit elements through a buffer descriptor: one load where they may be read as dwords
-template <bool VEC>
-__device__ __forceinline__ u32x2 load4(__amdgpu_buffer_rsrc_t r, u32 off) {
-    if (VEC) return __builtin_amdgcn_raw_buffer_load_b64(r, off, 0, 0);
-    u32 h[4];
-#pragma unroll
-    for (int e = 0; e < 4; ++e) h[e] = (unsigned short)__builtin_amdgcn_raw_buffer_load_b16(r, off + 2 * e, 0, 0);
-    return u32x2{h[0] | h[1] << 16, h[2] | h[3] << 16};
 }
 
 }  // namespace dreg
