@@ -684,7 +684,6 @@ static hipError_t launch_bwd(const void *grad_out, const void *q, const void *ke
                              int H, int W, int P, int G, hipStream_t st) {
     const int strips_x = (W + RPX - 1) / RPX;
     const long columns = (long)strips_x * G * B;
-    if (columns * H > (1L << 30)) return hipErrorNotSupported;
     // A workgroup fills a CU and walks down a strip of parent rows; its first band and the window rows beyond
     // its own cost about as much as 4 steps.  As many segments per column as make the whole shortest.
     constexpr int CUS = 256, OVER = 4;
@@ -716,8 +715,8 @@ bool deform_bwd_region16_serves(int B, int Cq, int C, int H, int W, int P, int s
     const int d = Cq / G, cg = C / G;
     if (d % 8 != 0 || d > 32 || cg % 8 != 0 || cg > 64) return false;
     const long plane = (long)H * W * 2, hpl = plane * 4;
-    // one image's key / value, a group's planes of the hi-res tensors, in bytes
-    return plane * Cq < (1L << 31) && plane * C < (1L << 31) && 64 * hpl < (1L << 31);
+    // workgroups; one image's key / value, a group's planes of the hi-res tensors, in bytes
+    return (long)B * G * ((W + dreg::RPX - 1) / dreg::RPX) * H <= (1L << 30) && plane * Cq < (1L << 31) && plane * C < (1L << 31) && 64 * hpl < (1L << 31);
 }
 
 // key_cl, value_cl: channels-last copies, aligned to 16 bytes; grad_key, grad_value: fp32 [B, H, W, channels],
