@@ -23,7 +23,8 @@
 // (430 MB each way at B=16, 100x168 in fp32) for the 2 x 29 % more matrix work that this costs.
 //
 // Operands: A and E enter the products as a 16-bit value plus a 16-bit remainder (f16: of values brought
-// into its range, see Fit), everything else is exact in 16 bits; sums are fp32.
+// into its range, see Fit) and, with odd W, a second remainder: calls with even W have had pairs since these
+// kernels serve them, those with odd W had fp32 weights before.  Everything else is exact in 16 bits; sums are fp32.
 //
 // What a non-finite operand does to the products' cells and children outside a window is mended behind them
 // (wm16_exact.hpp): the masked logits are selected, so that the maximum and 1 / sum are the child's own
@@ -33,9 +34,10 @@
 // Measured (B=16, C=256, d=64, 100x168, bf16): pixel kernel 295 us, cell kernel 429 us, a training step
 // 970 us against 1211 for the chain over K * K tensors (similarity and its softmax backward 274 us,
 // grad_q 92, grad_value and grad_key by vector fmas 544, the weights 86).  Odd W: key and value are copied into rows
-// of an even number of cells first (direct loads begin on dwords); B=16, 100x167 1597 -> 1170 us for a step,
-// of which the copies 108 and the cell kernel 503 (hi-res pieces across cache lines, results moved by half
-// a dword; 560 with a 2-byte store per result); B=8, d=64, 51x83 441 -> 198, B=4, C=512, d=32, 97x165 916 -> 540.
+// of an even number of cells first (direct loads begin on dwords); B=16, 100x167 1592 -> 1206 us for a step (1171 with
+// pairs), of which the copies 108 and the cell kernel, of pairs, 503 (hi-res pieces across cache lines, results moved by
+// half a dword; 560 with a 2-byte store per result); B=8, d=64, 51x83 412 -> 192, B=4, C=512, d=32, 97x165 915 -> 551.
+// The third operand costs the cell kernel 8 registers spilled in bf16, 16 in fp16.
 #include "wm16_exact.hpp"
 
 namespace sapa {
@@ -88,6 +90,9 @@ pad_rows_kernel(const unsigned short *__restrict__ a, const unsigned short *__re
     }
 }
 
+// Operands that hold A and E: two, with odd rows three, i.e. all 24 bits of them
+constexpr int pieces_of(bool odd) { return odd ? 3 : 2; }
+
 // position of the 16-byte piece of row r, channel ch in the swizzled tile of bwd_pixel_kernel
 __device__ __forceinline__ int swz(int ch, int r) { return ((ch & 7) << 1) | ((r + (ch >> 3)) & 1); }
 
@@ -124,6 +129,7 @@ bwd_pixel_kernel(const Args<T> args) {
               ns = args.ns, nblocks = args.nblocks, per_xcd = args.per_xcd;
     constexpr int NT = 128 * NSW;
     constexpr bool SCALED = __is_same(T, f16_t);             // E is brought into the type's range (Fit)
+    constexpr int NP = pieces_of(ODD);
     constexpr int NBUF = 3;
     constexpr int LROW = (4 * NSW + 4 + 7) / 8 * 4;          // dwords per staged window row: whole pieces of 8 cells
     constexpr int LOWBUF = WROWS * CHK * LROW;               // dwords per low-res buffer
@@ -334,7 +340,7 @@ bwd_pixel_kernel(const Args<T> args) {
     }
 
     // ---- gradient of the logits; what the cell kernel needs to form it again ----
-    u32x4 whi[2][2], wlo[2][2];
+    u32x4 we[2][2][NP];
     NonFinite seen;
     float down[2][4];           // f16: what the results of child 4 g + v of block nb are multiplied by
     if (active) {
@@ -372,7 +378,7 @@ bwd_pixel_kernel(const Args<T> args) {
                 for (int k = 0; k < 16; ++k) e[k / 8][k % 8] *= f.up;
             }
 #pragma unroll
-            for (int s = 0; s < 2; ++s) split8<T>(e[s], whi[nb][s], wlo[nb][s]);
+            for (int s = 0; s < 2; ++s) split8<T>(e[s], we[nb][s]);
         }
     }
 
@@ -395,10 +401,9 @@ bwd_pixel_kernel(const Args<T> args) {
             for (int nb = 0; nb < 2; ++nb) {
                 f32x4 o = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-                for (int s = 0; s < 2; ++s) {
-                    o = Mma<T>::k32(whi[nb][s], b[s], o);
-                    o = Mma<T>::k32(wlo[nb][s], b[s], o);
-                }
+                for (int s = 0; s < 2; ++s)
+#pragma unroll
+                    for (int i = 0; i < NP; ++i) o = Mma<T>::k32(we[nb][s][i], b[s], o);
                 // (a key that is not finite makes its channel's results so for every child of the block)
                 if (nb == 0) seen.see(o[0]);
                 if (SCALED) {
@@ -506,6 +511,7 @@ bwd_cell_kernel(const Args<T> args) {
     const int B = args.B, d = args.d, C = args.C, H = args.H, W = args.W, tiles_x = args.tiles_x, tiles_y = args.tiles_y,
               nblocks = args.nblocks, per_xcd = args.per_xcd;
     constexpr bool SCALED = __is_same(T, f16_t);             // A and E are brought into the type's range (Fit)
+    constexpr int NP = pieces_of(ODD);
     __shared__ __attribute__((aligned(16))) u32 lds[CBUF * (CHI + CLOW) + CSTAT + 4 * COUT + 4];
     u32 *const hibuf = lds, *const lowbuf = lds + CBUF * CHI;
     const u32 hi_base = lds_address((const __attribute__((address_space(3))) u32 *)lds), low_at = hi_base + CBUF * CHI * 4;
@@ -596,7 +602,7 @@ bwd_cell_kernel(const Args<T> args) {
     // the gathered sum over this wave's 128 children of 16 channels: reduction step (qx, s) covers parent
     // rows 2 s and 2 s + 1 of the quadrant, in the order the weights are held in; element v of the
     // result: cell (row g, column v), channel i16
-    u32x4 whi[2][2], wlo[2][2];
+    u32x4 wp[2][2][NP];
     Fit f = {1.f, 1.f};         // f16: the factors of this lane's cell, the results' of cells (g, v)
     float down[4];
     auto hold = [&](float (&w)[2][2][8]) __attribute__((always_inline)) {
@@ -613,7 +619,7 @@ bwd_cell_kernel(const Args<T> args) {
 #pragma unroll
         for (int qx = 0; qx < 2; ++qx)
 #pragma unroll
-            for (int s = 0; s < 2; ++s) split8<T>(w[qx][s], whi[qx][s], wlo[qx][s]);
+            for (int s = 0; s < 2; ++s) split8<T>(w[qx][s], wp[qx][s]);
     };
     NonFinite seen;
     auto gather = [&](int j) __attribute__((always_inline)) {
@@ -625,8 +631,8 @@ bwd_cell_kernel(const Args<T> args) {
             for (int s = 0; s < 2; ++s) {
                 const u32x2 lo = *(const u32x2 *)(hb + gat_at[qx][2 * s]), hi = *(const u32x2 *)(hb + gat_at[qx][2 * s + 1]);
                 const u32x4 b = u32x4{lo[0], lo[1], hi[0], hi[1]};
-                o = Mma<T>::k32(whi[qx][s], b, o);
-                o = Mma<T>::k32(wlo[qx][s], b, o);
+#pragma unroll
+                for (int i = 0; i < NP; ++i) o = Mma<T>::k32(wp[qx][s][i], b, o);
             }
         // (what is not finite in a child makes its channel's results so for every cell of the block)
         seen.see(o[0]);
@@ -789,7 +795,7 @@ bwd_cell_kernel(const Args<T> args) {
                         const f32x4 dsum = child_stats(0, qx, nb);
 #pragma unroll
                         for (int v = 0; v < 4; ++v)
-                            w[qx][s][4 * k + v] = joined<T>(whi[qx][s], wlo[qx][s], 4 * k + v) * f.down * (acc[qx][nb][v] - dsum[v]);
+                            w[qx][s][4 * k + v] = joined<T>(wp[qx][s], 4 * k + v) * f.down * (acc[qx][nb][v] - dsum[v]);
                     }
             hold(w);
         }

@@ -52,16 +52,26 @@ __device__ __forceinline__ u32 pack2(float a, float b) {
     return __builtin_bit_cast(u32, __builtin_convertvector(f32x2{a, b}, tx2));
 }
 
-// 8 fp32 values as a 16-bit operand plus the operand of their remainders
-template <typename T>
-__device__ __forceinline__ void split8(const float *p, u32x4 &hi, u32x4 &lo) {
+// 8 fp32 values as a 16-bit operand plus the operands of the remainders: N in all
+template <typename T, int N>
+__device__ __forceinline__ void split8(const float *p, u32x4 (&o)[N]) {
     typedef T tx8 __attribute__((ext_vector_type(8)));
-    hi = u32x4{pack2<T>(p[0], p[1]), pack2<T>(p[2], p[3]), pack2<T>(p[4], p[5]), pack2<T>(p[6], p[7])};
-    const tx8 h = __builtin_bit_cast(tx8, hi);
     float r[8];
 #pragma unroll
-    for (int k = 0; k < 8; ++k) r[k] = p[k] - (float)h[k];
-    lo = u32x4{pack2<T>(r[0], r[1]), pack2<T>(r[2], r[3]), pack2<T>(r[4], r[5]), pack2<T>(r[6], r[7])};
+    for (int k = 0; k < 8; ++k) r[k] = p[k];
+#pragma unroll
+    for (int i = 0; i < N; ++i) {
+        o[i] = u32x4{pack2<T>(r[0], r[1]), pack2<T>(r[2], r[3]), pack2<T>(r[4], r[5]), pack2<T>(r[6], r[7])};
+        const tx8 h = __builtin_bit_cast(tx8, o[i]);
+#pragma unroll
+        for (int k = 0; k < 8; ++k) r[k] -= (float)h[k];
+    }
+}
+template <typename T>
+__device__ __forceinline__ void split8(const float *p, u32x4 &hi, u32x4 &lo) {
+    u32x4 o[2];
+    split8<T>(p, o);
+    hi = o[0], lo = o[1];
 }
 
 // f16 holds a pair of operands to 2^-25 only and nothing beyond 65504, whatever its values' own size: a set
@@ -83,11 +93,19 @@ __device__ __forceinline__ float over_groups(float m) {
     return fmaxf(m, __shfl_xor(m, 32));
 }
 
-// value k of a pair of operands made by split8
+// value k of the operands made by split8
+template <typename T, int N>
+__device__ __forceinline__ float joined(const u32x4 (&o)[N], int k) {
+    typedef T tx8 __attribute__((ext_vector_type(8)));
+    float v = (float)__builtin_bit_cast(tx8, o[N - 1])[k];
+#pragma unroll
+    for (int i = N - 2; i >= 0; --i) v += (float)__builtin_bit_cast(tx8, o[i])[k];
+    return v;
+}
 template <typename T>
 __device__ __forceinline__ float joined(u32x4 hi, u32x4 lo, int k) {
-    typedef T tx8 __attribute__((ext_vector_type(8)));
-    return (float)__builtin_bit_cast(tx8, hi)[k] + (float)__builtin_bit_cast(tx8, lo)[k];
+    const u32x4 o[2] = {hi, lo};
+    return joined<T>(o, k);
 }
 
 // a 4 x 4 block of 16-bit values out of LDS, transposed: lane L of a 16-lane block addresses 4

@@ -39,6 +39,24 @@ def test_gradients_of_odd_rows(dtype, B, d, C, H, W):
             assert rel <= bar and a.is_contiguous(), (needs, a.shape, rel)
 
 
+def test_weights_hold_fp32s_precision():
+    """Every cell in the window of one child with a query and a gradient: each of grad_value and grad_key is one weight
+    times a bf16 number, rounded once.  fp32 arithmetic puts less than 2^-12 of them on the other side of a rounding
+    (errors of 2^-20 at most, of a spacing of 2^-7 .. 2^-8); weights of 16 bits put more than 2^-11 there."""
+    B, d, C, H, W = 16, 16, 16, 50, 85
+    q, key, v, go = _operands(torch.bfloat16, B, d, C, H, W)
+    child = torch.zeros(2 * H, 2 * W, dtype=torch.bool, device='cuda')
+    child[4::10, 5::10] = True
+    q, go = q * child, go * child
+    wide = [t.double().requires_grad_() for t in (q, key, v)]
+    want = torch.autograd.grad(sapa_amd.sapa_fused(*wide, 5, 2), wide, go.double())
+    leaves = [t.clone().requires_grad_() for t in (q, key, v)]
+    got = torch.autograd.grad(sapa_amd.sapa_fused(*leaves, 5, 2), leaves, go)
+    for a, b in zip(got[1:], want[1:]):
+        differ = (a != b.bfloat16()).double().mean().item()
+        assert differ < 2.0 ** -12, differ
+
+
 def test_scratch_of_three_floats_per_pixel_does_not_serve_odd_rows():
     """The entry point whose scratch holds no padded copies refuses them and writes nothing."""
     q, key, v, go = _operands(torch.bfloat16, 1, 16, 16, 4, 17)
