@@ -166,6 +166,9 @@ int sapa_fused_backward(const void *grad_out, const void *query, const void *key
 int sapa_fused_forward_attn(const void *query, const void *key, const void *value,
                             void *attn, void *out, int B, int d, int C, int H, int W,
                             int K, int s, int dtype, void *stream);
+/* 1 where it aggregates 16-bit tensors with the fp32 weights (some sizes with an odd W)
+ * although the one-launch forward, which enters them into 16-bit products, serves them. */
+int sapa_fused_forward_attn_aggregates(int B, int C, int H, int W, int K, int s, int dtype);
 long long sapa_fused_backward_attn_workspace(int B, int H, int W, int K, int s);
 int sapa_fused_backward_attn(const void *grad_out, const void *query, const void *key,
                              const void *value, const void *attn, void *workspace,

@@ -45,6 +45,7 @@ SIGNATURES = {
     'sapa_fused_backward_direct': [_vp] * 8 + [_i] * 9 + [_vp],
     'sapa_fused_backward_direct_workspace': [_i] * 9,       # (a size)
     'sapa_fused_backward_direct_ws': [_vp] * 8 + [_i] * 9 + [_vp],
+    'sapa_fused_forward_attn_aggregates': [_i] * 7,
     'sapa_fused_forward_attn': [_vp, _vp, _vp, _vp, _vp, _i, _i, _i, _i, _i, _i, _i, _i, _vp],
     'sapa_fused_backward_attn': [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _i, _i, _i, _i, _i, _i, _i, _i, _vp],
     'sapa_qk_forward_nhwc': [_vp, _vp, _vp, _i, _i, _i, _i, _i, _i, _i, _vp],

@@ -412,6 +412,20 @@ int sapa_fused_backward_direct_ws(const void *grad_out, const void *query, const
                            grad_key, grad_value, B, d, C, H, W, K, s, channels_last, dtype, stream);
 }
 
+// The output of 16-bit tensors next to their weights comes from the one-launch forward where it runs on the matrix
+// instructions (its weights are the same fp32 softmax of the same fp32 sums): 208 us against
+// 285 for the aggregation with the fp32 weights at B=16, C=256, 100x168.  With odd W (low-res rows
+// through registers) not between 3.7 and 8.9 M value elements of at most 35000 cells, where that kernel's tiles
+// leave half of the chip idle: weights and output by the aggregation / the one launch, as parts of training steps with
+// the chain over the weights, bf16, d=64, 13 sizes in between 441 / 448 us (B=8, C=256, 51x83), 373 / 387 (16, 256,
+// 43x29), 269 / 283 (8, 128, 51x83) to equal; below, 230 / 227 (16, 128, 43x29), 154 / 151 (8, 64, 51x83), above
+// 455 / 433 (16, 256, 50x45), 1689 / 1595 (16, 256, 100x167), 369 / 359 (3, 128, 159x117)
+int sapa_fused_forward_attn_aggregates(int B, int C, int H, int W, int K, int s, int dtype) {
+    const long cells = (long)B * H * W;
+    return K == 5 && s == 2 && (dtype == SAPA_F16 || dtype == SAPA_BF16) && W % 2 != 0 && cells <= 35000 &&
+           cells * C > 7L << 19 && cells * C < 17L << 19;
+}
+
 int sapa_fused_forward_attn(const void *query, const void *key, const void *value, void *attn,
                             void *out, int B, int d, int C, int H, int W, int K, int s, int dtype,
                             void *stream) {
@@ -430,19 +444,9 @@ int sapa_fused_forward_attn(const void *query, const void *key, const void *valu
                                 st, true);
     SAPA_STAGE(e);
     if (!out) return SAPA_OK;
-    // the output of 16-bit tensors from the one-launch forward where it runs on the matrix
-    // instructions (its weights are the same fp32 softmax of the same fp32 sums): 208 us against
-    // 285 for the aggregation with the fp32 weights at B=16, C=256, 100x168.  With odd W (low-res rows
-    // through registers) not between 3.7 and 8.9 M value elements of at most 35000 cells, where that kernel's tiles
-    // leave half of the chip idle: training steps with the aggregation / the one launch, bf16, d=64, 13 sizes in between
-    // 441 / 448 us (B=8, C=256, 51x83), 373 / 387 (16, 256, 43x29), 269 / 283 (8, 128, 51x83) to equal; below,
-    // 230 / 227 (16, 128, 43x29), 154 / 151 (8, 64, 51x83), above 455 / 433 (16, 256, 50x45), 1689 / 1595 (16, 256,
-    // 100x167), 369 / 359 (3, 128, 159x117)
-    const long cells = (long)B * H * W;
-    const bool aggregate = W % 2 != 0 && cells <= 35000 && cells * C > 7L << 19 && cells * C < 17L << 19;
     e = hipErrorNotSupported;
 #ifndef SAPA_WMAT16_OFF
-    if (!aggregate) e = sapa_b_wmat16_launch(TILED_FUSED, query, key, value, out, B, d, C, H, W, K, s, dtype, st);
+    if (!sapa_fused_forward_attn_aggregates(B, C, H, W, K, s, dtype)) e = sapa_b_wmat16_launch(TILED_FUSED, query, key, value, out, B, d, C, H, W, K, s, dtype, st);
 #endif
     if (e == hipErrorNotSupported)
         e = sapa_b_tiled_launch(TILED_AV, nullptr, nullptr, attn, value, out, B, 0, C, H, W, K, s, dtype, st, true);

@@ -385,18 +385,23 @@ class SAPAFusedFunction(Function):
         output = _lib.new_out(value, (n, c, h * scale_factor, w * scale_factor), nhwc)
         # (who says where the weights come from gets gradients that chain over them)
         ctx.direct = save_attention is None or nhwc
+        keep, passing = save_attention, False
         if save_attention is None:
-            save_attention = SAVE_ATTENTION and not (
-                wants_grad and _direct_serves(query, key, value, kernel_size, scale_factor, nhwc))
-        if wants_grad and not nhwc and save_attention:
+            keep = SAVE_ATTENTION
+            if wants_grad and keep and _direct_serves(query, key, value, kernel_size, scale_factor, nhwc):
+                # (weights that need not be kept are still aggregated with in fp32 where kept ones would be: the
+                # one-launch forward holds them in two 16-bit operands; B=8, C=256, 51x83 in bf16 250 us a step, 192 so)
+                keep, passing = False, not nhwc and bool(_lib.lib().sapa_fused_forward_attn_aggregates(
+                    n, c, h, w, kernel_size, scale_factor, _lib.dtype_code(value)))
+        if wants_grad and not nhwc and (keep or passing):
             attn = torch.empty((n, kernel_size * kernel_size, h * scale_factor, w * scale_factor),
                                dtype=torch.float32, device=value.device)
             status = _lib.call_status('sapa_fused_forward_attn', value.device, _lib.ptr(query), _lib.ptr(key),
                                       _lib.ptr(value), _lib.ptr(attn), _lib.ptr(output), n, d, c, h, w,
                                       kernel_size, scale_factor, _lib.dtype_code(value))
             if status != _lib.UNSUPPORTED:
-                ctx.has_attn = True
-                ctx.save_for_backward(*(saved + (attn,)))
+                ctx.has_attn = bool(keep)
+                ctx.save_for_backward(*(saved + (attn,) if keep else saved))
                 return output
             del attn
         if wants_grad:

@@ -66,3 +66,16 @@ def test_scratch_of_three_floats_per_pixel_does_not_serve_odd_rows():
     status = _lib.call_status('sapa_fused_backward_direct', q.device, *args, 1, 16, 16, 4, 17, 5, 2, 0,
                               _lib.dtype_code(q))
     assert status == _lib.UNSUPPORTED and all(bool((t == 7.0).all()) for t in grads)
+
+
+@pytest.mark.parametrize('dtype', [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize('B,C,H,W', [(16, 256, 43, 29), (8, 128, 51, 83), (4, 64, 51, 83), (16, 128, 43, 29)])
+def test_training_output_of_odd_rows_as_with_kept_weights(dtype, B, C, H, W):
+    """The output of a training step is, bit for bit, that of the one that keeps its fp32 weights, both where it is
+    aggregated with them (the first two sizes) and where it comes from the one-launch forward."""
+    q, key, v, _ = _operands(dtype, B, 32, C, H, W)
+    leaves = [t.requires_grad_() for t in (q, key, v)]
+    out = sapa_amd.sapa_fused(*leaves, 5, 2)
+    kept = sapa_amd.sapa_fused(*leaves, 5, 2, save_attention=True)
+    assert torch.equal(out, kept)
+    assert not any(t.size(1) == 25 for t in out.grad_fn.saved_tensors)
