@@ -211,6 +211,8 @@ def _direct_scratch(query, key, value, K, s, nhwc):
     if not (value.dtype in (torch.float16, torch.bfloat16) and query.dtype == key.dtype == value.dtype):
         return 0
     n, c, h, w = value.size()
+    if not nhwc and w % 2 and query.data_ptr() % 16:
+        return 0            # (read in pieces of 16 bytes; its weights are kept by the forward pass)
     return _lib.lib().sapa_fused_backward_direct_workspace(n, key.size(1), c, h, w, K, s, int(nhwc), _lib.dtype_code(value))
 
 
@@ -231,6 +233,8 @@ def _direct_backward(grad_output, query, key, value, K, s, needs):
         return None
     grad_output = _lib.layout_copy(grad_output, nhwc)
     n, c, h, w = value.size()
+    if not nhwc and w % 2 and grad_output.data_ptr() % 16:
+        grad_output = grad_output.clone()       # (it is read in pieces of 16 bytes)
     scratch = torch.empty(nbytes, dtype=torch.uint8, device=value.device)
     grads = [_lib.new_out(t, channels_last=nhwc) if need else None for t, need in zip((query, key, value), needs)]
     status = _lib.call_status('sapa_fused_backward_direct_ws', value.device, _lib.ptr(grad_output), _lib.ptr(query),
@@ -339,7 +343,7 @@ class SAPAFusedFunction(Function):
     """av(softmax(qk(query, key), dim=1), value) -- SAPA.attention
     (sapa_base.py:38-40) -- as one launch in the forward pass.  The gradients of
     16-bit operands that sapa_fused_backward_direct_ws serves come straight from them
-    (nothing kept, no K*K tensor at any time), unless the call says where its
+    (nothing kept; no K*K tensor but in the forward pass of some sizes with odd rows), unless the call says where its
     attention weights are to come from: with save_attention=True the
     forward pass runs as two launches that leave the fp32 weights
     [B,K*K,sH,sW] behind for the backward pass, as the reference's autograd graph

@@ -79,3 +79,35 @@ def test_training_output_of_odd_rows_as_with_kept_weights(dtype, B, C, H, W):
     kept = sapa_amd.sapa_fused(*leaves, 5, 2, save_attention=True)
     assert torch.equal(out, kept)
     assert not any(t.size(1) == 25 for t in out.grad_fn.saved_tensors)
+
+
+def _behind(t, k):
+    """t's values behind k others."""
+    return torch.empty(t.numel() + k, dtype=t.dtype, device=t.device)[k:].copy_(t.reshape(-1)).view_as(t)
+
+
+def test_tensors_that_begin_anywhere(monkeypatch):
+    """Key, value and the output's gradient: the same gradients from the operands, also from the middle of a dword on.
+    A query between two 16-byte pieces: the forward pass keeps the weights, and the backward pass chains over them."""
+    q, key, v, go = _operands(torch.bfloat16, 2, 17, 33, 9, 33)
+    names, call = [], _lib.call_status
+    monkeypatch.setattr(_lib, 'call_status', lambda name, *a: names.append(name) or call(name, *a))
+
+    def step(q, key, v, go):
+        names.clear()
+        leaves = [t.detach().requires_grad_() for t in (q, key, v)]
+        out = sapa_amd.sapa_fused(*leaves, 5, 2)
+        return (out,) + torch.autograd.grad(out, leaves, go), list(names)
+    want, route = step(q, key, v, go)
+    assert route == ['sapa_fused_backward_direct_ws']
+    for k, at in ((1, 1), (1, 2), (1, 3), (4, 3)):
+        ops = [q, key, v, go]
+        ops[at] = _behind(ops[at], k)
+        got, route = step(*ops)
+        assert route == ['sapa_fused_backward_direct_ws']
+        # (the output's low-res rows come through another kernel where they begin inside a dword)
+        assert all(torch.equal(a, b) for a, b in zip(got[1:], want[1:]))
+    got, route = step(_behind(q, 4), key, v, go)
+    assert route == ['sapa_fused_forward_attn', 'sapa_fused_backward_attn']
+    bar = torch.finfo(q.dtype).eps / 2 / 3 ** 0.5 * 1.2 * 2         # (one rounding of each)
+    assert all(((a.double() - b.double()).norm() / b.double().norm()).item() <= bar for a, b in zip(got, want))
