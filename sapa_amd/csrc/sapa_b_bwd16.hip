@@ -74,10 +74,11 @@ pad_rows_kernel(const unsigned short *__restrict__ a, const unsigned short *__re
         const u32 x = 4 * (u32)(i - row * pieces);           // first dword
         const unsigned short *const p = src + row * w + 2 * x;
         u32 *const o = dst + row * per_row + x;
-        if (x + 4 < per_row) {
+        const bool half = (uintptr_t)p % 4 != 0;
+        // (a tensor may begin in the middle of a dword: nothing in front of it is read)
+        if (x + 4 < per_row && !(half && i == 0)) {
             // (cells 2 x .. 2 x + 7 and one more are the row's own)
             typedef u32x4 __attribute__((aligned(4))) u32x4_a4;
-            const bool half = (uintptr_t)p % 4 != 0;
             const u32 *const q = (const u32 *)(p - half);
             const u32x4 v = *(const u32x4_a4 *)q;
             const u32 next = half ? q[4] : 0u;
@@ -85,7 +86,7 @@ pad_rows_kernel(const unsigned short *__restrict__ a, const unsigned short *__re
                                           __builtin_amdgcn_alignbit(v[3], v[2], 16), __builtin_amdgcn_alignbit(next, v[3], 16)}
                                   : v;
         } else {
-            for (u32 k = 0; k < per_row - x; ++k) o[k] = p[2 * k] | (2 * (x + k) + 1 < (u32)w ? (u32)p[2 * k + 1] << 16 : 0u);
+            for (u32 k = 0; k < 4 && k < per_row - x; ++k) o[k] = p[2 * k] | (2 * (x + k) + 1 < (u32)w ? (u32)p[2 * k + 1] << 16 : 0u);
         }
     }
 }
