@@ -5,6 +5,7 @@ import torch
 import sapa_amd
 from sapa_amd import _lib
 from sapa_amd.sapa_func import _direct_serves
+from test_gpu_fused16_range import exact_gradients, gradients, one_rounding, rel, same_non_finite
 
 pytestmark = pytest.mark.gpu
 
@@ -55,6 +56,25 @@ def test_weights_hold_fp32s_precision():
     for a, b in zip(got[1:], want[1:]):
         differ = (a != b.bfloat16()).double().mean().item()
         assert differ < 2.0 ** -12, differ
+
+
+@pytest.mark.parametrize('dtype', [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize('value', [float('nan'), float('inf')])
+@pytest.mark.parametrize('which', [0, 1, 2, 3])
+@pytest.mark.parametrize('C,H,W', [(40, 11, 23), (33, 9, 67)])
+def test_non_finite_values_stay_where_they_belong(C, H, W, which, value, dtype):
+    """Results that are stored half a dword over and formed again term by term behind it: at the ends of rows and
+    images, one tile of cell blocks and several."""
+    *ops, go = _operands(dtype, 2, 24, C, H, W)
+    t = (*ops, go)[which]
+    t[0, 3, 5, 0] = value
+    t[1, 7, -1, -1] = value
+    t[1, 2, 4, t.size(3) // 2] = -value
+    assert _direct_serves(*ops, 5, 2, False)
+    for got, want in zip(gradients(ops, go), exact_gradients(ops, go)[1:]):
+        assert same_non_finite(got, want)
+        ok = torch.isfinite(want)
+        assert rel(got[ok], want[ok]) <= one_rounding(dtype)
 
 
 def test_scratch_of_three_floats_per_pixel_does_not_serve_odd_rows():
