@@ -7,7 +7,7 @@ import sapa_amd
 pytestmark = pytest.mark.gpu
 
 
-# (slices of 8 channels, the last of 5; of 12, the last of 10; one slice of all; a single channel)
+# (slices of 8 channels, the last of 5; of 16, the last of 2; of 20, the last of 13; a single channel)
 @pytest.mark.parametrize('B,C,H,W', [(1, 37, 21, 70), (8, 130, 29, 47), (16, 33, 50, 84), (1, 1, 24, 50)])
 @pytest.mark.parametrize('dtype', [torch.float32, torch.bfloat16])
 def test_every_channel_of_every_slice(dtype, B, C, H, W):
