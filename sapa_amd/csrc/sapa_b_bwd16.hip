@@ -34,9 +34,10 @@
 // Measured (B=16, C=256, d=64, 100x168, bf16): pixel kernel 295 us, cell kernel 429 us, a training step
 // 970 us against 1211 for the chain over K * K tensors (similarity and its softmax backward 274 us,
 // grad_q 92, grad_value and grad_key by vector fmas 544, the weights 86).  Odd W: key and value are copied into rows
-// of an even number of cells first (direct loads begin on dwords); B=16, 100x167 1592 -> 1206 us for a step (1171 with
-// pairs), of which the copies 108 and the cell kernel, of pairs, 503 (hi-res pieces across cache lines, results moved by
-// half a dword; 560 with a 2-byte store per result); B=8, d=64, 51x83 412 -> 192, B=4, C=512, d=32, 97x165 915 -> 551.
+// of an even number of cells first (direct loads begin on dwords); B=16, 100x167 1593 -> 1193 us for a step (1166 with
+// pairs), of which the copies 98 and the cell kernel 526 (hi-res pieces across cache lines, results moved by half a
+// dword; of pairs 503, and 560 with a 2-byte store per result); B=4, C=512, d=32, 97x165 911 -> 543; B=8, d=64, 51x83
+// 409 -> 242, with 100 for a forward pass that aggregates with fp32 weights (175 with pairs and the one-launch forward).
 // The third operand costs the cell kernel 8 registers spilled in bf16, 16 in fp16.
 #include "wm16_exact.hpp"
 
@@ -61,7 +62,7 @@ template <typename T> struct Args {
 
 // Rows of w 16-bit cells -> rows of w + 1 (w odd), the added cell 0; two tensors in one launch.  A thread moves 4
 // dwords of a row, from the dword before where the row begins in the middle of one (B=16, d=64, C=256,
-// 100x167: 108 us = 3.2 TB/s; 131 with a thread per dword).
+// 100x167: 98 us = 3.5 TB/s; 131 with a thread per dword).
 __global__ __launch_bounds__(256) void
 pad_rows_kernel(const unsigned short *__restrict__ a, const unsigned short *__restrict__ b, u32 *__restrict__ pa,
                 u32 *__restrict__ pb, long rows_a, long rows_b, int w) {

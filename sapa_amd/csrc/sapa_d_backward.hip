@@ -238,8 +238,8 @@ hipError_t deform_fused_backward_launch(const void *grad_out, const void *q, con
         const long esize = wide ? 2 : 4;
         char *key_cl = rest, *value_cl = rest + align256((long)B * Cq * lpix * esize);
         // 16-bit tensors at s = 2: all four gradients in one kernel, which adds into the channels-last
-        // accumulators (faster than the three below at every size: B=16, C=64, 20x20, 9 points 252 -> 149 us for a
-        // training step, B=1, C=256, 180x190 887 -> 661; single small images are bound by the host, 149 -> 143)
+        // accumulators (faster than the three below at every size: B=16, C=64, 20x20, 9 points 252 -> 150 us for a
+        // training step, B=1, C=256, 180x190 873 -> 634; single small images are bound by the host, 149 -> 143)
         if (deform_bwd_region16_serves(B, Cq, C, H, W, P, s, G, dtype) &&
             ((uintptr_t)grad_out | (uintptr_t)q | (uintptr_t)offset | (uintptr_t)grad_q | (uintptr_t)grad_offset) % 4 == 0) {
             SAPA_STEP(nchw_to_nhwc_launch(key, key_cl, Cq, value, value_cl, C, B, lpix, (int)esize, st,

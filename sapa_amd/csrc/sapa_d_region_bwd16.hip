@@ -24,11 +24,11 @@
 // strip, not once per 16 x 16 pixels (a form of this kernel on such squares, windows whole in LDS: 9 us
 // per square in front of its first step, 115 us of 665 for the additions).
 //
-// Measured (B=8, C=256, 4 groups, d=32, 64x64 -> 128x128, bf16): this part of a training step 780 -> 470 us with
-// 25 points (step 1033 -> 718), 560 -> 330 with 9 (811 -> 574); C=128, 90x121, 9 points, channels-last
-// 1634 -> 1106 (whole step).  What bounds it is the chain of a step's three phases, each behind a barrier
-// with the 16 waves that one CU's LDS holds (of 470: A 35, B 150, C 175, memory 60, barriers 50): half
-// the vector instructions that it issues at the most, a tenth of the matrix rate, 1 TB/s.
+// Measured (B=8, C=256, 4 groups, d=32, 64x64 -> 128x128, bf16): this kernel 457 us with 25 points and 379 with 9, a
+// training step 1016 -> 693 and 800 -> 551; C=128, 90x121, 9 points, channels-last 2600 -> 1712.  What bounds it is
+// the chain of a step's three phases, each behind a barrier with the 16 waves that one CU's LDS holds (timed apart
+// in a form of 470 us: A 35, B 150, C 175, memory 60, barriers 50): 54 % of the vector instructions that it could
+// issue, a tenth of the matrix rate, 1 TB/s.
 //
 // Numerics: products of 16-bit values are exact in fp32, sums are fp32.  The integers (30 bits of a row's
 // largest possible sum; Wg's scaled by a power of two per pixel) enter the products as three 16-bit
