@@ -460,8 +460,10 @@ __device__ __forceinline__ f32x4 mma32(u32x4 a, u32x4 b, f32x4 c) {
 // to channels-last 8), 512 -> 32 2 to 5, 64 -> 64 2 to 11, 128 -> 64 from planes 11 and from channels-last
 // features 19 registers.
 // The tiles of a workgroup: wave after wave, so that the waves read neighbouring pieces of a plane (a plane of no whole
-// cache lines is otherwise read twice at every piece's end: 128 -> 128, 3 images 150x134 28.3 -> 22.1 us); eight waves
-// on channels-last features a run of them each (neighbouring tiles: 64 -> 32, one image 32x32 4.05 -> 4.6 us).
+// cache lines is otherwise read twice at every piece's end: 128 -> 128, 3 images 150x134 28.3 -> 22.1 us, 14 images 66x82
+// 41.7 -> 33.1); eight waves on planes of whole lines or on channels-last features a run of them each (neighbouring
+// tiles: 256 -> 64, 8 images 128x128 38.3 -> 43.0 us, 256 -> 128, 4 images 31.3 -> 34.3; channels-last 64 -> 32, one
+// image 32x32 4.05 -> 4.6).
 template <int C, int O, bool IN_CL, bool OUT_CL, bool WIDE, int NW>
 __global__ void __launch_bounds__(64 * NW)
 project32_kernel(const float *__restrict__ x, const float *__restrict__ w, const float *__restrict__ bias,
@@ -488,12 +490,12 @@ project32_kernel(const float *__restrict__ x, const float *__restrict__ w, const
 
     const long ntiles = (HW + 31) / 32;
     // tiles t0, t0 + stride .. below t1 (waves past `waves` help with the weights only)
-    constexpr bool NEIGHBOURS = !IN_CL || NW > 8;
+    const bool neighbours = NW > 8 || (!IN_CL && HW % 32 != 0);
     const long first = (long)blockIdx.x * waves * tiles_per_wave, last = first + (long)waves * tiles_per_wave;
-    const long t0 = NEIGHBOURS ? first + wave : ((long)blockIdx.x * waves + wave) * tiles_per_wave;
-    const long t1 = wave >= waves ? t0 : NEIGHBOURS ? (last < ntiles ? last : ntiles)
+    const long t0 = neighbours ? first + wave : ((long)blockIdx.x * waves + wave) * tiles_per_wave;
+    const long t1 = wave >= waves ? t0 : neighbours ? (last < ntiles ? last : ntiles)
                                                     : (t0 + tiles_per_wave < ntiles ? t0 + tiles_per_wave : ntiles);
-    const long stride = NEIGHBOURS ? waves : 1;
+    const long stride = neighbours ? waves : 1;
     const int r16 = lane & 15, kg = lane >> 4;    // row / column of a 16 x 16 tile, k group
     float bv[NT];
 #pragma unroll
@@ -747,13 +749,16 @@ static hipError_t launch32_co(const void *x, const void *w, const void *bias, vo
     const Spread s8 = spread32(ntiles, sets, 8), s12 = spread32(ntiles, sets, 12);
     // Twelve waves where they shorten a wave's chain of tiles to what is asked for below (eight have twice the steps of
     // x in flight and no bar to moving work between steps).  us with 8 / 12 waves, from planes: 5 tiles to 3 each
-    // (256 -> 64, 16 images 100x168) 66 / 60, 7 to 5 (128 -> 144, 8 images 128x128) 42.7 / 40.5, but 4 to 3
-    // (256 -> 400, 8 images 64x64) 45.3 / 46.5; from channels-last features 5 to 3 (256 -> 64) 64.9 / 61.9, but 7 to 5
-    // (256 -> 288, 14 images 72x68) 70 / 74 and, spilling, 5 to 3 at 128 -> 64 37 / 38.5 .. 42; 128 -> 32 with 2 tiles
-    // to 1 (16 images 50x84) 11.7 / 14.1.  Tenths of eight waves' tiles per tile of twelve waves:
-    constexpr int ASKED = C == 128 && O == 32 ? 1 << 20 : !IN_CL ? 14 : C == 128 ? 20 : 15;
-    // (and 256 -> 64 from channels-last features over one tile each for 3 to 6 waves: 8 images 64x64 13.9 / 12.5)
-    if (10 * s8.per >= ASKED * s12.per || (IN_CL && C == 256 && O == 64 && s8.per == 1 && s8.waves > 2 && s8.waves <= 6))
+    // (256 -> 64, 16 images 100x168) 66 / 60, 3 to 2 (256 -> 288, 8 images 64x64) 41.8 / 38.6, but 4 to 3
+    // (256 -> 400, 8 images 64x64) 45.3 / 46.5 and 11 to 8 (14 images 66x82, 800 outputs) 160 / 187 of 128 channels, 242 / 265
+    // of 256; from channels-last features 5 to 3 (256 -> 64) 64.9 / 61.9, but 7 to 5 (256 -> 288, 14 images 72x68) 70 / 74
+    // and, spilling, 5 to 3 at 128 -> 64 37 / 38.5 .. 42; of 64 channels 5 to 3 (64 -> 64, 16 images 100x168) 24.7 / 23.6, 9
+    // to 6 (64 -> 800, 16 images 50x84) 70.7 / 73.3; 128 -> 32 with 2 tiles to 1 (16 images 50x84) 11.7 / 14.1.  Tenths
+    // of eight waves' tiles per tile of twelve waves:
+    constexpr int ASKED = C == 128 && O == 32 ? 1 << 20 : !IN_CL ? 15 : C == 128 ? 20 : C == 64 ? 16 : 15;
+    // (of 64 channels not to a single tile: 2 images 192x192, 64 -> 32 / 64, 7.7 / 8.3 and 10.1 / 10.8; 256 -> 64 from
+    // channels-last features also over one tile each for 3 to 6 waves: 8 images 64x64 13.9 / 12.5)
+    if ((10 * s8.per >= ASKED * s12.per && (C > 64 || s12.per > 1)) || (IN_CL && C == 256 && O == 64 && s8.per == 1 && s8.waves > 2 && s8.waves <= 6))
         return launch32_waves<C, O, IN_CL, OUT_CL, WIDE, C == 128 && O == 32 ? 8 : 12>(x, w, bias, out, B, HW, st, outputs, s12);
     return launch32_waves<C, O, IN_CL, OUT_CL, WIDE, 8>(x, w, bias, out, B, HW, st, outputs, s8);
 }

@@ -35,9 +35,10 @@ def test_both_numbers_of_waves(B, C, O, H, W):
 
 
 # (eight waves on channels-last features: runs of 2 tiles of each of 8 waves, and of 3 tiles of 7 waves, a ragged last tile
-# in both; weights shared by the images: 7 of 8 waves; 12 waves and a last block of 8 outputs; planes of no whole lines)
+# in both; weights shared by the images: 7 of 8 waves; 12 waves and a last block of 8 outputs; planes of no whole lines;
+# planes of whole lines, runs of 2 tiles of 7 waves)
 @pytest.mark.parametrize('B,C,O,H,W', [(16, 128, 32, 50, 84), (9, 128, 32, 100, 169), (2, 512, 72, 100, 168), (2, 256, 264, 100, 168),
-                                       (3, 64, 40, 150, 134)])
+                                       (3, 64, 40, 150, 134), (8, 64, 160, 64, 64)])
 def test_runs_of_tiles_and_shared_weights(B, C, O, H, W):
     """As above; weights shared by the images through project_shared."""
     if O == 32:
