@@ -24,10 +24,10 @@
 // strip, not once per 16 x 16 pixels (a form of this kernel on such squares, windows whole in LDS: 9 us
 // per square in front of its first step, 115 us of 665 for the additions).
 //
-// Measured (B=8, C=256, 4 groups, d=32, 64x64 -> 128x128, bf16): this kernel 457 us with 25 points and 379 with 9, a
-// training step 1016 -> 693 and 800 -> 551; C=128, 90x121, 9 points, channels-last 2600 -> 1712.  What bounds it is
+// Measured (B=8, C=256, 4 groups, d=32, 64x64 -> 128x128, bf16): this kernel 427 us with 25 points and 351 with 9, a
+// training step 656 and 536, by the chain before 1016 and 800; C=128, 90x121, 9 points, channels-last 2600 -> 1712.  What bounds it is
 // the chain of a step's three phases, each behind a barrier with the 16 waves that one CU's LDS holds (timed apart
-// in a form of 470 us: A 35, B 150, C 175, memory 60, barriers 50): 54 % of the vector instructions that it could
+// in a form of 470 us, whose 60 for memory are no more waited for: A 35, B 150, C 175, barriers 50): 54 % of the vector instructions that it could
 // issue, a tenth of the matrix rate, 1 TB/s.
 //
 // Numerics: products of 16-bit values are exact in fp32, sums are fp32.  The integers (30 bits of a row's
@@ -164,15 +164,12 @@ deform_bwd_region16_kernel(const BwdArgs<T> A) {
     }
     // (columns behind a row's end are the next row's)
     const bool tail = hires && x0 + 4 * uj + 2 >= hW;
-    u32x4 hr = {0u, 0u, 0u, 0u};
-    u32x2 ofr = {0u, 0u};
-    // (both loads of the window row: one of them is out of range; a branch would wait for what is in flight)
-    auto load_row = [&](int gy) __attribute__((always_inline)) {
-        const bool ok = gy >= 0 && gy < H;
-        const u32 row = ok ? (u32)(gy * W) * 2u : 0u;           // (no row beside the image is ever an offset)
-        const u32x4 a = __builtin_amdgcn_raw_buffer_load_b128(rsa, ok ? offa : OUTSIDE, row * (u32)Cq, 0);
-        const u32x4 b = __builtin_amdgcn_raw_buffer_load_b128(rsb, ok ? offb : OUTSIDE, row * (u32)C, 0);
-        return u32x4{a[0] | b[0], a[1] | b[1], a[2] | b[2], a[3] | b[3]};
+    // A step's loads as they leave them.  Whatever joins two of them or moves one waits for it, and is done where they
+    // are put into LDS; and all waves issue the same two loads, of which those of pixels use half, or registers
+    // would be moved where the branches meet (each step waited for its own requests then, and for the stores
+    // of the step before: the kernel 454 us, 426 so).
+    struct Fetched {
+        u32x4 a, b;                 // pixels, offsets; or a piece of the key, of the value (one of them zeros)
     };
     auto put_piece = [&](int row, u32x4 v) __attribute__((always_inline)) {
         const int at = (int)((u32)((p0 + row) * WWX + pwl) % RING);
@@ -183,26 +180,23 @@ deform_bwd_region16_kernel(const BwdArgs<T> A) {
             *(u32x4 *)(Vl + at * VSB + pc8) = v;
         }
     };
-    auto fetch = [&](int step) __attribute__((always_inline)) {
-        if (hires) {
-            // (all of the offset in the lane's part, which the descriptor's check is made for dword by dword: where
-            // a row ends two pixels into a piece, the tensor's last one runs over its end)
-            const u32 so = (u32)(step * 4 * hW);
-            const bool ok = step < nstep;
-            const u32x2 v = __builtin_amdgcn_raw_buffer_load_b64(rsa, ok ? offa + so : OUTSIDE, 0, 0);
-            ofr = __builtin_amdgcn_raw_buffer_load_b64(rsb, ok ? offb + so : OUTSIDE, 0, 0);
-            hr[0] = v[0], hr[1] = v[1];
-        } else {
-            hr = load_row(step + AHEAD - 1 < nstep + 2 * RCH + 1 ? wy0 + step + AHEAD - 1 : -1);
-        }
+    auto fetch = [&](int step, Fetched &f) __attribute__((always_inline)) {
+        // (pixels: all of the offset in the lane's part, which the descriptor's check is made for dword by dword: where
+        // a row ends two pixels into a piece, the tensor's last one runs over its end)
+        const u32 lane_part = hires ? (u32)(step * 4 * hW) : 0u;
+        const int gy = step + AHEAD - 1 < nstep + 2 * RCH + 1 ? wy0 + step + AHEAD - 1 : -1;
+        const bool ok = hires ? step < nstep : gy >= 0 && gy < H;
+        const u32 row = !hires && ok ? (u32)(gy * W) * 2u : 0u;  // (no row beside the image is ever an offset)
+        f.a = __builtin_amdgcn_raw_buffer_load_b128(rsa, ok ? offa + lane_part : OUTSIDE, row * (u32)Cq, 0);
+        f.b = __builtin_amdgcn_raw_buffer_load_b128(rsb, ok ? offb + lane_part : OUTSIDE, row * (u32)C, 0);
     };
-    auto put = [&](int step) __attribute__((always_inline)) {
+    auto put = [&](int step, const Fetched &f) __attribute__((always_inline)) {
         const int buf = step & 1;
         if (hires) {
-            if (tail) hr[1] = 0u;
+            const u32 hr[2] = {f.a[0], tail ? 0u : f.a[1]};
             if (!isq) {
                 *(u32x2 *)(Dl[buf] + uch * PXS + upos) = u32x2{hr[0], hr[1]};
-                *(u32x2 *)(Of[buf] + uch * OFS + upos) = ofr;
+                *(u32x2 *)(Of[buf] + uch * OFS + upos) = u32x2{f.b[0], f.b[1]};
             } else {
                 *(u32x2 *)(Ql[buf] + uch * PXS + upos) = u32x2{hr[0], hr[1]};
             }
@@ -213,7 +207,7 @@ deform_bwd_region16_kernel(const BwdArgs<T> A) {
                 atomicOr(&badpx[buf], m << upos);
             }
         } else if (pwl < WWX) {
-            put_piece(step + AHEAD - 1, hr);
+            put_piece(step + AHEAD - 1, u32x4{f.a[0] | f.b[0], f.a[1] | f.b[1], f.a[2] | f.b[2], f.a[3] | f.b[3]});
         }
     };
 
@@ -246,7 +240,8 @@ deform_bwd_region16_kernel(const BwdArgs<T> A) {
             const int u = i * NTB + t, cp = cell_pix(u >> 3), c8 = 8 * (u & 7);
             vw[i] = __builtin_amdgcn_raw_buffer_load_b128(vr, cp >= 0 && c8 < cg ? (u32)((cp * C + g * cg + c8) * 2) : OUTSIDE, 0, 0);
         }
-        if (hires) fetch(0);
+        Fetched f;
+        if (hires) fetch(0, f);
         __syncthreads();            // (the flags are clear)
         bool bad = false;
 #pragma unroll
@@ -261,7 +256,7 @@ deform_bwd_region16_kernel(const BwdArgs<T> A) {
             if (u < NPC * 8) *(u32x4 *)(Vl + (c00 + (u >> 3)) % RING * VSB + 8 * (u & 7)) = vw[i];
         }
         if (bad) kbad = 1;
-        if (hires) put(0);
+        if (hires) put(0, f);
     }
     __syncthreads();
 
@@ -328,7 +323,8 @@ deform_bwd_region16_kernel(const BwdArgs<T> A) {
 
     for (int step = 0; step < nstep; ++step) {
         const int buf = step & 1;
-        fetch(step + 1);
+        Fetched next;
+        fetch(step + 1, next);
         const int base = band_base(p0 + step), cb0 = base / 16;
         const bool exact_q = kbad != 0;
 
@@ -643,9 +639,10 @@ deform_bwd_region16_kernel(const BwdArgs<T> A) {
                 __builtin_amdgcn_raw_buffer_store_b32(v[1], r, off == OUTSIDE || tail ? OUTSIDE : at + 4, 0, 0);
             }
         };
+        // (the store behind the loads that it does not wait for)
+        put(step + 1, next);
         if (want_o && wave < 8)
             store(args()->grad_offset + oplane * hpl, 2L * P * hpl * 2, offb, *(const u32x2 *)(Of[buf] + uch * OFS + upos));
-        put(step + 1);
         __syncthreads();
         if (any_fb) {
             if (fbq && want_q) {
