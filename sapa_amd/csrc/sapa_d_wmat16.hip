@@ -262,7 +262,9 @@ deform_fused_wmat16_kernel(const T *__restrict__ q, const T *__restrict__ key,
     u32x4 qa[NCHW ? 1 : NMB][DP / 32];
     constexpr int QN = NCHW ? NPX * DP / 2 / NT : 1;     // pixel pairs per thread
     static_assert(!NCHW || (NPX * DP / 2) % NT == 0, "the q tile divides over the threads");
-    u32 qraw[QN];
+    // (as loaded, the second pixel's element in a register of its own where pairs are no dwords: taken apart where
+    // they are loaded, they and the key window requested before them would be waited for there)
+    u32 qraw[QN], qodd[QN];
     const bool q32 = hW % 2 == 0 && (uintptr_t)q % 4 == 0;           // pairs are aligned dwords
     auto load_q = [&](int g) __attribute__((always_inline)) {
         if (NCHW) {
@@ -271,18 +273,12 @@ deform_fused_wmat16_kernel(const T *__restrict__ q, const T *__restrict__ key,
                 const int item = i * NT + tid;
                 const int ch = item / (NPX / 2), pr = item % (NPX / 2);
                 const int qh = y0 + pr / (TW / 2), qw = x0 + 2 * (pr % (TW / 2));
-                qraw[i] = 0u;
+                qraw[i] = qodd[i] = 0u;
                 if (ch < d && qh < hH && qw < hW) {
                     const T *qp = q + ((long)n * Cq + g * d + ch) * hpl + (long)qh * hW + qw;
-                    if (q32) {
-                        qraw[i] = *(const u32 *)qp;
-                    } else {
-                        union { T h[2]; u32 u; } x;
-                        x.u = 0u;
-                        x.h[0] = qp[0];
-                        if (qw + 1 < hW) x.h[1] = qp[1];
-                        qraw[i] = x.u;
-                    }
+                    if (!q32 && qw + 1 < hW) qodd[i] = *(const unsigned short *)(qp + 1);
+                    if (q32) qraw[i] = *(const u32 *)qp;
+                    else qraw[i] = *(const unsigned short *)qp;
                 }
             }
         } else {
@@ -306,10 +302,20 @@ deform_fused_wmat16_kernel(const T *__restrict__ q, const T *__restrict__ key,
             const int item = i * NT + tid;
             const int ch = item / (NPX / 2), pr = item % (NPX / 2);
             const int pi = (pr / (TW / 2)) * TW + 2 * (pr % (TW / 2));
-            union { u32 u; T h[2]; } x;
-            x.u = qraw[i];
-            Ql[pi * QSB + ch] = x.h[0];
-            Ql[(pi + 1) * QSB + ch] = x.h[1];
+            const u32 raw = q32 ? qraw[i] : qraw[i] | qodd[i] << 16;
+            if constexpr (NPX == 16) {
+                // the lane 8 further has the neighbouring channel: the even channel's lane writes both of the first
+                // pixel, the odd one's of the second
+                const u32 other = (u32)__builtin_amdgcn_update_dpp(0, (int)raw, 0x128, 0xf, 0xf, false);     // row_ror:8
+                const bool odd = ch & 1;
+                *(u32 *)(Ql + (pi + (odd ? 1 : 0)) * QSB + (ch & ~1)) =
+                    __builtin_amdgcn_perm(odd ? raw : other, odd ? other : raw, odd ? 0x07060302u : 0x05040100u);
+            } else {
+                union { u32 u; T h[2]; } x;
+                x.u = raw;
+                Ql[pi * QSB + ch] = x.h[0];
+                Ql[(pi + 1) * QSB + ch] = x.h[1];
+            }
         }
     };
 
@@ -324,7 +330,7 @@ deform_fused_wmat16_kernel(const T *__restrict__ q, const T *__restrict__ key,
     // a group's offsets (dx, dy of this lane's point, per pass) are fetched while the
     // group before it is aggregated, and stay as loaded until their use: nothing
     // waits for them where they are issued
-    u32 offraw[NSP], offnext[NSP];
+    u32 offraw[NSP], offnext[NSP], offdy[NSP];       // (offdy: dy where it does not come with dx)
     // Contiguous hi-res offsets whose tile rows are whole aligned vectors come in as
     // such: thread t fetches the 4 x-neighbours of tile row (t / 2) % 4 in the dx
     // (t even) or dy plane of point t / 8 -- one 8-byte load per thread instead of
@@ -360,7 +366,7 @@ deform_fused_wmat16_kernel(const T *__restrict__ q, const T *__restrict__ key,
         asm volatile("" : "+v"(prow_o));
 #pragma unroll
         for (int ps = 0; ps < NSP; ++ps) {
-            offnext[ps] = 0u;
+            offnext[ps] = offdy[ps] = 0u;
             if (ps < nsp) {
                 const Pix px = pixel(ps * ppp + prow_o);
                 if (px.active && pt < P) {
@@ -382,10 +388,8 @@ deform_fused_wmat16_kernel(const T *__restrict__ q, const T *__restrict__ key,
                             op = offset + cx * hpl + px.pp;
                             dy = hpl;
                         }
-                        union { T h[2]; u32 u; } x;
-                        x.h[0] = op[0];
-                        x.h[1] = op[dy];
-                        offnext[ps] = x.u;
+                        offnext[ps] = *(const unsigned short *)op;
+                        offdy[ps] = *(const unsigned short *)(op + dy);
                     } else {
                         offnext[ps] = *(const u32 *)(offset + px.hp * (2L * G * P) + 2L * ((long)g * P + pt));
                     }
@@ -403,12 +407,15 @@ deform_fused_wmat16_kernel(const T *__restrict__ q, const T *__restrict__ key,
         stage_store_key();
         stage_store_q();
         if (ovec) {
-            // Ost[point][pixel][dx, dy]
+            // Ost[point][pixel][dx, dy]: the neighbouring lanes hold dx and dy of 4 pixels, the first one writes two
+            // of them, the second one the others
             const int xy = tid & 1, row = (tid >> 1) & 3, opt = tid >> 3;
-            union { u32x2 u; T h[4]; } x;
-            x.u = u32x2{offnext[0], offnext[NSP > 1 ? 1 : 0]};
-#pragma unroll
-            for (int e = 0; e < 4; ++e) Ost[((opt * NPX) + row * 4 + e) * 2 + xy] = x.h[e];
+            const u32 lo = offnext[0], hi = offnext[NSP > 1 ? 1 : 0];
+            const u32 mine = xy ? hi : lo;
+            const u32 other = (u32)__builtin_amdgcn_update_dpp(0, (int)(xy ? lo : hi), 0xb1, 0xf, 0xf, false);    // quad_perm:[1,0,3,2]
+            const u32 dx = xy ? other : mine, dy = xy ? mine : other;
+            *(u32x2 *)(Ost + (opt * NPX + row * 4 + 2 * xy) * 2) =
+                u32x2{__builtin_amdgcn_perm(dy, dx, 0x05040100u), __builtin_amdgcn_perm(dy, dx, 0x07060302u)};
         }
         if (tid == 0) fb_flag = 0;
         __syncthreads();
@@ -417,7 +424,7 @@ deform_fused_wmat16_kernel(const T *__restrict__ q, const T *__restrict__ key,
         f32x2 off2[NSP];
 #pragma unroll
         for (int ps = 0; ps < NSP; ++ps) {
-            offraw[ps] = offnext[ps];
+            offraw[ps] = NCHW && !ovec ? offnext[ps] | offdy[ps] << 16 : offnext[ps];
             if (ovec) offraw[ps] = ps < nsp ? ((const u32 *)Ost)[pt * NPX + ps * ppp + prow] : 0u;
             off2[ps] = widen_pair<T>(offraw[ps]);
         }
@@ -513,16 +520,6 @@ deform_fused_wmat16_kernel(const T *__restrict__ q, const T *__restrict__ key,
                 __hip_atomic_fetch_add(wp + WWX, (u32)fma_(sc, t.w3, 0.5f), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
                 __hip_atomic_fetch_add(wp + WWX + 1, (u32)fma_(sc, t.w4, 0.5f), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
             }
-            // 8 entries (32 bytes) -> their 8 high parts, then their 8 remainders
-#pragma unroll
-            for (int i8 = 0; i8 < (KP / 8 + NL - 1) / NL; ++i8)
-                if (i8 * NL + pt < KP / 8) {
-                    u32x4 *blk = (u32x4 *)(wrow + 8 * (i8 * NL + pt));
-                    u32x4 hi, lo;
-                    split8<T>(blk[0], blk[1], hi, lo);
-                    blk[0] = hi;
-                    blk[1] = lo;
-                }
         };
 #pragma unroll
         for (int ps = 0; ps < NSP; ++ps) {
@@ -531,6 +528,20 @@ deform_fused_wmat16_kernel(const T *__restrict__ q, const T *__restrict__ key,
             } else {
                 sample(std::integral_constant<int, 32>{}, ps);
             }
+        }
+        // the wave's pixels, 16 lanes each: 8 entries (32 bytes) -> their 8 high parts, then their 8 remainders
+#pragma unroll
+        for (int j4 = 0; j4 < NPX / 16; ++j4) {
+            const int j = 4 * j4 + mk, pi = narrow ? 16 * j4 + 4 * wave + mk : 8 * (j >> 1) + 2 * wave + (j & 1);
+#pragma unroll
+            for (int i8 = 0; i8 < (KP / 8 + 15) / 16; ++i8)
+                if (i8 * 16 + mi < KP / 8) {
+                    u32x4 *blk = (u32x4 *)(SWl + pi * WS + 8 * (i8 * 16 + mi));
+                    u32x4 hi, lo;
+                    split8<T>(blk[0], blk[1], hi, lo);
+                    blk[0] = hi;
+                    blk[1] = lo;
+                }
         }
 
         // ---- (d) value chunks: out tile = Wm . value window (the key window is done with)
