@@ -99,13 +99,17 @@ sapa_b_wmat16_kernel(const T *__restrict__ q, const T *__restrict__ key, const T
     static_assert(NSW == 16 || NSW == 8, "piece swizzle");
     constexpr int NPC = 2 * NSW / 2;                         // 16-byte pieces per tile row = NSW
 
-    // two buffers of each kind (three, i.e. requests two chunks ahead, measured slower: 208 against
-    // 199 us at FPN-large)
-    __shared__ __attribute__((aligned(16))) u32 lds[2 * (LOWBUF + HIBUF) + 4];
-    u32 *const lowbuf = lds, *const hibuf = lds + 2 * LOWBUF;
+    // Buffers of each kind, one chunk per buffer.  Streamed tensors come from memory, not from a cache:
+    // requests two chunks ahead, and stores waited for two chunks later (B=16, C=256, d=64, 100x168 in bf16, inputs
+    // not in the memory-side cache 257 -> 245 us; read again and again, as no program does, 211 -> 213).  What fits
+    // the cache has two, and so two workgroups per CU.
+    constexpr int NB = STREAM && !ODD ? 3 : 2;
+    __shared__ __attribute__((aligned(16))) u32 lds[NB * (LOWBUF + HIBUF) + 4];
+    u32 *const lowbuf = lds, *const hibuf = lds + NB * LOWBUF;
+    const u32 low_at = lds_address((const __attribute__((address_space(3))) u32 *)lds), hi_base = low_at + NB * LOWBUF * 4;
     // blocks of the tile with a non-finite result (in the same array: with a variable of its own the
     // compiler waits for direct loads in other places, 258 -> 268 us at FPN-large)
-    u32 *const non_finite = lds + 2 * (LOWBUF + HIBUF);
+    u32 *const non_finite = lds + NB * (LOWBUF + HIBUF);
 
     const int logical = (int)(blockIdx.x % 8) * per_xcd + (int)(blockIdx.x / 8);
     if (logical >= nblocks) return;
@@ -154,8 +158,6 @@ sapa_b_wmat16_kernel(const T *__restrict__ q, const T *__restrict__ key, const T
 
     const int nKc = (d + CHK - 1) / CHK, allV = (C + CHK - 1) / CHK;
     const int nVc = allV - vbase < slice_chunks ? allV - vbase : slice_chunks, ntot = nKc + nVc;
-    const __amdgpu_buffer_rsrc_t rq = __builtin_amdgcn_make_buffer_rsrc(
-        (void *)(q + (long)n * d * SS * lpix), 0, (int)(d * hplane), 0x00020000);
     // (HALF: an image ends with half a dword, which lies outside: nothing behind a tensor is read, and
     // low_end puts that element in its place)
     const __amdgpu_buffer_rsrc_t rk = __builtin_amdgcn_make_buffer_rsrc(
@@ -165,35 +167,33 @@ sapa_b_wmat16_kernel(const T *__restrict__ q, const T *__restrict__ key, const T
     const __amdgpu_buffer_rsrc_t ro = __builtin_amdgcn_make_buffer_rsrc(
         (void *)(out + (long)n * C * SS * lpix), 0, (int)(C * hplane), 0x00020000);
 
-    (void)rq, (void)rk, (void)rv;
+    (void)rk, (void)rv;
     // Chunk j is the key + q channels 16 j .. for j < nKc and the value channels 16 (j - nKc) ..
-    // after; it lives in buffer j % 2 and is requested two chunks ahead, as soon as every wave is
+    // after; it lives in buffer j % NB and is requested NB chunks ahead, as soon as every wave is
     // done with that buffer.  A channel past the tensor's last lies past the descriptor: zeros.
-    auto stage_low = [&](__amdgpu_buffer_rsrc_t r, u32 c0, int buf) __attribute__((always_inline)) {
-#if defined(__HIP_DEVICE_COMPILE__)
-        u32 *lb = lowbuf + buf * LOWBUF + wave * 256;
+    const u32x4 dq = dma_rsrc(q + (long)n * d * SS * lpix, d * hplane);
+    const u32x4 dk = dma_rsrc(key + (long)n * d * lpix, d * lplane);
+    const u32x4 dv = dma_rsrc(value + (long)n * C * lpix, C * lplane);
+    auto stage_low = [&](u32x4 r, u32 c0, int buf) __attribute__((always_inline)) {
 #pragma unroll
         for (int i = 0; i < NLI; ++i)
             if ((i + 1) * NT <= NLP || i * NT + wave * 64 < NLP)
-                __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (__attribute__((address_space(3))) void *)(lb + i * NT * 4), 16,
-                                                         off_low[i] + c0 * lplane, 0, 0, 0);
-#endif
+                load_lds(r, low_at + (buf * LOWBUF + wave * 256 + i * NT * 4) * 4, off_low[i] + c0 * lplane);
     };
     auto stage_q = [&](u32 c0, int buf) __attribute__((always_inline)) {
-#if defined(__HIP_DEVICE_COMPILE__)
-        u32 *hb = hibuf + buf * HIBUF + wave * 256;
 #pragma unroll
-        for (int i = 0; i < NHI; ++i)
-            __builtin_amdgcn_raw_ptr_buffer_load_lds(rq, (__attribute__((address_space(3))) void *)(hb + i * NT * 4), 16,
-                                                     off_hi[i] + c0 * hplane, 0, 0, STREAM ? 2 : 0);
-#endif
+        for (int i = 0; i < NHI; ++i) load_lds<STREAM>(dq, hi_base + (buf * HIBUF + wave * 256 + i * NT * 4) * 4, off_hi[i] + c0 * hplane);
+    };
+    // operations that this wave issues for chunk j
+    auto loads_of = [&](int j) __attribute__((always_inline)) {
+        return j < ntot ? (ODD ? 0 : (NLP - wave * 64 + NT - 1) / NT) + (j < nKc ? NHI : 0) : 0;
     };
     auto stage = [&](int j) __attribute__((always_inline)) {
         if (j < nKc) {
-            if (!ODD) stage_low(rk, (u32)(j * CHK), j & 1);
-            stage_q((u32)(j * CHK), j & 1);
+            if (!ODD) stage_low(dk, (u32)(j * CHK), j % NB);
+            stage_q((u32)(j * CHK), j % NB);
         } else if (!ODD && j < ntot) {
-            stage_low(rv, (u32)((j - nKc + vbase) * CHK), j & 1);
+            stage_low(dv, (u32)((j - nKc + vbase) * CHK), j % NB);
         }
     };
     // ODD: an odd W puts every other row of a low-res plane in the middle of a dword, where direct loads
@@ -234,7 +234,7 @@ sapa_b_wmat16_kernel(const T *__restrict__ q, const T *__restrict__ key, const T
                         : u32x4{0u, v[0] << 16, __builtin_amdgcn_alignbyte(v[1], v[0], 2),
                                 __builtin_amdgcn_alignbyte(v[2], v[1], 2)};
             const int at = OWN ? slot / LPC * LROW + slot % LPC * 4 : slot * 4;
-            if (NLP % NT == 0 || slot < NLP) *(u32x4 *)(lowbuf + (j & 1) * LOWBUF + at) = m;
+            if (NLP % NT == 0 || slot < NLP) *(u32x4 *)(lowbuf + (j % NB) * LOWBUF + at) = m;
         }
     };
     // behind low_commit(j), by the wave that wrote the piece: the last element of an image of an odd number
@@ -246,7 +246,7 @@ sapa_b_wmat16_kernel(const T *__restrict__ q, const T *__restrict__ key, const T
         for (int i = 0; i < NLI; ++i) {
             const int slot = i * NT + tid, at = OWN ? slot / LPC * LROW + slot % LPC * 4 : slot * 4;
             const u32 e = (u32)((long)(nch - c0) * lpix) - 1u - (u32)(((int)off_low[i] >> 1) + (low_odd[i] ? 1 : 0));
-            if (e < 8u) ((T *)(lowbuf + (j & 1) * LOWBUF + at))[e] = last;
+            if (e < 8u) ((T *)(lowbuf + (j % NB) * LOWBUF + at))[e] = last;
         }
     };
     // chunk jn (the first of the keys or of the values) has landed in this wave's slots: the 6
@@ -255,7 +255,7 @@ sapa_b_wmat16_kernel(const T *__restrict__ q, const T *__restrict__ key, const T
     auto patch_low = [&](int jn) __attribute__((always_inline)) {
         if (!OWN && tx == 0 && ty == 0 && patch_slot >= 0 && (jn < nKc || vbase == 0)) {
             const __amdgpu_buffer_rsrc_t r = jn < nKc ? rk : rv;
-            u32 *dst = lowbuf + (jn & 1) * LOWBUF + patch_slot * 4;
+            u32 *dst = lowbuf + (jn % NB) * LOWBUF + patch_slot * 4;
 #pragma unroll
             for (int k = 1; k < 4; ++k) dst[k] = __builtin_amdgcn_raw_buffer_load_b32(r, 4 * (k - 1), 0, 0);
         }
@@ -270,8 +270,9 @@ sapa_b_wmat16_kernel(const T *__restrict__ q, const T *__restrict__ key, const T
     low_end(0);
     stage(0);
     stage(1);
-    // chunk 0: all but chunk 1's loads
-    wait_all_but(ODD ? 0 : ntot < 2 ? 0 : (NLP - wave * 64 + NT - 1) / NT + (1 < nKc ? NHI : 0));
+    if (NB > 2) stage(2);
+    // chunk 0: all but the loads of the chunks after it
+    wait_all_but(ODD ? 0 : loads_of(1) + (NB > 2 ? loads_of(2) : 0));
     patch_low(0);
     lds_barrier();
 
@@ -289,7 +290,7 @@ sapa_b_wmat16_kernel(const T *__restrict__ q, const T *__restrict__ key, const T
     for (int j = 0; j < nKc; ++j) {
         low_load(j + 1);
         if (active) {
-            const u32 *kb = lowbuf + (j & 1) * LOWBUF, *qb = hibuf + (j & 1) * HIBUF;
+            const u32 *kb = lowbuf + (j % NB) * LOWBUF, *qb = hibuf + (j % NB) * HIBUF;
             u32x2 a[4], b[4];
 #pragma unroll
             for (int mb = 0; mb < 4; ++mb)
@@ -306,11 +307,11 @@ sapa_b_wmat16_kernel(const T *__restrict__ q, const T *__restrict__ key, const T
         }
         low_commit(j + 1);
         low_end(j + 1);
-        // chunk j + 1: nothing was issued after its loads
-        wait_all_but(0);
+        // chunk j + 1: all but the loads of a chunk requested since
+        wait_all_but(NB > 2 ? loads_of(j + 2) : 0);
         if (j + 1 == nKc) patch_low(nKc);
         lds_barrier();
-        stage(j + 2);
+        stage(j + NB);
     }
 
     // ---- softmax over each child's 5 x 5 cells; the weights as A operands of the aggregation ----
@@ -402,7 +403,7 @@ sapa_b_wmat16_kernel(const T *__restrict__ q, const T *__restrict__ key, const T
         u32 *ob = hibuf + (j & 1) * HIBUF;                      // no loads into this ring any more
         low_load(j + 1);
         if (active) {
-            const u32 *vb = lowbuf + (j & 1) * LOWBUF;
+            const u32 *vb = lowbuf + (j % NB) * LOWBUF;
             // B operand of step s: lane (g, channel i16) holds the cells of rows 4 s + g / 2 and
             // 4 s + 2 + g / 2, columns 4 (g % 2) .. + 3 -- the order the weights are held in
             u32x4 b[2];
@@ -434,8 +435,8 @@ sapa_b_wmat16_kernel(const T *__restrict__ q, const T *__restrict__ key, const T
         }
         low_commit(j + 1);
         low_end(j + 1);
-        // chunk j + 1: its loads were the last operations issued
-        wait_all_but(0);
+        // chunk j + 1: all but the stores of chunk j - 1 (at least NHI) and the loads requested behind them
+        wait_all_but(NB > 2 ? loads_of(j + 2) + (j > nKc ? NHI : 0) : 0);
         lds_barrier();
         // the tile's 16 channels x 8 rows, 16 bytes per lane, right after the barrier that completes
         // them (sending them behind the next chunk's matrix instructions measured slower); a piece
@@ -459,7 +460,7 @@ sapa_b_wmat16_kernel(const T *__restrict__ q, const T *__restrict__ key, const T
             else __builtin_amdgcn_raw_buffer_store_b128(o, ro, off, 0, 0);
         }
         // (the next request behind the stores: 208 us at FPN-large against 216 with the loads first)
-        if (!ODD && j + 2 < ntot) stage_low(rv, (u32)((j + 2 - nKc + vbase) * CHK), j & 1);
+        if (!ODD && j + NB < ntot) stage_low(dv, (u32)((j + NB - nKc + vbase) * CHK), j % NB);
     }
 
     // ---- blocks with a non-finite result: again, term by term ----
