@@ -425,24 +425,31 @@ lowgrad_shift_kernel(const T *__restrict__ hi, const WT *__restrict__ w, T *__re
     }
 }
 
+// What tiles of nw waves of rw lanes cost, and the channels per workgroup that cost the least: the rounds of
+// workgroups (a CU holds 16 waves) times a workgroup's channels and the tile's weights, which every
+// workgroup of the tile reads again (as long as 6 channels take), times the waves that share a CU (fewer than 10 do not fill it).
+// 16 images, 256 channels, 50x84, 8 waves: 16 / 32 / 64 / 128 channels 164 / 153 / 148 / 145 us; 64 channels,
+// 8 / 16 / 32: 51 / 42 / 39.
+static double lowgrad_shift_cost(int nw, int rw, int K, int B, int C, int H, int W, int CH, int &cper) {
+    const int R = (K - 1) / 2, vx = rw - 2 * R, vy = 64 / rw * nw - 2 * R, resident = 16 / nw;
+    const double tiles = (double)((W + vx - 1) / vx) * ((H + vy - 1) / vy) * B;
+    cper = C < 8 ? (C + CH - 1) / CH * CH : 8;
+    double least = 0;
+    for (int c = cper; c < C + 4; c += 4) {
+        const double load = tiles * ((C + c - 1) / c) / (256 * resident);
+        const int waves = load > 0.5 ? nw * resident : nw;
+        const double time = (load <= 1 ? 1 : 0.5 * (load + __builtin_ceil(load))) * (c + 6) * (waves > 10 ? waves : 10);
+        if (least == 0 || time < least) least = time, cper = c;
+    }
+    return least;
+}
+
 template <typename T, typename WT, int K, int NW, int CH, int WPE, int RW>
 static hipError_t lowgrad_shift_launch(const void *hi, const void *w, void *out, int B, int C, int H, int W,
-                                       hipStream_t st) {
+                                       int cper, hipStream_t st) {
     constexpr int R = (K - 1) / 2, VX = RW - 2 * R, VY = 64 / RW * NW - 2 * R;
     const int tiles_x = (W + VX - 1) / VX, tiles_y = (H + VY - 1) / VY;
     const long tiles = (long)tiles_x * tiles_y * B;
-    // Channels per workgroup, so that the rounds of workgroups (two are resident on each of 256 CUs) times what one
-    // costs are the fewest: its channels, and the tile's weights, which every workgroup of the tile reads
-    // again (as long as 6 channels take).  16 images, 256 channels, 50x84: 16 / 32 / 64 / 128 channels
-    // 164 / 153 / 148 / 145 us, the estimate 170 / 147 / 136 / 134; 64 channels, 8 / 16 / 32: 51 / 42 / 39
-    // and 54 / 43 / 38.
-    int cper = C < 8 ? (C + CH - 1) / CH * CH : 8;
-    double least = 0;
-    for (int c = cper; c < C + 4; c += 4) {
-        const double load = (double)tiles * ((C + c - 1) / c) / 512;
-        const double time = (load <= 1 ? 1 : 0.5 * (load + __builtin_ceil(load))) * (c + 6);
-        if (least == 0 || time < least) least = time, cper = c;
-    }
     const int cgroups = (C + cper - 1) / cper;
     const long nb = tiles * cgroups;
     if (nb > (1L << 30)) return hipErrorNotSupported;
@@ -507,7 +514,7 @@ static hipError_t lowgrad_launch_t(const void *hi, const void *w, void *out, int
         // a 32-bit buffer descriptor per image.  Tiles of 8 waves with chunks of 2
         // channels keep it within 128 registers (four waves per SIMD, two workgroups per
         // CU), as 32 x 16 lanes (rows of whole cache lines) unless 16 x 32 wastes
-        // clearly fewer lanes on the shape.
+        // clearly fewer lanes on the shape (where 12 or 15 waves are better, below).
         constexpr int NW = 8, CH = 2, WPE = 4;
         const int R = (K - 1) / 2;
         auto lanes = [&](int rw) {
@@ -521,11 +528,24 @@ static hipError_t lowgrad_launch_t(const void *hi, const void *w, void *out, int
         const double lanes_gather = (double)((W + tw - 1) / tw) * ((H + 7) / 8) * (tw * 8);
         if ((long)C * H * 2 * W * 2 * (long)sizeof(T) < (1L << 31) &&
             lanes_gather >= SAPA_LOWGRAD_SHIFT_GAIN * lanes_shift) {
+            // Rows of 32 lanes and K = 5: of tiles of 8, 12 or 15 waves (12, 20 or 26 rows of cells from 16, 24 or 30 of
+            // lanes; 8 waves twice on a CU) those that the estimate prefers.  Sums are formed in the same order.  fp32,
+            // 256 channels, 8 / 12 / 15 waves: 16 images 50x84 126 / 129 / 109 us, 16 of 100x168 465 / 403 / 405,
+            // 4 of 100x168 127 / 101 / 112, 6 of 91x97 106 / 98 / 107, 16 of 25x42 51 / 50 / 36.
+            int cper8 = 0, cper12 = 0, cper15 = 0;
+            const double cost8 = lowgrad_shift_cost(NW, rows32 ? 32 : 16, K, B, C, H, W, CH, cper8);
+            if (K == 5 && rows32) {
+                const double cost12 = lowgrad_shift_cost(12, 32, K, B, C, H, W, CH, cper12);
+                const double cost15 = lowgrad_shift_cost(15, 32, K, B, C, H, W, CH, cper15);
+                if (cost15 < cost8 && cost15 < cost12)
+                    return lowgrad_shift_launch<T, WT, 5, 15, CH, WPE, 32>(hi, w, out, B, C, H, W, cper15, st);
+                if (cost12 < cost8) return lowgrad_shift_launch<T, WT, 5, 12, CH, WPE, 32>(hi, w, out, B, C, H, W, cper12, st);
+            }
             if (rows32)
-                return K == 3 ? lowgrad_shift_launch<T, WT, 3, NW, CH, WPE, 32>(hi, w, out, B, C, H, W, st)
-                              : lowgrad_shift_launch<T, WT, 5, NW, CH, WPE, 32>(hi, w, out, B, C, H, W, st);
-            return K == 3 ? lowgrad_shift_launch<T, WT, 3, NW, CH, WPE, 16>(hi, w, out, B, C, H, W, st)
-                          : lowgrad_shift_launch<T, WT, 5, NW, CH, WPE, 16>(hi, w, out, B, C, H, W, st);
+                return K == 3 ? lowgrad_shift_launch<T, WT, 3, NW, CH, WPE, 32>(hi, w, out, B, C, H, W, cper8, st)
+                              : lowgrad_shift_launch<T, WT, 5, NW, CH, WPE, 32>(hi, w, out, B, C, H, W, cper8, st);
+            return K == 3 ? lowgrad_shift_launch<T, WT, 3, NW, CH, WPE, 16>(hi, w, out, B, C, H, W, cper8, st)
+                          : lowgrad_shift_launch<T, WT, 5, NW, CH, WPE, 16>(hi, w, out, B, C, H, W, cper8, st);
         }
     }
 #endif

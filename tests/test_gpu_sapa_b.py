@@ -340,6 +340,13 @@ def test_tiled_lowres_gradient_integer_inputs_exact(shape):
     assert torch.equal(vd.grad.cpu().double(), want)
 
 
+# tiles of 12 and of 15 waves, ragged in x and y, channels that are no whole groups
+@pytest.mark.parametrize('shape', [(5, 62, 40, 55, 5), (9, 39, 21, 85, 5), (11, 30, 21, 85, 5), (11, 15, 43, 84, 5)],
+                         ids=lambda s: '-'.join(map(str, s)))
+def test_tall_lowres_gradient_tiles_integer_inputs_exact(shape):
+    test_tiled_lowres_gradient_integer_inputs_exact(shape)
+
+
 def test_backward_16bit_tensors():
     """16-bit tensors: gradients come back in the tensors' dtype and agree
     with the fp32 gradients at the same (rounded) inputs."""
