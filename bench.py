@@ -80,7 +80,7 @@ MEASURED_TRAFFIC = {
                                      'deform_fused_wmat16_kernel'),
     ('deform_p25', 'fp32', 'nchw_reference_order'): (828689742, 'profiles/sapa_d_lds_fused_deform_p25_fp32.md',
                                                      'deform_lds_kernel'),
-    ('deform_p9', 'fp32', 'nchw'): (399849952, 'profiles/sapa_d_lds_fused_deform_p9_fp32.md', 'deform_lds_kernel'),
+    ('deform_p9', 'fp32', 'nchw'): (289832257, 'profiles/sapa_d_gather_fused_deform_p9_fp32.md', 'deform_gather_kernel'),
     ('deform_p25', 'fp32', 'channels_last'): (356737114, 'profiles/sapa_d_nhwc_fused_deform_p25_fp32.md',
                                               'deform_fused_wmat_kernel'),
     ('deform_p25', 'bf16', 'channels_last'): (178447650, 'profiles/sapa_d_wmat16_fused_deform_p25_bf16.md',
@@ -756,7 +756,7 @@ def main():
                      else c_oracle.sapa_fused(*cpu0, K, s, 'f32'))
             e32 = (got - ref32).abs()
             outside = int((e32 > 1e-6 + 1e-5 * ref32.abs()).sum().item())
-            same_order = main_kernel in ('sapa_b_tiled_kernel', 'deform_lds_kernel', 'sapa_b_mfma_kernel')
+            same_order = main_kernel in ('sapa_b_tiled_kernel', 'deform_lds_kernel', 'deform_gather_kernel', 'sapa_b_mfma_kernel')
             rec['parity_image0'] = {
                 'against': "oracle/c_oracle 'f32' (the reference kernels' arithmetic and order of sums)",
                 'bar': '1e-6 + 1e-5 |b|', 'outside_bar': outside, 'elements': e32.numel(),

@@ -16,7 +16,7 @@ OBJ = os.path.join(CSRC, '_obj')
 LIBDIR = os.path.join(HERE, 'lib')
 LIB = os.path.join(LIBDIR, 'libsapa_hip.so')
 SOURCES = ['capi.hip', 'sapa_b_generic.hip', 'sapa_b_tiled.hip', 'sapa_b_dot2.hip', 'sapa_b_wmat16.hip', 'sapa_b_nhwc.hip', 'sapa_b_nhwc_mm.hip', 'sapa_b_nhwc16.hip', 'sapa_b_nhwc_wm16.hip', 'sapa_b_mfma.hip', 'sapa_b_lowgrad.hip', 'sapa_b_bwd16.hip', 'sapa_b_nhwc_bwd16.hip', 'sapa_d.hip', 'sapa_d_lowgrad.hip', 'sapa_d_nhwc.hip', 'sapa_d_wmat16.hip', 'sapa_d_backward.hip', 'sapa_d_bwdmat.hip', 'sapa_d_region_bwd16.hip', 'sapa_d_scatter.hip', 'sapa_moments.hip', 'sapa_project.hip', 'sapa_layout.hip', 'sapa_stream.hip',
-           'sapa_d_lds.hip']
+           'sapa_d_lds.hip', 'sapa_d_gather.hip']
 
 HIPCC = os.environ.get('HIPCC', '/opt/rocm/bin/hipcc')
 # packed-fp32 VALU ops are switched off for every kernel in this library

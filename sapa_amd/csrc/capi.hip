@@ -153,8 +153,11 @@ hipError_t deform_av_any(const void *attn, const void *value, const void *offset
 hipError_t deform_fused_any(const void *q, const void *key, const void *value, const void *offset,
                             void *out, int B, int Cq, int C, int H, int W, int P, int s, int G,
                             int olayout, int dtype, hipStream_t st) {
-    hipError_t e = took("deform_lds_kernel", deform_lds_launch(2, q, key, nullptr, value, offset, out, B, Cq,
-                                                                C, H, W, P, s, G, olayout, dtype, st));
+    hipError_t e = took("deform_gather_kernel", deform_gather_launch(q, key, value, offset, out, B, Cq, C, H, W, P, s,
+                                                                      G, olayout, dtype, st));
+    if (e == hipErrorNotSupported)
+        e = took("deform_lds_kernel", deform_lds_launch(2, q, key, nullptr, value, offset, out, B, Cq,
+                                                        C, H, W, P, s, G, olayout, dtype, st));
     if (e == hipErrorNotSupported)
         e = took("deform_fused_forward_kernel",
                  deform_fused_forward_launch(q, key, value, offset, out, B, Cq, C, H, W, P, s, G, olayout,

@@ -236,6 +236,8 @@ hipError_t lowres_grad_tiled_launch(const void *hi, const void *w, void *out, in
 // window; mode 0 = deform_qk (out = logits), 1 = deform_av (attn_in given),
 // 2 = fused.  hipErrorNotSupported when (s, dtype, P) has no instance / does
 // not fit LDS; the caller then takes the global-memory kernels below.
+hipError_t deform_gather_launch(const void *q, const void *key, const void *value, const void *offset, void *out, int B, int Cq,
+                                int C, int H, int W, int P, int s, int G, int olayout, int dtype, hipStream_t st);
 hipError_t deform_lds_launch(int mode, const void *q, const void *key, const void *attn_in,
                              const void *value, const void *offset, void *out, int B, int Cq, int C,
                              int H, int W, int P, int s, int G, int olayout, int dtype,

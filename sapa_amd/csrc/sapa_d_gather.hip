@@ -1,0 +1,324 @@
+// Fused SAPA-D (deform_qk -> softmax -> deform_av) of contiguous fp32 tensors, up_factor 2 and at most 12
+// sample points: every sample is gathered from a window in LDS, a pixel's points stay in registers.
+//
+// As in sapa_d_lds.hip a workgroup owns TPW x TPH low-res parents of one (image, group), a thread one
+// output pixel, and the window -- the tile plus 4 cells on every side, one more behind for the +1 corners --
+// passes through LDS in chunks of 16 channels as [cell][16 channels], zeros outside the image.  What differs
+// is where the rest lives.  A sample's place and fractions and its logit (then weight) are registers, formed
+// once: that kernel fetched the offsets again and formed floor, guard and window test again for each chunk of
+// channels (6 times with 32 query and 64 value channels: a third of its vector instructions), and another
+// third went into staging element by element.  Here a thread stages four channels of a cell at a time through
+// four buffer loads whose offsets are fixed for the whole kernel, requested a chunk ahead, into the second of two
+// buffers: one barrier per chunk.  A sample outside the image or the window points at cells that are always
+// zero, so the channel loops have no selects; the rare one inside the image but outside the window is added
+// from memory in its turn.
+//
+// Arithmetic and order of sums are those of sapa_d_lds.hip, bit for bit (reference:
+// deformsapa/deformsapa/src/cuda/deform_qk_cuda_kernel.cu:180-193, deform_av_cuda_kernel.cu:178-192).
+#include "deform_tap.hpp"
+#include "kernels.hpp"
+
+namespace sapa {
+
+namespace dgather {
+
+typedef unsigned u32;
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+
+constexpr int S = 2, HR = 4, CH = 16;
+constexpr int CST = CH + 4;                         // floats per cell: 16-byte reads spread over all bank groups
+constexpr u32 OUTSIDE = 0x80000000u;                // a buffer offset beyond any extent
+
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t planes(const void *p, long bytes) {
+    return __builtin_amdgcn_make_buffer_rsrc((void *)p, 0, (int)bytes, 0x00020000);
+}
+
+// PM: the most sample points
+template <int PM, int TPW, int TPH>
+__global__ void __launch_bounds__(TPW * TPH * S * S) __attribute__((amdgpu_waves_per_eu(4, 4)))
+deform_gather_kernel(const float *__restrict__ q, const float *__restrict__ key, const float *__restrict__ value,
+                     const float *__restrict__ offset, float *__restrict__ out, int Cq, int C, int H, int W, int P,
+                     int G, int olayout, int tiles_x, int tiles_y, int nblocks, int per_xcd) {
+    constexpr int NT = TPW * TPH * S * S, TXP = TPW * S;
+    constexpr int WW = TPW + 2 * HR + 1, WH = TPH + 2 * HR + 1, WIN = WW * WH;
+    constexpr int RS = WW * CST;                    // floats between window rows
+    constexpr int NOWHERE = WIN * CST;              // where samples that contribute nothing read zeros
+    constexpr int BUF = NOWHERE + RS + CST + CH;
+    constexpr int TASKS = WIN * (CH / 4), NST = (TASKS + NT - 1) / NT;
+
+    __shared__ __attribute__((aligned(16))) float lds[2 * BUF];
+
+    const int logical = (int)(blockIdx.x % 8) * per_xcd + (int)(blockIdx.x / 8);
+    if (logical >= nblocks) return;
+    const int tx = logical % tiles_x;
+    const int ty = (logical / tiles_x) % tiles_y;
+    const int g = (logical / (tiles_x * tiles_y)) % G;
+    const int b = logical / (tiles_x * tiles_y * G);
+
+    const int tid = threadIdx.x;
+    const int hH = H * S, hW = W * S, GP = G * P, d = Cq / G, cg = C / G;
+    const u32 lplane = (u32)(H * W) * 4u, hplane = (u32)(hH * hW) * 4u;         // bytes
+    const int qw = tx * TXP + tid % TXP, qh = ty * TPH * S + tid / TXP;
+    const bool active = qw < hW && qh < hH;
+    // idle threads of a partial tile read through clamped coordinates
+    const int cw = qw < hW ? qw : hW - 1, chh = qh < hH ? qh : hH - 1;
+    const u32 pix = (u32)(chh * hW + cw) * 4u;
+    const float ph = (float)(chh / S), pw = (float)(cw / S);
+    const int wx0 = tx * TPW - HR, wy0 = ty * TPH - HR;
+    const float *const qg = q + ((long)b * Cq + (long)g * d) * (hplane / 4);
+    const float *const kg = key + ((long)b * Cq + (long)g * d) * (lplane / 4);
+    const float *const vg = value + ((long)b * C + (long)g * cg) * (lplane / 4);
+    const int nK = (d + CH - 1) / CH, ntot = nK + (cg + CH - 1) / CH;
+
+    // ---- staging: task i of a thread is four channels of one cell ----
+    u32 from[NST];
+    int to[NST];
+#pragma unroll
+    for (int i = 0; i < NST; ++i) {
+        const int task = tid + i * NT, four = task / WIN, cell = task % WIN;
+        const int gy = wy0 + cell / WW, gx = wx0 + cell % WW;
+        const bool ok = task < TASKS && gy >= 0 && gy < H && gx >= 0 && gx < W;
+        from[i] = ok ? (u32)(4 * four) * lplane + (u32)(gy * W + gx) * 4u : OUTSIDE;
+        to[i] = task < TASKS ? cell * CST + 4 * four : -1;
+    }
+    f32x4 st[NST];
+    auto stage_load = [&](int j) __attribute__((always_inline)) {
+        const bool is_key = j < nK;
+        const int c0 = (is_key ? j : j - nK) * CH, nc = (is_key ? d : cg) - c0;
+        const __amdgpu_buffer_rsrc_t r = planes((const char *)(is_key ? kg : vg) + (long)c0 * lplane, (long)(nc < CH ? nc : CH) * lplane);
+#pragma unroll
+        for (int i = 0; i < NST; ++i) {
+            u32 at = from[i];                       // (opaque: or all four sums are kept)
+            asm volatile("" : "+v"(at));
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+                st[i][e] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(r, at + (u32)e * lplane, 0, 0));
+        }
+    };
+    auto stage_store = [&](int j) __attribute__((always_inline)) {
+        float *const dst = lds + (j & 1) * BUF;
+#pragma unroll
+        for (int i = 0; i < NST; ++i)
+            if ((i + 1) * NT <= TASKS || to[i] >= 0) *(f32x4 *)(dst + to[i]) = st[i];
+    };
+    // channel c of the chunk's queries of this pixel; those behind the last are 0
+    const __amdgpu_buffer_rsrc_t rq = planes(qg, (long)d * hplane);
+    auto load_q = [&](int j, float (&v)[CH]) __attribute__((always_inline)) {
+        u32 at = (u32)(j * CH) * hplane;
+        const u32 end = (u32)d * hplane;
+#pragma unroll
+        for (int c = 0; c < CH; ++c) {
+            v[c] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(rq, pix, at, 0));
+            at += at + hplane < end ? hplane : 0u;  // (no plane behind the last)
+        }
+    };
+    auto clear_q = [&](int j, float (&v)[CH]) __attribute__((always_inline)) {
+        const int nc = d - j * CH;
+        if (nc < CH)
+#pragma unroll
+            for (int c = 0; c < CH; ++c) v[c] = c < nc ? v[c] : 0.f;
+    };
+
+    stage_load(0);
+    // ---- the samples ----
+    float lh[PM], lw[PM], lg[PM];
+    int at[PM];
+    u32 far = 0;                                    // this pixel's samples in the image, but not in the window
+    {
+        const OffsetRef<float> op = offset_ref(offset, olayout, (long)b * GP + (long)g * P, chh, cw, S, H, W);
+        float ow[PM], oh[PM];
+#pragma unroll
+        for (int p = 0; p < PM; ++p) {
+            const int pp = p < P ? p : P - 1;
+            ow[p] = op.base[(long)(2 * pp) * op.stride];
+            oh[p] = op.base[(long)(2 * pp + 1) * op.stride];
+        }
+#pragma unroll
+        for (int p = 0; p < PM; ++p) {
+            const float kh = ph + oh[p], kw = pw + ow[p];
+            const bool guard = active && p < P && kh > -1.f && kh < (float)H && kw > -1.f && kw < (float)W;
+            const float fh = floor_(kh), fw = floor_(kw);
+            const int hl = (int)fh - wy0, wl = (int)fw - wx0;
+            const bool in = guard && hl >= 0 && hl <= WH - 2 && wl >= 0 && wl <= WW - 2;
+            at[p] = in ? hl * RS + wl * CST : NOWHERE;
+            lh[p] = in ? kh - fh : 0.f;
+            lw[p] = in ? kw - fw : 0.f;
+            lg[p] = 0.f;
+            far |= guard && !in ? 1u << p : 0u;
+        }
+    }
+    u32 far_wave = 0;                               // ... of any lane of the wave
+#pragma unroll
+    for (int p = 0; p < PM; ++p) far_wave |= __ballot(far >> p & 1u) ? 1u << p : 0u;
+    // add(c, value) for the channels c0 + c, c < 16, of such a sample
+    auto far_sample = [&](int p, const float *src, int c0, int channels, auto &&add) __attribute__((always_inline)) {
+        // (all of it formed again: kept from above, it does not fit the registers)
+        int t = tid;
+        asm volatile("" : "+v"(t));
+        const int x = tx * TXP + t % TXP, y = ty * TPH * S + t / TXP;
+        const OffsetRef<float> op = offset_ref(offset, olayout, (long)b * GP + (long)g * P, y, x, S, H, W);
+        Tap<float> tap;
+        tap_setup((float)(y / S) + op.base[(long)(2 * p + 1) * op.stride], (float)(x / S) + op.base[(long)(2 * p) * op.stride], H, W, tap);
+        const float *plane = src + (long)c0 * (lplane / 4);
+#pragma unroll
+        for (int c = 0; c < CH; ++c) {
+            if (c0 + c < channels) add(c, tap_sample(plane, tap));
+            plane += lplane / 4;
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    };
+
+    for (int i = tid; i < 2 * (BUF - NOWHERE); i += NT)
+        lds[i < BUF - NOWHERE ? NOWHERE + i : 2 * NOWHERE + i] = 0.f;
+    float qv[CH];
+    load_q(0, qv);
+    stage_store(0);
+
+    // ---- logits ----
+    for (int j = 0; j < nK; ++j) {
+        stage_load(j + 1);
+        __syncthreads();
+        clear_q(j, qv);
+        const float *const win = lds + (j & 1) * BUF;
+#pragma unroll
+        for (int p = 0; p < PM; ++p) {
+            if (p >= P) continue;
+            const float *const wp = win + at[p];
+            float fy = lh[p], fx = lw[p];
+            asm volatile("" : "+v"(fy), "+v"(fx));
+            const float hh = 1.f - fy, hw = 1.f - fx;
+            const float w1 = hh * hw, w2 = hh * fx, w3 = fy * hw, w4 = fy * fx;
+            float acc = lg[p];
+#pragma unroll
+            for (int c4 = 0; c4 < CH; c4 += 4) {
+                const f32x4 a1 = *(const f32x4 *)(wp + c4), a2 = *(const f32x4 *)(wp + CST + c4);
+                const f32x4 a3 = *(const f32x4 *)(wp + RS + c4), a4 = *(const f32x4 *)(wp + RS + CST + c4);
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    float val = w1 * a1[e];
+                    val = fma_(w2, a2[e], val);
+                    val = fma_(w3, a3[e], val);
+                    val = fma_(w4, a4[e], val);
+                    acc = fma_(val, qv[c4 + e], acc);
+                }
+            }
+            // (a query that is not finite times the zeros of a sample that contributes nothing)
+            lg[p] = at[p] != NOWHERE ? acc : lg[p];
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        for (u32 left = far_wave; left; left &= left - 1) {
+            const int p = __builtin_ctz(left);
+            if (far >> p & 1u) {
+                float acc = 0.f;
+#pragma unroll
+                for (int i = 0; i < PM; ++i) acc = i == p ? lg[i] : acc;
+                far_sample(p, kg, j * CH, d, [&](int c, float val) __attribute__((always_inline)) { acc = fma_(val, qv[c], acc); });
+#pragma unroll
+                for (int i = 0; i < PM; ++i) lg[i] = i == p ? acc : lg[i];
+            }
+        }
+        if (j + 1 < nK) load_q(j + 1, qv);
+        stage_store(j + 1);
+    }
+
+    // ---- softmax over the points (one outside the image keeps logit 0 and takes part) ----
+    {
+        float m = lg[0];
+#pragma unroll
+        for (int p = 1; p < PM; ++p) m = p < P ? max_(m, lg[p]) : m;
+        float sum = 0.f;
+#pragma unroll
+        for (int p = 0; p < PM; ++p) {
+            lg[p] = exp_(lg[p] - m);
+            sum = p < P ? sum + lg[p] : sum;
+        }
+        const float inv = 1.f / sum;
+        // (a sample that contributes nothing: its weight times the zeros may not be NaN)
+#pragma unroll
+        for (int p = 0; p < PM; ++p) lg[p] = at[p] != NOWHERE || (far >> p & 1u) ? lg[p] * inv : 0.f;
+    }
+
+    // ---- aggregation ----
+    const __amdgpu_buffer_rsrc_t ro = planes(out + ((long)b * C + (long)g * cg) * (hplane / 4), (long)cg * hplane);
+    const u32 opix = active ? pix : OUTSIDE;
+    for (int j = nK; j < ntot; ++j) {
+        if (j + 1 < ntot) stage_load(j + 1);
+        __syncthreads();
+        const float *const win = lds + (j & 1) * BUF;
+        const int c0 = (j - nK) * CH, nc = cg - c0;
+        float o[CH];
+#pragma unroll
+        for (int c = 0; c < CH; ++c) o[c] = 0.f;
+#pragma unroll
+        for (int p = 0; p < PM; ++p) {
+            if (p >= P) continue;
+            const float *const wp = win + at[p];
+            // (opaque: the weights of all samples kept over the loop do not fit the registers)
+            float fy = lh[p], fx = lw[p];
+            asm volatile("" : "+v"(fy), "+v"(fx));
+            const float hh = 1.f - fy, hw = 1.f - fx, wa = lg[p];
+            const float w1 = hh * hw, w2 = hh * fx, w3 = fy * hw, w4 = fy * fx;
+#pragma unroll
+            for (int c4 = 0; c4 < CH; c4 += 4) {
+                const f32x4 a1 = *(const f32x4 *)(wp + c4), a2 = *(const f32x4 *)(wp + CST + c4);
+                const f32x4 a3 = *(const f32x4 *)(wp + RS + c4), a4 = *(const f32x4 *)(wp + RS + CST + c4);
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    float val = w1 * a1[e];
+                    val = fma_(w2, a2[e], val);
+                    val = fma_(w3, a3[e], val);
+                    val = fma_(w4, a4[e], val);
+                    o[c4 + e] = fma_(val, wa, o[c4 + e]);
+                }
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        for (u32 left = far_wave; left; left &= left - 1) {
+            const int p = __builtin_ctz(left);
+            if (far >> p & 1u) {
+                float wa = 0.f;
+#pragma unroll
+                for (int i = 0; i < PM; ++i) wa = i == p ? lg[i] : wa;
+                far_sample(p, vg, c0, cg, [&](int c, float val) __attribute__((always_inline)) { o[c] = fma_(val, wa, o[c]); });
+            }
+        }
+        u32 plane = (u32)c0 * hplane;
+        asm volatile("" : "+s"(plane));
+#pragma unroll
+        for (int c = 0; c < CH; ++c) {
+            if (c < nc) __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(o[c]), ro, opix, plane, 0);
+            plane += hplane;
+        }
+        if (j + 1 < ntot) stage_store(j + 1);
+    }
+}
+
+template <int PM>
+static hipError_t launch(const void *q, const void *key, const void *value, const void *offset, void *out, int B, int Cq, int C,
+                         int H, int W, int P, int G, int olayout, hipStream_t st) {
+    constexpr int TPW = 16, TPH = 8;
+    const int tiles_x = (W + TPW - 1) / TPW, tiles_y = (H + TPH - 1) / TPH;
+    const long nb = (long)tiles_x * tiles_y * G * B;
+    if (nb > (1L << 30)) return hipErrorNotSupported;
+    const int per_xcd = (int)((nb + 7) / 8);
+    hipLaunchKernelGGL((deform_gather_kernel<PM, TPW, TPH>), dim3(per_xcd * 8), dim3(TPW * TPH * S * S), 0, st,
+                       (const float *)q, (const float *)key, (const float *)value, (const float *)offset, (float *)out, Cq, C, H,
+                       W, P, G, olayout, tiles_x, tiles_y, (int)nb, per_xcd);
+    return hipGetLastError();
+}
+
+}  // namespace dgather
+
+// Up to 9 points: a point takes four registers, and with 12 they spill at the 16 waves per CU that two windows of 36 KB
+// allow; from 13 the matrix form serves default calls.  Images at most 8 cells wide would leave half of each tile idle
+// (8 x 8 tiles of sapa_d_lds.hip).  A group's planes lie within the reach of a buffer descriptor's 32-bit offsets.
+hipError_t deform_gather_launch(const void *q, const void *key, const void *value, const void *offset, void *out, int B, int Cq,
+                                int C, int H, int W, int P, int s, int G, int olayout, int dtype, hipStream_t st) {
+    if (dtype != 0 || s != dgather::S || P < 1 || P > 9 || W <= 8) return hipErrorNotSupported;
+    const long most = Cq > C ? Cq / G : C / G;
+    if (most * H * W * (s * s) * 4L >= (1L << 31) || (most + 16) * (long)H * W * 4L >= (1L << 31)) return hipErrorNotSupported;
+    if (P <= 5) return dgather::launch<5>(q, key, value, offset, out, B, Cq, C, H, W, P, G, olayout, st);
+    return dgather::launch<9>(q, key, value, offset, out, B, Cq, C, H, W, P, G, olayout, st);
+}
+
+}  // namespace sapa

@@ -359,6 +359,7 @@ static hipError_t launch_t(int mode, const void *q, const void *key, const void 
     switch (s) {
         case 1: return launch_geom<T, TS, 1, 16, 16, 8>(mode, q, key, attn_in, value, offset, out, B, Cq, C, H, W, P, G, olayout, st, accumulate, partial);
         case 2:
+            // (the fused operator of fp32 tensors with up to 9 points: sapa_d_gather.hip)
             // few points leave LDS room for a 16 x 8-parent tile (512 threads): a
             // smaller share of halo cells per staged window (measured at P = 9: 12 % faster;
             // at P = 25 the [P][thread] logits of 512 threads cost a workgroup per CU)
