@@ -512,6 +512,15 @@ static hipError_t launch_mode(int mode, bool wide, const void *q, const void *ke
         // relatively less -- measured on the FPN levels)
         const long limit = sizeof(T) == 2 ? 1024 : 512;
         while (cgroups * 2 <= max_groups && tiles * cgroups * 2 <= limit) cgroups *= 2;
+        // The aggregation of fp32 tensors that are staged straight into LDS recomputes nothing in a slice: where those
+        // workgroups would leave CUs idle in their last round, slices of 4 chunks (256 channels, us before and
+        // now: 16 images 50x84, 336 tiles, 134 -> 109; 4 of 100x168, 312 tiles, 139 -> 113; 5 of 64x64, 80 tiles,
+        // 32 -> 26; full rounds are not better off: 2 of 120x120, 120 tiles in 4 slices, 37 -> 41).  Beyond 384 tiles the tile's weights, which every slice reads again, cost more than that (468
+        // tiles 155 and 160, 702 tiles 214 and 243).
+        const long round = 256, rounds = (tiles * cgroups + round - 1) / round;
+        if (mode == TILED_AV && std::is_same<T, float>::value && VEC == 4 && tiles <= 384 &&
+            10 * tiles * cgroups < 9 * round * rounds)
+            cgroups = max_groups;
 #ifdef SAPA_TUNE_CGROUPS
         cgroups = SAPA_TUNE_CGROUPS;
 #endif

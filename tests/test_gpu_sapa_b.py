@@ -581,6 +581,20 @@ def test_fused_and_av_with_sliced_value_channels(coracle, C):
     assert torch.equal(sapa_amd.av(*dev(attn, v), K, s).cpu(), coracle.av(attn, v, K, s, 'f32'))
 
 
+# tiles that would leave the last round of workgroups part empty: slices of 32 channels, the last one whole, short, alone
+@pytest.mark.parametrize('shape', [(12, 256, 20, 36), (12, 100, 20, 36), (40, 68, 17, 64), (5, 36, 64, 64)])
+def test_av_in_slices_of_32_channels(coracle, shape):
+    B, C, H, W = shape
+    g = gen(141)
+    attn, v = randn(g, B, 25, 2 * H, 2 * W), randn(g, B, C, H, W)
+    got = sapa_amd.av(*dev(attn, v), 5, 2).cpu()
+    for n in (0, B - 1):
+        assert torch.equal(got[n:n + 1], coracle.av(attn[n:n + 1], v[n:n + 1], 5, 2, 'f32'))
+    # every channel by itself: whatever the slice, the same sum
+    one = torch.cat([sapa_amd.av(attn.to(DEV), v[:, c:c + 1].to(DEV).contiguous(), 5, 2).cpu() for c in (0, C // 2, C - 1)], 1)
+    assert torch.equal(got[:, [0, C // 2, C - 1]], one)
+
+
 @pytest.mark.parametrize('W', [20, 22, 21, 36, 34, 33])
 def test_window_staging_vector_widths(coracle, W):
     """Row lengths that are multiples of 4, of 2 only, and odd select the
