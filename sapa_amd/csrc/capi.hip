@@ -918,12 +918,10 @@ int norm_project(const NormProject *f, int n, void *scratch, int B, int C, int O
         p = next;
     }
     hipError_t e = norm_fold_launch(nf, n, B, C, O, groups, eps, x_channels_last != 0, dtype, st);
-    for (int i = 0; i < n && e == hipSuccess; ++i) {
-        const void *b_b = f[i].bias_out ? nullptr : nf[i].b_out;
-        e = x_channels_last ? project_nhwc_launch(f[i].x, nf[i].w_out, b_b, f[i].out, B, C, O, (long)f[i].HW, dtype, st)
-                            : project_nchw_launch(f[i].x, nf[i].w_out, b_b, f[i].out, B, C, O, (long)f[i].HW,
-                                                  out_channels_last, dtype, st);
-    }
+    ProjectFeature pf[2] = {};
+    for (int i = 0; i < n; ++i)
+        pf[i] = ProjectFeature{f[i].x, nf[i].w_out, f[i].bias_out ? nullptr : nf[i].b_out, f[i].out, (long)f[i].HW};
+    if (e == hipSuccess) e = project_launch(pf, n, B, C, O, x_channels_last != 0, out_channels_last != 0, dtype, st);
     if (e == hipErrorNotSupported) return SAPA_ERR_UNSUPPORTED;
     return finish(e);
 }

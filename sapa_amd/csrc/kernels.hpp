@@ -103,7 +103,16 @@ hipError_t stream_mix_launch(const void *src, void *dst, long units, int reads, 
 // and 16 writing workgroups, each with one contiguous run of reps * 64 KiB
 hipError_t stream_split_launch(const void *src, void *dst, long groups, int reps, int nt, hipStream_t st);
 
-// sapa_project.hip: 1x1 projection of a channels-last 16-bit feature with per-image weights
+// sapa_project.hip: 1x1 projections with per-image weights of one feature, or in one launch of two with
+// the same B, C and O
+struct ProjectFeature {
+    const void *x, *w, *bias;
+    void *out;
+    long HW;
+};
+hipError_t project_launch(const ProjectFeature *f, int n, int B, int C, int O, bool x_channels_last, bool out_channels_last,
+                          int dtype, hipStream_t st);
+// ... of a channels-last feature
 hipError_t project_nhwc_launch(const void *x, const void *w, const void *bias, void *out, int B,
                                int C, int O, long HW, int dtype, hipStream_t st);
 // ... of a contiguous feature [B, C, HW] into [B, HW, O] (out_channels_last) or [B, O, HW]; fp32

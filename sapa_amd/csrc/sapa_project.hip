@@ -52,6 +52,15 @@ __device__ __forceinline__ Span span_of(int outputs) {
     return Span{outputs, o0, outputs - o0 < O ? outputs - o0 : O};
 }
 
+// A launch serves one feature, or two of the same B, C and O (a module's query and key features; blocks = 0: none), the
+// second's workgroups of an image behind the first's.  (Two that together do not fill the chip, see project_launch.)
+template <typename T> struct Feature {
+    const T *x, *w, *bias;
+    T *out;
+    long HW;
+    int tiles, blocks;                            // tiles per wave, workgroups per image
+};
+
 typedef unsigned u32;
 typedef u32 u32x2 __attribute__((ext_vector_type(2)));
 typedef u32 u32x4 __attribute__((ext_vector_type(4)));
@@ -87,8 +96,15 @@ __device__ __forceinline__ u32 pack2(float a, float b) {
 // C input channels, O outputs (both multiples of 16); tiles of 16 pixels
 template <typename T, int C, int O, bool WIDE>
 __global__ void __launch_bounds__(256)
-project_kernel(const T *__restrict__ x, const T *__restrict__ w, const T *__restrict__ bias,
-               T *__restrict__ out, long HW, int tiles_per_block, int outputs) {
+project_kernel(Feature<T> f0, Feature<T> f1, int outputs) {
+    const bool second = (int)blockIdx.x >= f0.blocks;
+    const Feature<T> f = second ? f1 : f0;
+    const long block = (int)blockIdx.x - (second ? f0.blocks : 0);
+    const int b = blockIdx.y;
+    const T *__restrict__ const x = f.x, *__restrict__ const w = f.w, *__restrict__ const bias = f.bias;
+    T *__restrict__ const out = f.out;
+    const long HW = f.HW;
+    const int tiles_per_wave = f.tiles;
     constexpr int RW = C / 2 + 4;                 // dwords per padded row of C 16-bit values
     constexpr int NL = C / 32;                    // 16-byte loads per lane and tile (16 rows of 2 C bytes)
     constexpr int NT = O / 16;                    // output tiles of 16 columns
@@ -98,7 +114,6 @@ project_kernel(const T *__restrict__ x, const T *__restrict__ w, const T *__rest
     u32 *wl = sh;                                 // weights: O rows of RW dwords
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     u32 *xt = sh + O * RW + wave * XT;            // this wave's tile
-    const int b = blockIdx.y;
     const T *xb = x + (long)b * HW * C;
     const Span sp = span_of<O, WIDE>(outputs);
     T *ob = out + (long)b * HW * sp.OT;
@@ -117,8 +132,8 @@ project_kernel(const T *__restrict__ x, const T *__restrict__ w, const T *__rest
     __syncthreads();
 
     const long ntiles = (HW + 15) / 16;
-    const long t0 = ((long)blockIdx.x * 4 + wave) * tiles_per_block;
-    const long t1 = t0 + tiles_per_block < ntiles ? t0 + tiles_per_block : ntiles;
+    const long t0 = (block * 4 + wave) * tiles_per_wave;
+    const long t1 = t0 + tiles_per_wave < ntiles ? t0 + tiles_per_wave : ntiles;
     const int r16 = lane & 15, kg = lane >> 4;    // row / column of a 16 x 16 tile, k group
     float bv[NT];
 #pragma unroll
@@ -196,22 +211,35 @@ project_kernel(const T *__restrict__ x, const T *__restrict__ w, const T *__rest
     }
 }
 
+// n features in tiles of `pixels`: tiles per wave and workgroups per image; false: too many workgroups.  At most 512
+// workgroups of 4 waves; a tile per wave only where all of them are resident, `resident` on each of 256 CUs (us with 2 tiles
+// per wave at least and so, modules: 256 channels, 1 image 50x84, planes 41 -> 36, 2 of 48x48 38 -> 34, 512 channels, 2 of
+// 32x32 42 -> 36; in two rounds, SAPA-D channels-last, 512 channels, 2 of 32x32, 53 -> 56).
+template <typename T>
+static bool spread16(const ProjectFeature *p, int n, Feature<T> (&f)[2], int B, int pixels, int blocks_o, int resident) {
+    long tiles[2] = {0, 0}, blocks[2] = {0, 0};
+    for (int i = 0; i < n; ++i) tiles[i] = (p[i].HW + pixels - 1) / pixels;
+    const long all = (tiles[0] + tiles[1]) * B * blocks_o;
+    long per = (all + 4L * 512 - 1) / (4L * 512);
+    if (per < 2 && all > 4L * 256 * resident) per = 2;
+    for (int i = 0; i < n; ++i) blocks[i] = (tiles[i] + 4 * per - 1) / (4 * per);
+    for (int i = 0; i < n; ++i)
+        f[i] = Feature<T>{(const T *)p[i].x, (const T *)p[i].w, (const T *)p[i].bias, (T *)p[i].out, p[i].HW, (int)per, (int)blocks[i]};
+    return blocks[0] <= 65535 * 32L && blocks[1] <= 65535 * 32L && B <= 65535 && blocks_o <= 65535;
+}
+
 template <typename T, int C, int O, bool WIDE = false>
-static hipError_t launch_co(const void *x, const void *w, const void *bias, void *out, int B, long HW,
-                            hipStream_t st, int outputs = O) {
+static hipError_t launch_co(const ProjectFeature *p, int n, int B, hipStream_t st, int outputs = O) {
     constexpr int RW = C / 2 + 4, OW = O / 2 + 4;
     constexpr int XT = 16 * RW > 16 * OW ? 16 * RW : 16 * OW;
     constexpr size_t lds = (size_t)(O * RW + 4 * XT) * 4;
     static_assert(lds <= 160 * 1024, "weights and tiles must fit LDS");
-    const long ntiles = (HW + 15) / 16;
     const int blocks_o = (outputs + O - 1) / O;
     // two workgroups are resident per CU (LDS) and the part has 256 CUs: one round of at most 512
-    // workgroups, at least 2 tiles per wave (16 images of 100 x 168 pixels, 256 -> 64: 37 us against
+    // workgroups (16 images of 100 x 168 pixels, 256 -> 64: 37 us against
     // 46 with a fixed 8 tiles per wave; 200 x 336 pixels: 141 against 146)
-    long per = (ntiles * B * blocks_o + 4L * 512 - 1) / (4L * 512);
-    if (per < 2) per = 2;
-    const long blocks = (ntiles + 4 * per - 1) / (4 * per);
-    if (blocks > 65535 * 32L || B > 65535 || blocks_o > 65535) return hipErrorNotSupported;
+    Feature<T> f[2] = {};
+    if (!spread16(p, n, f, B, 16, blocks_o, lds > 80 * 1024 ? 1 : 2)) return hipErrorNotSupported;
     auto kern = project_kernel<T, C, O, WIDE>;
     if (lds > 64 * 1024) {
         // more than the default 64 KB per workgroup: ask for it; a device that
@@ -226,8 +254,8 @@ static hipError_t launch_co(const void *x, const void *w, const void *bias, void
             return hipErrorNotSupported;
         }
     }
-    hipLaunchKernelGGL(kern, dim3((unsigned)blocks, B, blocks_o), dim3(256), lds, st, (const T *)x, (const T *)w,
-                       (const T *)bias, (T *)out, HW, (int)per, outputs);
+    hipLaunchKernelGGL(kern, dim3((unsigned)(f[0].blocks + f[1].blocks), B, blocks_o), dim3(256), lds, st, f[0], f[1],
+                       outputs);
     return hipGetLastError();
 }
 
@@ -241,8 +269,15 @@ static hipError_t launch_co(const void *x, const void *w, const void *bias, void
 // HW a multiple of 8 (16-byte pieces never run from one plane into the next).
 template <typename T, int C, int O, bool OUT_CL, bool WIDE>
 __global__ void __launch_bounds__(256)
-project16p_kernel(const T *__restrict__ x, const T *__restrict__ w, const T *__restrict__ bias,
-                  T *__restrict__ out, long HW, int tiles_per_wave, int outputs) {
+project16p_kernel(Feature<T> f0, Feature<T> f1, int outputs) {
+    const bool second = (int)blockIdx.x >= f0.blocks;
+    const Feature<T> f = second ? f1 : f0;
+    const long block = (int)blockIdx.x - (second ? f0.blocks : 0);
+    const int b = blockIdx.y;
+    const T *__restrict__ const x = f.x, *__restrict__ const w = f.w, *__restrict__ const bias = f.bias;
+    T *__restrict__ const out = f.out;
+    const long HW = f.HW;
+    const int tiles_per_wave = f.tiles;
     typedef short s16x4 __attribute__((ext_vector_type(4)));
     constexpr int NW = 4;
     constexpr int RW = C / 2 + 4;                 // dwords per padded row of C 16-bit values
@@ -259,8 +294,6 @@ project16p_kernel(const T *__restrict__ x, const T *__restrict__ w, const T *__r
     u32 *wl = sh;                                 // weights: O rows of RW dwords
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     u32 *xt = sh + O * RW + wave * WF;            // this wave's x tile / result tile
-    const int b = blockIdx.y;
-
     const Span sp = span_of<O, WIDE>(outputs);
     // the image's weights -> LDS, 8 channels per thread and step: two groups of 4, which lie 8
     // places apart in the step's order
@@ -281,7 +314,7 @@ project16p_kernel(const T *__restrict__ x, const T *__restrict__ w, const T *__r
     __syncthreads();
 
     const long ntiles = (HW + 63) / 64;
-    const long t0 = ((long)blockIdx.x * NW + wave) * tiles_per_wave;
+    const long t0 = (block * NW + wave) * tiles_per_wave;
     const long t1 = t0 + tiles_per_wave < ntiles ? t0 + tiles_per_wave : ntiles;
     if (t0 >= t1) return;
     const int r16 = lane & 15, kg = lane >> 4;
@@ -385,31 +418,27 @@ project16p_kernel(const T *__restrict__ x, const T *__restrict__ w, const T *__r
 }
 
 template <typename T, int C, int O, bool OUT_CL, bool WIDE = false>
-static hipError_t launch16p_co(const void *x, const void *w, const void *bias, void *out, int B, long HW,
-                               hipStream_t st, int outputs = O) {
+static hipError_t launch16p_co(const ProjectFeature *p, int n, int B, hipStream_t st, int outputs = O) {
     constexpr int RT = OUT_CL ? 16 * (O / 2 + 4) : 16 * 36, XT = 32 * 40;
     constexpr size_t lds = (size_t)(O * (C / 2 + 4) + 4 * (RT > XT ? RT : XT)) * 4;
     static_assert(lds <= 64 * 1024, "weights and tiles within the default LDS of a workgroup");
-    if (HW % 8 != 0 || HW * (long)(C > outputs ? C : outputs) * 2 >= (1L << 31)) return hipErrorNotSupported;
-    const long ntiles = (HW + 63) / 64;
+    for (int i = 0; i < n; ++i)
+        if (p[i].HW % 8 != 0 || p[i].HW * (long)(C > outputs ? C : outputs) * 2 >= (1L << 31)) return hipErrorNotSupported;
     const int blocks_o = (outputs + O - 1) / O;
     // two workgroups are resident per CU (their registers) and the part has 256 CUs: one round of
-    // at most 512 workgroups, at least 2 tiles per wave (q projection at 16 x 200 x 336 pixels:
+    // at most 512 workgroups (q projection at 16 x 200 x 336 pixels:
     // 140 us against 152 with 704 workgroups)
-    long per = (ntiles * B * blocks_o + 4L * 512 - 1) / (4L * 512);
-    if (per < 2) per = 2;
-    const long blocks = (ntiles + 4 * per - 1) / (4 * per);
-    if (blocks > 65535 * 32L || B > 65535 || blocks_o > 65535) return hipErrorNotSupported;
-    hipLaunchKernelGGL((project16p_kernel<T, C, O, OUT_CL, WIDE>), dim3((unsigned)blocks, B, blocks_o), dim3(256), lds,
-                       st, (const T *)x, (const T *)w, (const T *)bias, (T *)out, HW, (int)per, outputs);
+    Feature<T> f[2] = {};
+    if (!spread16(p, n, f, B, 64, blocks_o, 2)) return hipErrorNotSupported;
+    hipLaunchKernelGGL((project16p_kernel<T, C, O, OUT_CL, WIDE>), dim3((unsigned)(f[0].blocks + f[1].blocks), B, blocks_o),
+                       dim3(256), lds, st, f[0], f[1], outputs);
     return hipGetLastError();
 }
 
 template <typename T, bool OUT_CL>
-static hipError_t launch16p(const void *x, const void *w, const void *bias, void *out, int B, int C, int O,
-                            long HW, hipStream_t st) {
+static hipError_t launch16p(const ProjectFeature *p, int n, int B, int C, int O, hipStream_t st) {
 #define SAPA_PROJECT_CASE(CV, OV) \
-    if (C == CV && O == OV) return launch16p_co<T, CV, OV, OUT_CL>(x, w, bias, out, B, HW, st);
+    if (C == CV && O == OV) return launch16p_co<T, CV, OV, OUT_CL>(p, n, B, st);
     SAPA_PROJECT_CASE(64, 32) SAPA_PROJECT_CASE(64, 64)
     SAPA_PROJECT_CASE(128, 32) SAPA_PROJECT_CASE(128, 64)
     SAPA_PROJECT_CASE(256, 32) SAPA_PROJECT_CASE(256, 64)
@@ -466,8 +495,15 @@ __device__ __forceinline__ f32x4 mma32(u32x4 a, u32x4 b, f32x4 c) {
 // image 32x32 4.05 -> 4.6).
 template <int C, int O, bool IN_CL, bool OUT_CL, bool WIDE, int NW>
 __global__ void __launch_bounds__(64 * NW)
-project32_kernel(const float *__restrict__ x, const float *__restrict__ w, const float *__restrict__ bias,
-                 float *__restrict__ out, long HW, int tiles_per_wave, int waves, int outputs) {
+project32_kernel(Feature<float> f0, Feature<float> f1, int waves, int outputs) {
+    const bool second = (int)blockIdx.x >= f0.blocks;
+    const Feature<float> f = second ? f1 : f0;
+    const long block = (int)blockIdx.x - (second ? f0.blocks : 0);
+    const int b = blockIdx.y;
+    const float *__restrict__ const x = f.x, *__restrict__ const w = f.w, *__restrict__ const bias = f.bias;
+    float *__restrict__ const out = f.out;
+    const long HW = f.HW;
+    const int tiles_per_wave = f.tiles;
     static_assert(IN_CL ? OUT_CL : true, "channels-last features give channels-last projections");
     constexpr int RW = C / 2 + 4;                 // dwords per padded row of C bf16 values
     constexpr int PLANE = O * RW;                 // dwords per piece plane
@@ -484,15 +520,13 @@ project32_kernel(const float *__restrict__ x, const float *__restrict__ w, const
     u32 *wl = sh;                                 // weights: 3 planes of O rows of RW dwords
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     float *rt = (float *)(sh + 3 * PLANE) + wave * WF;          // this wave's x tile / result tile
-    const int b = blockIdx.y;
-
     const Span sp = span_of<O, WIDE>(outputs);
 
     const long ntiles = (HW + 31) / 32;
     // tiles t0, t0 + stride .. below t1 (waves past `waves` help with the weights only)
     const bool neighbours = NW > 8 || (!IN_CL && HW % 32 != 0);
-    const long first = (long)blockIdx.x * waves * tiles_per_wave, last = first + (long)waves * tiles_per_wave;
-    const long t0 = neighbours ? first + wave : ((long)blockIdx.x * waves + wave) * tiles_per_wave;
+    const long first = block * waves * tiles_per_wave, last = first + (long)waves * tiles_per_wave;
+    const long t0 = neighbours ? first + wave : (block * waves + wave) * tiles_per_wave;
     const long t1 = wave >= waves ? t0 : neighbours ? (last < ntiles ? last : ntiles)
                                                     : (t0 + tiles_per_wave < ntiles ? t0 + tiles_per_wave : ntiles);
     const long stride = neighbours ? waves : 1;
@@ -688,14 +722,15 @@ project32_kernel(const float *__restrict__ x, const float *__restrict__ w, const
 
 // How a projection's tiles are spread: tiles per wave, waves per workgroup that have some, workgroups per image
 struct Spread {
-    long per, blocks;
+    long per, blocks[2];
     int waves;
 };
 // One workgroup is resident per CU (its weight planes fill most of the LDS) and the part has
 // 256 CUs: two full rounds of workgroups where that leaves a wave 8 tiles or more (6 of 12 waves), else one
 // (16 images: 200x336 pixels 301 us in two rounds against 315 in one; 100x168 pixels 71 us in
 // one round against 98 in 272 workgroups; 256 -> 288, 8 images 128x128, 8 waves, 119 us in one against 130)
-static Spread spread32(long ntiles, long sets, int nw) {
+static Spread spread32(const long (&tiles)[2], long sets, int nw) {
+    const long ntiles = tiles[0] + tiles[1];
     const long slots = 256;
     long blocks = 2 * slots / sets > 1 ? 2 * slots / sets : 1;
     long per = (ntiles + nw * blocks - 1) / (nw * blocks);
@@ -711,17 +746,20 @@ static Spread spread32(long ntiles, long sets, int nw) {
     int waves = (int)((ntiles + blocks * per - 1) / (blocks * per));
     waves = waves < 1 ? 1 : waves > nw ? nw : waves;
     if (nw == 8 && per > 1 && waves < 6) waves = nw;
-    return Spread{per, (ntiles + waves * per - 1) / (waves * per), waves};
+    return Spread{per, {(tiles[0] + waves * per - 1) / (waves * per), (tiles[1] + waves * per - 1) / (waves * per)}, waves};
 }
 
 template <int C, int O, bool IN_CL, bool OUT_CL, bool WIDE, int NW>
-static hipError_t launch32_waves(const void *x, const void *w, const void *bias, void *out, int B, long HW,
-                                 hipStream_t st, int outputs, const Spread &s) {
+static hipError_t launch32_waves(const ProjectFeature *p, int n, int B, hipStream_t st, int outputs, const Spread &s) {
     constexpr int RT = OUT_CL ? 16 * (O + 4) : 16 * 36, XB = IN_CL ? 0 : 32 * 32;
     constexpr size_t lds = (size_t)(3 * O * (C / 2 + 4) + NW * (RT > XB ? RT : XB)) * 4;
     static_assert(lds <= 160 * 1024, "weights and tiles must fit LDS");
     const int blocks_o = (outputs + O - 1) / O;
-    if (s.blocks > 65535 * 32L || B > 65535 || blocks_o > 65535) return hipErrorNotSupported;
+    Feature<float> f[2] = {};
+    for (int i = 0; i < n; ++i)
+        f[i] = Feature<float>{(const float *)p[i].x, (const float *)p[i].w, (const float *)p[i].bias, (float *)p[i].out, p[i].HW,
+                              (int)s.per, (int)s.blocks[i]};
+    if (s.blocks[0] > 65535 * 32L || s.blocks[1] > 65535 * 32L || B > 65535 || blocks_o > 65535) return hipErrorNotSupported;
     auto kern = project32_kernel<C, O, IN_CL, OUT_CL, WIDE, NW>;
     if (lds > 64 * 1024) {
         int dev = 0, most = 0;
@@ -734,18 +772,21 @@ static hipError_t launch32_waves(const void *x, const void *w, const void *bias,
             return hipErrorNotSupported;
         }
     }
-    hipLaunchKernelGGL(kern, dim3((unsigned)s.blocks, B, blocks_o), dim3(64 * NW), lds, st, (const float *)x, (const float *)w,
-                       (const float *)bias, (float *)out, HW, (int)s.per, s.waves, outputs);
+    hipLaunchKernelGGL(kern, dim3((unsigned)(f[0].blocks + f[1].blocks), B, blocks_o), dim3(64 * NW), lds, st, f[0], f[1],
+                       s.waves, outputs);
     return hipGetLastError();
 }
 
 template <int C, int O, bool IN_CL, bool OUT_CL, bool WIDE = false>
-static hipError_t launch32_co(const void *x, const void *w, const void *bias, void *out, int B, long HW,
-                              hipStream_t st, int outputs = O) {
-    if (!OUT_CL && HW % 4 != 0) return hipErrorNotSupported;
-    // 32-bit byte offsets inside an image
-    if (HW * (long)(C > outputs ? C : outputs) * 4 >= (1L << 31)) return hipErrorNotSupported;
-    const long ntiles = (HW + 31) / 32, sets = (long)B * ((outputs + O - 1) / O);     // sets: workgroups that share a pixel range's place
+static hipError_t launch32_co(const ProjectFeature *p, int n, int B, hipStream_t st, int outputs = O) {
+    long ntiles[2] = {0, 0};
+    for (int i = 0; i < n; ++i) {
+        if (!OUT_CL && p[i].HW % 4 != 0) return hipErrorNotSupported;
+        // 32-bit byte offsets inside an image
+        if (p[i].HW * (long)(C > outputs ? C : outputs) * 4 >= (1L << 31)) return hipErrorNotSupported;
+        ntiles[i] = (p[i].HW + 31) / 32;
+    }
+    const long sets = (long)B * ((outputs + O - 1) / O);     // sets: workgroups that share a pixel range's place
     const Spread s8 = spread32(ntiles, sets, 8), s12 = spread32(ntiles, sets, 12);
     // Twelve waves where they shorten a wave's chain of tiles to what is asked for below (eight have twice the steps of
     // x in flight and no bar to moving work between steps).  us with 8 / 12 waves, from planes: 5 tiles to 3 each
@@ -759,15 +800,14 @@ static hipError_t launch32_co(const void *x, const void *w, const void *bias, vo
     // (of 64 channels not to a single tile: 2 images 192x192, 64 -> 32 / 64, 7.7 / 8.3 and 10.1 / 10.8; 256 -> 64 from
     // channels-last features also over one tile each for 3 to 6 waves: 8 images 64x64 13.9 / 12.5)
     if ((10 * s8.per >= ASKED * s12.per && (C > 64 || s12.per > 1)) || (IN_CL && C == 256 && O == 64 && s8.per == 1 && s8.waves > 2 && s8.waves <= 6))
-        return launch32_waves<C, O, IN_CL, OUT_CL, WIDE, C == 128 && O == 32 ? 8 : 12>(x, w, bias, out, B, HW, st, outputs, s12);
-    return launch32_waves<C, O, IN_CL, OUT_CL, WIDE, 8>(x, w, bias, out, B, HW, st, outputs, s8);
+        return launch32_waves<C, O, IN_CL, OUT_CL, WIDE, C == 128 && O == 32 ? 8 : 12>(p, n, B, st, outputs, s12);
+    return launch32_waves<C, O, IN_CL, OUT_CL, WIDE, 8>(p, n, B, st, outputs, s8);
 }
 
 template <bool IN_CL, bool OUT_CL>
-static hipError_t launch32(const void *x, const void *w, const void *bias, void *out, int B, int C, int O,
-                           long HW, hipStream_t st) {
+static hipError_t launch32(const ProjectFeature *p, int n, int B, int C, int O, hipStream_t st) {
 #define SAPA_PROJECT_CASE(CV, OV) \
-    if (C == CV && O == OV) return launch32_co<CV, OV, IN_CL, OUT_CL>(x, w, bias, out, B, HW, st);
+    if (C == CV && O == OV) return launch32_co<CV, OV, IN_CL, OUT_CL>(p, n, B, st);
     SAPA_PROJECT_CASE(64, 32) SAPA_PROJECT_CASE(64, 64)
     SAPA_PROJECT_CASE(128, 32) SAPA_PROJECT_CASE(128, 64)
     SAPA_PROJECT_CASE(256, 32) SAPA_PROJECT_CASE(256, 64)
@@ -777,10 +817,9 @@ static hipError_t launch32(const void *x, const void *w, const void *bias, void 
 }
 
 template <typename T>
-static hipError_t launch_t(const void *x, const void *w, const void *bias, void *out, int B, int C,
-                           int O, long HW, hipStream_t st) {
+static hipError_t launch_t(const ProjectFeature *p, int n, int B, int C, int O, hipStream_t st) {
 #define SAPA_PROJECT_CASE(CV, OV) \
-    if (C == CV && O == OV) return launch_co<T, CV, OV>(x, w, bias, out, B, HW, st);
+    if (C == CV && O == OV) return launch_co<T, CV, OV>(p, n, B, st);
     SAPA_PROJECT_CASE(64, 32) SAPA_PROJECT_CASE(64, 64)
     SAPA_PROJECT_CASE(128, 32) SAPA_PROJECT_CASE(128, 64) SAPA_PROJECT_CASE(128, 128)
     SAPA_PROJECT_CASE(256, 32) SAPA_PROJECT_CASE(256, 64) SAPA_PROJECT_CASE(256, 128)
@@ -791,13 +830,12 @@ static hipError_t launch_t(const void *x, const void *w, const void *bias, void 
 
 // one output block per 64 outputs (32 where 512 channels' weights leave no room for more)
 template <typename T, bool IN_CL, bool OUT_CL>
-static hipError_t launch_shared(const void *x, const void *w, const void *bias, void *out, int B, int C, int O,
-                                long HW, hipStream_t st) {
+static hipError_t launch_shared(const ProjectFeature *p, int n, int B, int C, int O, hipStream_t st) {
 #define SAPA_SHARED_CASE(CV, OV)                                                                                     \
     if (C == CV) {                                                                                                   \
-        if constexpr (sizeof(T) == 4) return launch32_co<CV, OV, IN_CL, OUT_CL, true>(x, w, bias, out, B, HW, st, O); \
-        else if constexpr (IN_CL) return launch_co<T, CV, OV, true>(x, w, bias, out, B, HW, st, O);                  \
-        else return launch16p_co<T, CV, OV, OUT_CL, true>(x, w, bias, out, B, HW, st, O);                            \
+        if constexpr (sizeof(T) == 4) return launch32_co<CV, OV, IN_CL, OUT_CL, true>(p, n, B, st, O); \
+        else if constexpr (IN_CL) return launch_co<T, CV, OV, true>(p, n, B, st, O);                  \
+        else return launch16p_co<T, CV, OV, OUT_CL, true>(p, n, B, st, O);                            \
     }
     SAPA_SHARED_CASE(64, 64) SAPA_SHARED_CASE(128, 64) SAPA_SHARED_CASE(256, 64) SAPA_SHARED_CASE(512, 32)
 #undef SAPA_SHARED_CASE
@@ -814,11 +852,12 @@ hipError_t project_shared_launch(const void *x, const void *w, const void *bias,
     const void *ptrs[3] = {x, w, out};
     for (const void *p : ptrs)
         if ((uintptr_t)p % 16 != 0) return hipErrorNotSupported;
+    const ProjectFeature f{x, w, bias, out, HW};
     if (O % 8 != 0 || (x_channels_last && !out_channels_last)) return hipErrorNotSupported;
 #define SAPA_SHARED(TV)                                                                                       \
-    return x_channels_last ? project::launch_shared<TV, true, true>(x, w, bias, out, B, C, O, HW, st)         \
-           : out_channels_last ? project::launch_shared<TV, false, true>(x, w, bias, out, B, C, O, HW, st)    \
-                               : project::launch_shared<TV, false, false>(x, w, bias, out, B, C, O, HW, st)
+    return x_channels_last ? project::launch_shared<TV, true, true>(&f, 1, B, C, O, st)         \
+           : out_channels_last ? project::launch_shared<TV, false, true>(&f, 1, B, C, O, st)    \
+                               : project::launch_shared<TV, false, false>(&f, 1, B, C, O, st)
     if (dtype == 0) SAPA_SHARED(float);
     if (dtype == 2) SAPA_SHARED(f16_t);
     if (dtype == 3) SAPA_SHARED(bf16_t);
@@ -826,39 +865,49 @@ hipError_t project_shared_launch(const void *x, const void *w, const void *bias,
     return hipErrorNotSupported;
 }
 
-// x [B, HW, C], w [B, O, C], bias [B, O] or null, out [B, HW, O]; f16 / bf16 / fp32;
-// (C, O) among the instantiated pairs (C in {64, 128, 256, 512}, O in {32, 64, 128}; fp32:
-// those whose three weight planes fit LDS); every pointer aligned to 16 bytes.
-// hipErrorNotSupported otherwise.
-hipError_t project_nhwc_launch(const void *x, const void *w, const void *bias, void *out, int B,
-                               int C, int O, long HW, int dtype, hipStream_t st) {
-    const void *ptrs[3] = {x, w, out};
-    for (const void *p : ptrs)
-        if ((uintptr_t)p % 16 != 0) return hipErrorNotSupported;
-    if (dtype == 0) return project::launch32<true, true>(x, w, bias, out, B, C, O, HW, st);
-    if (dtype == 2) return project::launch_t<f16_t>(x, w, bias, out, B, C, O, HW, st);
-    if (dtype == 3) return project::launch_t<bf16_t>(x, w, bias, out, B, C, O, HW, st);
-    return hipErrorNotSupported;
+// One projection, or two of the same B, C and O, with per-image weights w [B, O, C] and bias [B, O] or null:
+//   x_channels_last: x [B, HW, C] -> out [B, HW, O]; f16 / bf16 / fp32; (C, O) among the instantiated pairs (C in
+//     {64, 128, 256, 512}, O in {32, 64, 128}; fp32: those whose three weight planes fit LDS);
+//   else x [B, C, HW] (planes) -> out [B, HW, O] (out_channels_last) or [B, O, HW]; the (C, O) pairs of the fp32
+//     kernel; fp32: HW a multiple of 4 for a planar result; f16 / bf16: HW a multiple of 8.
+// x, w and out aligned to 16 bytes.  hipErrorNotSupported otherwise (nothing is launched then).
+hipError_t project_launch(const ProjectFeature *f, int n, int B, int C, int O, bool x_channels_last, bool out_channels_last,
+                          int dtype, hipStream_t st) {
+    for (int i = 0; i < n; ++i)
+        if (((uintptr_t)f[i].x | (uintptr_t)f[i].w | (uintptr_t)f[i].out) % 16 != 0) return hipErrorNotSupported;
+    // Two that together have no more tiles than the chip's waves (2048) go as one launch: the smaller one's latencies
+    // lie beside the other's.  Modules, us before and so: bf16, 8 images 16x16, C=256, 35 -> 26 (29 with 2 tiles per wave
+    // at least), channels-last 41 -> 36; fp32 45 -> 36, 4 of 24x24 47 -> 40.  Larger ones take a launch each: 16 of 50x84
+    // in fp32 102 -> 109 for the two projections, 100x168 in channels-last bf16 176 -> 172 and the operator behind them 3 more.
+    const long tile = dtype == 0 ? 32 : x_channels_last ? 16 : 64;
+    if (n == 2 && ((f[0].HW + tile - 1) / tile + (f[1].HW + tile - 1) / tile) * B > 2048) {
+        const hipError_t e = project_launch(f, 1, B, C, O, x_channels_last, out_channels_last, dtype, st);
+        return e == hipSuccess ? project_launch(f + 1, 1, B, C, O, x_channels_last, out_channels_last, dtype, st) : e;
+    }
+    if (x_channels_last) {
+        if (dtype == 0) return project::launch32<true, true>(f, n, B, C, O, st);
+        if (dtype == 2) return project::launch_t<f16_t>(f, n, B, C, O, st);
+        if (dtype == 3) return project::launch_t<bf16_t>(f, n, B, C, O, st);
+        return hipErrorNotSupported;
+    }
+    if (dtype == 2)
+        return out_channels_last ? project::launch16p<f16_t, true>(f, n, B, C, O, st) : project::launch16p<f16_t, false>(f, n, B, C, O, st);
+    if (dtype == 3)
+        return out_channels_last ? project::launch16p<bf16_t, true>(f, n, B, C, O, st) : project::launch16p<bf16_t, false>(f, n, B, C, O, st);
+    if (dtype != 0) return hipErrorNotSupported;
+    return out_channels_last ? project::launch32<false, true>(f, n, B, C, O, st) : project::launch32<false, false>(f, n, B, C, O, st);
 }
 
-// The same projection of a contiguous feature x [B, C, HW] (planes): out [B, HW, O]
-// (out_channels_last) or [B, O, HW]; the (C, O) pairs of the fp32 kernel above; fp32: HW a
-// multiple of 4 for a planar result; f16 / bf16: HW a multiple of 8; x and out aligned to 16
-// bytes.  hipErrorNotSupported otherwise.
-hipError_t project_nchw_launch(const void *x, const void *w, const void *bias, void *out, int B, int C,
-                               int O, long HW, int out_channels_last, int dtype, hipStream_t st) {
-    const void *ptrs[3] = {x, w, out};
-    for (const void *p : ptrs)
-        if ((uintptr_t)p % 16 != 0) return hipErrorNotSupported;
-    if (dtype == 2)
-        return out_channels_last ? project::launch16p<f16_t, true>(x, w, bias, out, B, C, O, HW, st)
-                                 : project::launch16p<f16_t, false>(x, w, bias, out, B, C, O, HW, st);
-    if (dtype == 3)
-        return out_channels_last ? project::launch16p<bf16_t, true>(x, w, bias, out, B, C, O, HW, st)
-                                 : project::launch16p<bf16_t, false>(x, w, bias, out, B, C, O, HW, st);
-    if (dtype != 0) return hipErrorNotSupported;
-    return out_channels_last ? project::launch32<false, true>(x, w, bias, out, B, C, O, HW, st)
-                             : project::launch32<false, false>(x, w, bias, out, B, C, O, HW, st);
+hipError_t project_nhwc_launch(const void *x, const void *w, const void *bias, void *out, int B, int C, int O, long HW,
+                               int dtype, hipStream_t st) {
+    const ProjectFeature f{x, w, bias, out, HW};
+    return project_launch(&f, 1, B, C, O, true, true, dtype, st);
+}
+
+hipError_t project_nchw_launch(const void *x, const void *w, const void *bias, void *out, int B, int C, int O, long HW,
+                               int out_channels_last, int dtype, hipStream_t st) {
+    const ProjectFeature f{x, w, bias, out, HW};
+    return project_launch(&f, 1, B, C, O, false, out_channels_last != 0, dtype, st);
 }
 
 // Whether project_nhwc_launch (x_channels_last; the result is channels-last then) / project_nchw_launch

@@ -169,6 +169,8 @@ def test_small_separate_operators(dtype, B, d, C, H, W):
     (1, 64, 32, 2, 4),         # one chunk per feature
     (2, 256, 64, 100, 168),    # chunks shared by several threads in one feature, a thread per channel in the other
     (3, 512, 32, 24, 20),      # more channels than the threads of a block of few chunks
+    # both projections in one launch, a last tile of few pixels each; 2041 tiles, the most for it in fp32; 2198
+    (8, 256, 64, 25, 40), (13, 256, 64, 25, 40), (14, 256, 64, 25, 40),
 ])
 def test_norm_project_of_two_features(dtype, channels_last, B, C, O, h, w):
     """sapa_norm_project_pair gives what sapa_norm_project gives for each feature.  (Where one feature
