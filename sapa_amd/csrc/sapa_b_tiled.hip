@@ -55,7 +55,7 @@ __global__ void __launch_bounds__(64 * NWX * NWY * (S / CY))
 sapa_b_tiled_kernel(const T *__restrict__ q, const T *__restrict__ key,
                     const T *__restrict__ attn_in, const T *__restrict__ value,
                     T *__restrict__ out, int d, int C, int H, int W, int tiles_x, int tiles_y,
-                    int nblocks, int per_xcd, int cgroups, int cper) {
+                    int nblocks, int per_xcd, int cgroups, int cper, int whole) {
     typedef float A;
     constexpr int KK = K * K, R = (K - 1) / 2;
     constexpr int NSUB = S / CY;           // waves sharing one band of parent rows
@@ -128,17 +128,21 @@ sapa_b_tiled_kernel(const T *__restrict__ q, const T *__restrict__ key,
     // Workgroups are handed to the 8 XCDs round-robin; give each XCD a
     // contiguous run of tiles so that neighbouring tiles (which share halo
     // rows) meet in the same L2.
-    const int logical = (int)(blockIdx.x % 8) * per_xcd + (int)(blockIdx.x / 8);
+    // (whole >= 0: the first `whole` tiles of an XCD's run take all channels, the others `cgroups` slices each)
+    const int at = (int)(blockIdx.x / 8);
+    const bool sliced = whole >= 0 && at >= whole;
+    const int rest = per_xcd - whole;
+    const int logical = (int)(blockIdx.x % 8) * per_xcd + (sliced ? whole + (at - whole) % rest : at);
     if (logical >= nblocks) return;
     // logical = ((n * cgroups + cg) * tiles_y + ty) * tiles_x + tx; a small
     // problem is split over `cgroups` slices of `cper` value channels each
     // (every slice recomputes the logits) so that the chip is still filled
     const int tx = logical % tiles_x;
     const int ty = (logical / tiles_x) % tiles_y;
-    const int cg = (logical / (tiles_x * tiles_y)) % cgroups;
-    const int n = logical / (tiles_x * tiles_y * cgroups);
+    const int cg = whole >= 0 ? (sliced ? (at - whole) / rest : 0) : (logical / (tiles_x * tiles_y)) % cgroups;
+    const int n = logical / (tiles_x * tiles_y * (whole >= 0 ? 1 : cgroups));
     const int cbeg = cg * cper;                      // first value channel of this slice
-    const int cend = cbeg + cper < C ? cbeg + cper : C;
+    const int cend = cbeg + cper < C && (whole < 0 || sliced) ? cbeg + cper : C;
     if (DO_AV && cbeg >= C) return;                  // rounding left this slice empty
 
     const int tid = threadIdx.x;
@@ -504,9 +508,10 @@ static hipError_t launch_mode(int mode, bool wide, const void *q, const void *ke
     // up to two workgroups per CU (256 CUs) -- beyond that the recomputed
     // logits cost more than the added parallelism gains (measured).  A slice
     // is a multiple of CH channels and at least 4 chunks long.
+    const long tiles = (long)tiles_x * tiles_y * B;
+    int whole = -1;
     int cgroups = 1;
     if (mode == TILED_FUSED || mode == TILED_AV) {
-        const long tiles = (long)tiles_x * tiles_y * B;
         const int max_groups = C / (4 * CH) > 0 ? C / (4 * CH) : 1;
         // (16-bit tensors: up to four per CU -- their recomputed logits cost
         // relatively less -- measured on the FPN levels)
@@ -515,27 +520,37 @@ static hipError_t launch_mode(int mode, bool wide, const void *q, const void *ke
         // The aggregation of fp32 tensors that are staged straight into LDS recomputes nothing in a slice: where those
         // workgroups would leave CUs idle in their last round, slices of 4 chunks (256 channels, us before and
         // now: 16 images 50x84, 336 tiles, 134 -> 109; 4 of 100x168, 312 tiles, 139 -> 113; 5 of 64x64, 80 tiles,
-        // 32 -> 26; full rounds are not better off: 2 of 120x120, 120 tiles in 4 slices, 37 -> 41).  Beyond 384 tiles the tile's weights, which every slice reads again, cost more than that (468
-        // tiles 155 and 160, 702 tiles 214 and 243).
+        // 32 -> 26; full rounds are not better off: 2 of 120x120, 120 tiles in 4 slices, 37 -> 41).  Beyond 384 tiles
+        // the tile's weights, which every slice reads again, cost more than that (468 tiles 155 and 160, 702 tiles 214
+        // and 243).
         const long round = 256, rounds = (tiles * cgroups + round - 1) / round;
-        if (mode == TILED_AV && std::is_same<T, float>::value && VEC == 4 && tiles <= 384 &&
-            10 * tiles * cgroups < 9 * round * rounds)
+        const bool direct = std::is_same<T, float>::value && VEC == 4, aggregate = mode == TILED_AV;
+        if (direct && aggregate && tiles <= 384 && 10 * tiles * cgroups < 9 * round * rounds &&
+            (tiles <= round || max_groups > 2))
             cgroups = max_groups;
+        // Else only the tiles behind the last full round, in two or three slices each: aggregation, 6 images 100x168, 468
+        // tiles, 154 -> 142 us, 9 images 214 -> 205, 16 images 357 -> 350; 64 channels, 16 of 50x84, 31 -> 28.  Fused, whose
+        // slices recompute the logits, with at most 8 tiles per XCD behind one full round (16, 17, 20 images 64x64, 256 /
+        // 272 / 320 tiles, 93 / 135 / 157 -> 93 / 123 / 139; 4 of 100x168, 312 tiles, 133 -> 123; 336 tiles 132 -> 139).
+        else if (direct && cgroups == 1 && max_groups > 1 && tiles > round && (aggregate || tiles <= 320)) {
+            const int run = (int)((tiles + 7) / 8);           // an XCD's tiles, for its 32 CUs
+            if (run % 32) whole = run - run % 32, cgroups = aggregate && max_groups > 2 ? 3 : 2;
+        }
 #ifdef SAPA_TUNE_CGROUPS
         cgroups = SAPA_TUNE_CGROUPS;
 #endif
     }
     const int cper = ((C + cgroups - 1) / cgroups + CH - 1) / CH * CH;
-    const long nb = (long)tiles_x * tiles_y * B * cgroups;
+    const long nb = tiles * (whole >= 0 ? 1 : cgroups);
     if (nb > (1L << 30)) return hipErrorNotSupported;
     // the output leaves through 32-bit byte offsets inside one chunk of CH planes
     if ((long)CH * H * S * W * S * (long)sizeof(T) > (1L << 31)) return hipErrorNotSupported;
     const int per_xcd = (int)((nb + 7) / 8);
-    const dim3 grid(per_xcd * 8), block(NT);
+    const dim3 grid((whole >= 0 ? whole + (per_xcd - whole) * cgroups : per_xcd) * 8), block(NT);
 #define SAPA_TM_LAUNCH(M, WD)                                                                 \
     hipLaunchKernelGGL((sapa_b_tiled_kernel<T, K, S, CY, NWX, NWY, CH, VEC, WLX, M, WD>), grid, block, 0, st, \
                        (const T *)q, (const T *)key, (const T *)attn_in, (const T *)value,    \
-                       (T *)out, d, C, H, W, tiles_x, tiles_y, (int)nb, per_xcd, cgroups, cper)
+                       (T *)out, d, C, H, W, tiles_x, tiles_y, (int)nb, per_xcd, cgroups, cper, whole)
 #define SAPA_TM_CASE(M)                                                                       \
     case M:                                                                                   \
         SAPA_TM_LAUNCH(M, false);                                                             \

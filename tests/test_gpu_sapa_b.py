@@ -595,6 +595,24 @@ def test_av_in_slices_of_32_channels(coracle, shape):
     assert torch.equal(got[:, [0, C // 2, C - 1]], one)
 
 
+# more tiles than fit one round: the ones behind it in two or three slices, in runs of tiles whose last one is short
+@pytest.mark.parametrize('B,C,H,W', [(67, 70, 32, 32), (100, 40, 32, 32), (65, 64, 29, 28), (260, 96, 8, 32)])
+def test_tiles_behind_the_last_full_round_in_slices(coracle, B, C, H, W):
+    g = gen(142)
+    q, key = randn(g, B, 8, 2 * H, 2 * W), randn(g, B, 8, H, W)
+    attn, v = torch.softmax(randn(g, B, 25, 2 * H, 2 * W), 1), randn(g, B, C, H, W)
+    got, fused = sapa_amd.av(*dev(attn, v), 5, 2).cpu(), sapa_amd.sapa_fused(*dev(q, key, v), 5, 2).cpu()
+    for n in (0, B // 2, B - 1):
+        s = slice(n, n + 1)
+        assert torch.equal(got[s], coracle.av(attn[s], v[s], 5, 2, 'f32'))
+        assert_f32_close(fused[s], coracle.sapa_fused(q[s], key[s], v[s], 5, 2, 'f32'), 'fused')
+    # every channel by itself: whatever the slice, the same sums
+    for c in (0, C // 2, C - 1):
+        vc = v[:, c:c + 1].to(DEV).contiguous()
+        assert torch.equal(got[:, c:c + 1], sapa_amd.av(attn.to(DEV), vc, 5, 2).cpu())
+        assert torch.equal(fused[:, c:c + 1], sapa_amd.sapa_fused(q.to(DEV), key.to(DEV), vc, 5, 2).cpu())
+
+
 @pytest.mark.parametrize('W', [20, 22, 21, 36, 34, 33])
 def test_window_staging_vector_widths(coracle, W):
     """Row lengths that are multiples of 4, of 2 only, and odd select the
