@@ -492,6 +492,12 @@ static hipError_t launch_geom(const void *q, const void *key, const void *value,
     // 256 / 512 workgroups; 32x32: 16.6, 12.6 / 11.1 / 13.2; B=2, d=64, 50x84: 18.7, 18.4 / 13.6 / 14.8)
     const int allV = (C + CHK - 1) / CHK;
     long want = 256 / tiles;
+    // ... and from 129 tiles, each CU with room for two workgroups of 8 blocks, in three slices where those are still
+    // resident at once and many enough channels share a tile's weights (bf16, d=64, one slice / two / three: 4 images 50x84,
+    // 156 tiles, 256 channels 21.6 / 20.6 / 18.6 us, 512 of them 51x83 53.2 / 47.4 / 44.5; K=7, s=4, 160 tiles 31.5 / 27.2
+    // / 25.6; but 128 channels, d=32, 160 tiles 13.7 / 14.9 / 14.4, and 224 or 234 tiles 19.8 / 18.9 / 24.5, 29.9 / 32.0
+    // / 37.9)
+    if (NSW == 8 && tiles > 128 && 3 * tiles <= 512 && allV >= 16) want = 3;
     want = want < 1 ? 1 : want > allV ? allV : want;
     const int slice_chunks = (int)((allV + want - 1) / want), nslices = (allV + slice_chunks - 1) / slice_chunks;
     const long nb = tiles * nslices;

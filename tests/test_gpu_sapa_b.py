@@ -238,6 +238,20 @@ def test_16bit_dense_window_kernel(coracle, shape, dtype):
     assert rel <= 1.05 * half_ulp + 1e-6, f'{shape} {dtype} box filter: {rel / half_ulp:.2f} half-spacings'
 
 
+# 129 .. 170 tiles: value channels in three slices, of whole chunks, of chunks that do not divide, the last one partial
+@pytest.mark.parametrize('B,C,H,W,K,s', [(33, 256, 16, 16, 5, 2), (42, 280, 13, 19, 5, 2), (34, 517, 15, 14, 5, 2),
+                                         (35, 256, 8, 6, 7, 4), (43, 264, 16, 16, 3, 2)])
+def test_16bit_dense_window_kernel_in_three_slices(B, C, H, W, K, s):
+    g = gen(143)
+    q, key, v = (randn(g, B, c, *hw).bfloat16().to(DEV) for c, hw in ((16, (s * H, s * W)), (16, (H, W)), (C, (H, W))))
+    got = sapa_amd.sapa_fused(q, key, v, K, s)
+    for n in (0, B // 2, B - 1):        # an image by itself, in other slices: the same sums
+        i = slice(n, n + 1)
+        assert torch.equal(got[i], sapa_amd.sapa_fused(q[i].contiguous(), key[i].contiguous(), v[i].contiguous(), K, s))
+        exact = sapa_amd.sapa_fused(q[i].double(), key[i].double(), v[i].double(), K, s)
+        assert_rel_rms_close(got[i].cpu(), exact.cpu(), BF16_REL, 'three slices')
+
+
 @pytest.mark.parametrize('shape', [SHAPES[0], SHAPES[6]], ids=[IDS[0], IDS[6]])
 def test_fp64(coracle, shape):
     B, d, C, H, W, K, s = shape
