@@ -49,7 +49,7 @@ template <typename T, int NSW, bool STREAM, bool QB>
 __global__ __launch_bounds__(64 * NSW) void
 sapa_b_nhwc_wm16_kernel(const T *__restrict__ q, const T *__restrict__ key, const T *__restrict__ value,
                         const T *__restrict__ qbias, T *__restrict__ out, int d, int C, int H, int W, int tiles_x, int tiles_y, int ns,
-                        int nblocks, int per_xcd) {
+                        int nslices, int slice_chunks, int nblocks, int per_xcd) {
     constexpr int NT = 64 * NSW;
     constexpr int WC = 4 * NSW + 4;                          // window cells per row of the tile
     constexpr int NCELL = WROWS * WC;
@@ -65,7 +65,9 @@ sapa_b_nhwc_wm16_kernel(const T *__restrict__ q, const T *__restrict__ key, cons
 
     const int logical = (int)(blockIdx.x % 8) * per_xcd + (int)(blockIdx.x / 8);
     if (logical >= nblocks) return;
-    const int tx = logical % tiles_x, ty = (logical / tiles_x) % tiles_y, n = logical / (tiles_x * tiles_y);
+    // logical = tile * nslices + slice of the value chunks: a tile's slices share its window and queries through L2
+    const int slice = logical % nslices, tile = logical / nslices;
+    const int tx = tile % tiles_x, ty = (tile / tiles_x) % tiles_y, n = tile / (tiles_x * tiles_y);
     const int X0 = tx * 4 * ns, Y0 = ty * 4;                 // first parent of the tile
     const int nsx = (W + 3) / 4;
     const int ns_here = nsx - tx * ns < ns ? nsx - tx * ns : ns;
@@ -101,15 +103,16 @@ sapa_b_nhwc_wm16_kernel(const T *__restrict__ q, const T *__restrict__ key, cons
         (void *)(out + (long)n * C * 4 * lpix), 0, (int)(C * 4 * lpix * (long)sizeof(T)), 0x00020000);
     (void)rk, (void)rv;
 
-    const int nKc = (d + CHK - 1) / CHK, nVc = (C + CHK - 1) / CHK, ntot = nKc + nVc;
-    // chunk j: key channels 64 j .. for j < nKc, value channels 64 (j - nKc) .. after; buffer j % 2,
+    const int nKc = (d + CHK - 1) / CHK, allV = (C + CHK - 1) / CHK, firstV = slice * slice_chunks;
+    const int ntot = nKc + (allV - firstV < slice_chunks ? allV - firstV : slice_chunks);
+    // chunk j: key channels 64 j .. for j < nKc, value channels 64 (j - nKc + firstV) .. after; buffer j % 2,
     // requested two chunks ahead.  A piece past the tensor's last channel would be the next
     // cell's: out of range instead (zeros).
     auto stage = [&](int j) __attribute__((always_inline)) {
 #if defined(__HIP_DEVICE_COMPILE__)
         if (j >= ntot) return;
         const bool is_key = j < nKc;
-        const int cx = is_key ? d : C, c0 = (is_key ? j : j - nKc) * CHK;
+        const int cx = is_key ? d : C, c0 = (is_key ? j : j - nKc + firstV) * CHK;
         const __amdgpu_buffer_rsrc_t r = is_key ? rk : rv;
         u32 *lb = lowbuf + (j & 1) * LOWBUF + wave * 256;
 #pragma unroll
@@ -281,7 +284,7 @@ sapa_b_nhwc_wm16_kernel(const T *__restrict__ q, const T *__restrict__ key, cons
         ch_out[i] = 8 * (p & 7);
     }
     for (int j = nKc; j < ntot; ++j) {
-        const int c0 = (j - nKc) * CHK;
+        const int c0 = (j - nKc + firstV) * CHK;
         if (active) {
             const u32 *vb = lowbuf + (j & 1) * LOWBUF;
             // A operand of (channel block mk, step s): lane (g, channel i16) holds the cells of rows
@@ -339,17 +342,25 @@ static hipError_t launch_geom(const void *q, const void *key, const void *value,
     const int nsx = (W + 3) / 4;
     const int tiles_x = (nsx + NSW - 1) / NSW, tiles_y = (H + 3) / 4;
     const int ns = (nsx + tiles_x - 1) / tiles_x;             // blocks per tile, balanced over the row
-    const long nb = (long)tiles_x * tiles_y * B;
+    const long tiles = (long)tiles_x * tiles_y * B;
+    const int allV = (C + CHK - 1) / CHK;
+    // Tiles that leave room on the CUs (three workgroups each): the value channels in two slices while those are all
+    // resident, in four while there is one per CU; each forms the weights again (bf16, C=256, one slice / two / four: 64 tiles
+    // 12.9 / 9.9 / 8.9 us, 78 13.3 / 10.5 / 11.0, 384 23.7 / 18.9 / 27, 468 23.8 / 25.8 / 31; C=512, 312 tiles 33 / 28 / 29)
+    int want = tiles <= 64 ? 4 : tiles <= 384 ? 2 : 1;
+    if (want > allV) want = allV;
+    const int slice_chunks = (allV + want - 1) / want, nslices = (allV + slice_chunks - 1) / slice_chunks;
+    const long nb = tiles * nslices;
     if (nb > (1L << 30)) return hipErrorNotSupported;
     const int per_xcd = (int)((nb + 7) / 8);
     if (qbias)
         hipLaunchKernelGGL((sapa_b_nhwc_wm16_kernel<T, NSW, STREAM, true>), dim3(per_xcd * 8), dim3(64 * NSW), 0, st,
                            (const T *)q, (const T *)key, (const T *)value, (const T *)qbias, (T *)out, d, C, H, W,
-                           tiles_x, tiles_y, ns, (int)nb, per_xcd);
+                           tiles_x, tiles_y, ns, nslices, slice_chunks, (int)nb, per_xcd);
     else
         hipLaunchKernelGGL((sapa_b_nhwc_wm16_kernel<T, NSW, STREAM, false>), dim3(per_xcd * 8), dim3(64 * NSW), 0, st,
                            (const T *)q, (const T *)key, (const T *)value, (const T *)nullptr, (T *)out, d, C, H, W,
-                           tiles_x, tiles_y, ns, (int)nb, per_xcd);
+                           tiles_x, tiles_y, ns, nslices, slice_chunks, (int)nb, per_xcd);
     return hipGetLastError();
 }
 

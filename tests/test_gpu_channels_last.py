@@ -146,6 +146,22 @@ def test_16bit_dense_window_kernel(coracle, shape, dtype):
         assert worst <= 1.05 * half_ulp, f'{shape} {dtype} with bias: {worst / half_ulp:.2f} half-spacings'
 
 
+# 36 and 144 tiles: value chunks of 64 channels in four and two slices, that divide, do not, the last one partial
+@pytest.mark.parametrize('B,C', [(1, 256), (1, 328), (1, 136), (4, 256), (4, 328), (11, 64), (11, 72)])
+@pytest.mark.parametrize('bias', [False, True])
+def test_16bit_dense_window_kernel_in_slices(B, C, bias):
+    g = gen(331)
+    q, key, v = cl(*(t.bfloat16() for t in inputs(g, B, 16, C, 46, 45, 5)[:3]))
+    qb = randn(g, B, 16).bfloat16().to(DEV) if bias else None
+    got = sapa_amd.sapa_fused(q, key, v, 5, 2, qb)
+    for c in (slice(0, 8), slice(64, 128), slice(C - 8, C)):     # channels of one chunk by themselves: the same sums
+        one = v[:, c].contiguous(memory_format=CL)
+        if one.shape[1]:
+            assert torch.equal(got[:, c], sapa_amd.sapa_fused(q, key, one, 5, 2, qb))
+    exact = sapa_amd.sapa_fused(*(t.double().contiguous() for t in (q if qb is None else q.double() + qb.double()[:, :, None, None], key, v)), 5, 2)
+    assert_rel_rms_close(got.cpu(), exact.cpu(), BF16_REL, 'slices')
+
+
 @pytest.mark.parametrize('dtype,rel', [(torch.bfloat16, BF16_REL), (torch.float16, F16_REL)])
 @pytest.mark.parametrize('K,s', [(5, 2), (7, 4)])
 def test_16bit_matches_contiguous_path_at_a_larger_shape(dtype, rel, K, s):
