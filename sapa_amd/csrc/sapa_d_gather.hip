@@ -1,4 +1,4 @@
-// Fused SAPA-D (deform_qk -> softmax -> deform_av) of contiguous fp32 tensors, up_factor 2 and at most 12
+// Fused SAPA-D (deform_qk -> softmax -> deform_av) of contiguous fp32 tensors, up_factor 2 and at most 9
 // sample points: every sample is gathered from a window in LDS, a pixel's points stay in registers.
 //
 // As in sapa_d_lds.hip a workgroup owns TPW x TPH low-res parents of one (image, group), a thread one
@@ -38,7 +38,7 @@ template <int PM, int TPW, int TPH>
 __global__ void __launch_bounds__(TPW * TPH * S * S) __attribute__((amdgpu_waves_per_eu(4, 4)))
 deform_gather_kernel(const float *__restrict__ q, const float *__restrict__ key, const float *__restrict__ value,
                      const float *__restrict__ offset, float *__restrict__ out, int Cq, int C, int H, int W, int P,
-                     int G, int olayout, int tiles_x, int tiles_y, int nblocks, int per_xcd) {
+                     int G, int olayout, int tiles_x, int tiles_y, int nslices, int slice_chunks, int nblocks, int per_xcd) {
     constexpr int NT = TPW * TPH * S * S, TXP = TPW * S;
     constexpr int WW = TPW + 2 * HR + 1, WH = TPH + 2 * HR + 1, WIN = WW * WH;
     constexpr int RS = WW * CST;                    // floats between window rows
@@ -50,10 +50,12 @@ deform_gather_kernel(const float *__restrict__ q, const float *__restrict__ key,
 
     const int logical = (int)(blockIdx.x % 8) * per_xcd + (int)(blockIdx.x / 8);
     if (logical >= nblocks) return;
-    const int tx = logical % tiles_x;
-    const int ty = (logical / tiles_x) % tiles_y;
-    const int g = (logical / (tiles_x * tiles_y)) % G;
-    const int b = logical / (tiles_x * tiles_y * G);
+    // logical = tile * nslices + slice of the value chunks: a tile's slices meet in an XCD's L2
+    const int slice = logical % nslices, tile = logical / nslices;
+    const int tx = tile % tiles_x;
+    const int ty = (tile / tiles_x) % tiles_y;
+    const int g = (tile / (tiles_x * tiles_y)) % G;
+    const int b = tile / (tiles_x * tiles_y * G);
 
     const int tid = threadIdx.x;
     const int hH = H * S, hW = W * S, GP = G * P, d = Cq / G, cg = C / G;
@@ -68,7 +70,8 @@ deform_gather_kernel(const float *__restrict__ q, const float *__restrict__ key,
     const float *const qg = q + ((long)b * Cq + (long)g * d) * (hplane / 4);
     const float *const kg = key + ((long)b * Cq + (long)g * d) * (lplane / 4);
     const float *const vg = value + ((long)b * C + (long)g * cg) * (lplane / 4);
-    const int nK = (d + CH - 1) / CH, ntot = nK + (cg + CH - 1) / CH;
+    const int nK = (d + CH - 1) / CH, firstV = slice * slice_chunks, leftV = (cg + CH - 1) / CH - firstV;
+    const int ntot = nK + (leftV < slice_chunks ? leftV : slice_chunks);
 
     // ---- staging: task i of a thread is four channels of one cell ----
     u32 from[NST];
@@ -84,7 +87,7 @@ deform_gather_kernel(const float *__restrict__ q, const float *__restrict__ key,
     f32x4 st[NST];
     auto stage_load = [&](int j) __attribute__((always_inline)) {
         const bool is_key = j < nK;
-        const int c0 = (is_key ? j : j - nK) * CH, nc = (is_key ? d : cg) - c0;
+        const int c0 = (is_key ? j : j - nK + firstV) * CH, nc = (is_key ? d : cg) - c0;
         const __amdgpu_buffer_rsrc_t r = planes((const char *)(is_key ? kg : vg) + (long)c0 * lplane, (long)(nc < CH ? nc : CH) * lplane);
 #pragma unroll
         for (int i = 0; i < NST; ++i) {
@@ -245,7 +248,7 @@ deform_gather_kernel(const float *__restrict__ q, const float *__restrict__ key,
         if (j + 1 < ntot) stage_load(j + 1);
         __syncthreads();
         const float *const win = lds + (j & 1) * BUF;
-        const int c0 = (j - nK) * CH, nc = cg - c0;
+        const int c0 = (j - nK + firstV) * CH, nc = cg - c0;
         float o[CH];
 #pragma unroll
         for (int c = 0; c < CH; ++c) o[c] = 0.f;
@@ -298,12 +301,20 @@ static hipError_t launch(const void *q, const void *key, const void *value, cons
                          int H, int W, int P, int G, int olayout, hipStream_t st) {
     constexpr int TPW = 16, TPH = 8;
     const int tiles_x = (W + TPW - 1) / TPW, tiles_y = (H + TPH - 1) / TPH;
-    const long nb = (long)tiles_x * tiles_y * G * B;
+    const long tiles = (long)tiles_x * tiles_y * G * B;
+    const int chunks = (C / G + CH - 1) / CH;
+    // Fewer tiles than CUs: a workgroup's time is a chain of one step per 16 channels, so the value channels are split over
+    // several workgroups per tile, each forming the weights again, up to one per CU (C=256, 9 points, one slice / two / four:
+    // 1 image 16x16, 8 tiles, 37 / 27 / 22 us; 4 of 32x32, 128 tiles, 39 / 30 / 37; 2 of 64x64, 256 tiles, 43 / 47 / 66)
+    long want = tiles > 0 ? 256 / tiles : 1;
+    want = want < 1 ? 1 : want > chunks ? chunks : want;
+    const int slice_chunks = (int)((chunks + want - 1) / want), nslices = (chunks + slice_chunks - 1) / slice_chunks;
+    const long nb = tiles * nslices;
     if (nb > (1L << 30)) return hipErrorNotSupported;
     const int per_xcd = (int)((nb + 7) / 8);
     hipLaunchKernelGGL((deform_gather_kernel<PM, TPW, TPH>), dim3(per_xcd * 8), dim3(TPW * TPH * S * S), 0, st,
                        (const float *)q, (const float *)key, (const float *)value, (const float *)offset, (float *)out, Cq, C, H,
-                       W, P, G, olayout, tiles_x, tiles_y, (int)nb, per_xcd);
+                       W, P, G, olayout, tiles_x, tiles_y, nslices, slice_chunks, (int)nb, per_xcd);
     return hipGetLastError();
 }
 
