@@ -10,8 +10,8 @@
 // third went into staging element by element.  Here a thread stages four channels of a cell at a time through
 // four buffer loads whose offsets are fixed for the whole kernel, requested a chunk ahead, into the second of two
 // buffers: one barrier per chunk.  A sample outside the image or the window points at cells that are always
-// zero, so the channel loops have no selects; the rare one inside the image but outside the window is added
-// from memory in its turn.
+// zero, so the channel loops have no selects; the rare one inside the image but outside the window comes from
+// memory.  It is added at its point's place in the order: waves that have one aggregate in a loop over the points.
 //
 // Arithmetic and order of sums are those of sapa_d_lds.hip, bit for bit (reference:
 // deformsapa/deformsapa/src/cuda/deform_qk_cuda_kernel.cu:180-193, deform_av_cuda_kernel.cu:178-192).
@@ -252,14 +252,10 @@ deform_gather_kernel(const float *__restrict__ q, const float *__restrict__ key,
         float o[CH];
 #pragma unroll
         for (int c = 0; c < CH; ++c) o[c] = 0.f;
-#pragma unroll
-        for (int p = 0; p < PM; ++p) {
-            if (p >= P) continue;
-            const float *const wp = win + at[p];
-            // (opaque: the weights of all samples kept over the loop do not fit the registers)
-            float fy = lh[p], fx = lw[p];
-            asm volatile("" : "+v"(fy), "+v"(fx));
-            const float hh = 1.f - fy, hw = 1.f - fx, wa = lg[p];
+        // sample of weight wa from the window, of place `cell` in it and fractions fy, fx
+        auto window_sample = [&](int cell, float fy, float fx, float wa) __attribute__((always_inline)) {
+            const float *const wp = win + cell;
+            const float hh = 1.f - fy, hw = 1.f - fx;
             const float w1 = hh * hw, w2 = hh * fx, w3 = fy * hw, w4 = fy * fx;
 #pragma unroll
             for (int c4 = 0; c4 < CH; c4 += 4) {
@@ -274,15 +270,32 @@ deform_gather_kernel(const float *__restrict__ q, const float *__restrict__ key,
                     o[c4 + e] = fma_(val, wa, o[c4 + e]);
                 }
             }
-            __builtin_amdgcn_sched_barrier(0);
-        }
-        for (u32 left = far_wave; left; left &= left - 1) {
-            const int p = __builtin_ctz(left);
-            if (far >> p & 1u) {
-                float wa = 0.f;
+        };
+        if (far_wave == 0) {
 #pragma unroll
-                for (int i = 0; i < PM; ++i) wa = i == p ? lg[i] : wa;
-                far_sample(p, vg, c0, cg, [&](int c, float val) __attribute__((always_inline)) { o[c] = fma_(val, wa, o[c]); });
+            for (int p = 0; p < PM; ++p) {
+                if (p >= P) continue;
+                // (opaque: the weights of all samples kept over the loop do not fit the registers)
+                float fy = lh[p], fx = lw[p];
+                asm volatile("" : "+v"(fy), "+v"(fx));
+                window_sample(at[p], fy, fx, lg[p]);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        } else {
+            // a sample beyond the window is added where its point stands: a loop with one body for all points, or
+            // the code of such a sample would be there nine times
+#pragma unroll 1
+            for (int p = 0; p < P; ++p) {
+                int cell = at[0];
+                float fy = lh[0], fx = lw[0], wa = lg[0];
+#pragma unroll
+                for (int i = 1; i < PM; ++i) {
+                    const bool here = i == p;
+                    cell = here ? at[i] : cell, fy = here ? lh[i] : fy, fx = here ? lw[i] : fx, wa = here ? lg[i] : wa;
+                }
+                window_sample(cell, fy, fx, cell != NOWHERE ? wa : 0.f);
+                if (far >> p & 1u)
+                    far_sample(p, vg, c0, cg, [&](int c, float val) __attribute__((always_inline)) { o[c] = fma_(val, wa, o[c]); });
             }
         }
         u32 plane = (u32)c0 * hplane;

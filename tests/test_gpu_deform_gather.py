@@ -59,3 +59,18 @@ def test_value_channels_in_slices(cg, scale):
         i = slice(n, n + 1)
         assert torch.equal(got[i], sapa_amd.deform_sapa_fused(*(t[i].contiguous() for t in (q, key, v, off)), P, 2, G))
         assert _lib.lib().sapa_hip_last_kernel() == b'deform_gather_kernel'
+
+
+@pytest.mark.parametrize('P', [2, 4, 8])
+@pytest.mark.parametrize('scale', [3.0, 6.0])
+def test_samples_beyond_the_window_are_added_in_the_order_of_the_points(coracle, P, scale):
+    """Equal logits make every weight exactly 1 / P: the output is deform_av's, in its order of sums, bit for bit,
+    also where samples lie in the image but not in the tile's window."""
+    G, cg, H, W = 2, 37, 33, 40
+    g = gen(74)
+    q, key = torch.zeros(1, G * 3, 2 * H, 2 * W), randn(g, 1, G * 3, H, W)
+    v, off = randn(g, 1, G * cg, H, W), randn(g, 1, 2 * G * P, 2 * H, 2 * W) * scale
+    got = sapa_amd.deform_sapa_fused(*(t.cuda() for t in (q, key, v, off)), P, 2, G, matrix_form=False).cpu()
+    assert _lib.lib().sapa_hip_last_kernel() == b'deform_gather_kernel'
+    attn = torch.full((1, G, P, 2 * H, 2 * W), 1. / P)
+    assert torch.equal(got, coracle.deform_av(attn, v, off, P, 2, G, 'f32'))
