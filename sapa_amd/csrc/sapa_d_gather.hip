@@ -28,6 +28,9 @@ typedef float f32x4 __attribute__((ext_vector_type(4)));
 constexpr int S = 2, HR = 4, CH = 16;
 constexpr int CST = CH + 4;                         // floats per cell: 16-byte reads spread over all bank groups
 constexpr u32 OUTSIDE = 0x80000000u;                // a buffer offset beyond any extent
+// a sample in the image, but not in the window: the rows and columns of its corners that are in the image, and the index
+// (y + 1) W + x + 1 of its low corner (below 2^26 where a group's planes are within a descriptor's reach)
+constexpr u32 FAR = 0x80000000u, FAR_Y0 = 1u << 30, FAR_Y1 = 1u << 29, FAR_X0 = 1u << 28, FAR_X1 = 1u << 27, FAR_INDEX = FAR_X1 - 1;
 
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t planes(const void *p, long bytes) {
     return __builtin_amdgcn_make_buffer_rsrc((void *)p, 0, (int)bytes, 0x00020000);
@@ -125,8 +128,8 @@ deform_gather_kernel(const float *__restrict__ q, const float *__restrict__ key,
     stage_load(0);
     // ---- the samples ----
     float lh[PM], lw[PM], lg[PM];
-    int at[PM];
-    u32 far = 0;                                    // this pixel's samples in the image, but not in the window
+    int at[PM];                                     // place in the window (NOWHERE: none), or FAR and where in the image
+    u32 far_wave = 0;                               // points with a sample in the image, but not in the window
     {
         const OffsetRef<float> op = offset_ref(offset, olayout, (long)b * GP + (long)g * P, chh, cw, S, H, W);
         float ow[PM], oh[PM];
@@ -144,30 +147,58 @@ deform_gather_kernel(const float *__restrict__ q, const float *__restrict__ key,
             const int hl = (int)fh - wy0, wl = (int)fw - wx0;
             const bool in = guard && hl >= 0 && hl <= WH - 2 && wl >= 0 && wl <= WW - 2;
             at[p] = in ? hl * RS + wl * CST : NOWHERE;
-            lh[p] = in ? kh - fh : 0.f;
-            lw[p] = in ? kw - fw : 0.f;
+            lh[p] = guard ? kh - fh : 0.f;
+            lw[p] = guard ? kw - fw : 0.f;
             lg[p] = 0.f;
-            far |= guard && !in ? 1u << p : 0u;
+            if (guard && !in) {
+                const int y = (int)fh, x = (int)fw;             // -1 .. H - 1, -1 .. W - 1
+                at[p] = (int)(FAR | (y >= 0 ? FAR_Y0 : 0u) | (y + 1 < H ? FAR_Y1 : 0u) | (x >= 0 ? FAR_X0 : 0u) |
+                              (x + 1 < W ? FAR_X1 : 0u) | (u32)((y + 1) * W + x + 1));
+            }
+            far_wave |= __ballot(at[p] < 0) ? 1u << p : 0u;
         }
     }
-    u32 far_wave = 0;                               // ... of any lane of the wave
+    // the sample of code `code` (at[p] < 0) and fractions fy, fx in the channels c0 .. c0 + 15: add(c, value).  What bounds
+    // it is the way to the cache and back: four channels at a time, 16 loads in flight, its place kept from the start (one
+    // channel at a time behind the offsets fetched again, 8 images 64x64, C=256, 9 points, offsets of standard deviation
+    // 2 / 3 / 4 / 6: 576 / 792 / 672 / 884 us, 235 / 306 / 449 / 803 so; sapa_d_lds.hip 520 / 601 / 619 / 857)
+    auto far_sample = [&](int code, float fy, float fx, const float *src, int c0, int channels, auto &&add) __attribute__((always_inline)) {
+        const __amdgpu_buffer_rsrc_t r = planes((const char *)src + (long)c0 * lplane, (long)(channels - c0 < CH ? channels - c0 : CH) * lplane);
+        const u32 u = (u32)code, first = ((u & FAR_INDEX) - (u32)(W + 1)) * 4u;
+        const bool y0 = u & FAR_Y0, y1 = u & FAR_Y1, x0 = u & FAR_X0, x1 = u & FAR_X1;
+        u32 i1 = y0 && x0 ? first : OUTSIDE, i2 = y0 && x1 ? first + 4u : OUTSIDE;
+        u32 i3 = y1 && x0 ? first + 4u * (u32)W : OUTSIDE, i4 = y1 && x1 ? first + 4u * (u32)W + 4u : OUTSIDE;
+        const float hh = 1.f - fy, hw = 1.f - fx;
+        const float w1 = hh * hw, w2 = hh * fx, w3 = fy * hw, w4 = fy * fx;
 #pragma unroll
-    for (int p = 0; p < PM; ++p) far_wave |= __ballot(far >> p & 1u) ? 1u << p : 0u;
-    // add(c, value) for the channels c0 + c, c < 16, of such a sample
-    auto far_sample = [&](int p, const float *src, int c0, int channels, auto &&add) __attribute__((always_inline)) {
-        // (all of it formed again: kept from above, it does not fit the registers)
-        int t = tid;
-        asm volatile("" : "+v"(t));
-        const int x = tx * TXP + t % TXP, y = ty * TPH * S + t / TXP;
-        const OffsetRef<float> op = offset_ref(offset, olayout, (long)b * GP + (long)g * P, y, x, S, H, W);
-        Tap<float> tap;
-        tap_setup((float)(y / S) + op.base[(long)(2 * p + 1) * op.stride], (float)(x / S) + op.base[(long)(2 * p) * op.stride], H, W, tap);
-        const float *plane = src + (long)c0 * (lplane / 4);
+        for (int c4 = 0; c4 < CH; c4 += 4) {
+            float v[4][4];
 #pragma unroll
-        for (int c = 0; c < CH; ++c) {
-            if (c0 + c < channels) add(c, tap_sample(plane, tap));
-            plane += lplane / 4;
+            for (int e = 0; e < 4; ++e) {
+                v[e][0] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(r, i1, 0, 0));
+                v[e][1] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(r, i2, 0, 0));
+                v[e][2] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(r, i3, 0, 0));
+                v[e][3] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(r, i4, 0, 0));
+                i1 += lplane, i2 += lplane, i3 += lplane, i4 += lplane;
+            }
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                float val = w1 * v[e][0];
+                val = fma_(w2, v[e][1], val);
+                val = fma_(w3, v[e][2], val);
+                val = fma_(w4, v[e][3], val);
+                add(c4 + e, val);
+            }
             __builtin_amdgcn_sched_barrier(0);
+        }
+    };
+    // of at, lh, lw and lg those of point p
+    auto point = [&](int p, int &code, float &fy, float &fx, float &l) __attribute__((always_inline)) {
+        code = at[0], fy = lh[0], fx = lw[0], l = lg[0];
+#pragma unroll
+        for (int i = 1; i < PM; ++i) {
+            const bool here = i == p;
+            code = here ? at[i] : code, fy = here ? lh[i] : fy, fx = here ? lw[i] : fx, l = here ? lg[i] : l;
         }
     };
 
@@ -186,7 +217,7 @@ deform_gather_kernel(const float *__restrict__ q, const float *__restrict__ key,
 #pragma unroll
         for (int p = 0; p < PM; ++p) {
             if (p >= P) continue;
-            const float *const wp = win + at[p];
+            const float *const wp = win + (at[p] < 0 ? NOWHERE : at[p]);
             float fy = lh[p], fx = lw[p];
             asm volatile("" : "+v"(fy), "+v"(fx));
             const float hh = 1.f - fy, hw = 1.f - fx;
@@ -206,16 +237,16 @@ deform_gather_kernel(const float *__restrict__ q, const float *__restrict__ key,
                 }
             }
             // (a query that is not finite times the zeros of a sample that contributes nothing)
-            lg[p] = at[p] != NOWHERE ? acc : lg[p];
+            lg[p] = (u32)at[p] < (u32)NOWHERE ? acc : lg[p];
             __builtin_amdgcn_sched_barrier(0);
         }
         for (u32 left = far_wave; left; left &= left - 1) {
             const int p = __builtin_ctz(left);
-            if (far >> p & 1u) {
-                float acc = 0.f;
-#pragma unroll
-                for (int i = 0; i < PM; ++i) acc = i == p ? lg[i] : acc;
-                far_sample(p, kg, j * CH, d, [&](int c, float val) __attribute__((always_inline)) { acc = fma_(val, qv[c], acc); });
+            int code;
+            float fy, fx, acc;
+            point(p, code, fy, fx, acc);
+            if (code < 0) {
+                far_sample(code, fy, fx, kg, j * CH, d, [&](int c, float val) __attribute__((always_inline)) { acc = fma_(val, qv[c], acc); });
 #pragma unroll
                 for (int i = 0; i < PM; ++i) lg[i] = i == p ? acc : lg[i];
             }
@@ -238,7 +269,7 @@ deform_gather_kernel(const float *__restrict__ q, const float *__restrict__ key,
         const float inv = 1.f / sum;
         // (a sample that contributes nothing: its weight times the zeros may not be NaN)
 #pragma unroll
-        for (int p = 0; p < PM; ++p) lg[p] = at[p] != NOWHERE || (far >> p & 1u) ? lg[p] * inv : 0.f;
+        for (int p = 0; p < PM; ++p) lg[p] = at[p] != NOWHERE ? lg[p] * inv : 0.f;
     }
 
     // ---- aggregation ----
@@ -286,16 +317,12 @@ deform_gather_kernel(const float *__restrict__ q, const float *__restrict__ key,
             // the code of such a sample would be there nine times
 #pragma unroll 1
             for (int p = 0; p < P; ++p) {
-                int cell = at[0];
-                float fy = lh[0], fx = lw[0], wa = lg[0];
-#pragma unroll
-                for (int i = 1; i < PM; ++i) {
-                    const bool here = i == p;
-                    cell = here ? at[i] : cell, fy = here ? lh[i] : fy, fx = here ? lw[i] : fx, wa = here ? lg[i] : wa;
-                }
-                window_sample(cell, fy, fx, cell != NOWHERE ? wa : 0.f);
-                if (far >> p & 1u)
-                    far_sample(p, vg, c0, cg, [&](int c, float val) __attribute__((always_inline)) { o[c] = fma_(val, wa, o[c]); });
+                int code;
+                float fy, fx, wa;
+                point(p, code, fy, fx, wa);
+                window_sample(code < 0 ? NOWHERE : code, fy, fx, code < 0 ? 0.f : wa);
+                if (code < 0)
+                    far_sample(code, fy, fx, vg, c0, cg, [&](int c, float val) __attribute__((always_inline)) { o[c] = fma_(val, wa, o[c]); });
             }
         }
         u32 plane = (u32)c0 * hplane;
