@@ -35,6 +35,7 @@
 // bias passes, 298 with these; 25 points 638, 492; bf16 channels-last 361, 239.  What is left there in
 // fp32 is the matrix work of the six piece products: 30 us per 8.6 GFLOP at the rate of a large product.)
 #include "kernels.hpp"
+#include "project_plan.hpp"
 
 namespace sapa {
 
@@ -211,21 +212,15 @@ project_kernel(Feature<T> f0, Feature<T> f1, int outputs) {
     }
 }
 
-// n features in tiles of `pixels`: tiles per wave and workgroups per image; false: too many workgroups.  At most 512
-// workgroups of 4 waves; a tile per wave only where all of them are resident, `resident` on each of 256 CUs (us with 2 tiles
-// per wave at least and so, modules: 256 channels, 1 image 50x84, planes 41 -> 36, 2 of 48x48 38 -> 34, 512 channels, 2 of
-// 32x32 42 -> 36; in two rounds, SAPA-D channels-last, 512 channels, 2 of 32x32, 53 -> 56).
+// n features in tiles of `pixels`: false where there are too many workgroups
 template <typename T>
 static bool spread16(const ProjectFeature *p, int n, Feature<T> (&f)[2], int B, int pixels, int blocks_o, int resident) {
-    long tiles[2] = {0, 0}, blocks[2] = {0, 0};
+    long tiles[2] = {0, 0};
     for (int i = 0; i < n; ++i) tiles[i] = (p[i].HW + pixels - 1) / pixels;
-    const long all = (tiles[0] + tiles[1]) * B * blocks_o;
-    long per = (all + 4L * 512 - 1) / (4L * 512);
-    if (per < 2 && all > 4L * 256 * resident) per = 2;
-    for (int i = 0; i < n; ++i) blocks[i] = (tiles[i] + 4 * per - 1) / (4 * per);
+    const Spread s = plan16(tiles, (long)B * blocks_o, resident);
     for (int i = 0; i < n; ++i)
-        f[i] = Feature<T>{(const T *)p[i].x, (const T *)p[i].w, (const T *)p[i].bias, (T *)p[i].out, p[i].HW, (int)per, (int)blocks[i]};
-    return blocks[0] <= 65535 * 32L && blocks[1] <= 65535 * 32L && B <= 65535 && blocks_o <= 65535;
+        f[i] = Feature<T>{(const T *)p[i].x, (const T *)p[i].w, (const T *)p[i].bias, (T *)p[i].out, p[i].HW, (int)s.per, (int)s.blocks[i]};
+    return s.blocks[0] <= 65535 * 32L && s.blocks[1] <= 65535 * 32L && B <= 65535 && blocks_o <= 65535;
 }
 
 template <typename T, int C, int O, bool WIDE = false>
@@ -720,35 +715,6 @@ project32_kernel(Feature<float> f0, Feature<float> f1, int waves, int outputs) {
     }
 }
 
-// How a projection's tiles are spread: tiles per wave, waves per workgroup that have some, workgroups per image
-struct Spread {
-    long per, blocks[2];
-    int waves;
-};
-// One workgroup is resident per CU (its weight planes fill most of the LDS) and the part has
-// 256 CUs: two full rounds of workgroups where that leaves a wave 8 tiles or more (6 of 12 waves), else one
-// (16 images: 200x336 pixels 301 us in two rounds against 315 in one; 100x168 pixels 71 us in
-// one round against 98 in 272 workgroups; 256 -> 288, 8 images 128x128, 8 waves, 119 us in one against 130)
-static Spread spread32(const long (&tiles)[2], long sets, int nw) {
-    const long ntiles = tiles[0] + tiles[1];
-    const long slots = 256;
-    long blocks = 2 * slots / sets > 1 ? 2 * slots / sets : 1;
-    long per = (ntiles + nw * blocks - 1) / (nw * blocks);
-    if (per < (nw == 8 ? 8 : 6)) {
-        blocks = slots / sets > 1 ? slots / sets : 1;
-        per = (ntiles + nw * blocks - 1) / (nw * blocks);
-    }
-    // ... and as few waves per workgroup as cover the image in that many tiles each, so that no workgroup of the
-    // round is missing (240 workgroups of 12 waves else 256 of 11; 512 -> 72, 2 images 100x168, 8 waves in 198
-    // workgroups 35.8 us, 7 in 228 31.3; fewer tiles than the chip has room for: a wave's matrix instructions are not
-    // queued behind a second wave's; 4 images of 33x20 pixels, 256 -> 128 / 288: SAPA-D module 113 -> 104 us), but over
-    // several tiles each not with less than 6 of 8 (128 -> 32, 16 images 50x84: 5 waves 12.4 us, 8 11.7)
-    int waves = (int)((ntiles + blocks * per - 1) / (blocks * per));
-    waves = waves < 1 ? 1 : waves > nw ? nw : waves;
-    if (nw == 8 && per > 1 && waves < 6) waves = nw;
-    return Spread{per, {(tiles[0] + waves * per - 1) / (waves * per), (tiles[1] + waves * per - 1) / (waves * per)}, waves};
-}
-
 template <int C, int O, bool IN_CL, bool OUT_CL, bool WIDE, int NW>
 static hipError_t launch32_waves(const ProjectFeature *p, int n, int B, hipStream_t st, int outputs, const Spread &s) {
     constexpr int RT = OUT_CL ? 16 * (O + 4) : 16 * 36, XB = IN_CL ? 0 : 32 * 32;
@@ -787,7 +753,7 @@ static hipError_t launch32_co(const ProjectFeature *p, int n, int B, hipStream_t
         ntiles[i] = (p[i].HW + 31) / 32;
     }
     const long sets = (long)B * ((outputs + O - 1) / O);     // sets: workgroups that share a pixel range's place
-    const Spread s8 = spread32(ntiles, sets, 8), s12 = spread32(ntiles, sets, 12);
+    const Spread s8 = plan32(ntiles, sets, 8), s12 = plan32(ntiles, sets, 12);
     // Twelve waves where they shorten a wave's chain of tiles to what is asked for below (eight have twice the steps of
     // x in flight and no bar to moving work between steps).  us with 8 / 12 waves, from planes: 5 tiles to 3 each
     // (256 -> 64, 16 images 100x168) 66 / 60, 3 to 2 (256 -> 288, 8 images 64x64) 41.8 / 38.6, but 4 to 3
