@@ -104,6 +104,9 @@ sapa_b_wmat16_kernel(const T *__restrict__ q, const T *__restrict__ key, const T
     // not in the memory-side cache 257 -> 245 us; read again and again, as no program does, 211 -> 213).  What fits
     // the cache has two, and so two workgroups per CU.
     constexpr int NB = STREAM && !ODD ? 3 : 2;
+    // (of two by the lowest bit: a signed remainder in the kernels whose registers spill cost K=7, s=4, B=4, C=512, 64x64
+    // in bf16 68.1 -> 68.7 us)
+    auto ring = [](int j) { return NB == 2 ? j & 1 : j % NB; };
     __shared__ __attribute__((aligned(16))) u32 lds[NB * (LOWBUF + HIBUF) + 4];
     u32 *const lowbuf = lds, *const hibuf = lds + NB * LOWBUF;
     const u32 low_at = lds_address((const __attribute__((address_space(3))) u32 *)lds), hi_base = low_at + NB * LOWBUF * 4;
@@ -190,10 +193,10 @@ sapa_b_wmat16_kernel(const T *__restrict__ q, const T *__restrict__ key, const T
     };
     auto stage = [&](int j) __attribute__((always_inline)) {
         if (j < nKc) {
-            if (!ODD) stage_low(dk, (u32)(j * CHK), j % NB);
-            stage_q((u32)(j * CHK), j % NB);
+            if (!ODD) stage_low(dk, (u32)(j * CHK), ring(j));
+            stage_q((u32)(j * CHK), ring(j));
         } else if (!ODD && j < ntot) {
-            stage_low(dv, (u32)((j - nKc + vbase) * CHK), j % NB);
+            stage_low(dv, (u32)((j - nKc + vbase) * CHK), ring(j));
         }
     };
     // ODD: an odd W puts every other row of a low-res plane in the middle of a dword, where direct loads
@@ -234,7 +237,7 @@ sapa_b_wmat16_kernel(const T *__restrict__ q, const T *__restrict__ key, const T
                         : u32x4{0u, v[0] << 16, __builtin_amdgcn_alignbyte(v[1], v[0], 2),
                                 __builtin_amdgcn_alignbyte(v[2], v[1], 2)};
             const int at = OWN ? slot / LPC * LROW + slot % LPC * 4 : slot * 4;
-            if (NLP % NT == 0 || slot < NLP) *(u32x4 *)(lowbuf + (j % NB) * LOWBUF + at) = m;
+            if (NLP % NT == 0 || slot < NLP) *(u32x4 *)(lowbuf + ring(j) * LOWBUF + at) = m;
         }
     };
     // behind low_commit(j), by the wave that wrote the piece: the last element of an image of an odd number
@@ -246,7 +249,7 @@ sapa_b_wmat16_kernel(const T *__restrict__ q, const T *__restrict__ key, const T
         for (int i = 0; i < NLI; ++i) {
             const int slot = i * NT + tid, at = OWN ? slot / LPC * LROW + slot % LPC * 4 : slot * 4;
             const u32 e = (u32)((long)(nch - c0) * lpix) - 1u - (u32)(((int)off_low[i] >> 1) + (low_odd[i] ? 1 : 0));
-            if (e < 8u) ((T *)(lowbuf + (j % NB) * LOWBUF + at))[e] = last;
+            if (e < 8u) ((T *)(lowbuf + ring(j) * LOWBUF + at))[e] = last;
         }
     };
     // chunk jn (the first of the keys or of the values) has landed in this wave's slots: the 6
@@ -255,7 +258,7 @@ sapa_b_wmat16_kernel(const T *__restrict__ q, const T *__restrict__ key, const T
     auto patch_low = [&](int jn) __attribute__((always_inline)) {
         if (!OWN && tx == 0 && ty == 0 && patch_slot >= 0 && (jn < nKc || vbase == 0)) {
             const __amdgpu_buffer_rsrc_t r = jn < nKc ? rk : rv;
-            u32 *dst = lowbuf + (jn % NB) * LOWBUF + patch_slot * 4;
+            u32 *dst = lowbuf + ring(jn) * LOWBUF + patch_slot * 4;
 #pragma unroll
             for (int k = 1; k < 4; ++k) dst[k] = __builtin_amdgcn_raw_buffer_load_b32(r, 4 * (k - 1), 0, 0);
         }
@@ -290,7 +293,7 @@ sapa_b_wmat16_kernel(const T *__restrict__ q, const T *__restrict__ key, const T
     for (int j = 0; j < nKc; ++j) {
         low_load(j + 1);
         if (active) {
-            const u32 *kb = lowbuf + (j % NB) * LOWBUF, *qb = hibuf + (j % NB) * HIBUF;
+            const u32 *kb = lowbuf + ring(j) * LOWBUF, *qb = hibuf + ring(j) * HIBUF;
             u32x2 a[4], b[4];
 #pragma unroll
             for (int mb = 0; mb < 4; ++mb)
@@ -403,7 +406,7 @@ sapa_b_wmat16_kernel(const T *__restrict__ q, const T *__restrict__ key, const T
         u32 *ob = hibuf + (j & 1) * HIBUF;                      // no loads into this ring any more
         low_load(j + 1);
         if (active) {
-            const u32 *vb = lowbuf + (j % NB) * LOWBUF;
+            const u32 *vb = lowbuf + ring(j) * LOWBUF;
             // B operand of step s: lane (g, channel i16) holds the cells of rows 4 s + g / 2 and
             // 4 s + 2 + g / 2, columns 4 (g % 2) .. + 3 -- the order the weights are held in
             u32x4 b[2];
@@ -460,7 +463,7 @@ sapa_b_wmat16_kernel(const T *__restrict__ q, const T *__restrict__ key, const T
             else __builtin_amdgcn_raw_buffer_store_b128(o, ro, off, 0, 0);
         }
         // (the next request behind the stores: 208 us at FPN-large against 216 with the loads first)
-        if (!ODD && j + NB < ntot) stage_low(dv, (u32)((j + NB - nKc + vbase) * CHK), j % NB);
+        if (!ODD && j + NB < ntot) stage_low(dv, (u32)((j + NB - nKc + vbase) * CHK), ring(j));
     }
 
     // ---- blocks with a non-finite result: again, term by term ----
