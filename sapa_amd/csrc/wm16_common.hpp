@@ -126,17 +126,21 @@ __device__ __forceinline__ u32x4 dma_rsrc(const void *p, u32 bytes) {
 // builtin: it knows that the instruction writes LDS, and in front of the next transposing LDS read (an
 // intrinsic, so without an address it could compare) it waits for every load in flight -- the loads just
 // issued for a later chunk among them, which ends all prefetching.  The waits are the kernel's own
-// (wait_all_but).  m0 is the compiler's scratch register for the same purpose: nothing else in these
-// kernels uses it.
+// (wait_all_but).  m0 is named as written, so that the compiler, which merges its own settings of m0 where nothing
+// writes it between them, sets it again for its own direct loads.  (It warns that m0 is a reserved register, whose value
+// is not kept for it: none is in it here.)
+#pragma clang diagnostic push
+#pragma clang diagnostic ignored "-Winline-asm"
 template <bool NT = false>
 __device__ __forceinline__ void load_lds(u32x4 r, u32 at, u32 off) {
 #if defined(__HIP_DEVICE_COMPILE__)
     if constexpr (NT)
-        asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, 0 offen nt lds" ::"s"(at), "v"(off), "s"(r) : "memory");
+        asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, 0 offen nt lds" ::"s"(at), "v"(off), "s"(r) : "memory", "m0");
     else
-        asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds" ::"s"(at), "v"(off), "s"(r) : "memory");
+        asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds" ::"s"(at), "v"(off), "s"(r) : "memory", "m0");
 #endif
 }
+#pragma clang diagnostic pop
 
 // LDS byte address of a __shared__ array
 __device__ __forceinline__ u32 lds_address(const __attribute__((address_space(3))) u32 *p) { return (u32)(unsigned long long)p; }
