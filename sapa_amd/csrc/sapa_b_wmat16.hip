@@ -71,7 +71,9 @@ __device__ __forceinline__ int swz(int ch, int r) { return ((ch & 7) << 1) | ((r
 //
 // HALF: images of the key or of the value of an odd number of elements (a kernel of its own: what it
 // takes in registers costs the others up to 10 % -- K=3, s=2, B=16, C=256, 50x84 in bf16 83 -> 91 us)
-template <typename T, int K, int S, int NSW, bool STREAM, bool ODD, bool HALF>
+//
+// DEEP: three buffers of each kind instead of two, requests two chunks ahead and stores waited for two chunks later
+template <typename T, int K, int S, int NSW, bool STREAM, bool ODD, bool HALF, bool DEEP>
 __global__ __launch_bounds__(64 * NSW, 4) void
 sapa_b_wmat16_kernel(const T *__restrict__ q, const T *__restrict__ key, const T *__restrict__ value,
                      T *__restrict__ out, int d, int C, int H, int W, int tiles_x, int tiles_y, int ns,
@@ -99,11 +101,9 @@ sapa_b_wmat16_kernel(const T *__restrict__ q, const T *__restrict__ key, const T
     static_assert(NSW == 16 || NSW == 8, "piece swizzle");
     constexpr int NPC = 2 * NSW / 2;                         // 16-byte pieces per tile row = NSW
 
-    // Buffers of each kind, one chunk per buffer.  Streamed tensors come from memory, not from a cache:
-    // requests two chunks ahead, and stores waited for two chunks later (B=16, C=256, d=64, 100x168 in bf16, inputs
-    // not in the memory-side cache 257 -> 245 us; read again and again, as no program does, 211 -> 213).  What fits
-    // the cache has two, and so two workgroups per CU.
-    constexpr int NB = STREAM && !ODD ? 3 : 2;
+    // buffers of each kind, one chunk per buffer
+    static_assert(!DEEP || (STREAM && !ODD), "three buffers: streamed tensors");
+    constexpr int NB = DEEP ? 3 : 2;
     // (of two by the lowest bit: a signed remainder in the kernels whose registers spill cost K=7, s=4, B=4, C=512, 64x64
     // in bf16 68.1 -> 68.7 us)
     auto ring = [](int j) { return NB == 2 ? j & 1 : j % NB; };
@@ -481,7 +481,7 @@ sapa_b_wmat16_kernel(const T *__restrict__ q, const T *__restrict__ key, const T
     }
 }
 
-template <typename T, int K, int S, int NSW, bool STREAM, bool ODD, bool HALF = false>
+template <typename T, int K, int S, int NSW, bool STREAM, bool ODD, bool HALF = false, bool DEEP = false>
 static hipError_t launch_geom(const void *q, const void *key, const void *value, void *out, int B, int d,
                               int C, int H, int W, hipStream_t st) {
     constexpr int PB = 8 / S;
@@ -506,7 +506,7 @@ static hipError_t launch_geom(const void *q, const void *key, const void *value,
     const long nb = tiles * nslices;
     if (nb > (1L << 30)) return hipErrorNotSupported;
     const int per_xcd = (int)((nb + 7) / 8);
-    hipLaunchKernelGGL((sapa_b_wmat16_kernel<T, K, S, NSW, STREAM, ODD, HALF>), dim3(per_xcd * 8), dim3(64 * NSW), 0, st, (const T *)q,
+    hipLaunchKernelGGL((sapa_b_wmat16_kernel<T, K, S, NSW, STREAM, ODD, HALF, DEEP>), dim3(per_xcd * 8), dim3(64 * NSW), 0, st, (const T *)q,
                        (const T *)key, (const T *)value, (T *)out, d, C, H, W, tiles_x, tiles_y, ns,
                        nslices, slice_chunks, (int)nb, per_xcd);
     return hipGetLastError();
@@ -532,7 +532,14 @@ hipError_t sapa_b_wmat16_launch(int mode, const void *q, const void *key, const 
     // (low-res rows through registers) has tiles of 8 blocks only: with 16 the registers do not suffice
     // (B=16, C=256, d=64, 42x25: 24 us, by vector fmas 65; 100x167: 289 us against 451; rows below 16
     // cells, 13x13 at B=8: 9 us against 19 on the one-block-per-parent matrix kernel).
-    const bool stream = 2L * ((long)B * H * W * (1L + s * s) * ((long)d + C)) > (256L << 20);
+    const long bytes = 2L * ((long)B * H * W * (1L + s * s) * ((long)d + C));
+    const bool stream = bytes > (256L << 20);
+    // Three buffers where the bytes are well beyond that cache and the chain of chunks is long enough for them (d=64 in
+    // bf16, three sets of tensors in turn, two buffers / three, us per call: C=256, 16 images 100x168, 820 MiB, 257 / 247,
+    // 10 of them, 513, 156 / 153, 16 of 96x96, 450, 134 / 126; but 8 of 100x168, 410, 118 / 122, 32 of 50x84, 410, 119 / 128,
+    // 3 of them with C=512, 277, 67 / 73; chains of 10 chunks, d=32, C=128: 16 images, 410 MiB, 123 / 133, 32, 820, 273 / 275,
+    // of 6 348 / 363.  One set again and again, partly from the cache: 16 of 100x168 215 / 220)
+    const bool deep = bytes > (432L << 20) && (d + wm16::CHK - 1) / wm16::CHK + (C + wm16::CHK - 1) / wm16::CHK >= 16;
     const bool odd = W % 2 != 0, half = ((d | C) & H & W & 1) != 0;
     // Other windows: streamed only where a tile's rows are whole 128-byte lines (s W a multiple of 64);
     // else parts of a line are written by two workgroups, and the caches put them together
@@ -547,6 +554,7 @@ hipError_t sapa_b_wmat16_launch(int mode, const void *q, const void *key, const 
     SAPA_WM16_OWN(T, 7, 4) SAPA_WM16_OWN(T, 5, 4) SAPA_WM16_OWN(T, 3, 2)                                         \
     return half     ? wm16::launch_geom<T, 5, 2, 8, false, true, true>(q, key, value, out, B, d, C, H, W, st)    \
            : odd    ? wm16::launch_geom<T, 5, 2, 8, false, true>(q, key, value, out, B, d, C, H, W, st)          \
+           : deep   ? wm16::launch_geom<T, 5, 2, 16, true, false, false, true>(q, key, value, out, B, d, C, H, W, st) \
            : stream ? wm16::launch_geom<T, 5, 2, 16, true, false>(q, key, value, out, B, d, C, H, W, st)         \
                     : wm16::launch_geom<T, 5, 2, 8, false, false>(q, key, value, out, B, d, C, H, W, st)
     if (dtype == 2) {

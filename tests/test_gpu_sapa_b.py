@@ -252,6 +252,21 @@ def test_16bit_dense_window_kernel_in_three_slices(B, C, H, W, K, s):
         assert_rel_rms_close(got[i].cpu(), exact.cpu(), BF16_REL, 'three slices')
 
 
+# streamed (beyond 256 MiB) with two buffers, up to 432 MiB or with a chain below 16 chunks, and with three: 17, 20 and
+# 21 chunks, the last ones partial, ragged tiles
+@pytest.mark.parametrize('B,d,C,H,W', [(13, 16, 256, 89, 90), (60, 24, 100, 70, 76), (22, 16, 256, 89, 90), (22, 64, 250, 77, 92),
+                                       (29, 70, 252, 64, 78)])
+def test_16bit_dense_window_kernel_of_streamed_tensors(B, d, C, H, W):
+    g = torch.Generator(device=DEV).manual_seed(144)
+    q, key, v = (torch.randn(B, c, *hw, generator=g, device=DEV).bfloat16() for c, hw in ((d, (2 * H, 2 * W)), (d, (H, W)), (C, (H, W))))
+    got = sapa_amd.sapa_fused(q, key, v, 5, 2)
+    for n in (0, B // 2, B - 1):        # an image by itself is not streamed: the same sums
+        i = slice(n, n + 1)
+        assert torch.equal(got[i], sapa_amd.sapa_fused(q[i].contiguous(), key[i].contiguous(), v[i].contiguous(), 5, 2))
+    exact = sapa_amd.sapa_fused(q[i].double(), key[i].double(), v[i].double(), 5, 2)
+    assert_rel_rms_close(got[i].cpu(), exact.cpu(), BF16_REL, 'streamed')
+
+
 @pytest.mark.parametrize('shape', [SHAPES[0], SHAPES[6]], ids=[IDS[0], IDS[6]])
 def test_fp64(coracle, shape):
     B, d, C, H, W, K, s = shape
