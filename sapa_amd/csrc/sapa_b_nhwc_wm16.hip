@@ -65,8 +65,10 @@ sapa_b_nhwc_wm16_kernel(const T *__restrict__ q, const T *__restrict__ key, cons
 
     const int logical = (int)(blockIdx.x % 8) * per_xcd + (int)(blockIdx.x / 8);
     if (logical >= nblocks) return;
-    // logical = tile * nslices + slice of the value chunks: a tile's slices share its window and queries through L2
-    const int slice = logical % nslices, tile = logical / nslices;
+    // logical = tile * nslices + slice of the value chunks: a tile's slices share its window and queries through L2 (no
+    // division in front of a tile that has one: B=8, C=64, 64x64 11.3 us with it, 11.1 without)
+    int slice = 0, tile = logical;
+    if (nslices > 1) tile = logical / nslices, slice = logical - tile * nslices;
     const int tx = tile % tiles_x, ty = (tile / tiles_x) % tiles_y, n = tile / (tiles_x * tiles_y);
     const int X0 = tx * 4 * ns, Y0 = ty * 4;                 // first parent of the tile
     const int nsx = (W + 3) / 4;
