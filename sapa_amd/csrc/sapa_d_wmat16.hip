@@ -451,9 +451,9 @@ deform_fused_wmat16_kernel(const T *__restrict__ q, const T *__restrict__ key,
 
         // ---- (c) per (pixel, point): logit from Sim, softmax over the points,
         // attention-weighted corner weights into Wm.  A pixel's row of Sim / Wm is
-        // touched by the lanes of that pixel only, all in one wave, whose LDS
-        // operations run in program order: gathers, then the row is cleared,
-        // then the adds, then the split -- no barrier in between.
+        // touched by the lanes of one wave only (the split by those of its other
+        // pixels, too), whose LDS operations run in program order: gathers, then the
+        // row is cleared, then the adds, then the split -- no barrier in between.
         u32 fbmask = 0;             // pass ps: the point passes the guard but leaves the window
         float fatt[NSP];
         auto sample = [&](auto nl, int ps) __attribute__((always_inline)) {

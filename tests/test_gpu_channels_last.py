@@ -146,8 +146,9 @@ def test_16bit_dense_window_kernel(coracle, shape, dtype):
         assert worst <= 1.05 * half_ulp, f'{shape} {dtype} with bias: {worst / half_ulp:.2f} half-spacings'
 
 
-# 36 and 144 tiles: value chunks of 64 channels in four and two slices, that divide, do not, the last one partial
-@pytest.mark.parametrize('B,C', [(1, 256), (1, 328), (1, 136), (4, 256), (4, 328), (11, 64), (11, 72)])
+# 36, 144 and 360 tiles: value chunks of 64 channels in four and two slices, that divide, do not, the last one partial;
+# 396 tiles: one slice
+@pytest.mark.parametrize('B,C', [(1, 256), (1, 328), (1, 136), (4, 256), (4, 328), (10, 72), (11, 64), (11, 72)])
 @pytest.mark.parametrize('bias', [False, True])
 def test_16bit_dense_window_kernel_in_slices(B, C, bias):
     g = gen(331)

@@ -45,17 +45,19 @@ def test_values_that_are_not_finite_stay_where_they_are_sampled(coracle):
     assert_f32_close(got[ok], want[ok], 'finite outputs')
 
 
-@pytest.mark.parametrize('cg,scale', [(20, 0.75), (33, 6.0), (64, 3.0), (100, 1.5)])
-def test_value_channels_in_slices(cg, scale):
+# slices of one chunk each; 100 tiles: of three chunks and two, of two and one that is partial
+@pytest.mark.parametrize('B,G,cg,H,W,scale', [(33, 2, 20, 16, 16, 0.75), (33, 2, 33, 16, 16, 6.0), (33, 2, 64, 16, 16, 3.0),
+                                              (33, 2, 100, 16, 16, 1.5), (3, 4, 80, 40, 80, 0.75), (3, 4, 44, 40, 80, 3.0)])
+def test_value_channels_in_slices(B, G, cg, H, W, scale):
     """An image by itself, its value channels in up to a slice per 16, gives what it gives in a batch whose tiles take all
     of them: whole chunks, a last one partial, samples beyond the window."""
-    B, G, P, H, W = 33, 2, 7, 16, 16
+    P = 7
     g = gen(73)
     q, key, v = randn(g, B, G * 20, 2 * H, 2 * W), randn(g, B, G * 20, H, W), randn(g, B, G * cg, H, W)
     off = randn(g, B, 2 * G * P, 2 * H, 2 * W) * scale
     q, key, v, off = (t.cuda() for t in (q, key, v, off))
     got = sapa_amd.deform_sapa_fused(q, key, v, off, P, 2, G)
-    for n in (0, 16, 32):
+    for n in (0, B // 2, B - 1):
         i = slice(n, n + 1)
         assert torch.equal(got[i], sapa_amd.deform_sapa_fused(*(t[i].contiguous() for t in (q, key, v, off)), P, 2, G))
         assert _lib.lib().sapa_hip_last_kernel() == b'deform_gather_kernel'
