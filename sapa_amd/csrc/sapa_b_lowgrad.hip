@@ -528,15 +528,19 @@ static hipError_t lowgrad_launch_t(const void *hi, const void *w, void *out, int
         const double lanes_gather = (double)((W + tw - 1) / tw) * ((H + 7) / 8) * (tw * 8);
         if ((long)C * H * 2 * W * 2 * (long)sizeof(T) < (1L << 31) &&
             lanes_gather >= SAPA_LOWGRAD_SHIFT_GAIN * lanes_shift) {
-            // Rows of 32 lanes and K = 5: of tiles of 8, 12 or 15 waves (12, 20 or 26 rows of cells from 16, 24 or 30 of
-            // lanes; 8 waves twice on a CU) those that the estimate prefers.  Sums are formed in the same order.  fp32,
-            // 256 channels, 8 / 12 / 15 waves: 16 images 50x84 126 / 129 / 109 us, 16 of 100x168 465 / 403 / 405,
-            // 4 of 100x168 127 / 101 / 112, 6 of 91x97 106 / 98 / 107, 16 of 25x42 51 / 50 / 36.
+            // Rows of 32 lanes and K = 5: tiles of 12 or 15 waves (20 or 26 rows of cells from 24 or 30 of lanes; 8 waves
+            // complete 12 from 16, twice on a CU) where the estimate prefers them by more than it is off: 10 and 6.5 % in fp32,
+            // 15 % in 16 bits.  Sums are formed in the same order.  256 channels, three sets of tensors in turn, 8 / 12 / 15
+            // waves: fp32, 16 images 50x84 124 / 130 / 109 us, 4 of 100x168 127 / 105 / 113, 6 of 91x97 107 / 99 / 108; on the
+            // other side of the lines 16 of 33x57 81 / 86 / 103, 5 of 91x97 87 / 90 / 87, with 128 channels 11 of 18x17 12.1 /
+            // 12.8 / 14.8 (15 for 16 waves at equal work: 244 for 256 us at 16 of 91x97, 39.9 for 38.6 at 8 with 64 channels);
+            // bf16, 16 of 50x84 115 / 121 / 101, 4 of 100x168 113 / 96 / 102, but 12 of 91x97 166 / 188 / 181, 16 of 33x57
+            // 71 / 79 / 96.
             int cper8 = 0, cper12 = 0, cper15 = 0;
             const double cost8 = lowgrad_shift_cost(NW, rows32 ? 32 : 16, K, B, C, H, W, CH, cper8);
             if (K == 5 && rows32) {
-                const double cost12 = lowgrad_shift_cost(12, 32, K, B, C, H, W, CH, cper12);
-                const double cost15 = lowgrad_shift_cost(15, 32, K, B, C, H, W, CH, cper15);
+                const double cost12 = (sizeof(T) == 2 ? 1.15 : 1.1) * lowgrad_shift_cost(12, 32, K, B, C, H, W, CH, cper12);
+                const double cost15 = (sizeof(T) == 2 ? 1.15 : 1.065) * lowgrad_shift_cost(15, 32, K, B, C, H, W, CH, cper15);
                 if (cost15 < cost8 && cost15 < cost12)
                     return lowgrad_shift_launch<T, WT, 5, 15, CH, WPE, 32>(hi, w, out, B, C, H, W, cper15, st);
                 if (cost12 < cost8) return lowgrad_shift_launch<T, WT, 5, 12, CH, WPE, 32>(hi, w, out, B, C, H, W, cper12, st);

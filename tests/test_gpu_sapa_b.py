@@ -369,8 +369,9 @@ def test_tiled_lowres_gradient_integer_inputs_exact(shape):
     assert torch.equal(vd.grad.cpu().double(), want)
 
 
-# tiles of 12 and of 15 waves, ragged in x and y, channels that are no whole groups
-@pytest.mark.parametrize('shape', [(5, 62, 40, 55, 5), (9, 39, 21, 85, 5), (11, 30, 21, 85, 5), (11, 15, 43, 84, 5)],
+# tiles of 8, of 12 (the fourth and fifth) and of 15 waves (the last two), ragged in x and y, channels that are no whole groups
+@pytest.mark.parametrize('shape', [(5, 62, 40, 55, 5), (9, 39, 21, 85, 5), (11, 30, 21, 85, 5), (11, 15, 43, 84, 5),
+                                   (11, 62, 19, 47, 5), (11, 37, 51, 53, 5), (8, 37, 50, 79, 5)],
                          ids=lambda s: '-'.join(map(str, s)))
 def test_tall_lowres_gradient_tiles_integer_inputs_exact(shape):
     test_tiled_lowres_gradient_integer_inputs_exact(shape)
