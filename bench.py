@@ -61,7 +61,7 @@ DEFORM_WORKLOADS = {
 # that kernel stops with an error instead of printing a stale figure.
 MEASURED_TRAFFIC = {
     ('fpn_large', 'fp32', 'nchw'): (1831119034, 'profiles/sapa_b_fused_fpn_large_fp32.md', 'sapa_b_tiled_kernel'),
-    ('fpn_large', 'bf16', 'nchw'): (944266161, 'profiles/sapa_b_fused_fpn_large_bf16.md', 'sapa_b_wmat16_kernel'),
+    ('fpn_large', 'bf16', 'nchw'): (955247572, 'profiles/sapa_b_fused_fpn_large_bf16.md', 'sapa_b_wmat16_kernel'),
     ('fpn_large', 'fp32', 'channels_last'): (1720501334, 'profiles/sapa_b_nhwc_fused_fpn_large_fp32.md',
                                              'sapa_b_nhwc_kernel'),
     ('fpn_large', 'bf16', 'channels_last'): (862391142, 'profiles/sapa_b_nhwc_fused_fpn_large_bf16.md',
@@ -76,14 +76,14 @@ MEASURED_TRAFFIC = {
                                           'sapa_b_nhwc16_kernel'),
     ('deform_p25', 'fp32', 'nchw'): (459730983, 'profiles/sapa_d_wmat_fused_deform_p25_fp32_nchw.md',
                                      'deform_fused_wmat_kernel'),
-    ('deform_p25', 'bf16', 'nchw'): (228881067, 'profiles/sapa_d_wmat16_fused_deform_p25_bf16_nchw.md',
+    ('deform_p25', 'bf16', 'nchw'): (228879126, 'profiles/sapa_d_wmat16_fused_deform_p25_bf16_nchw.md',
                                      'deform_fused_wmat16_kernel'),
     ('deform_p25', 'fp32', 'nchw_reference_order'): (828689742, 'profiles/sapa_d_lds_fused_deform_p25_fp32.md',
                                                      'deform_lds_kernel'),
-    ('deform_p9', 'fp32', 'nchw'): (289832257, 'profiles/sapa_d_gather_fused_deform_p9_fp32.md', 'deform_gather_kernel'),
+    ('deform_p9', 'fp32', 'nchw'): (289761759, 'profiles/sapa_d_gather_fused_deform_p9_fp32.md', 'deform_gather_kernel'),
     ('deform_p25', 'fp32', 'channels_last'): (356737114, 'profiles/sapa_d_nhwc_fused_deform_p25_fp32.md',
                                               'deform_fused_wmat_kernel'),
-    ('deform_p25', 'bf16', 'channels_last'): (178447650, 'profiles/sapa_d_wmat16_fused_deform_p25_bf16.md',
+    ('deform_p25', 'bf16', 'channels_last'): (178450883, 'profiles/sapa_d_wmat16_fused_deform_p25_bf16.md',
                                               'deform_fused_wmat16_kernel'),
 }
 

@@ -346,9 +346,10 @@ static hipError_t launch_geom(const void *q, const void *key, const void *value,
     const int ns = (nsx + tiles_x - 1) / tiles_x;             // blocks per tile, balanced over the row
     const long tiles = (long)tiles_x * tiles_y * B;
     const int allV = (C + CHK - 1) / CHK;
-    // Tiles that leave room on the CUs (three workgroups each): the value channels in two slices while those are all
-    // resident, in four while there is one per CU; each forms the weights again (bf16, C=256, one slice / two / four: 64 tiles
-    // 12.9 / 9.9 / 8.9 us, 78 13.3 / 10.5 / 11.0, 384 23.7 / 18.9 / 27, 468 23.8 / 25.8 / 31; C=512, 312 tiles 33 / 28 / 29)
+    // Tiles that leave room on the CUs (three workgroups each): the value channels in two slices, in four of one per CU at
+    // most; each forms the weights again (bf16, one slice / two / four: C=256, 64 tiles 12.9 / 9.9 / 8.9 us, 78 13.3 / 10.5 /
+    // 11.0, 384 23.7 / 18.9 / 27, 468 23.8 / 25.8 / 31; C=512, 312 tiles 33 / 28 / 29.  With 512 channels four are still
+    // ahead of two at 114 tiles, 14.6 for 15.1: the line is drawn for 256)
     int want = tiles <= 64 ? 4 : tiles <= 384 ? 2 : 1;
     if (want > allV) want = allV;
     const int slice_chunks = (allV + want - 1) / want, nslices = (allV + slice_chunks - 1) / slice_chunks;

@@ -529,9 +529,12 @@ static hipError_t launch_mode(int mode, bool wide, const void *q, const void *ke
             (tiles <= round || max_groups > 2))
             cgroups = max_groups;
         // Else only the tiles behind the last full round, in two or three slices each: aggregation, 6 images 100x168, 468
-        // tiles, 154 -> 142 us, 9 images 214 -> 205, 16 images 357 -> 350; 64 channels, 16 of 50x84, 31 -> 28.  Fused, whose
+        // tiles, 155 -> 142 us, 9 images 212 -> 205, 16 images 352 -> 346; 64 channels, 16 of 50x84, 31 -> 27.  Fused, whose
         // slices recompute the logits, with at most 8 tiles per XCD behind one full round (16, 17, 20 images 64x64, 256 /
-        // 272 / 320 tiles, 93 / 135 / 157 -> 93 / 123 / 139; 4 of 100x168, 312 tiles, 133 -> 123; 336 tiles 132 -> 139).
+        // 272 / 320 tiles, 91 / 141 / 152 -> 91 / 129 / 131; 4 of 100x168, 312 tiles, 132 -> 120; 336 tiles 132 -> 139).
+        // Both rules hold for tiles of 16 x 8 and 16 x 16 parents too, of which more are resident (aggregation, 34 images
+        // 24x48, 306 tiles of 16 x 8, 92 -> 46, 24 of 40x40, 360, 92 -> 53; 18, 30 and 44 of 48x48, 162, 270 and 396 of
+        // 16 x 16, 54 -> 47, 122 -> 91, 146 -> 130).
         else if (direct && cgroups == 1 && max_groups > 1 && tiles > round && (aggregate || tiles <= 320)) {
             const int run = (int)((tiles + 7) / 8);           // an XCD's tiles, for its 32 CUs
             if (run % 32) whole = run - run % 32, cgroups = aggregate && max_groups > 2 ? 3 : 2;
