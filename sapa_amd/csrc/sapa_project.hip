@@ -836,7 +836,8 @@ hipError_t project_shared_launch(const void *x, const void *w, const void *bias,
 //     {64, 128, 256, 512}, O in {32, 64, 128}; fp32: those whose three weight planes fit LDS);
 //   else x [B, C, HW] (planes) -> out [B, HW, O] (out_channels_last) or [B, O, HW]; the (C, O) pairs of the fp32
 //     kernel; fp32: HW a multiple of 4 for a planar result; f16 / bf16: HW a multiple of 8.
-// x, w and out aligned to 16 bytes.  hipErrorNotSupported otherwise (nothing is launched then).
+// x, w and out aligned to 16 bytes.  hipErrorNotSupported otherwise (of two that take a launch each, the first may have gone
+// out then: callers ask project_supported before).
 hipError_t project_launch(const ProjectFeature *f, int n, int B, int C, int O, bool x_channels_last, bool out_channels_last,
                           int dtype, hipStream_t st) {
     for (int i = 0; i < n; ++i)

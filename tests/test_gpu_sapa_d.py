@@ -114,6 +114,30 @@ def test_deform_fused_matrix_form_on_contiguous_tensors(coracle, shape, dtype):
         assert _lib.last_kernel() == kernel and torch.equal(a, b), layout
 
 
+# pixel pairs that are no dwords: rows of an odd number of pixels; a query and offsets that begin on half a dword
+@pytest.mark.parametrize('dtype', [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize('shape', [(1, 2, 32, 40, 9, 11, 9, 1), (2, 1, 16, 24, 6, 7, 25, 1), (2, 2, 16, 64, 7, 9, 9, 2),
+                                   (1, 2, 24, 72, 5, 6, 25, 2)])
+def test_16bit_matrix_form_of_pairs_that_are_no_dwords(coracle, shape, dtype):
+    from sapa_amd import _lib
+    B, G, dq, cg, H, W, P, s = shape
+    q, key, v, off = (t.to(dtype) for t in make(gen(234), shape)[:4])
+    want = coracle.deform_sapa_fused(q.float(), key.float(), v.float(), off.float(), P, s, G, 'f32')
+    args = dev(q, key, v, off)
+    got = sapa_amd.deform_sapa_fused(*args, P, s, G)
+    assert _lib.last_kernel() == 'deform_fused_wmat16_kernel'
+    assert_rel_rms_close(got.float(), want, BF16_REL if dtype == torch.bfloat16 else F16_REL, 'matrix form')
+
+    def half_a_dword_on(t):
+        room = torch.empty(t.numel() + 1, dtype=t.dtype, device=t.device)
+        room[1:] = t.flatten()
+        return room[1:].view(t.shape)
+    for which in ((0,), (3,), (0, 3)):
+        moved = [half_a_dword_on(t) if i in which else t for i, t in enumerate(args)]
+        assert all(moved[i].data_ptr() % 4 == 2 for i in which)
+        assert torch.equal(sapa_amd.deform_sapa_fused(*moved, P, s, G), got)
+
+
 def test_deform_fused_matrix_form_limits():
     """Too few points for the matrix form to pay, fp64, and the low-res offset
     layouts stay on the contiguous-layout kernels; asking for it explicitly raises."""
